@@ -49,7 +49,7 @@ EXPORTED_SYMBOLS = (
     "fa_reset_work_queues", "fa_release_work_queue", "run_flash_attention", "fa_strerror", "fa_last_device_error",
     "fa_sched_block_rows", "fa_sched_block_keys", "fa_sched_num_items", "fa_sched_item",
     "fa_sched_heads", "fa_sched_tile_range", "fa_sched_classify", "fa_count_pairs", "fa_algorithmic_flops",
-    "fa_dropout_threshold", "fa_dropout_keep", "fa_fwd_workspace_bytes", "fa_fwd_suggest_splits",
+    "fa_dropout_threshold", "fa_dropout_keep", "fa_fwd_workspace_bytes", "fa_fwd_suggest_splits", "fa_fwd_auto_splits",
     "fa_bwd_validate", "fa_bwd", "fa_bwd_workspace_bytes", "fa_bwd_fast_workspace_bytes", "fa_bwd_min_fast_workspace_bytes",
     "fa_bwd_algorithmic_flops",
     "fa_bwd_sched_query_tile_range", "fa_bwd_sched_classify",
@@ -135,6 +135,7 @@ def lib():
         L.fa_fwd_workspace_bytes.restype = ctypes.c_ulonglong
         L.fa_fwd_workspace_bytes.argtypes = [ctypes.POINTER(FaFwdParams)]
         L.fa_fwd_suggest_splits.argtypes = [ctypes.POINTER(FaFwdParams)]
+        L.fa_fwd_auto_splits.argtypes = [ctypes.POINTER(FaFwdParams)]
         L.run_flash_attention.argtypes = [ctypes.c_int] * 4 + [ctypes.c_void_p] * 6 + [ctypes.c_int] * 5 + [
             ctypes.c_void_p, ctypes.c_float, ctypes.c_void_p]
         L.fa_sched_block_rows.argtypes = [ctypes.c_int] * 7
@@ -287,7 +288,7 @@ def flash_attention_forward(q, k, v, softmax_scale=None, causal=False, window_le
                     q_st, k_st, v_st, o_st,
                     dropout_prob=dropout_prob, seed=seed, S_kv=0 if S_kv == S else S_kv, exact_first_rows=exact_first_rows)
     if splits == "auto":
-        splits = lib().fa_fwd_suggest_splits(ctypes.byref(p))
+        splits = lib().fa_fwd_auto_splits(ctypes.byref(p))
     workspace = None
     if splits and splits > 1:
         p.split_num = int(splits)

@@ -32,6 +32,9 @@ hipError_t fa_launch_forward_dropout(const FaKernelArgs &a, int bf16, int D, int
                                      hipStream_t stream);
 hipError_t fa_launch_forward_dropout_regular(const FaKernelArgs &a, int bf16, int D, int masked, int shape, unsigned grid,
                                              hipStream_t stream);
+hipError_t fa_launch_forward_decode(const FaKernelArgs &a, int bf16, int D, int rows, int streaming, hipStream_t stream,
+                                    bool configure_only = false);
+hipError_t fa_configure_forward_decode();
 hipError_t fa_launch_combine_splits(const FaKernelArgs &a, int bf16, int D, hipStream_t stream);
 hipError_t fa_launch_backward(const FaBwdArgs &a, int bf16, int D, int masked, int general, int alibi, int compute_units,
                               hipStream_t stream, bool configure_only = false);
@@ -310,6 +313,14 @@ int effective_splits(const fa_fwd_params *p)
     const int tiles = key_tiles(p);
     return p->split_num < tiles ? p->split_num : tiles;
 }
+// Whether the decoding kernel (fa_fwd_decode.hip) takes the problem: every query row of a K/V head fits its 32.
+// (Rows that the default forward computes in the verifier's arithmetic, and dropout, belong to the tile kernels.)
+bool decode_problem(const fa_fwd_params *p, bool causal_type)
+{
+    const int hk = p->n_kv_heads > 0 ? p->n_kv_heads : p->N, sk = p->S_kv > 0 ? p->S_kv : p->S;
+    if ((long long)(p->N / hk) * p->S > 32 || sk < p->S || fa_dropout_threshold(p->dropout_prob) != 0) return false;
+    return !(causal_type && sk - p->S < 32 && packed_group(p) == 1 && !p->exact_first_rows);
+}
 }  // namespace
 
 unsigned long long fa_fwd_workspace_bytes(const fa_fwd_params *p)
@@ -333,6 +344,27 @@ int fa_fwd_suggest_splits(const fa_fwd_params *p)
     long long n = (resident + items - 1) / items;
     const long long cap = key_tiles(p) / 4;
     if (n > cap) n = cap;
+    return n < 1 ? 1 : (int)n;
+}
+
+int fa_fwd_auto_splits(const fa_fwd_params *p)
+{
+    if (!p || p->B <= 0 || p->N <= 0 || p->S <= 0 || p->d <= 0) return 1;
+    const int hk = p->n_kv_heads > 0 ? p->n_kv_heads : p->N, sk = p->S_kv > 0 ? p->S_kv : p->S;
+    if (p->N % hk != 0) return 1;
+    const int s_max = sk > p->S ? sk : p->S;
+    int L, R;
+    fa_mask_bounds(s_max, p->is_causal, p->window_size_left, p->window_size_right, &L, &R);
+    if (!decode_problem(p, R == 0)) return fa_fwd_suggest_splits(p);
+    // The decoding kernel: two workgroups per CU, and no wave without at least one piece of its own (32 keys at head
+    // dimension 128, 64 at 64, four waves per workgroup) among the keys that some query sees.  Both launches of a call,
+    // splits: us -- B1 H32/8 S_kv 1003: 4: 9.9, 8: 8.3, 16: 8.1; B1 H16 S_kv 512 D64: 2: 8.2, 4: 7.5; B1 H64/8 S_kv 32768:
+    // 16: 43.5, 32: 30.2, 64: 29.2; B16 H32/8 S_kv 8192: 2: 86.8, 4: 87.4, 8: 88.7; B8 H32/8 S_kv 2048: 4: 17.7, 8: 16.8, 16: 17.9.
+    const long long heads = (long long)p->B * hk, visible = (long long)p->S + L < sk ? (long long)p->S + L : sk;
+    const long long most = visible / (p->d == 64 ? 256 : 128);
+    long long n = (2LL * kComputeUnits + heads - 1) / heads;
+    if (n > most) n = most;
+    if (n > key_tiles(p)) n = key_tiles(p);
     return n < 1 ? 1 : (int)n;
 }
 
@@ -467,6 +499,24 @@ int forward(const fa_fwd_params *p, void *workspace, const FaDeviceState *ds, vo
         if (grid > resident) grid = resident;
         if (sched == FA_SCHED_QUEUE) a.queue = work_queue_for_launch(ds, static_cast<hipStream_t>(stream));
     }
+    const bool decode = decode_problem(p, a.R == 0);
+    auto launch_decode = [&]() {
+        a.pack = p->N / a.Hk;
+        const long long heads = (long long)p->B * a.Hk;
+        a.n_items = heads * a.n_splits;
+        // (the streaming hint from where K and V do not stay in the 256 MB memory-side cache: measured beside the kernel)
+        const int streaming = heads * a.Sk * p->d * 4.0 > 128e6 ? 1 : 0;
+        hipError_t e = fa_launch_forward_decode(a, p->dtype == FA_DTYPE_BF16, p->d, a.pack * p->S, streaming, static_cast<hipStream_t>(stream));
+        if (e != hipSuccess) return device_fail(e, "decode launch");
+        if (a.n_splits > 1) {
+            e = fa_launch_combine_splits(a, p->dtype == FA_DTYPE_BF16, p->d, static_cast<hipStream_t>(stream));
+            if (e != hipSuccess) return device_fail(e, "combine launch");
+        }
+        return (int)FA_OK;
+    };
+#ifndef FA_CHECK_RING
+    if (decode) return launch_decode();
+#endif      // (the checking build runs the tile kernels, whose ring it checks, on these problems as well, in front)
     const int shape = waves == 8 ? 0 : 1;
     // dropout: p in units of 1/256 (a key is kept iff its random byte is >= the threshold)
     a.drop_threshold = (unsigned)fa_dropout_threshold(p->dropout_prob);
@@ -486,6 +536,9 @@ int forward(const fa_fwd_params *p, void *workspace, const FaDeviceState *ds, vo
         e = fa_launch_combine_splits(a, p->dtype == FA_DTYPE_BF16, p->d, static_cast<hipStream_t>(stream));
         if (e != hipSuccess) return device_fail(e, "combine launch");
     }
+#ifdef FA_CHECK_RING
+    if (decode) return launch_decode();
+#endif
     return FA_OK;
 }
 }  // namespace
@@ -497,7 +550,7 @@ int fa_init(void)
     if (e != hipSuccess) return device_fail(e, "device set-up");
     // everything a first launch would otherwise do besides the launch itself: after this call no entry point makes
     // a HIP call on this device that is not a stream operation (which is what a stream capture needs)
-    hipError_t (*const configure[])() = {fa_configure_forward_contiguous, fa_configure_forward_strided, fa_configure_forward_general,
+    hipError_t (*const configure[])() = {fa_configure_forward_contiguous, fa_configure_forward_strided, fa_configure_forward_general, fa_configure_forward_decode,
                                          fa_configure_forward_dropout, fa_configure_forward_dropout_regular, fa_configure_backward, fa_configure_backward_dropout,
                                          fa_configure_backward_strided, fa_configure_backward_dropout_regular, fa_configure_backward_alibi_regular};
     for (auto fn : configure) {

@@ -1229,42 +1229,6 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
     }
 }
 
-// Merges the partial results of a launch with key splits: for every query row,
-//   LSE = log sum_s exp(LSE_s),  O = sum_s exp(LSE_s - LSE) * O_s
-// (a split that saw no key of the row has LSE_s = -inf and weight 0).  One thread per four output elements.
-template <bool BF16, int D>
-__global__ void __launch_bounds__(256) fa_combine_splits(const FaKernelArgs a)
-{
-    constexpr int TPR = D / 4;                    // threads per row
-    const long long row = (long long)blockIdx.x * (256 / TPR) + threadIdx.x / TPR;
-    const int c4 = (threadIdx.x % TPR) * 4;
-    const long long n_rows = (long long)a.BH * a.S;
-    if (row >= n_rows) return;
-    const int bh = (int)(row / a.S), q = (int)(row % a.S);
-    float mx = -INFINITY;
-    for (int s = 0; s < a.n_splits; ++s) mx = fmaxf(mx, a.lse_part[(size_t)s * n_rows + row]);
-    float wsum = 0.0f;
-    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-    if (mx != -INFINITY) {
-        for (int s = 0; s < a.n_splits; ++s) {
-            const float w = __expf(a.lse_part[(size_t)s * n_rows + row] - mx);
-            if (w > 0.0f) {
-                const f32x4 o = *reinterpret_cast<const f32x4 *>(a.o_part + ((size_t)s * n_rows + row) * D + c4);
-                acc += o * w;
-                wsum += w;
-            }
-        }
-        acc *= 1.0f / wsum;
-    }
-    const int bi = bh / a.H, hi = bh - bi * a.H;
-    uint16_t *dst = a.O + (size_t)bi * a.o_bs + (size_t)hi * a.o_hs + (size_t)q * a.o_rs + c4;
-    u32x2 w2;
-    w2[0] = Num<BF16>::pack2(acc[0], acc[1]);
-    w2[1] = Num<BF16>::pack2(acc[2], acc[3]);
-    *reinterpret_cast<u32x2 *>(dst) = w2;
-    if (a.lse != nullptr && c4 == 0) a.lse[row] = mx == -INFINITY ? -INFINITY : mx + __logf(wsum);
-}
-
 template <bool BF16, int D, bool MASKED, bool ALIBI, bool GENERAL, bool DROPOUT, int NW, int NST, bool STRIDED = false, int NSTV = NST>
 hipError_t launch(const FaKernelArgs &a, unsigned grid, hipStream_t stream, bool configure_only)
 {

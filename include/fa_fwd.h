@@ -127,6 +127,10 @@ int fa_fwd_validate(const fa_fwd_params *p);
 unsigned long long fa_fwd_workspace_bytes(const fa_fwd_params *p);
 /* A split count that fills the device for these shapes (1 when the problem has enough work items anyway). */
 int fa_fwd_suggest_splits(const fa_fwd_params *p);
+/* The split count with which this library is fastest: that of fa_fwd_suggest_splits, and where the decoding kernel
+ * takes the problem (at most 32 query rows per K/V head) what suits that kernel, which splits short caches further and
+ * divides only the keys that a window leaves visible.  Set split_num to it before asking for the workspace. */
+int fa_fwd_auto_splits(const fa_fwd_params *p);
 
 /* Sets up the library's state for the current device: looks up the addresses of its two file-scope device
  * arrays and the CU count, and makes the LDS opt-in (hipFuncSetAttribute) of every kernel instantiation.  Optional
