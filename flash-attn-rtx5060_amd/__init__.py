@@ -51,7 +51,7 @@ EXPORTED_SYMBOLS = (
     "fa_sched_heads", "fa_sched_tile_range", "fa_sched_classify", "fa_count_pairs", "fa_algorithmic_flops",
     "fa_dropout_threshold", "fa_dropout_keep", "fa_fwd_workspace_bytes", "fa_fwd_suggest_splits", "fa_fwd_auto_splits",
     "fa_bwd_validate", "fa_bwd", "fa_bwd_workspace_bytes", "fa_bwd_fast_workspace_bytes", "fa_bwd_min_fast_workspace_bytes",
-    "fa_bwd_algorithmic_flops",
+    "fa_bwd_share_bytes", "fa_bwd_shared", "fa_bwd_algorithmic_flops",
     "fa_bwd_sched_query_tile_range", "fa_bwd_sched_classify",
     "fa_dev_count", "fa_dev_name", "fa_dev_malloc", "fa_dev_free", "fa_dev_h2d", "fa_dev_d2h",
     "fa_dev_memset", "fa_dev_sync", "fa_event_create", "fa_event_record", "fa_event_sync",
@@ -155,6 +155,9 @@ def lib():
         L.fa_dropout_threshold.argtypes = [ctypes.c_float]
         L.fa_bwd_validate.argtypes = [ctypes.POINTER(FaBwdParams)]
         L.fa_bwd.argtypes = [ctypes.POINTER(FaBwdParams), ctypes.c_void_p]
+        L.fa_bwd_shared.argtypes = [ctypes.POINTER(FaBwdParams), ctypes.c_void_p, ctypes.c_ulonglong, ctypes.c_void_p]
+        L.fa_bwd_share_bytes.restype = ctypes.c_ulonglong
+        L.fa_bwd_share_bytes.argtypes = [ctypes.POINTER(FaBwdParams)]
         L.fa_bwd_workspace_bytes.restype = ctypes.c_ulonglong
         L.fa_bwd_workspace_bytes.argtypes = [ctypes.POINTER(FaBwdParams)]
         L.fa_bwd_fast_workspace_bytes.restype = ctypes.c_ulonglong
@@ -375,9 +378,10 @@ def flash_attention_backward(q, k, v, o, lse, do, softmax_scale=None, causal=Fal
                         dropout_prob=dropout_prob, seed=seed)
     small = lib().fa_bwd_workspace_bytes(ctypes.byref(p))
     fast = lib().fa_bwd_fast_workspace_bytes(ctypes.byref(p)) if five_products else 0
-    sizes = [small]                       # tried from the back; the small workspace is what is left when nothing else fits
+    # (workspace, partial sums behind it), tried from the back; the small workspace is what is left when nothing else fits
+    sizes = [(small, 0)]
     if fast and five_products is True and workspace_limit is None:
-        sizes.append(fast)
+        sizes.append((fast, 0))
     elif fast:
         # "auto": whole chunks of eight K/V heads' dS blocks, about 2 GiB of them (chunks measure no slower than the
         # full size: B2 N32 S8192 D128 3.27 ms with 2.2 or 4.4 GB against 3.34 with 8.6), never fewer heads than the
@@ -388,27 +392,32 @@ def flash_attention_backward(q, k, v, o, lse, do, softmax_scale=None, causal=Fal
         off = (small + 255) // 256 * 256
         kv_total = q.shape[0] * k.shape[1]
         per_head = (fast - off) // kv_total
-        heads = max((least - off) // per_head, (2 << 30) // per_head // 8 * 8)
+        heads = min(kv_total, max((least - off) // per_head, (2 << 30) // per_head // 8 * 8))
         limit = workspace_limit if workspace_limit is not None else fast
         if off + heads * per_head > limit:
             heads = (limit - off) // per_head // 8 * 8 if limit > off else 0
         want = fast if heads >= kv_total else off + heads * per_head
         if least <= limit and want > least:
-            sizes.append(least)
+            sizes.append((least, 0))
         if heads > 0 and least <= want <= limit:
-            sizes.append(want)
+            sizes.append((want, 0))
+            if workspace_limit is None:
+                p.workspace_bytes = want
+                sizes.append((want, lib().fa_bwd_share_bytes(ctypes.byref(p))))
     workspace = None
     while workspace is None:              # stream-ordered: freed after the launch
-        need = sizes.pop()
+        need, parts = sizes.pop()
+        parts_at = (need + 255) // 256 * 256
         try:
-            workspace = torch.empty(max(need, 16), dtype=torch.uint8, device=q.device)
+            workspace = torch.empty(max(parts_at + parts if parts else need, 16), dtype=torch.uint8, device=q.device)
         except torch.cuda.OutOfMemoryError:
             if not sizes:
                 raise
     if poison_workspace:
         workspace.fill_(0xff)
     p.workspace, p.workspace_bytes = workspace.data_ptr(), need
-    st = lib().fa_bwd(ctypes.byref(p), ctypes.c_void_p(torch.cuda.current_stream(q.device).cuda_stream))
+    st = lib().fa_bwd_shared(ctypes.byref(p), workspace.data_ptr() + parts_at if parts else None, parts,
+                             ctypes.c_void_p(torch.cuda.current_stream(q.device).cuda_stream))
     if st != FA_OK:
         raise FaError(st, lib().fa_last_device_error().decode() if st == FA_ERR_DEVICE else "")
     return dq, dk, dv

@@ -390,7 +390,8 @@ __global__ void __launch_bounds__(kBwdWaves * 64, 2) fa_bwd_dq(const FaBwdArgs a
 // ---------------------------------------------------------------------------------------------------------
 // WRITE_DS (regular lengths, no ALiBi): every 32-query x 32-key block of dS that a wave forms is also written to
 // a.ds_blocks, in the wave's operand order, for fa_bwd_dq_from_ds.
-template <bool BF16, int D, bool MASKED, int LAYOUT, bool ALIBI, bool DROPOUT, bool WRITE_DS = false>
+// SHARES (with WRITE_DS): the walks cut into equal shares, see fa_bwd_layout.h.
+template <bool BF16, int D, bool MASKED, int LAYOUT, bool ALIBI, bool DROPOUT, bool WRITE_DS = false, bool SHARES = false>
 __global__ void __launch_bounds__(kBwdWaves * 64, 2) fa_bwd_dkdv(const FaBwdArgs a)
 {
     constexpr bool STRIDES = LAYOUT >= 1, GENERAL = LAYOUT == 2, ONE_ITEM = STRIDES && D == 128 && !(WRITE_DS && FA_DS_LOOP);
@@ -410,15 +411,33 @@ __global__ void __launch_bounds__(kBwdWaves * 64, 2) fa_bwd_dkdv(const FaBwdArgs
     // (work items as in fa_bwd_dq; the list here is ascending in the key block, which is longest first under a
     // causal mask: key block 0 is seen by every query)
     const long long n_items = (long long)a.heads * n_kblocks;
+    // Equal shares: the walks of all key blocks one behind the other, cut into as many shares as there are
+    // workgroups (fa_bwd_layout.h); a share covers the end of one walk, whole walks, and the beginning of another.
+    // (What this needs besides the position `share_at` is read and formed again at each place that uses it: scalar
+    // registers held through the tile loop are spilled into vector registers, which the 128-wide kernels do not have.)
+    int share_at = 0;
+    if (SHARES) share_at = fa_bwd_share_begin(fa_bwd_share_of((int)blockIdx.x, (int)gridDim.x), (int)gridDim.x, a.walk_total);
     for (int pass = 0; !ONE_ITEM || pass < 1; ++pass) {       // (128-wide strided and general instantiations: exactly one item, no loop)
     const long long item = (long long)pass * gridDim.x + ((pass & 1) ? gridDim.x - 1 - blockIdx.x : blockIdx.x);
-    if (item >= n_items) break;
+    if (!SHARES && item >= n_items) break;
     if (pass > 0) __syncthreads();
     int lane = ONE_ITEM ? (int)threadIdx.x & 63 : (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
     if (!ONE_ITEM) asm volatile("" : "+v"(lane));
     const int half = lane >> 5, l32 = lane & 31;
     int bhk, kblock;
-    fa_item_decode(item, a.heads, n_kblocks, 0, &bhk, &kblock);
+    int walk_from = 0, walk_pairs = 0;             // shares: the (query head, query tile) pairs of the walk this pass does
+    if (SHARES) {
+        const FaBwdArgs &f = args_reloaded();
+        const int end = fa_bwd_share_begin(fa_bwd_share_of((int)blockIdx.x, (int)gridDim.x) + 1, (int)gridDim.x, f.walk_total);
+        if (share_at >= end) break;
+        int walk_begin, walk_len;
+        fa_bwd_walk_at(share_at, f.walk_head, G, S, Sk, f.R + off, f.L - off, &bhk, &kblock, &walk_begin, &walk_len);
+        walk_from = share_at - walk_begin;
+        walk_pairs = end - share_at < walk_len - walk_from ? end - share_at : walk_len - walk_from;
+        share_at += walk_pairs;
+    } else {
+        fa_item_decode(item, a.heads, n_kblocks, 0, &bhk, &kblock);
+    }
     bhk += a.head0;
     const int b = bhk / a.Hk, hk = bhk - b * a.Hk;
     const int q_rs = STRIDES ? a.q.rs : D, g_rs = STRIDES ? a.dO_.rs : D, k_rs = STRIDES ? a.k.rs : D, v_rs = STRIDES ? a.v.rs : D;
@@ -639,7 +658,11 @@ __global__ void __launch_bounds__(kBwdWaves * 64, 2) fa_bwd_dkdv(const FaBwdArgs
         // from the last query tile down to the diagonal: every workgroup of a head then starts on the same tile
         // and the ones that run together keep reading the same tiles out of L2; then the next head of the group
         // (head, tile) pairs are fetched two ahead, as in fa_bwd_dq
-        int ig = 0, it = t1;                                    // the next pair to fetch
+        // (shares: from pair `walk_from` of the walk, `walk_pairs` of them)
+        const int per_head = t1 - t0 + 1;
+        const int first_g = SHARES ? walk_from / per_head : 0, first_t = SHARES ? t1 - (walk_from - first_g * per_head) : t1;
+        int pairs_left = SHARES ? walk_pairs : G * per_head;    // (WRITE_DS) pairs still to come
+        int ig = first_g, it = first_t;                         // the next pair to fetch
         auto issue_next = [&](int stage) __attribute__((always_inline)) {
             issue(ig, it, stage);
             if (--it < t0) {
@@ -647,9 +670,9 @@ __global__ void __launch_bounds__(kBwdWaves * 64, 2) fa_bwd_dkdv(const FaBwdArgs
                 if (STRIDES && ig < G) walk_head(ig);
             }
         };
-        if (STRIDES) walk_head(0);
+        if (STRIDES) walk_head(first_g);
         issue_next(0);
-        if (ig < G) issue_next(1);
+        if (SHARES ? pairs_left > 1 : ig < G) issue_next(1);
         wait_vm<0>();
 #pragma unroll
         for (int s = 0; s < KS; ++s) asm volatile("" : "+v"(kf[s]), "+v"(vf[s]));
@@ -665,12 +688,12 @@ __global__ void __launch_bounds__(kBwdWaves * 64, 2) fa_bwd_dkdv(const FaBwdArgs
         int stage = 0;
         // WRITE_DS: the dS stores this wave made in the last two iterations, and the pairs still to come.  The next
         // pair is then requested in front of an iteration's work instead of behind it.
-        int st1 = 0, st2 = 0, pairs_left = G * (t1 - t0 + 1);
+        int st1 = 0, st2 = 0;
         constexpr bool TOP = WRITE_DS;
-        for (int g = 0; g < G; ++g) {
+        for (int g = first_g, t_from = first_t; SHARES ? pairs_left > 0 : g < G; ++g, t_from = t1) {
             float slope_l2 = 0.0f;
             if (ALIBI) slope_l2 = a.alibi[hk * G + g] * kLog2e;
-            for (int t = t1; t >= t0; --t) {
+            for (int t = t_from; t >= t0 && (!SHARES || pairs_left > 0); --t) {
                 const int next = stage == NSTG - 1 ? 0 : stage + 1, prev = stage == 0 ? NSTG - 1 : stage - 1;
                 const bool more = t - 1 >= t0 || g + 1 < G;
                 --pairs_left;
@@ -685,7 +708,7 @@ __global__ void __launch_bounds__(kBwdWaves * 64, 2) fa_bwd_dkdv(const FaBwdArgs
                     if (wave < 2) wait_vm<2 * IPW + 1>(); else wait_vm<2 * IPW>();     // waves 0 and 1 also fetch lse / delta
                 } else wait_vm<0>();
                 phase_barrier();
-                if (TOP && ig < G) issue_next(prev);
+                if (TOP && (SHARES ? pairs_left > 1 : ig < G)) issue_next(prev);
                 st2 = st1;
                 st1 = (WRITE_DS && my_lo <= t && t <= my_hi) ? 4 : 0;
                 if (my_lo <= t && t <= my_hi) {
@@ -707,7 +730,25 @@ __global__ void __launch_bounds__(kBwdWaves * 64, 2) fa_bwd_dkdv(const FaBwdArgs
     int lane_e = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
     asm volatile("" : "+v"(lane_e));
     const int key_e = kw + (lane_e & 31), half_e = lane_e >> 5;
-    if (active && key_e < Sk) {
+    int part_slot = -1;
+    if (SHARES) {
+        const FaBwdArgs &f = args_reloaded();
+        const int share = fa_bwd_share_of((int)blockIdx.x, (int)gridDim.x), begin = fa_bwd_share_begin(share, (int)gridDim.x, f.walk_total);
+        int head, kb, walk_begin, walk_len;
+        fa_bwd_walk_at(share_at - 1, f.walk_head, G, S, Sk, f.R + off, f.L - off, &head, &kb, &walk_begin, &walk_len);
+        if (begin > walk_begin || share_at < walk_begin + walk_len) part_slot = fa_bwd_part_slot(share, begin > walk_begin ? 1 : 0);
+    }
+    if (SHARES && part_slot >= 0) {
+        // part of a walk: the fp32 sums as the registers hold them, 1 KiB per store instruction, for fa_bwd_add_parts
+        if (active) {
+            float *part = args_reloaded().partials + (size_t)part_slot * (2 * 256 * D) + wave * (32 * D) + 4 * lane_e;
+#pragma unroll
+            for (int i = 0; i < 4 * DB; ++i) {
+                *reinterpret_cast<f32x4 *>(part + 256 * i) = f32x4{dk[i / 4][4 * (i % 4)], dk[i / 4][4 * (i % 4) + 1], dk[i / 4][4 * (i % 4) + 2], dk[i / 4][4 * (i % 4) + 3]};
+                *reinterpret_cast<f32x4 *>(part + 256 * D + 256 * i) = f32x4{dv[i / 4][4 * (i % 4)], dv[i / 4][4 * (i % 4) + 1], dv[i / 4][4 * (i % 4) + 2], dv[i / 4][4 * (i % 4) + 3]};
+            }
+        }
+    } else if (active && key_e < Sk) {
         uint16_t *dKh, *dVh;
         int dk_rs = D, dv_rs = D;
         if (STRIDES) {
@@ -774,6 +815,49 @@ __global__ void __launch_bounds__(256) fa_bwd_prepare(const FaBwdArgs a)
         a.delta[row] = sum;
         const float l = a.lse[row];
         a.lse2[row] = l == -INFINITY ? INFINITY : l * kLog2e;
+    }
+}
+
+// The parts of the walks that fa_bwd_dkdv cut between its workgroups' shares: dK and dV of such a key block are the sums
+// of its parts, added in the order of the walk (the same bits every run).  Workgroup (share c, wave w, dK or dV): the 32
+// keys of wave w in the block that the boundary in front of share c cuts, if it cuts one and is the first to do so.
+// Bound by HBM: 256 KB per part at head dimension 128, read once; a thread has all its slots of a part in flight at once
+// (one slot after the other, the 57 parts of B1 H8/1 S2048's first block took 0.7 ms).
+template <bool BF16, int D, bool STRIDED>
+__global__ void __launch_bounds__(256) fa_bwd_add_parts(const FaBwdArgs a, int n_shares)
+{
+    constexpr int SLOTS = 8 * D / 256;            // 16-byte slots per thread: 32 keys x D floats over 256 threads
+    const int share = (int)blockIdx.x / (2 * kBwdWaves) + 1, wave = (int)blockIdx.x / 2 % kBwdWaves, which = (int)blockIdx.x % 2;
+    const int S = a.S, G = STRIDED ? a.H / a.Hk : 1;
+    const int cut = fa_bwd_share_begin(share, n_shares, a.walk_total);
+    int bhk, kblock, begin, len;
+    fa_bwd_walk_at(cut, a.walk_head, G, S, S, a.R, a.L, &bhk, &kblock, &begin, &len);
+    if (cut == begin || fa_bwd_share_begin(share - 1, n_shares, a.walk_total) > begin) return;
+    int last = share;                             // the share that holds the walk's end
+    while (fa_bwd_share_begin(last + 1, n_shares, a.walk_total) < begin + len) ++last;
+    constexpr size_t PART = 2 * 256 * D;
+    const float *src = a.partials + (size_t)which * (256 * D) + wave * (32 * D) + 4 * (int)threadIdx.x;
+    f32x4 sum[SLOTS];
+#pragma unroll
+    for (int n = 0; n < SLOTS; ++n) sum[n] = *reinterpret_cast<const f32x4 *>(src + fa_bwd_part_slot(share - 1, 0) * PART + 1024 * n);
+#pragma unroll 4
+    for (int s = share; s <= last; ++s)
+#pragma unroll
+        for (int n = 0; n < SLOTS; ++n) sum[n] += *reinterpret_cast<const f32x4 *>(src + fa_bwd_part_slot(s, 1) * PART + 1024 * n);
+    bhk += a.head0;
+    const int b = bhk / a.Hk, hk = bhk - b * a.Hk;
+    uint16_t *out = which == 0 ? (STRIDED ? head_ptr(a.dK, a.dk, b, hk) : a.dK + (size_t)bhk * S * D)
+                               : (STRIDED ? head_ptr(a.dV, a.dv, b, hk) : a.dV + (size_t)bhk * S * D);
+    const int rs = STRIDED ? (which == 0 ? a.dk.rs : a.dv.rs) : D, lane = (int)threadIdx.x % 64, key = kblock * 256 + wave * 32 + (lane & 31);
+    const float scale = which == 0 ? a.scale : 1.0f;
+    if (key >= S) return;
+#pragma unroll
+    for (int n = 0; n < SLOTS; ++n) {
+        const int i = n * 4 + (int)threadIdx.x / 64, col = 32 * (i / 4) + 8 * (i % 4) + 4 * (lane >> 5);
+        u32x2 w;
+        w[0] = Num<BF16>::pack2(sum[n][0] * scale, sum[n][1] * scale);
+        w[1] = Num<BF16>::pack2(sum[n][2] * scale, sum[n][3] * scale);
+        *reinterpret_cast<u32x2 *>(out + (size_t)key * rs + col) = w;
     }
 }
 
@@ -939,6 +1023,7 @@ hipError_t launch_bwd(const FaBwdArgs &a_in, int compute_units, hipStream_t stre
     // length S = S_kv without them
     constexpr bool FIVE = LAYOUT <= 1 || (!ALIBI && !DROPOUT);
     constexpr int FL = FIVE ? LAYOUT : 0;
+    constexpr bool CAN_SHARE = FIVE && fa_bwd_can_share(D, DROPOUT);
     const int smem_dq_ds = kBwdStages * (TILEB + kBwdWaves * 2 * kDsBlockBytes);
     // the LDS opt-in is per (instantiation, device) and is made once, not on every launch
     static std::atomic<unsigned long long> configured{0ull};
@@ -952,6 +1037,11 @@ hipError_t launch_bwd(const FaBwdArgs &a_in, int compute_units, hipStream_t stre
             e = hipFuncSetAttribute(reinterpret_cast<const void *>(fa_bwd_dkdv<BF16, D, MASKED, FL, ALIBI, DROPOUT, true>),
                                     hipFuncAttributeMaxDynamicSharedMemorySize, smem_dkdv_ds);
             if (e != hipSuccess) return e;
+            if constexpr (CAN_SHARE) {
+                e = hipFuncSetAttribute(reinterpret_cast<const void *>(fa_bwd_dkdv<BF16, D, MASKED, FL, ALIBI, DROPOUT, true, true>),
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, smem_dkdv_ds);
+                if (e != hipSuccess) return e;
+            }
             e = hipFuncSetAttribute(reinterpret_cast<const void *>(fa_bwd_dq_from_ds<BF16, D, MASKED, FL>),
                                     hipFuncAttributeMaxDynamicSharedMemorySize, smem_dq_ds);
             if (e != hipSuccess) return e;
@@ -970,13 +1060,12 @@ hipError_t launch_bwd(const FaBwdArgs &a_in, int compute_units, hipStream_t stre
     const unsigned resident = (unsigned)compute_units;
     // (the general instantiations always carry the mask code: without a bound on either side, L = R = S + S_kv, their
     // items are alike as well)
-    const long long unbounded = (long long)a.S + a.Sk;
     // (The 128-wide strided and general instantiations are launched one workgroup per item only: with the item loop
     // around them they spill ten times as much, and a reload inside the tile loop waits for every tile load in
     // flight: c3's shape stored [B,S,H,D] 4.1 ms against 3.8.  The 64-wide ones have the registers for the loop.)
     // (The kernels of the five-product form have the loop in every layout: the key-owning one keeps K^T / V^T
     // fragments in LDS and compiles with it without spilling, or with 12 bytes outside the tile loop.)
-    const bool uneven_items = MASKED && (a.L < unbounded || a.R < unbounded) && 2LL * a.L > (long long)a.S;
+    const bool uneven_items = MASKED && fa_bwd_uneven(a.S, a.Sk, a.L, a.R);
     const bool uneven = (LAYOUT == 0 || D == 64) && uneven_items;
     auto grid_if = [&](bool snake, long long items) {
         const unsigned g = (unsigned)items;
@@ -995,8 +1084,18 @@ hipError_t launch_bwd(const FaBwdArgs &a_in, int compute_units, hipStream_t stre
                 a.head0 = h0;
                 a.heads = all_heads - h0 < chunk ? all_heads - h0 : chunk;
                 const unsigned launch_k = grid_if(FA_DS_LOOP ? uneven_items : uneven, (long long)a.heads * ((a.Sk + 255) / 256));
+                unsigned n_shares = 0;
+                if constexpr (CAN_SHARE) {
+                    if (a.partials != nullptr) n_shares = (unsigned)fa_bwd_shares(a.heads, group, a.S, a.R, a.L, a.walk_head, (int)resident);
+                    if (n_shares != 0) {
+                        a.walk_total = a.heads * a.walk_head;
+                        hipLaunchKernelGGL((fa_bwd_dkdv<BF16, D, MASKED, FL, ALIBI, DROPOUT, true, true>), dim3(n_shares), dim3(kBwdWaves * 64), smem_dkdv_ds, stream, a);
+                        hipLaunchKernelGGL((fa_bwd_add_parts<BF16, D, FL >= 1>), dim3((n_shares - 1) * 2 * kBwdWaves), dim3(256), 0, stream, a, (int)n_shares);
+                    }
+                }
                 const unsigned launch_q = grid_if(uneven_items, (long long)a.heads * group * ((a.S + 255) / 256));
-                hipLaunchKernelGGL((fa_bwd_dkdv<BF16, D, MASKED, FL, ALIBI, DROPOUT, true>), dim3(launch_k), dim3(kBwdWaves * 64), smem_dkdv_ds, stream, a);
+                if (n_shares == 0)
+                    hipLaunchKernelGGL((fa_bwd_dkdv<BF16, D, MASKED, FL, ALIBI, DROPOUT, true>), dim3(launch_k), dim3(kBwdWaves * 64), smem_dkdv_ds, stream, a);
                 hipLaunchKernelGGL((fa_bwd_dq_from_ds<BF16, D, MASKED, FL>), dim3(launch_q), dim3(kBwdWaves * 64), smem_dq_ds, stream, a);
             }
             return hipGetLastError();

@@ -4,6 +4,8 @@
 #ifndef FA_BWD_LAYOUT_H
 #define FA_BWD_LAYOUT_H
 
+#include "fa_sched.h"
+
 #if defined(__HIPCC__)
 #define FA_LAYOUT_HD __host__ __device__ __forceinline__
 #else
@@ -60,6 +62,81 @@ FA_LAYOUT_HD long long fa_ds_blocks_per_head(int S) { return fa_ds_squares_per_s
 FA_LAYOUT_HD long long fa_ds_block_index(int S, int qb, int kb)
 {
     return (((long long)(qb >> 3) * fa_ds_squares_per_side(S) + (kb >> 3)) << 6) + ((qb & 7) << 3) + (kb & 7);
+}
+
+// ---- Equal shares of the key-owning kernel's work.  The walk of a key block (256 keys of a K/V head) visits the 64-query
+// tiles that see one of its keys, for each of the G query heads that share the K/V head: G * tiles pairs, in that order
+// (head by head, from the last tile down).  Under a causal mask block 0 walks all tiles and the last block four of
+// them; a problem with few key blocks leaves CUs idle.  The walks of all blocks, block by block and head by head, are
+// therefore laid end to end and cut into shares that differ by at most one pair (no more shares than pairs).
+FA_LAYOUT_HD int fa_bwd_walk_tiles(int S, int Sk, int Lq, int Rq, int kblock)
+{
+    int lo, hi;
+    fa_tile_range(S, 64, Lq, Rq, kblock * 256, Sk - kblock * 256 < 256 ? Sk - kblock * 256 : 256, &lo, &hi);
+    return hi - lo + 1;
+}
+// Share of workgroup `block`: with workgroups dealt round robin over the eight XCDs, each XCD gets consecutive shares
+// (a head or two of the list: what runs there at a time reads the same tiles).  `shares` is a multiple of eight.
+FA_LAYOUT_HD int fa_bwd_share_of(int block, int shares) { return (block & 7) * (shares >> 3) + (block >> 3); }
+FA_LAYOUT_HD int fa_bwd_share_begin(int share, int shares, int total) { return (int)((long long)share * total / shares); }
+// The walk that pair `at` (of the whole list) belongs to: K/V head (counted from the launch's first) and key block, its
+// first pair and its length.  per_head: pairs of one head's walks.
+FA_LAYOUT_HD void fa_bwd_walk_at(int at, int per_head, int G, int S, int Sk, int Lq, int Rq, int *head, int *kblock, int *begin, int *len)
+{
+    const int h = (int)((unsigned)at / (unsigned)per_head);
+    int from = h * per_head, kb = 0, n = G * fa_bwd_walk_tiles(S, Sk, Lq, Rq, 0);
+    while (at >= from + n) {
+        from += n;
+        n = G * fa_bwd_walk_tiles(S, Sk, Lq, Rq, ++kb);
+    }
+    *head = h; *kblock = kb; *begin = from; *len = n;
+}
+// Where a share leaves the fp32 sums of a walk it does only a part of: the end of a walk that an earlier share began
+// (from > 0, always the share's first walk) in the first of its two slots, a walk it begins and does not finish (its
+// last) in the second.
+#define FA_BWD_PARTS_PER_SHARE 2
+FA_LAYOUT_HD int fa_bwd_part_slot(int share, int from) { return FA_BWD_PARTS_PER_SHARE * share + (from > 0 ? 0 : 1); }
+
+// Whether the key-owning kernel with shares is built: not at head dimension 128 with dropout, which is out of registers
+// (the 80-260 bytes of scratch memory that the shares cost it are touched in the tile loop).
+#if defined(__cplusplus)
+constexpr
+#endif
+FA_LAYOUT_HD int fa_bwd_can_share(int D, int dropout) { return !(D == 128 && dropout); }
+// Whether the key-owning kernel's items differ in length: masked, and not a window of at most half the length.
+FA_LAYOUT_HD int fa_bwd_uneven(int S, int Sk, int L, int R) { return (L < S + Sk || R < S + Sk) && 2LL * L > (long long)S; }
+// How many equal shares the walks of a launch over `heads` K/V heads are cut into, or 0 to leave every walk to one
+// workgroup: cut when the longest of a few workgroups (walking the items as a snake, or nearly in rounds when the
+// hardware hands them out) has more than 4/3 of a share and 3 to 9 pairs, what writing and adding the parts costs, to do.
+// (Why 4/3: the chip is at its power cap, and compute units that idle leave their power to the others.)  Backward pass,
+// fp16, longest : share in pairs, cut against whole: causal D128 B1 H32/8 S4096 256 : 68 493 against 938 us, B1 H8 S2048
+// 32 : 4.5 102 against 157, B1 H16 S1024 16 : 2.5 77 against 93, B2 H8 S512 8 : 2 51 against 59, without a mask B1 H40 S2048
+// 64 : 40 330 against 370; and not cut: B1 H32 S2048 32 : 18 195 against 184, B6 H8 S2048 36 : 27 266 against 233, without a
+// mask B2 H16 S512 D64 8 : 2 47 against 44.
+FA_LAYOUT_HD int fa_bwd_shares(int heads, int G, int S, int Lq, int Rq, int walk_head, int compute_units)
+{
+    const int n_kblocks = (S + 255) / 256;
+    const long long total = (long long)heads * walk_head, items = (long long)heads * n_kblocks;
+    if (walk_head <= 0 || total > 0x3fffffffLL) return 0;
+    long long shares = total / 2 / 8 * 8;          // at least two pairs each
+    if (shares > compute_units) shares = compute_units / 8 * 8;
+    if (shares < 8) return 0;
+    const int snake = fa_bwd_uneven(S, S, Rq, Lq) && items < 16LL * compute_units;
+    const long long g = items < compute_units ? items : compute_units;
+    long long worst = 0;
+    for (int probe = 0; probe < 8; ++probe) {
+        const long long at = probe == 7 ? (items - 1) % g : probe * (g - 1) / 6;
+        long long sum = 0;
+        for (long long pass = 0; pass * g < items; ++pass) {
+            const long long item = pass * g + (snake && (pass & 1) ? g - 1 - at : at);
+            if (item >= items) continue;
+            int head, kblock;
+            fa_item_decode(item, heads, n_kblocks, 0, &head, &kblock);
+            sum += (long long)G * fa_bwd_walk_tiles(S, S, Lq, Rq, kblock);
+        }
+        if (sum > worst) worst = sum;
+    }
+    return 3 * worst > 4 * (total / shares) + 9 + 18 * shares / 256 ? (int)shares : 0;
 }
 
 #endif

@@ -799,10 +799,50 @@ int fa_bwd_validate(const fa_bwd_params *p)
     return FA_OK;
 }
 
-int fa_bwd(const fa_bwd_params *p, void *stream)
+namespace {
+// The K/V heads whose dS blocks fit a workspace of this size (whole chunks), 0 when it does not select the five-product form
+int ds_heads_for(const fa_bwd_params *p, unsigned long long workspace_bytes)
+{
+    if (fa_bwd_fast_workspace_bytes(p) == 0 || workspace_bytes < fa_bwd_min_fast_workspace_bytes(p)) return 0;
+    const long long all = kv_heads_total(p);
+    long long fit = (long long)((workspace_bytes - ds_blocks_offset(p)) / ds_bytes_per_kv_head(p));
+    if (fit < all) fit = fit / 8 * 8;
+    return (int)(fit < all ? fit : all);
+}
+// pairs in the walks of one K/V head's key blocks (0: too many to count in 31 bits)
+int walk_pairs_per_head(int S, int G, int L, int R)
+{
+    long long pairs = 0;
+    for (int kb = 0; kb < (S + 255) / 256; ++kb) pairs += (long long)G * fa_bwd_walk_tiles(S, S, R, L, kb);
+    return pairs <= 0x3fffffffLL ? (int)pairs : 0;
+}
+}  // namespace
+
+unsigned long long fa_bwd_share_bytes(const fa_bwd_params *p)
+{
+    if (!p) return 0;
+    const int heads = ds_heads_for(p, p->workspace_bytes);
+    if (heads == 0 || !fa_bwd_can_share(p->d, fa_dropout_threshold(p->dropout_prob) != 0)) return 0;
+    const int G = p->n_kv_heads > 0 ? p->N / p->n_kv_heads : 1;
+    int L, R;
+    fa_mask_bounds(2 * p->S, p->is_causal, p->window_size_left, p->window_size_right, &L, &R);
+    const int per_head = walk_pairs_per_head(p->S, G, L, R);
+    // the launches: whole chunks and a smaller last one
+    const int rest = (int)(kv_heads_total(p) % heads);
+    int shares = fa_bwd_shares(heads, G, p->S, R, L, per_head, kComputeUnits);
+    const int of_rest = rest != 0 ? fa_bwd_shares(rest, G, p->S, R, L, per_head, kComputeUnits) : 0;
+    if (of_rest > shares) shares = of_rest;
+    return (unsigned long long)shares * FA_BWD_PARTS_PER_SHARE * 2ull * 256ull * (unsigned long long)p->d * 4ull;
+}
+
+int fa_bwd(const fa_bwd_params *p, void *stream) { return fa_bwd_shared(p, nullptr, 0, stream); }
+
+int fa_bwd_shared(const fa_bwd_params *p, void *partials, unsigned long long partials_bytes, void *stream)
 {
     const int st = fa_bwd_validate(p);
     if (st != FA_OK) return st;
+    const unsigned long long share_bytes = partials != nullptr ? fa_bwd_share_bytes(p) : 0;
+    if (partials != nullptr && (reinterpret_cast<uintptr_t>(partials) % 16 != 0 || partials_bytes < share_bytes)) return FA_ERR_WORKSPACE;
     const FaDeviceState *ds = nullptr;
     {
         const hipError_t de = fa_device_state(&ds);
@@ -820,18 +860,12 @@ int fa_bwd(const fa_bwd_params *p, void *stream)
     // a workspace large enough for the dS blocks selects the five-product form
     // (all of them at once when it holds fa_bwd_fast_workspace_bytes, else for as many K/V heads' groups at a time as
     // fit, a multiple of eight and not fewer than fa_bwd_min_fast_workspace_bytes allows)
-    const unsigned long long fast_bytes = fa_bwd_fast_workspace_bytes(p);
-    a.ds_blocks = nullptr;
+    a.ds_heads = ds_heads_for(p, p->workspace_bytes);
+    a.ds_blocks = a.ds_heads > 0 ? reinterpret_cast<uint16_t *>(static_cast<char *>(p->workspace) + ds_blocks_offset(p)) : nullptr;
     a.head0 = 0;
     a.heads = (int)kv_heads_total(p);
-    a.ds_heads = 0;
-    if (fast_bytes != 0 && p->workspace_bytes >= fa_bwd_min_fast_workspace_bytes(p)) {
-        const unsigned long long off = ds_blocks_offset(p);
-        long long fit = (long long)((p->workspace_bytes - off) / ds_bytes_per_kv_head(p));
-        if (fit < kv_heads_total(p)) fit = fit / 8 * 8;
-        a.ds_heads = (int)(fit < kv_heads_total(p) ? fit : kv_heads_total(p));
-        a.ds_blocks = reinterpret_cast<uint16_t *>(static_cast<char *>(p->workspace) + off);
-    }
+    a.partials = share_bytes != 0 ? static_cast<float *>(partials) : nullptr;
+    a.walk_head = a.walk_total = 0;
     a.dQ = static_cast<uint16_t *>(p->dQ);
     a.dK = static_cast<uint16_t *>(p->dK);
     a.dV = static_cast<uint16_t *>(p->dV);
@@ -866,6 +900,7 @@ int fa_bwd(const fa_bwd_params *p, void *stream)
     // "unbounded" must stay unbounded after the shift by Sk - S that the key-owning kernel applies
     const int far = a.S + a.Sk;
     fa_mask_bounds(far, p->is_causal, p->window_size_left, p->window_size_right, &a.L, &a.R);
+    if (a.partials != nullptr) a.walk_head = walk_pairs_per_head(a.S, a.H / a.Hk, a.L, a.R);
     a.scale = p->softmax_scale;
     a.drop_threshold = (unsigned)fa_dropout_threshold(p->dropout_prob);
     a.drop_scale = 256.0f / (256.0f - (float)a.drop_threshold);

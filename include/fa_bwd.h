@@ -75,6 +75,14 @@ unsigned long long fa_bwd_min_fast_workspace_bytes(const fa_bwd_params *p);
  * dS blocks; dQ from the blocks: five products).  No atomics either way: every output element has one writer and
  * the same inputs give the same bits on every run. */
 int fa_bwd(const fa_bwd_params *p, void *stream);
+/* fa_bwd with room for partial sums of dK and dV (fp32, device, 16-byte aligned, fa_bwd_share_bytes(); NULL and 0 =
+ * fa_bwd).  Where one workgroup per key block leaves compute units idle -- few K/V heads, blocks of unequal work --, the
+ * five-product form then cuts the key blocks' work into equal shares, and one more kernel adds the parts of the blocks
+ * that were cut, in a fixed order: the same inputs give the same bits, but dK and dV of those blocks are summed in
+ * another order than by fa_bwd.  fa_bwd_share_bytes depends on p->workspace_bytes (which heads a launch works on) and
+ * is 0 where nothing would be cut. */
+unsigned long long fa_bwd_share_bytes(const fa_bwd_params *p);
+int fa_bwd_shared(const fa_bwd_params *p, void *partials, unsigned long long partials_bytes, void *stream);
 /* Host mirror of the arithmetic with which the key-owning kernel finds its work (csrc/fa_sched.h with the two
  * sides of the mask exchanged and shifted by S_kv - S): the inclusive range of 64-query tiles that contain a
  * query seeing at least one of the keys [k_begin, k_begin + rows), lo > hi when there is none; and the class of
