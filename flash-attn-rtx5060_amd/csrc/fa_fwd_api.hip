@@ -356,16 +356,30 @@ int fa_fwd_auto_splits(const fa_fwd_params *p)
     int L, R;
     fa_mask_bounds(s_max, p->is_causal, p->window_size_left, p->window_size_right, &L, &R);
     if (!decode_problem(p, R == 0)) return fa_fwd_suggest_splits(p);
-    // The decoding kernel: two workgroups per CU, and no wave without at least one piece of its own (32 keys at head
-    // dimension 128, 64 at 64, four waves per workgroup) among the keys that some query sees.  Both launches of a call,
-    // splits: us -- B1 H32/8 S_kv 1003: 4: 9.9, 8: 8.3, 16: 8.1; B1 H16 S_kv 512 D64: 2: 8.2, 4: 7.5; B1 H64/8 S_kv 32768:
-    // 16: 43.5, 32: 30.2, 64: 29.2; B16 H32/8 S_kv 8192: 2: 86.8, 4: 87.4, 8: 88.7; B8 H32/8 S_kv 2048: 4: 17.7, 8: 16.8, 16: 17.9.
+    // The decoding kernel: the splits with the least estimated time.  The chip's bandwidth is shared by its CUs, so K and V
+    // take as long as the CU with the most workgroups: (their bytes at 6.5 TB/s) * ceil(load) / load with load workgroups
+    // per CU, 5 % more where a CU has only one (four waves do not keep enough bytes in flight); a second launch costs 4 us
+    // and the partial results' traffic, one more trip to memory per 64 splits.  No wave without at least one piece of its own
+    // (32 keys at head dimension 128, 64 at 64, four waves per workgroup) among the keys that some query sees.  Both
+    // launches of a call, splits (workgroups per CU): us -- B17 H4 S_kv 27819 8 (2.1): 195, 15 (3.98): 149; B14 H32 S_kv
+    // 8806 D64 2 (3.5): 169, 4 (7.0): 155; B33 H4 S_kv 10356 4 (2.06): 140, 5 (2.6): 117; B26 H32 S4 S_kv 1616 D64 1 (3.25): 86,
+    // 4 (13): 63; B38 H32/4 S_kv 6599 4 (2.4): 94, 5 (2.97): 84.5; B4 H32 S_kv 32768 2 (1): 327, 4 (2): 308; B1 H32/8 S_kv 1003
+    // 4: 9.9, 8: 8.3; B10 H16 S_kv 1000 D64 1 (0.6): 12.2, 3 (1.9): 13.8.
     const long long heads = (long long)p->B * hk, visible = (long long)p->S + L < sk ? (long long)p->S + L : sk;
-    const long long most = visible / (p->d == 64 ? 256 : 128);
-    long long n = (2LL * kComputeUnits + heads - 1) / heads;
-    if (n > most) n = most;
-    if (n > key_tiles(p)) n = key_tiles(p);
-    return n < 1 ? 1 : (int)n;
+    long long most = visible / (p->d == 64 ? 256 : 128);
+    if (most > key_tiles(p)) most = key_tiles(p);
+    const long long loaded = (4LL * kComputeUnits + heads - 1) / heads;         // beyond four workgroups per CU: up to eight splits
+    if (most > (loaded > 8 ? loaded : 8)) most = loaded > 8 ? loaded : 8;
+    const double base = heads * (double)visible * p->d * 4.0 / 6.5e6, partial = (double)p->B * p->N * p->S * p->d * 8.0 / 5e6;
+    long long best = 1;
+    double best_us = 0.0;
+    for (long long n = 1; n <= most || n == 1; ++n) {
+        const long long groups = heads * n, per_cu = (groups + kComputeUnits - 1) / kComputeUnits;
+        double us = base * (double)(per_cu * kComputeUnits) / (double)groups * (per_cu == 1 ? 1.05 : 1.0);
+        if (n > 1) us += 4.0 + partial * (double)n + (double)((n - 1) / 64);
+        if (n == 1 || us < best_us) { best = n; best_us = us; }
+    }
+    return (int)best;
 }
 
 namespace {
