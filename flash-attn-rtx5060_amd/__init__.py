@@ -249,6 +249,41 @@ def abi_strides(t):
     return t, tuple(norm)
 
 
+# What a call needs besides its pointers follows from shapes, strides, types and options: it is worked out once per such
+# combination and kept (a small call's time was this Python code: B1 H4 S256 D64 11.4 us a call around a 7 us kernel, one
+# new token behind 1003 keys 16.5 around 9).  The entries hold sizes and a filled parameter block as bytes, never a tensor,
+# an address or an object's identity; they are made only from calls that succeeded with plain numbers for options.
+_plans = {}
+_PLANS_MAX = 1024
+_PLAIN = frozenset((int, float, bool, str, type(None)))
+_WHOLE = frozenset((int, bool))            # (a float is refused for these, and 1.0 would find the entry of 1)
+_torch_module = None
+
+
+def _torch():
+    global _torch_module
+    if _torch_module is None:
+        import torch
+        _torch_module = torch
+    return _torch_module
+
+
+def _raw_stream(torch, t):
+    """Handle of the current stream of t's device."""
+    get = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    return get(t.get_device()) if get is not None else torch.cuda.current_stream(t.device).cuda_stream
+
+
+def _slopes_key(alibi_slopes):
+    return None if alibi_slopes is None else (alibi_slopes.shape, alibi_slopes.stride(), alibi_slopes.dtype, alibi_slopes.device)
+
+
+def _keep_plan(key, plan):
+    if len(_plans) >= _PLANS_MAX:
+        _plans.clear()
+    _plans[key] = plan
+
+
 def flash_attention_forward(q, k, v, softmax_scale=None, causal=False, window_left=-1, window_right=-1,
                             return_lse=True, out=None, lse=None, sched=FA_SCHED_AUTO, alibi_slopes=None,
                             dropout_prob=0.0, seed=0, splits=1, exact_first_rows=False, static_scratch=False):
@@ -261,7 +296,33 @@ def flash_attention_forward(q, k, v, softmax_scale=None, causal=False, window_le
     ``alibi_slopes``: fp32 GPU tensor [N]; slope[h]*|i-j| is subtracted from every scaled score (mask.h:21-26).
     ``exact_first_rows``: see fa_fwd_params.exact_first_rows.  ``static_scratch``: go through
     fa_fwd_split_static (the key splits' partial results in the library's own static device array)."""
-    import torch
+    torch = _torch()
+    key = None
+    if (out is None and lse is None and {type(window_left), type(window_right), type(sched), type(seed)} <= _WHOLE and
+            {type(softmax_scale), type(causal), type(return_lse), type(dropout_prob), type(splits), type(exact_first_rows),
+             type(static_scratch)} <= _PLAIN):
+        key = (q.shape, q.stride(), q.dtype, q.device, k.shape, k.stride(), k.dtype, k.device, v.shape, v.stride(), v.dtype, v.device,
+               softmax_scale, causal, window_left, window_right, return_lse, sched, dropout_prob, seed, splits, exact_first_rows,
+               static_scratch, _slopes_key(alibi_slopes))
+        plan = _plans.get(key)
+        if plan is not None:
+            block, lse_shape, need, entry = plan
+            p = FaFwdParams.from_buffer_copy(block)
+            out = torch.empty_like(q)
+            p.Q, p.K, p.V, p.O = q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr()
+            if return_lse:
+                lse = torch.empty(lse_shape, dtype=torch.float32, device=q.device)
+                p.L = lse.data_ptr()
+            if alibi_slopes is not None:
+                p.alibi_slopes_ptr = alibi_slopes.data_ptr()
+            if need:
+                workspace = torch.empty(need, dtype=torch.uint8, device=q.device)   # stream-ordered: freed after the launch
+                p.workspace = workspace.data_ptr()
+            st = entry(ctypes.byref(p), _raw_stream(torch, q))
+            if st != FA_OK:
+                raise FaError(st, lib().fa_last_device_error().decode() if st == FA_ERR_DEVICE else "")
+            return (out, lse) if return_lse else out
+    given = (q, k, v)
     if not (q.is_cuda and k.is_cuda and v.is_cuda):
         raise ValueError("q, k, v must live on the GPU")
     if q.dtype not in (torch.float16, torch.bfloat16) or k.dtype != q.dtype or v.dtype != q.dtype:
@@ -299,11 +360,12 @@ def flash_attention_forward(q, k, v, softmax_scale=None, causal=False, window_le
         if need and not static_scratch:
             workspace = torch.empty(need, dtype=torch.uint8, device=q.device)   # stream-ordered: freed after the launch
             p.workspace, p.workspace_bytes = workspace.data_ptr(), need
-    stream = torch.cuda.current_stream(q.device).cuda_stream
     entry = lib().fa_fwd_split_static if static_scratch else lib().fa_fwd
-    st = entry(ctypes.byref(p), ctypes.c_void_p(stream))
+    st = entry(ctypes.byref(p), _raw_stream(torch, q))
     if st != FA_OK:
         raise FaError(st, lib().fa_last_device_error().decode() if st == FA_ERR_DEVICE else "")
+    if key is not None and q is given[0] and k is given[1] and v is given[2]:         # (no dense copy was needed)
+        _keep_plan(key, (bytes(p), (B, N, S), 0 if workspace is None else p.workspace_bytes, entry))
     return (out, lse) if return_lse else out
 
 
@@ -342,7 +404,35 @@ def flash_attention_backward(q, k, v, o, lse, do, softmax_scale=None, causal=Fal
     NaN bit patterns first: the kernels must not read anything in it that they have not written.
     Shapes and strides as in flash_attention_forward (q, o, do [B, N, S, d]; k, v [B, Nk, S_kv, d]; lse
     [B, N, S] float32 contiguous); dq, dk, dv come back with the strides of q, k, v."""
-    import torch
+    torch = _torch()
+    key = None
+    if (type(five_products) is str and five_products == "auto" and not poison_workspace and workspace_limit is None and
+            {type(window_left), type(window_right), type(seed)} <= _WHOLE and {type(softmax_scale), type(causal), type(dropout_prob)} <= _PLAIN):
+        key = (q.shape, q.stride(), q.dtype, q.device, k.shape, k.stride(), k.dtype, k.device, v.shape, v.stride(), v.dtype, v.device,
+               o.shape, o.stride(), o.dtype, o.device, do.shape, do.stride(), do.dtype, do.device, lse.shape, lse.stride(), lse.dtype, lse.device,
+               softmax_scale, causal, window_left, window_right, dropout_prob, seed, _slopes_key(alibi_slopes))
+        plan = _plans.get(key)
+        workspace = None
+        if plan is not None:
+            block, total, parts_at, parts = plan
+            try:
+                workspace = torch.empty(total, dtype=torch.uint8, device=q.device)      # stream-ordered: freed after the launch
+            except torch.cuda.OutOfMemoryError:
+                pass                                                                    # (the smaller sizes are tried below)
+        if workspace is not None:
+            p = FaBwdParams.from_buffer_copy(block)
+            dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
+            p.Q, p.K, p.V, p.O, p.dO, p.L = q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), do.data_ptr(), lse.data_ptr()
+            p.dQ, p.dK, p.dV = dq.data_ptr(), dk.data_ptr(), dv.data_ptr()
+            at = workspace.data_ptr()
+            p.workspace = at
+            if alibi_slopes is not None:
+                p.alibi_slopes_ptr = alibi_slopes.data_ptr()
+            st = lib().fa_bwd_shared(ctypes.byref(p), at + parts_at if parts else None, parts, _raw_stream(torch, q))
+            if st != FA_OK:
+                raise FaError(st, lib().fa_last_device_error().decode() if st == FA_ERR_DEVICE else "")
+            return dq, dk, dv
+    given = (q, k, v, o, do)
     if not all(t.is_cuda and t.dtype == q.dtype and t.dim() == 4 for t in (q, k, v, o, do)):
         raise ValueError("q, k, v, o, do must be 4-d GPU tensors of one dtype")
     if q.dtype not in (torch.float16, torch.bfloat16):
@@ -363,10 +453,13 @@ def flash_attention_backward(q, k, v, o, lse, do, softmax_scale=None, causal=Fal
     for n, t in dict(q=q, k=k, v=v, o=o, do=do).items():
         tensors[n], strides[n] = abi_strides(t)
     q, k, v, o, do = (tensors[n] for n in ("q", "k", "v", "o", "do"))
+    if any(t is not was for t, was in zip((q, k, v, o, do), given)):
+        key = None
     for n, like in (("dq", q), ("dk", k), ("dv", v)):
         g = torch.empty_like(like)                    # keeps a dense or permuted layout
         g_abi, g_st = abi_strides(g)
         if g_abi is not g:
+            key = None
             g, g_st = torch.empty(like.shape, dtype=like.dtype, device=like.device), None
         tensors[n], strides[n] = g, g_st
     dq, dk, dv = tensors["dq"], tensors["dk"], tensors["dv"]
@@ -404,8 +497,9 @@ def flash_attention_backward(q, k, v, o, lse, do, softmax_scale=None, causal=Fal
             if workspace_limit is None:
                 p.workspace_bytes = want
                 sizes.append((want, lib().fa_bwd_share_bytes(ctypes.byref(p))))
-    workspace = None
+    workspace, choices = None, len(sizes)
     while workspace is None:              # stream-ordered: freed after the launch
+        first_choice = len(sizes) == choices
         need, parts = sizes.pop()
         parts_at = (need + 255) // 256 * 256
         try:
@@ -416,10 +510,11 @@ def flash_attention_backward(q, k, v, o, lse, do, softmax_scale=None, causal=Fal
     if poison_workspace:
         workspace.fill_(0xff)
     p.workspace, p.workspace_bytes = workspace.data_ptr(), need
-    st = lib().fa_bwd_shared(ctypes.byref(p), workspace.data_ptr() + parts_at if parts else None, parts,
-                             ctypes.c_void_p(torch.cuda.current_stream(q.device).cuda_stream))
+    st = lib().fa_bwd_shared(ctypes.byref(p), workspace.data_ptr() + parts_at if parts else None, parts, _raw_stream(torch, q))
     if st != FA_OK:
         raise FaError(st, lib().fa_last_device_error().decode() if st == FA_ERR_DEVICE else "")
+    if key is not None and first_choice:
+        _keep_plan(key, (bytes(p), workspace.numel(), parts_at, parts))
     return dq, dk, dv
 
 

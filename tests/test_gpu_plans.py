@@ -1,0 +1,61 @@
+"""What the binding keeps per combination of shapes, strides and options: a call that finds an entry gives what the first
+one gave, for other tensors, other strides and other options, and what was refused stays refused."""
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _inputs(torch, seed, bshd, B=2, H=4, Hk=2, S=200, D=64):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    t = [torch.randn((B, S, h, D) if bshd else (B, h, S, D), device="cuda", generator=g).half() for h in (H, Hk, Hk, H)]
+    return [x.transpose(1, 2) for x in t] if bshd else t
+
+
+@pytest.mark.parametrize("bshd", [False, True])
+@pytest.mark.parametrize("kw", [dict(), dict(causal=True), dict(causal=True, window_left=40), dict(causal=True, splits=3),
+                                dict(splits="auto", return_lse=False), dict(dropout_prob=0.2, seed=5), dict(softmax_scale=0.3), "slopes"])
+def test_second_call_equals_the_first(fa, kw, bshd):
+    import torch
+    results = []
+    for kept in (False, True):
+        fa._plans.clear()
+        if kept:            # entries of this shape made from other tensors (and, beside them, of other options and strides)
+            for s, other in ((11, bshd), (12, not bshd)):
+                q, k, v, do = _inputs(torch, s, other)
+                for o in (dict(), dict(causal=True), dict(softmax_scale=0.5), dict() if kw == "slopes" else kw):
+                    fa.flash_attention_forward(q, k, v, **o)
+                if kw == "slopes":
+                    fa.flash_attention_forward(q, k, v, alibi_slopes=torch.full((4,), 3.0, device="cuda"))
+        q, k, v, do = _inputs(torch, 1, bshd)
+        o = dict(alibi_slopes=torch.tensor([0.5, 0.25, 0.1, 0.0], device="cuda")) if kw == "slopes" else kw
+        got = fa.flash_attention_forward(q, k, v, **o)
+        out = list(got) if isinstance(got, tuple) else [got]
+        o = {n: x for n, x in o.items() if n not in ("splits", "return_lse")}
+        fwd, lse = fa.flash_attention_forward(q, k, v, exact_first_rows=True, **o)
+        for _ in range(2):
+            out += fa.flash_attention_backward(q, k, v, fwd, lse, do, **o)
+        torch.cuda.synchronize()
+        assert out[0].stride() == q.stride() and out[-1].stride() == v.stride()
+        results.append(out)
+    for a, b in zip(*results):
+        assert a.stride() == b.stride()
+        assert torch.equal(a.contiguous().view(torch.uint8), b.contiguous().view(torch.uint8))
+
+
+def test_what_was_refused_stays_refused(fa):
+    import torch
+    q, k, v, _ = _inputs(torch, 1, False)
+    fa.flash_attention_forward(q, k, v, causal=True, window_left=1, seed=1)
+    for bad in (dict(window_left=1.0), dict(seed=1.0)):
+        with pytest.raises(TypeError):
+            fa.flash_attention_forward(q, k, v, **{**dict(causal=True, window_left=1, seed=1), **bad})
+    scale = torch.tensor(0.25)
+    a = fa.flash_attention_forward(q, k, v, softmax_scale=scale, return_lse=False).clone()
+    scale.fill_(0.5)        # the same object with another value
+    b = fa.flash_attention_forward(q, k, v, softmax_scale=scale, return_lse=False)
+    assert torch.equal(b, fa.flash_attention_forward(q, k, v, softmax_scale=0.5, return_lse=False)) and not torch.equal(a, b)
+    with pytest.raises(ValueError):
+        fa.flash_attention_forward(q, k.cpu(), v)
+    shifted = torch.empty(q.numel() + 8, dtype=q.dtype, device="cuda")[1:1 + q.numel()].view(q.shape)      # 2 bytes off
+    with pytest.raises(fa.FaError):
+        fa.flash_attention_forward(shifted, k, v, causal=True, window_left=1, seed=1)
