@@ -82,9 +82,9 @@ template <int D> struct TileReader {
     }
 };
 
-// one 64-row tile global -> LDS: wave w issues instructions w, w+8, ...
-template <int D> struct TileLoader {
-    static constexpr int CPR = D / 8, ROWB = D * 2, TILEB = 64 * ROWB, IPW = TILEB / 1024 / kBwdWaves;
+// one 64-row tile global -> LDS: wave w of NW issues instructions w, w + NW, ...
+template <int D, int NW = kBwdWaves> struct TileLoader {
+    static constexpr int CPR = D / 8, ROWB = D * 2, TILEB = 64 * ROWB, IPW = TILEB / 1024 / NW;
     uint32_t g[IPW];
     int wave, lane;
     // row_bytes: distance between consecutive rows of the source in bytes
@@ -93,14 +93,14 @@ template <int D> struct TileLoader {
         wave = wave_; lane = lane_;
 #pragma unroll
         for (int i = 0; i < IPW; ++i) {
-            g[i] = (uint32_t)fa_bwd_load_source(D, (i * kBwdWaves + wave) * 64 + lane, row_bytes);
+            g[i] = (uint32_t)fa_bwd_load_source(D, (i * NW + wave) * 64 + lane, row_bytes);
         }
     }
     __device__ __forceinline__ void load(const uint16_t *tile_src, uint32_t lds_tile) const
     {
 #pragma unroll
         for (int i = 0; i < IPW; ++i)
-            dma_16(reinterpret_cast<const char *>(tile_src), g[i], lds_tile + (i * kBwdWaves + wave) * 1024);
+            dma_16(reinterpret_cast<const char *>(tile_src), g[i], lds_tile + (i * NW + wave) * 1024);
     }
     // a tile whose last rows lie past the end of the tensor: they are filled with copies of row `valid - 1`
     __device__ __forceinline__ void load_ragged(const uint16_t *tile_src, uint32_t lds_tile, int valid, int row_bytes) const
@@ -111,10 +111,10 @@ template <int D> struct TileLoader {
         asm volatile("" : "+v"(ln));
 #pragma unroll
         for (int i = 0; i < IPW; ++i) {
-            const int P = (i * kBwdWaves + wave) * 64 + ln, row = P / CPR, pos = P % CPR;
+            const int P = (i * NW + wave) * 64 + ln, row = P / CPR, pos = P % CPR;
             const int src_row = row < valid ? row : valid - 1;
             dma_16(reinterpret_cast<const char *>(tile_src), (uint32_t)(src_row * row_bytes + ((pos ^ fa_u_swz(CPR, row)) << 4)),
-                   lds_tile + (i * kBwdWaves + wave) * 1024);
+                   lds_tile + (i * NW + wave) * 1024);
         }
     }
 };
@@ -139,7 +139,7 @@ __device__ __forceinline__ void wait_vm_upto(int n)
 #define FA_WAIT_CASE(k) case k: wait_vm<k>(); break;
     FA_WAIT_CASE(0) FA_WAIT_CASE(1) FA_WAIT_CASE(2) FA_WAIT_CASE(3) FA_WAIT_CASE(4) FA_WAIT_CASE(5) FA_WAIT_CASE(6) FA_WAIT_CASE(7)
     FA_WAIT_CASE(8) FA_WAIT_CASE(9) FA_WAIT_CASE(10) FA_WAIT_CASE(11) FA_WAIT_CASE(12) FA_WAIT_CASE(13) FA_WAIT_CASE(14) FA_WAIT_CASE(15)
-    FA_WAIT_CASE(16)
+    FA_WAIT_CASE(16) FA_WAIT_CASE(17) FA_WAIT_CASE(18)
 #undef FA_WAIT_CASE
     default: wait_vm<0>(); break;
     }
@@ -861,27 +861,29 @@ __global__ void __launch_bounds__(256) fa_bwd_add_parts(const FaBwdArgs a, int n
     }
 }
 
-// dQ^T += K^T dS^T over the dS blocks fa_bwd_dkdv<WRITE_DS> wrote.  A workgroup owns 256 queries (8 waves x one
+// dQ^T += K^T dS^T over the dS blocks fa_bwd_dkdv<WRITE_DS> wrote.  A workgroup owns 32 NW queries (NW waves x one
 // 32-query block, lane = query) and walks the key tiles of its visible range.  LDS stage: the K tile (read
 // transposed, as in fa_bwd_dq) and, per wave, the two 2 KiB dS blocks of its query block against the tile's keys,
 // fetched by that wave alone.  A block comes in as it lies in memory except that the 64-byte groups of four keys
 // are XOR-permuted among the four 512-byte planes, so that the transposing read of a half-wave -- four keys, all
 // 32 queries, i.e. one group in each plane -- touches every LDS bank once.
-template <bool BF16, int D, bool MASKED, int LAYOUT>
-__global__ void __launch_bounds__(kBwdWaves * 64, 2) fa_bwd_dq_from_ds(const FaBwdArgs a)
+template <bool BF16, int D, bool MASKED, int LAYOUT, int NW, int NST>
+__global__ void __launch_bounds__(NW * 64, 2) fa_bwd_dq_from_ds(const FaBwdArgs a)
 {
     constexpr bool STRIDED = LAYOUT >= 1, GENERAL = LAYOUT == 2;      // (general: any length S = S_kv)
     typedef Num<BF16> N;
     typedef TileReader<D> Reader;
-    typedef TileLoader<D> Loader;
+    typedef TileLoader<D, NW> Loader;
     constexpr int DB = Reader::DB, TILEB = Loader::TILEB, IPW = Loader::IPW;
     constexpr int WAVE_DS = 2 * kDsBlockBytes;                 // a wave's two blocks of a key tile
-    constexpr int STAGEB = TILEB + kBwdWaves * WAVE_DS;
+    constexpr int STAGEB = TILEB + NW * WAVE_DS, ROWS = 32 * NW;
+    constexpr int AHEAD = NST - 1;                             // tiles are requested this many ahead
+    static_assert((AHEAD - 1) * (IPW + 4) <= 18, "more requests in flight than wait_vm_upto counts");
     extern __shared__ __attribute__((aligned(1024))) char smem[];
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)smem;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int S = a.S;
-    const int n_qblocks = (S + 255) / 256;
+    const int n_qblocks = (S + ROWS - 1) / ROWS;
     const int group = STRIDED ? a.H / a.Hk : 1, heads_q = a.heads * group, head0_q = a.head0 * group;
     const long long n_items = (long long)heads_q * n_qblocks;
     for (int pass = 0;; ++pass) {
@@ -903,10 +905,10 @@ __global__ void __launch_bounds__(kBwdWaves * 64, 2) fa_bwd_dq_from_ds(const FaB
         dQh = head_ptr(a.dQ, a.dq, b, h);
         k_rs = a.k.rs; dq_rs = a.dq.rs;
     }
-    const int q0 = qblock * 256, qw = q0 + wave * 32;
-    const bool active = qw < S;                    // the last block may own fewer than 256 rows
+    const int q0 = qblock * ROWS, qw = q0 + wave * 32;
+    const bool active = qw < S;                    // the last block may own fewer rows
     int t0, t1, my_lo = 1, my_hi = 0;
-    fa_tile_range(S, 64, a.L, a.R, q0, S - q0 < 256 ? S - q0 : 256, &t0, &t1);
+    fa_tile_range(S, 64, a.L, a.R, q0, S - q0 < ROWS ? S - q0 : ROWS, &t0, &t1);
     if (active) fa_tile_range(S, 64, a.L, a.R, qw, GENERAL && S - qw < 32 ? S - qw : 32, &my_lo, &my_hi);
     // this head's dS blocks; this wave reads those of query block qw / 32
     const char *ds_head = reinterpret_cast<const char *>(a.ds_blocks) + (long long)(bh - head0_q) * fa_ds_blocks_per_head(S) * kDsBlockBytes;
@@ -961,15 +963,18 @@ __global__ void __launch_bounds__(kBwdWaves * 64, 2) fa_bwd_dq_from_ds(const FaB
     for (int db = 0; db < DB; ++db) dq[db] = zero16();
 
     if (t0 <= t1) {
-        issue(t0, 0);
-        if (t0 + 1 <= t1) issue(t0 + 1, 1);
-        wait_vm<0>();
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u)
+            if (t0 + u <= t1) issue(t0 + u, u);
         int stage = 0;
         for (int t = t0; t <= t1; ++t) {
-            const int next = stage == kBwdStages - 1 ? 0 : stage + 1;
-            if (t + 1 <= t1) {              // tile t has landed, tile t+1 may still be in flight
-                if (my_lo <= t + 1 && t + 1 <= my_hi) wait_vm<IPW + 4>(); else wait_vm<IPW>();
-            } else wait_vm<0>();
+            const int next = stage == NST - 1 ? 0 : stage + 1;
+            // tile t has landed when at most the requests of the tiles behind it are outstanding
+            int later = 0;
+#pragma unroll
+            for (int u = 1; u < AHEAD; ++u)
+                if (t + u <= t1) later += my_lo <= t + u && t + u <= my_hi ? IPW + 4 : IPW;
+            wait_vm_upto(later);
             phase_barrier();
             if (my_lo <= t && t <= my_hi) {
 #pragma unroll
@@ -985,8 +990,8 @@ __global__ void __launch_bounds__(kBwdWaves * 64, 2) fa_bwd_dq_from_ds(const FaB
                     }
                 }
             }
-            if (t + 2 <= t1) issue(t + 2, next == kBwdStages - 1 ? 0 : next + 1);
-            const int delta = next == 0 ? -(kBwdStages - 1) * STAGEB : STAGEB;
+            if (t + AHEAD <= t1) issue(t + AHEAD, stage == 0 ? NST - 1 : stage - 1);       // (the stage tile t - 1 was read from)
+            const int delta = next == 0 ? -(NST - 1) * STAGEB : STAGEB;
             rd.advance(delta);
             ds_rd[0] += delta; ds_rd[1] += delta;
             stage = next;
@@ -1024,7 +1029,8 @@ hipError_t launch_bwd(const FaBwdArgs &a_in, int compute_units, hipStream_t stre
     constexpr bool FIVE = LAYOUT <= 1 || (!ALIBI && !DROPOUT);
     constexpr int FL = FIVE ? LAYOUT : 0;
     constexpr bool CAN_SHARE = FIVE && fa_bwd_can_share(D, DROPOUT);
-    const int smem_dq_ds = kBwdStages * (TILEB + kBwdWaves * 2 * kDsBlockBytes);
+    // the query-owning kernel from dS blocks: 8 waves (256 queries) and three LDS stages, or 4 waves and four stages
+    auto smem_dq_ds = [](int waves, int stages) { return stages * (TILEB + waves * 2 * kDsBlockBytes); };
     // the LDS opt-in is per (instantiation, device) and is made once, not on every launch
     static std::atomic<unsigned long long> configured{0ull};
     const unsigned long long dev_bit = 1ull << fa_launch_device();
@@ -1042,8 +1048,11 @@ hipError_t launch_bwd(const FaBwdArgs &a_in, int compute_units, hipStream_t stre
                                         hipFuncAttributeMaxDynamicSharedMemorySize, smem_dkdv_ds);
                 if (e != hipSuccess) return e;
             }
-            e = hipFuncSetAttribute(reinterpret_cast<const void *>(fa_bwd_dq_from_ds<BF16, D, MASKED, FL>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, smem_dq_ds);
+            e = hipFuncSetAttribute(reinterpret_cast<const void *>(fa_bwd_dq_from_ds<BF16, D, MASKED, FL, 8, 3>),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, smem_dq_ds(8, 3));
+            if (e != hipSuccess) return e;
+            e = hipFuncSetAttribute(reinterpret_cast<const void *>(fa_bwd_dq_from_ds<BF16, D, MASKED, FL, 4, 4>),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, smem_dq_ds(4, 4));
             if (e != hipSuccess) return e;
         }
         configured.fetch_or(dev_bit, std::memory_order_relaxed);
@@ -1093,10 +1102,21 @@ hipError_t launch_bwd(const FaBwdArgs &a_in, int compute_units, hipStream_t stre
                         hipLaunchKernelGGL((fa_bwd_add_parts<BF16, D, FL >= 1>), dim3((n_shares - 1) * 2 * kBwdWaves), dim3(256), 0, stream, a, (int)n_shares);
                     }
                 }
-                const unsigned launch_q = grid_if(uneven_items, (long long)a.heads * group * ((a.S + 255) / 256));
                 if (n_shares == 0)
                     hipLaunchKernelGGL((fa_bwd_dkdv<BF16, D, MASKED, FL, ALIBI, DROPOUT, true>), dim3(launch_k), dim3(kBwdWaves * 64), smem_dkdv_ds, stream, a);
-                hipLaunchKernelGGL((fa_bwd_dq_from_ds<BF16, D, MASKED, FL>), dim3(launch_q), dim3(kBwdWaves * 64), smem_dq_ds, stream, a);
+                // Fewer than two 256-query items per CU: 128-query ones, twice as many, and a deeper ring, since a CU that
+                // walks one item waits for the latency of its tiles.  Backward pass, causal, 128 against 256 queries: B2 H16
+                // S2048 D128 (256 items) 162 against 177 us, B1 H8 S2048 D128 88 against 97, B1 H4 S4096 D64 86 against 98, B1 H16
+                // S1024 D64 45 against 50; with 512 items level (B8 H16 S1000 D64 108 both), with 1024 K is read twice as often
+                // for nothing (B2 H32/8 S4096 D128 910 against 887).
+                const long long heads_q = (long long)a.heads * group, items_q = heads_q * ((a.S + 255) / 256);
+                if (items_q < 2LL * compute_units) {
+                    const unsigned launch_q = grid_if(uneven_items, heads_q * ((a.S + 127) / 128));
+                    hipLaunchKernelGGL((fa_bwd_dq_from_ds<BF16, D, MASKED, FL, 4, 4>), dim3(launch_q), dim3(4 * 64), smem_dq_ds(4, 4), stream, a);
+                } else {
+                    const unsigned launch_q = grid_if(uneven_items, items_q);
+                    hipLaunchKernelGGL((fa_bwd_dq_from_ds<BF16, D, MASKED, FL, 8, 3>), dim3(launch_q), dim3(8 * 64), smem_dq_ds(8, 3), stream, a);
+                }
             }
             return hipGetLastError();
         }
