@@ -352,7 +352,9 @@ def flash_attention_forward(q, k, v, softmax_scale=None, causal=False, window_le
                     q_st, k_st, v_st, o_st,
                     dropout_prob=dropout_prob, seed=seed, S_kv=0 if S_kv == S else S_kv, exact_first_rows=exact_first_rows)
     if splits == "auto":
-        splits = lib().fa_fwd_auto_splits(ctypes.byref(p))
+        splits = p.split_num = lib().fa_fwd_auto_splits(ctypes.byref(p))
+        if static_scratch and lib().fa_fwd_workspace_bytes(ctypes.byref(p)) > lib().fa_fwd_static_scratch_bytes():
+            splits = p.split_num = lib().fa_fwd_suggest_splits(ctypes.byref(p))     # (fewer of them may fit)
     workspace = None
     if splits and splits > 1:
         p.split_num = int(splits)

@@ -59,3 +59,24 @@ def test_decode_kernel_with_streaming_loads(fa):
     ref = (p[..., None] * v.float()).sum(2, keepdim=True)
     assert float((o.float() - ref).abs().max()) <= 2e-3
     assert float((lse[..., 0] - torch.logsumexp(s, dim=-1)).abs().max()) <= 2e-3
+
+
+def test_auto_splits_fit_the_static_scratch(fa):
+    """splits="auto" through the static scratch: where the partial results of the fastest split count do not fit the
+    32 MiB, the count that fills the device once is used, whose do."""
+    import ctypes
+    import torch
+    B, H, Hk, S, Skv, D = 146, 64, 2, 1, 4000, 128
+    L = fa.lib()
+    p = fa.make_params(B, H, S, D, causal=True, n_kv_heads=Hk, S_kv=Skv)
+    need = {}
+    for name, splits in (("auto", L.fa_fwd_auto_splits), ("fill", L.fa_fwd_suggest_splits)):
+        p.split_num = splits(ctypes.byref(p))
+        need[name] = L.fa_fwd_workspace_bytes(ctypes.byref(p))
+    assert need["auto"] > L.fa_fwd_static_scratch_bytes() >= need["fill"] > 0
+    g = torch.Generator(device="cuda").manual_seed(6)
+    q = torch.randn((B, H, S, D), device="cuda", generator=g, dtype=torch.float16)
+    k, v = (torch.randn((B, Hk, Skv, D), device="cuda", generator=g, dtype=torch.float16) for _ in range(2))
+    o = fa.flash_attention_forward(q, k, v, causal=True, splits="auto", static_scratch=True, return_lse=False)
+    ref = fa.flash_attention_forward(q, k, v, causal=True, splits=p.split_num, return_lse=False)
+    assert torch.equal(o, ref)
