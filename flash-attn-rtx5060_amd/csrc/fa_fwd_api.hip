@@ -355,7 +355,30 @@ int fa_fwd_auto_splits(const fa_fwd_params *p)
     const int s_max = sk > p->S ? sk : p->S;
     int L, R;
     fa_mask_bounds(s_max, p->is_causal, p->window_size_left, p->window_size_right, &L, &R);
-    if (!decode_problem(p, R == 0)) return fa_fwd_suggest_splits(p);
+    if (!decode_problem(p, R == 0)) {
+        // The tile kernels, 128-row blocks, queries behind a cache (what else ran is left at the count that fills the device):
+        // the least estimated time as well.  Workgroups per compute unit times (key tiles of a split, 0.85 us each at head
+        // dimension 128 and 0.55 at 64, + 1.4), 1.4 of that per workgroup where a unit has only one; a second launch costs
+        // 4.6 us and the partial results' traffic.  Filling the device once took just over one round to two: 512 slots for
+        // 528 items are as slow as 1024.  Causal bf16 [B,S,H,D], items before splits, filled once against this, splits: us --
+        // B1 H32/8 S700 S_kv 4700 192 3: 94.9, 4: 82.4; B1 H32 S300 S_kv 4000 D64 96 6: 38.9, 5: 29.1; B3 H8/2 S150 S_kv 10000 48 11:
+        // 61.3, 10: 43.9; B4 H32/8 S256 S_kv 2000 256 2: 54.4, 1: 48.9; B4 H16 S600 S_kv 3000 320 2: 94.1, 1: 82.8; B1 H32/8 S500
+        // S_kv 4596 128 4: 55.6 both.  Sixty random shapes where the two differ: 0.97 to 1.68 times as fast, 1.21 on average.
+        const long long items = base_items(p);
+        const int tiles = key_tiles(p);
+        if (sk <= p->S || L < s_max || waves_of(p) == 8 || items >= 2 * kComputeUnits) return fa_fwd_suggest_splits(p);
+        const double tile_us = p->d == 64 ? 0.55 : 0.85, partial = (double)p->B * p->N * p->S * p->d * 8.0 / 5.2e6;
+        int best = 1;
+        double best_us = 0.0;
+        // (at least three tiles a split, B2 H16/4 S91 S_kv 636 5: 19.1, 2: 18.6; at most four workgroups on every slot)
+        for (int n = 1; n == 1 || (3 * n <= tiles && items * n <= 8 * kComputeUnits); ++n) {
+            const long long per_cu = (items * n + kComputeUnits - 1) / kComputeUnits;
+            double us = (double)per_cu * ((tiles + n - 1) / n * tile_us + 1.4) * (per_cu == 1 ? 1.4 : 1.0);
+            if (n > 1) us += 4.6 + partial * n;
+            if (n == 1 || us < best_us) { best = n; best_us = us; }
+        }
+        return best;
+    }
     // The decoding kernel: the splits with the least estimated time.  The chip's bandwidth is shared by its CUs, so K and V
     // take as long as the CU with the most workgroups: (their bytes at 6.5 TB/s) * ceil(load) / load with load workgroups
     // per CU, 5 % more where a CU has only one (four waves do not keep enough bytes in flight); a second launch costs 4 us

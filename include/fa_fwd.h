@@ -129,7 +129,8 @@ unsigned long long fa_fwd_workspace_bytes(const fa_fwd_params *p);
 int fa_fwd_suggest_splits(const fa_fwd_params *p);
 /* The split count with which this library is fastest: that of fa_fwd_suggest_splits, and where the decoding kernel
  * takes the problem (at most 32 query rows per K/V head) what suits that kernel, which splits short caches further and
- * divides only the keys that a window leaves visible.  Set split_num to it before asking for the workspace. */
+ * divides only the keys that a window leaves visible, or where a few hundred query rows stand behind a cache what
+ * leaves no compute unit with more work than the others.  Set split_num to it before asking for the workspace. */
 int fa_fwd_auto_splits(const fa_fwd_params *p);
 
 /* Sets up the library's state for the current device: looks up the addresses of its two file-scope device
