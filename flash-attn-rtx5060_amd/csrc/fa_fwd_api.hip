@@ -471,7 +471,6 @@ int forward(const fa_fwd_params *p, void *workspace, const FaDeviceState *ds, vo
     a.Hk = p->n_kv_heads > 0 ? p->n_kv_heads : p->N;
     a.Sk = p->S_kv > 0 ? p->S_kv : p->S;
     a.n_splits = effective_splits(p);
-    a.tiles_per_split = (key_tiles(p) + a.n_splits - 1) / a.n_splits;
     a.o_part = static_cast<float *>(workspace);
     a.lse_part = a.o_part != nullptr ? a.o_part + (size_t)a.n_splits * p->B * p->N * p->S * p->d : nullptr;
     a.pack = packed_group(p);

@@ -601,8 +601,12 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
     fa_tile_range(Sk, kBlockKeys, a.L, a.R, block_pos0 + pos_off, rows_in_block, &t0, &t1);
     int my_lo = 1, my_hi = 0;   // key tiles with at least one visible pair for this wave (contiguous)
     if (wave_live) fa_tile_range(Sk, kBlockKeys, a.L, a.R, wave_pos0 + pos_off, wave_npos, &my_lo, &my_hi);
-    if (n_splits > 1) {         // this item's share of the key tiles; may leave nothing
-        const int s_lo = split * a.tiles_per_split, s_hi = s_lo + a.tiles_per_split - 1;
+    if (n_splits > 1) {         // this item's share of the key tiles that the block visits; may leave nothing
+        // (of the block's own range, not of all keys: under a window most shares of the whole cache hold nothing that the
+        // block sees, and one or two did all the work.  Causal bf16 [B,S,H,D], shares of all keys against these, us: window
+        // 1024 B1 H32/8 S500 S_kv 16000 54.5 / 33.7, window 2000 B1 H8 S2048 S_kv 32768 78.6 / 41.0, window 512 B2 H8 S256
+        // S_kv 8000 D64 24.3 / 21.0; no window B1 H32/8 S500 S_kv 4596 58.3 / 55.4, B1 H64/16 S40 S_kv 6000 31.3 / 30.6)
+        const int share = (t1 - t0 + n_splits) / n_splits, s_lo = t0 + split * share, s_hi = s_lo + share - 1;
         t0 = t0 > s_lo ? t0 : s_lo;
         t1 = t1 < s_hi ? t1 : s_hi;
         my_lo = my_lo > s_lo ? my_lo : s_lo;

@@ -30,8 +30,8 @@ struct FaKernelArgs {
     long long q_bs, q_hs, k_bs, k_hs;           // batch and head strides
     long long v_bs, v_hs, o_bs, o_hs;
     int Sk;              // keys per head (S is the number of queries); query i sits at key position i + Sk - S
-    int n_splits;        // > 1: every (head, query block) is n_splits consecutive work items, each over
-    int tiles_per_split; //      tiles_per_split key tiles, writing partial results:
+    int n_splits;        // > 1: every (head, query block) is n_splits consecutive work items, each over an equal
+                         //      share of the key tiles that the block visits, writing partial results:
     float *o_part;       //      [n_splits][BH][S][D] fp32, normalised over the split's own keys
     float *lse_part;     //      [n_splits][BH][S] fp32, -inf where the split saw no key of the row
     int pack;            // > 1: work items are (batch, K/V head) and their rows the queries of the `pack` query

@@ -44,3 +44,26 @@ def test_chunks_with_auto_splits(fa, oracle, B, H, Hk, S, Skv, D, dtype, causal)
     torch.cuda.synchronize()
     err = errors(oracle.to_f32(from_torch(o), dtype), oracle.to_f32(o_ref, dtype), lse.cpu().numpy(), lse_ref)
     assert_within(err, dtype, f"S={S} Skv={Skv} splits={both(fa, B, H, Hk, S, Skv, D, causal)[0]}")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,H,Hk,S,Skv,D,dtype,wl,splits", [
+    (1, 2, 2, 150, 1500, 64, 0, 100, 3),          # every block sees four or five of 24 tiles
+    (1, 2, 1, 150, 1500, 128, 1, 40, 7),          # more splits than tiles: some shares hold nothing
+    (1, 4, 1, 30, 2000, 128, 0, 300, 4),          # four heads' rows in one block
+    (1, 2, 2, 256, 300, 64, 0, 0, 5),             # every row sees one key
+    (1, 2, 2, 300, 310, 128, 0, 64, 4),           # the first rows' arithmetic (queries from position 10 on)
+])
+def test_windows_with_splits(fa, oracle, B, H, Hk, S, Skv, D, dtype, wl, splits):
+    import torch
+    q, _, _ = make_inputs(fa, (B, H, S, D), dtype, seed=4000 + S)
+    _, k, v = make_inputs(fa, (B, Hk, Skv, D), dtype, seed=4001 + Skv)
+    o_ref, lse_ref = oracle_rect(oracle, q, k, v, dtype, True, wl, -1, None)
+    o, lse = fa.flash_attention_forward(*(to_torch(x, dtype) for x in (q, k, v)), causal=True, window_left=wl, splits=splits)
+    torch.cuda.synchronize()
+    got = oracle.to_f32(from_torch(o), dtype)
+    err = errors(got, oracle.to_f32(o_ref, dtype), lse.cpu().numpy(), lse_ref)
+    if wl == 0:                                   # |O| as large as the values: one ulp of the result
+        assert err["nonfinite"] == 0 and err["max_abs"] <= max(2e-3, 2.0 ** -10 * abs(got).max())
+    else:
+        assert_within(err, dtype, f"S={S} Skv={Skv} wl={wl} splits={splits}")
