@@ -331,7 +331,8 @@ __global__ void __launch_bounds__(NW * 64, NB == 1 ? 4 : 2) fa_fwd_decode(const 
 // (a split that saw no key of the row has LSE_s = -inf and weight 0).  A thread has four output elements of a row and
 // takes eight splits at a time, logsumexps and partial rows requested together: one trip to memory for up to eight
 // splits.  With more of them GROUPS threads share the four elements, taking eight splits in turn, and their sums meet
-// in LDS.
+// in LDS.  A part of weight 0 is left out, not multiplied: what it holds may be infinite (a split's own keys decide),
+// and the places of the last batch behind the last split hold that split's part once more.
 template <bool BF16, int D, int GROUPS>
 __global__ void __launch_bounds__(256) fa_combine_splits(const FaKernelArgs a)
 {
@@ -346,6 +347,10 @@ __global__ void __launch_bounds__(256) fa_combine_splits(const FaKernelArgs a)
     const int n = a.n_splits;
     const float *lse_row = a.lse_part + row, *o_row = a.o_part + row * D + 4 * t;
     const size_t o_step = (size_t)n_rows * D;
+    auto weighted = [](f32x4 part, float w) __attribute__((always_inline)) {
+        const f32x4 none = {0.0f, 0.0f, 0.0f, 0.0f};
+        return w > 0.0f ? part * w : none;
+    };
     float m = kNoReference, l = 0.0f;             // running reference point and sum of weights
     f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
     for (int s0 = BATCH * group; s0 < n; s0 += BATCH * GROUPS) {
@@ -364,13 +369,13 @@ __global__ void __launch_bounds__(256) fa_combine_splits(const FaKernelArgs a)
             mx = fmaxf(mx, lse[u]);
         }
         const float alpha = __expf(m - mx);
-        acc *= alpha;
+        acc = weighted(acc, alpha);
         l *= alpha;
         m = mx;
 #pragma unroll
         for (int u = 0; u < BATCH; ++u) {
             const float w = __expf(lse[u] - mx);
-            acc += o[u] * w;
+            acc += weighted(o[u], w);
             l += w;
         }
     }
@@ -388,7 +393,7 @@ __global__ void __launch_bounds__(256) fa_combine_splits(const FaKernelArgs a)
 #pragma unroll
         for (int i = 0; i < GROUPS; ++i) {
             const float w = __expf(sm[r * GROUPS + i] - m);
-            acc += so[(r * GROUPS + i) * TPR + t] * w;
+            acc += weighted(so[(r * GROUPS + i) * TPR + t], w);
             l += sl[r * GROUPS + i] * w;
         }
     }

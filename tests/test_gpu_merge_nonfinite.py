@@ -1,0 +1,44 @@
+"""The merge of key splits where a part holds an infinity: only parts that carry weight reach the result."""
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(1, 4, 2, 1, 704, 64), (2, 4, 4, 3, 704, 128),          # the decoding kernel
+          (1, 4, 2, 200, 704, 64), (1, 2, 2, 200, 704, 128)]      # 128-row blocks
+
+
+def _inputs(torch, B, H, Hk, S, Skv, D):
+    g = torch.Generator(device="cuda").manual_seed(9)
+    q = torch.randn((B, H, S, D), device="cuda", generator=g).half()
+    k, v = (torch.randn((B, Hk, Skv, D), device="cuda", generator=g).half() for _ in range(2))
+    return q, k, v
+
+
+@pytest.mark.parametrize("splits", [3, 8, 11])        # a last batch of eight parts with five, no and five free places
+@pytest.mark.parametrize("B,H,Hk,S,Skv,D", SHAPES)
+def test_infinite_value_in_the_last_split(fa, B, H, Hk, S, Skv, D, splits):
+    import torch
+    q, k, v = _inputs(torch, B, H, Hk, S, Skv, D)
+    want, lse_want = fa.flash_attention_forward(q, k, v, splits=splits)
+    v[:, :, -1, 5] = float("inf")
+    got, lse = fa.flash_attention_forward(q, k, v, splits=splits)
+    torch.cuda.synchronize()
+    assert bool((got[..., 5] == float("inf")).all())
+    got[..., 5] = want[..., 5]
+    assert torch.equal(got, want) and torch.equal(lse, lse_want)
+
+
+@pytest.mark.parametrize("splits", [3, 8, 11])
+@pytest.mark.parametrize("B,H,Hk,S,Skv,D", SHAPES)
+def test_infinite_value_in_a_split_without_weight(fa, B, H, Hk, S, Skv, D, splits):
+    """The last key's score is two thousand above all others: every other split's weight is exactly zero, and the result
+    the last key's value, but for one rounding of the probability and one of the output to fp16 (2^-11 each)."""
+    import torch
+    q, k, v = _inputs(torch, B, H, Hk, S, Skv, D)
+    q[..., 3] = 8.0
+    k[:, :, -1, 3] = 2000.0 * D ** 0.5 / 8.0
+    v[:, :, 7, 5] = float("inf")
+    got, lse = fa.flash_attention_forward(q, k, v, splits=splits)
+    torch.cuda.synchronize()
+    want = v[:, :, -1:].repeat_interleave(H // Hk, 1).float()
+    assert bool(((got.float() - want).abs() <= 2.0 ** -9 * want.abs() + 1e-6).all()) and bool(torch.isfinite(lse).all())
