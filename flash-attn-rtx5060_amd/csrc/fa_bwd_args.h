@@ -32,6 +32,7 @@ struct FaBwdArgs {
     // Five-product form with the key blocks' walks cut into equal shares (fa_bwd_layout.h), or null: fp32 dK and dV of
     // the walks that were cut, FA_BWD_PARTS_PER_SHARE slots of 2 * 256 * D floats per share.
     float *partials;
+    int share_slots;                        // shares whose parts it holds
     int walk_head, walk_total;              // pairs in the walks of one K/V head and of all heads of the launch
     int S, Sk;                              // queries, keys; query i sits at key position i + Sk - S
     int L, R;                               // key j visible to the query at position p iff p - L <= j <= p + R

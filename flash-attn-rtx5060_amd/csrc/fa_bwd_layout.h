@@ -138,5 +138,22 @@ FA_LAYOUT_HD int fa_bwd_shares(int heads, int G, int S, int Lq, int Rq, int walk
     }
     return 3 * worst > 4 * (total / shares) + 9 + 18 * shares / 256 ? (int)shares : 0;
 }
+// The buffer of the parts is sized on the host without a device, for FA_BWD_SHARE_UNITS compute units (a whole MI355X):
+// the shares of the larger of the launches over a whole chunk of K/V heads and over the `rest` that is left (0: none).
+#define FA_BWD_SHARE_UNITS 256
+FA_LAYOUT_HD int fa_bwd_share_slots(int chunk, int rest, int G, int S, int Lq, int Rq, int walk_head)
+{
+    const int whole = fa_bwd_shares(chunk, G, S, Lq, Rq, walk_head, FA_BWD_SHARE_UNITS);
+    const int last = rest > 0 ? fa_bwd_shares(rest, G, S, Lq, Rq, walk_head, FA_BWD_SHARE_UNITS) : 0;
+    return whole > last ? whole : last;
+}
+// The shares of one launch: by the compute units of the device it runs on, which may cut what FA_BWD_SHARE_UNITS would
+// leave whole (a partition with 32 units: S 512, causal, chunks of 264 heads and a rest of 2, 32 shares where the buffer
+// holds 8), and none when the buffer has fewer slots than that.
+FA_LAYOUT_HD int fa_bwd_launch_shares(int heads, int G, int S, int Lq, int Rq, int walk_head, int compute_units, int slots)
+{
+    const int shares = fa_bwd_shares(heads, G, S, Lq, Rq, walk_head, compute_units);
+    return shares <= slots ? shares : 0;
+}
 
 #endif

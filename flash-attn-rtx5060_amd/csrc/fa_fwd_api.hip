@@ -852,6 +852,8 @@ int walk_pairs_per_head(int S, int G, int L, int R)
     for (int kb = 0; kb < (S + 255) / 256; ++kb) pairs += (long long)G * fa_bwd_walk_tiles(S, S, R, L, kb);
     return pairs <= 0x3fffffffLL ? (int)pairs : 0;
 }
+// fp32 dK and dV parts of one share
+unsigned long long bytes_per_share(const fa_bwd_params *p) { return FA_BWD_PARTS_PER_SHARE * 2ull * 256ull * (unsigned long long)p->d * 4ull; }
 }  // namespace
 
 unsigned long long fa_bwd_share_bytes(const fa_bwd_params *p)
@@ -865,10 +867,8 @@ unsigned long long fa_bwd_share_bytes(const fa_bwd_params *p)
     const int per_head = walk_pairs_per_head(p->S, G, L, R);
     // the launches: whole chunks and a smaller last one
     const int rest = (int)(kv_heads_total(p) % heads);
-    int shares = fa_bwd_shares(heads, G, p->S, R, L, per_head, kComputeUnits);
-    const int of_rest = rest != 0 ? fa_bwd_shares(rest, G, p->S, R, L, per_head, kComputeUnits) : 0;
-    if (of_rest > shares) shares = of_rest;
-    return (unsigned long long)shares * FA_BWD_PARTS_PER_SHARE * 2ull * 256ull * (unsigned long long)p->d * 4ull;
+    const int slots = fa_bwd_share_slots(heads, rest, G, p->S, R, L, per_head);
+    return (unsigned long long)slots * bytes_per_share(p);
 }
 
 int fa_bwd(const fa_bwd_params *p, void *stream) { return fa_bwd_shared(p, nullptr, 0, stream); }
@@ -901,6 +901,7 @@ int fa_bwd_shared(const fa_bwd_params *p, void *partials, unsigned long long par
     a.head0 = 0;
     a.heads = (int)kv_heads_total(p);
     a.partials = share_bytes != 0 ? static_cast<float *>(partials) : nullptr;
+    a.share_slots = a.partials != nullptr ? (int)(share_bytes / bytes_per_share(p)) : 0;
     a.walk_head = a.walk_total = 0;
     a.dQ = static_cast<uint16_t *>(p->dQ);
     a.dK = static_cast<uint16_t *>(p->dK);

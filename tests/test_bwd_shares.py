@@ -23,6 +23,17 @@ def test_shares_cover_every_walk_once():
     assert out.returncode == 0, out.stdout
 
 
+def test_launches_fit_the_buffer_of_the_parts():
+    """tests/c/check_bwd_share_slots.c: the shares of every launch against what fa_bwd_share_bytes sizes, for devices of
+    other compute unit counts as well."""
+    with tempfile.TemporaryDirectory() as tmp:
+        exe = os.path.join(tmp, "check_bwd_share_slots")
+        subprocess.run(["gcc", "-O2", "-Wall", "-Wextra", "-I", os.path.join(REPO, "flash-attn-rtx5060_amd", "csrc"),
+                        os.path.join(REPO, "tests", "c", "check_bwd_share_slots.c"), "-o", exe], check=True)
+        out = subprocess.run([exe], stdout=subprocess.PIPE, text=True)
+    assert out.returncode == 0, out.stdout
+
+
 def test_share_bytes_and_refusals(fa):
     import ctypes
     L = fa.lib()
