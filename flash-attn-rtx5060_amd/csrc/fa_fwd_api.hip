@@ -321,7 +321,56 @@ bool decode_problem(const fa_fwd_params *p, bool causal_type)
     if ((long long)(p->N / hk) * p->S > 32 || sk < p->S || fa_dropout_threshold(p->dropout_prob) != 0) return false;
     return !(causal_type && sk - p->S < 32 && packed_group(p) == 1 && !p->exact_first_rows);
 }
+// Workgroups of the tile kernels that a device keeps resident
+long long resident_groups(int compute_units, int waves) { return (long long)compute_units * (waves == 8 ? 1 : 2); }
+// How a call reaches the device: by the decoding kernel, whose workgroups (one per K/V head and key split) the hardware
+// hands out, with the streaming hint or without; else the schedule of the tile kernels' work items.
+struct Launch {
+    bool decode, streaming;
+    int sched;
+};
+Launch launch_of(const fa_fwd_params *p, int compute_units)
+{
+    const int sk = p->S_kv > 0 ? p->S_kv : p->S, hk = p->n_kv_heads > 0 ? p->n_kv_heads : p->N;
+    const int s_max = sk > p->S ? sk : p->S, waves = waves_of(p), pack = packed_group(p);
+    int L, R;
+    fa_mask_bounds(s_max, p->is_causal, p->window_size_left, p->window_size_right, &L, &R);
+    Launch l;
+    l.decode = decode_problem(p, R == 0);
+    // (the streaming hint from where K and V do not stay in the 256 MB memory-side cache: measured beside the kernel)
+    l.streaming = l.decode && (double)p->B * hk * sk * p->d * 4.0 > 128e6;
+    // FA_SCHED_AUTO: with at most one item per resident workgroup there is nothing to schedule (and the
+    // queue's counter round trips, 2.3 us each, would double the run time of a 7 us problem).  With fewer than
+    // eight items per workgroup the fixed snake wins: it pairs every long item with a short one, knows its next
+    // item without asking, and its items' loads can be requested before the current item's epilogue without a
+    // counter in between -- causal fp16 problems, snake against queue: B8 H32 S1024 D64 (four items per workgroup)
+    // 67 against 100 us, B4 H32 S2048 D64 (four) 111 against 138, B2 H32 S4096 D128 (four) 290 against 312, c2 (two)
+    // 611 against 448 TFLOP/s.  At eight per workgroup the two are level (c3 1016 against 1018 TFLOP/s, B1 H32 S16384
+    // 2097 us both); beyond, the queue's balancing is worth more than its counters cost (c5, 32 items per workgroup:
+    // 16.2 against 17.0 ms; B8 H32 S8192 D64 2.75 against 2.80 ms).
+    l.sched = p->sched;
+    // Items that are all alike (no mask, or a window of at most half the length: all but the first few query blocks
+    // of a head see the same number of tiles) need no balancing either, and the fixed order saves them the
+    // counters' barriers: c4 766 against 748 TFLOP/s, c3's shape without a mask 1101 against 1096.
+    if (l.sched == FA_SCHED_AUTO) {
+        const long long blocks = pack > 1 ? 1 : (p->S + 32 * waves - 1) / (32 * waves);
+        const long long items = (long long)p->B * p->N / pack * blocks * effective_splits(p), resident = resident_groups(compute_units, waves);
+        const bool alike = !(L < s_max || R < s_max) || 2LL * L <= (long long)p->S;
+        l.sched = items <= resident ? FA_SCHED_DISPATCH : (items < 8 * resident || alike) ? FA_SCHED_PERSISTENT : FA_SCHED_QUEUE;
+    }
+    return l;
+}
 }  // namespace
+
+int fa_sched_launch(const fa_fwd_params *p, int compute_units, int *decoding, int *streaming)
+{
+    const int st = fa_fwd_validate(p);
+    if (st != FA_OK) return st;
+    const Launch l = launch_of(p, compute_units);
+    if (decoding) *decoding = l.decode;
+    if (streaming) *streaming = l.streaming;
+    return l.decode ? FA_SCHED_DISPATCH : l.sched;
+}
 
 unsigned long long fa_fwd_workspace_bytes(const fa_fwd_params *p)
 {
@@ -508,41 +557,12 @@ int forward(const fa_fwd_params *p, void *workspace, const FaDeviceState *ds, vo
     a.scale_log2e = p->softmax_scale * 1.44269504088896340736f;
     a.n_items = (long long)(a.BH / a.pack) * a.n_qblocks * a.n_splits;
 
-    // Dispatch mode launches one workgroup per item, in list order; the hardware hands them to CUs as these
-    // free up, which is a longest-first greedy schedule.  Persistent mode launches one resident set of
-    // workgroups that walk the list themselves.
-    long long grid = a.n_items;
-    a.queue = nullptr;
-    const long long resident = (long long)ds->compute_units * (waves == 8 ? 1 : 2);
-    // FA_SCHED_AUTO: with at most one item per resident workgroup there is nothing to schedule (and the
-    // queue's counter round trips, 2.3 us each, would double the run time of a 7 us problem).  With fewer than
-    // eight items per workgroup the fixed snake wins: it pairs every long item with a short one, knows its next
-    // item without asking, and its items' loads can be requested before the current item's epilogue without a
-    // counter in between -- causal fp16 problems, snake against queue: B8 H32 S1024 D64 (four items per workgroup)
-    // 67 against 100 us, B4 H32 S2048 D64 (four) 111 against 138, B2 H32 S4096 D128 (four) 290 against 312, c2 (two)
-    // 611 against 448 TFLOP/s.  At eight per workgroup the two are level (c3 1016 against 1018 TFLOP/s, B1 H32 S16384
-    // 2097 us both); beyond, the queue's balancing is worth more than its counters cost (c5, 32 items per workgroup:
-    // 16.2 against 17.0 ms; B8 H32 S8192 D64 2.75 against 2.80 ms).
-    int sched = p->sched;
-    // Items that are all alike (no mask, or a window of at most half the length: all but the first few query blocks
-    // of a head see the same number of tiles) need no balancing either, and the fixed order saves them the
-    // counters' barriers: c4 766 against 748 TFLOP/s, c3's shape without a mask 1101 against 1096.
-    if (sched == FA_SCHED_AUTO) {
-        const bool alike = !a.descending || 2LL * a.L <= (long long)p->S;
-        sched = a.n_items <= resident ? FA_SCHED_DISPATCH : (a.n_items < 8 * resident || alike) ? FA_SCHED_PERSISTENT : FA_SCHED_QUEUE;
-    }
-    if (sched == FA_SCHED_PERSISTENT || sched == FA_SCHED_QUEUE) {
-        if (grid > resident) grid = resident;
-        if (sched == FA_SCHED_QUEUE) a.queue = work_queue_for_launch(ds, static_cast<hipStream_t>(stream));
-    }
-    const bool decode = decode_problem(p, a.R == 0);
+    const Launch launch = launch_of(p, ds->compute_units);
     auto launch_decode = [&]() {
         a.pack = p->N / a.Hk;
         const long long heads = (long long)p->B * a.Hk;
         a.n_items = heads * a.n_splits;
-        // (the streaming hint from where K and V do not stay in the 256 MB memory-side cache: measured beside the kernel)
-        const int streaming = heads * a.Sk * p->d * 4.0 > 128e6 ? 1 : 0;
-        hipError_t e = fa_launch_forward_decode(a, p->dtype == FA_DTYPE_BF16, p->d, a.pack * p->S, streaming, static_cast<hipStream_t>(stream));
+        hipError_t e = fa_launch_forward_decode(a, p->dtype == FA_DTYPE_BF16, p->d, a.pack * p->S, launch.streaming ? 1 : 0, static_cast<hipStream_t>(stream));
         if (e != hipSuccess) return device_fail(e, "decode launch");
         if (a.n_splits > 1) {
             e = fa_launch_combine_splits(a, p->dtype == FA_DTYPE_BF16, p->d, static_cast<hipStream_t>(stream));
@@ -551,8 +571,18 @@ int forward(const fa_fwd_params *p, void *workspace, const FaDeviceState *ds, vo
         return (int)FA_OK;
     };
 #ifndef FA_CHECK_RING
-    if (decode) return launch_decode();
+    if (launch.decode) return launch_decode();      // (before a work queue is asked for: this kernel uses none)
 #endif      // (the checking build runs the tile kernels, whose ring it checks, on these problems as well, in front)
+    // Dispatch mode launches one workgroup per item, in list order; the hardware hands them to CUs as these
+    // free up, which is a longest-first greedy schedule.  Persistent mode launches one resident set of
+    // workgroups that walk the list themselves.
+    long long grid = a.n_items;
+    a.queue = nullptr;
+    if (launch.sched == FA_SCHED_PERSISTENT || launch.sched == FA_SCHED_QUEUE) {
+        const long long resident = resident_groups(ds->compute_units, waves);
+        if (grid > resident) grid = resident;
+        if (launch.sched == FA_SCHED_QUEUE) a.queue = work_queue_for_launch(ds, static_cast<hipStream_t>(stream));
+    }
     const int shape = waves == 8 ? 0 : 1;
     // dropout: p in units of 1/256 (a key is kept iff its random byte is >= the threshold)
     a.drop_threshold = (unsigned)fa_dropout_threshold(p->dropout_prob);
@@ -573,7 +603,7 @@ int forward(const fa_fwd_params *p, void *workspace, const FaDeviceState *ds, vo
         if (e != hipSuccess) return device_fail(e, "combine launch");
     }
 #ifdef FA_CHECK_RING
-    if (decode) return launch_decode();
+    if (launch.decode) return launch_decode();
 #endif
     return FA_OK;
 }

@@ -91,7 +91,7 @@ typedef struct fa_fwd_params {
     /* --- beyond mykernelParamType --- */
     int dtype;                /* FA_DTYPE_F16 / FA_DTYPE_BF16                                 */
     int is_causal;            /* keys with j > i are masked (mask.h:27-38)                    */
-    int sched;                /* FA_SCHED_*                                                   */
+    int sched;                /* FA_SCHED_*; without effect where the decoding kernel runs (fa_sched_launch) */
     /* --- layouts beyond the reference's contiguous [B,N,S,d] (main.cu:182); all zero = that layout --- */
     int n_kv_heads;           /* K/V heads per batch entry, 0 = N.  Must divide N: query head h reads K/V
                                  head h / (N / n_kv_heads) (grouped-query / multi-query attention)      */
@@ -236,6 +236,11 @@ int fa_sched_item(int B, int N, int S, int d, int is_causal, int window_left,
  * n_kv_heads = 0 or N the position is the head.  No counterpart in the reference, which has one K/V head per
  * query head (flash_forward.h:378-381). */
 int fa_sched_heads(int N, int n_kv_heads, int bh, int *batch, int *q_head, int *kv_head);
+/* How a call with these parameters reaches a device of `compute_units`: the schedule of its work items
+ * (FA_SCHED_DISPATCH, _PERSISTENT or _QUEUE), or a negative status for parameters that fa_fwd refuses.  *decoding
+ * (may be NULL): the decoding kernel runs it, one workgroup per K/V head and key split that the hardware hands out
+ * (FA_SCHED_DISPATCH), and *streaming: that kernel reads K and V with the non-temporal hint. */
+int fa_sched_launch(const fa_fwd_params *p, int compute_units, int *decoding, int *streaming);
 /* Key-tile range [*tile_lo, *tile_hi] (inclusive) visited for query rows
  * [q_begin, q_begin + rows).  Same clipping as flash_forward.h:52-61. */
 void fa_sched_tile_range(int S, int block_keys, int is_causal, int window_left,

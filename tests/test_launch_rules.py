@@ -1,0 +1,33 @@
+"""Which way a call reaches the device (fa_sched_launch, the rule the launch itself asks), on the host."""
+import ctypes
+
+import pytest
+
+CUS = 256
+
+
+def launch(fa, B, H, Hk, S, Skv, D, causal=True, wl=-1, splits=1, sched=0, cus=CUS, strides=None):
+    """(schedule, decoding kernel, streaming hint)"""
+    p = fa.make_params(B, H, S, D, 0x1000, 0x2000, 0x3000, 0x4000, causal=causal, window_left=wl, n_kv_heads=0 if Hk == H else Hk,
+                       S_kv=0 if Skv == S else Skv, split_num=splits, workspace_ptr=0x5000, workspace_bytes=1 << 62, sched=sched,
+                       **(strides or {}))
+    dec, nt = ctypes.c_int(-1), ctypes.c_int(-1)
+    st = fa.lib().fa_sched_launch(ctypes.byref(p), cus, ctypes.byref(dec), ctypes.byref(nt))
+    return st, dec.value, nt.value
+
+
+def test_schedules_of_the_tile_kernels(fa):
+    """At most one item per resident workgroup, fewer than eight, more; a named schedule; refusals."""
+    assert launch(fa, 1, 4, 4, 512, 512, 64)[:2] == (fa.FA_SCHED_DISPATCH, 0)
+    assert launch(fa, 4, 16, 16, 2048, 2048, 64)[:2] == (fa.FA_SCHED_PERSISTENT, 0)
+    assert launch(fa, 2, 32, 32, 8192, 8192, 128)[:2] == (fa.FA_SCHED_QUEUE, 0)
+    assert launch(fa, 2, 32, 32, 8192, 8192, 128, causal=False)[:2] == (fa.FA_SCHED_PERSISTENT, 0)
+    assert launch(fa, 1, 4, 4, 512, 512, 64, sched=fa.FA_SCHED_QUEUE)[0] == fa.FA_SCHED_QUEUE
+    assert launch(fa, 1, 4, 3, 512, 512, 64)[0] == fa.FA_ERR_LAYOUT
+
+
+@pytest.mark.parametrize("sched", [0, 1, 2, 3])
+def test_decoding_takes_no_work_queue(fa, sched):
+    """Causal decoding with as many items as would make the tile kernels balance through a queue, and with a queue asked for."""
+    assert launch(fa, 64, 32, 32, 1, 2048, 128, splits=2, sched=sched)[:2] == (fa.FA_SCHED_DISPATCH, 1)
+    assert launch(fa, 512, 16, 16, 1, 2048, 128, sched=sched)[:2] == (fa.FA_SCHED_DISPATCH, 1)
