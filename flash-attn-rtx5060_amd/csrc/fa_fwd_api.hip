@@ -314,10 +314,13 @@ int effective_splits(const fa_fwd_params *p)
     return p->split_num < tiles ? p->split_num : tiles;
 }
 // Whether the decoding kernel (fa_fwd_decode.hip) takes the problem: every query row of a K/V head fits its 32.
-// (Rows that the default forward computes in the verifier's arithmetic, and dropout, belong to the tile kernels.)
-bool decode_problem(const fa_fwd_params *p, bool causal_type)
+// (Rows that the default forward computes in the verifier's arithmetic, and dropout, belong to the tile kernels.  So do
+// 2^24 and more K/V heads times `splits`: a workgroup each, of 256 threads, and a launch has fewer than 2^32 of them.)
+constexpr long long kDecodeMostGroups = (1LL << 24) - 1;
+bool decode_problem(const fa_fwd_params *p, bool causal_type, int splits)
 {
     const int hk = p->n_kv_heads > 0 ? p->n_kv_heads : p->N, sk = p->S_kv > 0 ? p->S_kv : p->S;
+    if ((long long)p->B * hk * splits > kDecodeMostGroups) return false;
     if ((long long)(p->N / hk) * p->S > 32 || sk < p->S || fa_dropout_threshold(p->dropout_prob) != 0) return false;
     return !(causal_type && sk - p->S < 32 && packed_group(p) == 1 && !p->exact_first_rows);
 }
@@ -336,7 +339,7 @@ Launch launch_of(const fa_fwd_params *p, int compute_units)
     int L, R;
     fa_mask_bounds(s_max, p->is_causal, p->window_size_left, p->window_size_right, &L, &R);
     Launch l;
-    l.decode = decode_problem(p, R == 0);
+    l.decode = decode_problem(p, R == 0, effective_splits(p));
     // (the streaming hint from where K and V do not stay in the 256 MB memory-side cache: measured beside the kernel)
     l.streaming = l.decode && (double)p->B * hk * sk * p->d * 4.0 > 128e6;
     // FA_SCHED_AUTO: with at most one item per resident workgroup there is nothing to schedule (and the
@@ -404,7 +407,7 @@ int fa_fwd_auto_splits(const fa_fwd_params *p)
     const int s_max = sk > p->S ? sk : p->S;
     int L, R;
     fa_mask_bounds(s_max, p->is_causal, p->window_size_left, p->window_size_right, &L, &R);
-    if (!decode_problem(p, R == 0)) {
+    if (!decode_problem(p, R == 0, 1)) {
         // The tile kernels, 128-row blocks, queries behind a cache (what else ran is left at the count that fills the device):
         // the least estimated time as well.  Workgroups per compute unit times (key tiles of a split, 0.85 us each at head
         // dimension 128 and 0.55 at 64, + 1.4), 1.4 of that per workgroup where a unit has only one; a second launch costs
@@ -442,6 +445,7 @@ int fa_fwd_auto_splits(const fa_fwd_params *p)
     if (most > key_tiles(p)) most = key_tiles(p);
     const long long loaded = (4LL * kComputeUnits + heads - 1) / heads;         // beyond four workgroups per CU: up to eight splits
     if (most > (loaded > 8 ? loaded : 8)) most = loaded > 8 ? loaded : 8;
+    if (most * heads > kDecodeMostGroups) most = kDecodeMostGroups / heads;
     const double base = heads * (double)visible * p->d * 4.0 / 6.5e6, partial = (double)p->B * p->N * p->S * p->d * 8.0 / 5e6;
     long long best = 1;
     double best_us = 0.0;

@@ -31,3 +31,17 @@ def test_decoding_takes_no_work_queue(fa, sched):
     """Causal decoding with as many items as would make the tile kernels balance through a queue, and with a queue asked for."""
     assert launch(fa, 64, 32, 32, 1, 2048, 128, splits=2, sched=sched)[:2] == (fa.FA_SCHED_DISPATCH, 1)
     assert launch(fa, 512, 16, 16, 1, 2048, 128, sched=sched)[:2] == (fa.FA_SCHED_DISPATCH, 1)
+
+
+def test_decoding_grid_stays_below_2_to_the_32_threads(fa):
+    """One 256-thread workgroup per K/V head and split: from 2^24 of them on the tile kernels take the call, and "auto"
+    never splits a decoding call beyond that."""
+    heads = 1 << 23
+    assert launch(fa, heads // 8, 8, 8, 1, 1, 64, causal=False)[1] == 1
+    assert launch(fa, heads // 8, 8, 8, 1, 512, 64, splits=2)[:2] == (fa.FA_SCHED_QUEUE, 0)
+    assert launch(fa, heads // 8 - 1, 8, 8, 1, 512, 64, splits=2)[1] == 1
+    assert launch(fa, heads // 4, 8, 8, 1, 1, 64, causal=False)[:2] == (fa.FA_SCHED_PERSISTENT, 0)
+    for b in (heads // 8, heads // 24, heads // 9):
+        p = fa.make_params(b, 8, 1, 64, causal=True, S_kv=4096)
+        n = fa.lib().fa_fwd_auto_splits(ctypes.byref(p))
+        assert n >= 1 and launch(fa, b, 8, 8, 1, 4096, 64, splits=n)[1] == 1
