@@ -464,8 +464,8 @@ hipError_t fa_configure_forward_decode()
 hipError_t fa_launch_combine_splits(const FaKernelArgs &a, int bf16, int D, hipStream_t stream)
 {
     const long long n_rows = (long long)a.BH * a.S;
-    const int groups = a.n_splits > 8 ? 8 : 1;
-    const int rows_per_block = 256 / (D / 4 * groups);
+    const int groups = fa_combine_groups(n_rows, D, a.n_splits);
+    const int rows_per_block = fa_combine_rows(D, groups);
     const unsigned grid = (unsigned)((n_rows + rows_per_block - 1) / rows_per_block);
 #define FA_COMBINE(BF, DD, GR) \
     if (bf16 == BF && D == DD && groups == GR) hipLaunchKernelGGL((fa_combine_splits<BF != 0, DD, GR>), dim3(grid), dim3(256), 0, stream, a);

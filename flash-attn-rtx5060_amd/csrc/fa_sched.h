@@ -102,4 +102,14 @@ FA_HD int fa_strided_heads(int bh, int H, int Hk, int *hi, int *hk)
     return (int)bi;
 }
 
+// Threads that share four output elements of a row in the merge of key splits: eight where a thread alone would make
+// more than one trip to memory (more than eight splits), as long as the launch stays below 2^32 threads, which it does
+// up to 2^24 rows at head dimension 128; so many rows fill the chip without sharing.
+FA_HD int fa_combine_groups(long long n_rows, int D, int n_splits)
+{
+    return n_splits > 8 && n_rows < (1LL << 32) / (D / 4 * 8) - 256 ? 8 : 1;
+}
+// Rows per workgroup of 256 threads
+FA_HD int fa_combine_rows(int D, int groups) { return 256 / (D / 4 * groups); }
+
 #endif

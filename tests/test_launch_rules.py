@@ -1,9 +1,12 @@
 """Which way a call reaches the device (fa_sched_launch, the rule the launch itself asks), on the host."""
 import ctypes
+import os
+import subprocess
 
 import pytest
 
 CUS = 256
+REPO = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
 def launch(fa, B, H, Hk, S, Skv, D, causal=True, wl=-1, splits=1, sched=0, cus=CUS, strides=None):
@@ -45,3 +48,12 @@ def test_decoding_grid_stays_below_2_to_the_32_threads(fa):
         p = fa.make_params(b, 8, 1, 64, causal=True, S_kv=4096)
         n = fa.lib().fa_fwd_auto_splits(ctypes.byref(p))
         assert n >= 1 and launch(fa, b, 8, 8, 1, 4096, 64, splits=n)[1] == 1
+
+
+def test_grid_of_the_merge_of_key_splits(tmp_path):
+    """tests/c/check_combine_grid.c: every row covered, fewer than 2^32 threads."""
+    exe = str(tmp_path / "check_combine_grid")
+    subprocess.run(["gcc", "-O2", "-Wall", "-Wextra", "-I", os.path.join(REPO, "flash-attn-rtx5060_amd", "csrc"),
+                    os.path.join(REPO, "tests", "c", "check_combine_grid.c"), "-o", exe], check=True)
+    out = subprocess.run([exe], stdout=subprocess.PIPE, text=True)
+    assert out.returncode == 0, out.stdout
