@@ -250,10 +250,11 @@ def abi_strides(t):
     return t, tuple(norm)
 
 
-# What a call needs besides its pointers follows from shapes, strides, types and options: it is worked out once per such
-# combination and kept (a small call's time was this Python code: B1 H4 S256 D64 11.4 us a call around a 7 us kernel, one
-# new token behind 1003 keys 16.5 around 9).  The entries hold sizes and a filled parameter block as bytes, never a tensor,
-# an address or an object's identity; they are made only from calls that succeeded with plain numbers for options.
+# What a call needs besides its pointers and its dropout seed (another one in every step of a training) follows from shapes,
+# strides, types and the other options: it is worked out once per such combination and kept (a small call's time was this
+# Python code: B1 H4 S256 D64 11.4 us a call around a 7 us kernel, one new token behind 1003 keys 16.5 around 9).  The
+# entries hold sizes and a filled parameter block as bytes, never a tensor, an address or an object's identity; they are
+# made only from calls that succeeded with plain numbers for options.
 _plans = {}
 _PLANS_MAX = 1024
 _PLAIN = frozenset((int, float, bool, str, type(None)))
@@ -303,14 +304,14 @@ def flash_attention_forward(q, k, v, softmax_scale=None, causal=False, window_le
             {type(softmax_scale), type(causal), type(return_lse), type(dropout_prob), type(splits), type(exact_first_rows),
              type(static_scratch)} <= _PLAIN):
         key = (q.shape, q.stride(), q.dtype, q.device, k.shape, k.stride(), k.dtype, k.device, v.shape, v.stride(), v.dtype, v.device,
-               softmax_scale, causal, window_left, window_right, return_lse, sched, dropout_prob, seed, splits, exact_first_rows,
+               softmax_scale, causal, window_left, window_right, return_lse, sched, dropout_prob, splits, exact_first_rows,
                static_scratch, _slopes_key(alibi_slopes))
         plan = _plans.get(key)
         if plan is not None:
             block, lse_shape, need, entry = plan
             p = FaFwdParams.from_buffer_copy(block)
             out = torch.empty_like(q)
-            p.Q, p.K, p.V, p.O = q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr()
+            p.Q, p.K, p.V, p.O, p.seed = q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), seed
             if return_lse:
                 lse = torch.empty(lse_shape, dtype=torch.float32, device=q.device)
                 p.L = lse.data_ptr()
@@ -413,7 +414,7 @@ def flash_attention_backward(q, k, v, o, lse, do, softmax_scale=None, causal=Fal
             {type(window_left), type(window_right), type(seed)} <= _WHOLE and {type(softmax_scale), type(causal), type(dropout_prob)} <= _PLAIN):
         key = (q.shape, q.stride(), q.dtype, q.device, k.shape, k.stride(), k.dtype, k.device, v.shape, v.stride(), v.dtype, v.device,
                o.shape, o.stride(), o.dtype, o.device, do.shape, do.stride(), do.dtype, do.device, lse.shape, lse.stride(), lse.dtype, lse.device,
-               softmax_scale, causal, window_left, window_right, dropout_prob, seed, _slopes_key(alibi_slopes))
+               softmax_scale, causal, window_left, window_right, dropout_prob, _slopes_key(alibi_slopes))
         plan = _plans.get(key)
         workspace = None
         if plan is not None:
@@ -426,7 +427,7 @@ def flash_attention_backward(q, k, v, o, lse, do, softmax_scale=None, causal=Fal
             p = FaBwdParams.from_buffer_copy(block)
             dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
             p.Q, p.K, p.V, p.O, p.dO, p.L = q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), do.data_ptr(), lse.data_ptr()
-            p.dQ, p.dK, p.dV = dq.data_ptr(), dk.data_ptr(), dv.data_ptr()
+            p.dQ, p.dK, p.dV, p.seed = dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), seed
             at = workspace.data_ptr()
             p.workspace = at
             if alibi_slopes is not None:

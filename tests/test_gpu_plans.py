@@ -42,6 +42,27 @@ def test_second_call_equals_the_first(fa, kw, bshd):
         assert torch.equal(a.contiguous().view(torch.uint8), b.contiguous().view(torch.uint8))
 
 
+def test_seeds_share_an_entry(fa):
+    """A training with dropout has another seed every step: one entry for the forward and one for the backward pass serve
+    them all, each with its own mask."""
+    import torch
+    q, k, v, do = _inputs(torch, 3, False)
+    results = []
+    for kept in (False, True):
+        fa._plans.clear()
+        for seed in (7, 0, (1 << 64) - 1, 8):
+            if not kept:
+                fa._plans.clear()
+            kw = dict(dropout_prob=0.2, seed=seed)
+            o, lse = fa.flash_attention_forward(q, k, v, exact_first_rows=True, **kw)
+            results.append((o,) + fa.flash_attention_backward(q, k, v, o, lse, do, **kw))
+    assert len(fa._plans) == 2
+    torch.cuda.synchronize()
+    for a, b in zip(results[:4], results[4:]):
+        assert all(torch.equal(x.view(torch.int16), y.view(torch.int16)) for x, y in zip(a, b))
+    assert not any(torch.equal(results[0][0], r[0]) for r in results[1:4])
+
+
 def test_what_was_refused_stays_refused(fa):
     import torch
     q, k, v, _ = _inputs(torch, 1, False)
