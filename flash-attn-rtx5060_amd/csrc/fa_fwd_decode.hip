@@ -351,7 +351,9 @@ __global__ void __launch_bounds__(256) fa_combine_splits(const FaKernelArgs a)
         const f32x4 none = {0.0f, 0.0f, 0.0f, 0.0f};
         return w > 0.0f ? part * w : none;
     };
-    float m = kNoReference, l = 0.0f;             // running reference point and sum of weights
+    // running reference point and sum of weights (logsumexps are scaled scores, of any size: kNoReference is one for raw
+    // scores; from the lowest finite number the differences below are never NaN)
+    float m = -__FLT_MAX__, l = 0.0f;
     f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
     for (int s0 = BATCH * group; s0 < n; s0 += BATCH * GROUPS) {
         float lse[BATCH];

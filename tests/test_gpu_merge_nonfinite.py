@@ -1,4 +1,5 @@
-"""The merge of key splits where a part holds an infinity: only parts that carry weight reach the result."""
+"""The merge of key splits where a part holds an infinity -- only parts that carry weight reach the result -- and where the
+logsumexps are far from zero."""
 import pytest
 
 pytestmark = pytest.mark.gpu
@@ -42,3 +43,21 @@ def test_infinite_value_in_a_split_without_weight(fa, B, H, Hk, S, Skv, D, split
     torch.cuda.synchronize()
     want = v[:, :, -1:].repeat_interleave(H // Hk, 1).float()
     assert bool(((got.float() - want).abs() <= 2.0 ** -9 * want.abs() + 1e-6).all()) and bool(torch.isfinite(lse).all())
+
+
+@pytest.mark.parametrize("sign", [1.0, -1.0])
+@pytest.mark.parametrize("B,H,Hk,S,Skv,D", SHAPES)
+def test_logsumexps_of_any_size(fa, B, H, Hk, S, Skv, D, sign):
+    """All scores alike, a power of two of about 1e32 or its negative (exact in fp32, and so is the difference of two of
+    them): the values, alike for all keys of a head, come back as they are."""
+    import torch
+    q, k, v = _inputs(torch, B, H, Hk, S, Skv, D)
+    q.fill_(8.0)
+    k.fill_(8.0 * sign)
+    v.copy_(v[:, :, :1].expand_as(v).clone())
+    for splits in (3, 11):
+        got, lse = fa.flash_attention_forward(q, k, v, softmax_scale=2.0 ** 95, splits=splits)
+        torch.cuda.synchronize()
+        want = v[:, :, :1].repeat_interleave(H // Hk, 1).expand_as(got).float()
+        assert bool(((got.float() - want).abs() <= 2.0 ** -10 * want.abs()).all())
+        assert bool((lse == sign * 64.0 * D * 2.0 ** 95).all())
