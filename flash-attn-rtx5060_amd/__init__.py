@@ -419,13 +419,13 @@ def flash_attention_backward(q, k, v, o, lse, do, softmax_scale=None, causal=Fal
         workspace = None
         if plan is not None:
             block, total, parts_at, parts = plan
+            dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)  # (first: they need no less when memory is short)
             try:
                 workspace = torch.empty(total, dtype=torch.uint8, device=q.device)      # stream-ordered: freed after the launch
             except torch.cuda.OutOfMemoryError:
-                pass                                                                    # (the smaller sizes are tried below)
+                dq = dk = dv = None                                                     # (the smaller sizes are tried below)
         if workspace is not None:
             p = FaBwdParams.from_buffer_copy(block)
-            dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
             p.Q, p.K, p.V, p.O, p.dO, p.L = q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), do.data_ptr(), lse.data_ptr()
             p.dQ, p.dK, p.dV, p.seed = dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), seed
             at = workspace.data_ptr()

@@ -63,6 +63,44 @@ def test_seeds_share_an_entry(fa):
     assert not any(torch.equal(results[0][0], r[0]) for r in results[1:4])
 
 
+def test_backward_with_an_entry_when_memory_is_short(fa, monkeypatch):
+    """Room for the gradients and the small workspace, or for the kept entry's workspace alone: the call takes the smaller
+    workspace, as it does without an entry.  (The limit is counted here; the device has memory enough.)"""
+    import torch
+    import weakref
+    q, k, v, do = _inputs(torch, 4, False, B=1, H=8, Hk=8, S=512)
+    o, lse = fa.flash_attention_forward(q, k, v, exact_first_rows=True)
+    fa._plans.clear()
+    want = fa.flash_attention_backward(q, k, v, o, lse, do)
+    (_, total, _, _), = fa._plans.values()
+    limit, used = total + (1 << 20), [0]
+    assert total > (2 << 20) and 3 * q.numel() * 2 > (1 << 20)
+
+    def counted(make):
+        def wrapper(*args, **kw):
+            t = make(*args, **kw)
+            n = t.numel() * t.element_size()
+            if used[0] + n > limit:
+                raise torch.cuda.OutOfMemoryError("limit of this test")
+            used[0] += n
+            weakref.finalize(t, lambda: used.__setitem__(0, used[0] - n))
+            return t
+        return wrapper
+
+    got = []
+    for kept in (False, True):
+        if not kept:
+            plan = dict(fa._plans)
+            fa._plans.clear()
+        with monkeypatch.context() as m:
+            m.setattr(torch, "empty", counted(torch.empty))
+            m.setattr(torch, "empty_like", counted(torch.empty_like))
+            got.append([x.clone() for x in fa.flash_attention_backward(q, k, v, o, lse, do)])
+        fa._plans.update(plan)
+    for a, b, w in zip(*got, want):
+        assert torch.equal(a, b) and (a.float() - w.float()).norm() <= 2e-3 * w.float().norm()      # (each is within 1e-3 of the exact gradients)
+
+
 def test_what_was_refused_stays_refused(fa):
     import torch
     q, k, v, _ = _inputs(torch, 1, False)
