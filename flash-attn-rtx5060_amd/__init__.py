@@ -280,10 +280,14 @@ def _slopes_key(alibi_slopes):
     return None if alibi_slopes is None else (alibi_slopes.shape, alibi_slopes.stride(), alibi_slopes.dtype, alibi_slopes.device)
 
 
-def _keep_plan(key, plan):
+def _keep_plan(key, p, *rest):
+    block = type(p).from_buffer_copy(p)
+    for name, kind in p._fields_:
+        if kind is ctypes.c_void_p:
+            setattr(block, name, None)      # (every call sets its own)
     if len(_plans) >= _PLANS_MAX:
         _plans.clear()
-    _plans[key] = plan
+    _plans[key] = (bytes(block),) + rest
 
 
 def flash_attention_forward(q, k, v, softmax_scale=None, causal=False, window_left=-1, window_right=-1,
@@ -369,7 +373,7 @@ def flash_attention_forward(q, k, v, softmax_scale=None, causal=False, window_le
     if st != FA_OK:
         raise FaError(st, lib().fa_last_device_error().decode() if st == FA_ERR_DEVICE else "")
     if key is not None and q is given[0] and k is given[1] and v is given[2]:         # (no dense copy was needed)
-        _keep_plan(key, (bytes(p), (B, N, S), 0 if workspace is None else p.workspace_bytes, entry))
+        _keep_plan(key, p, (B, N, S), 0 if workspace is None else p.workspace_bytes, entry)
     return (out, lse) if return_lse else out
 
 
@@ -518,7 +522,7 @@ def flash_attention_backward(q, k, v, o, lse, do, softmax_scale=None, causal=Fal
     if st != FA_OK:
         raise FaError(st, lib().fa_last_device_error().decode() if st == FA_ERR_DEVICE else "")
     if key is not None and first_choice:
-        _keep_plan(key, (bytes(p), workspace.numel(), parts_at, parts))
+        _keep_plan(key, p, workspace.numel(), parts_at, parts)
     return dq, dk, dv
 
 

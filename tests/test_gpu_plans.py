@@ -63,6 +63,21 @@ def test_seeds_share_an_entry(fa):
     assert not any(torch.equal(results[0][0], r[0]) for r in results[1:4])
 
 
+def test_entries_hold_no_address(fa):
+    import ctypes
+    import torch
+    fa._plans.clear()
+    q, k, v, do = _inputs(torch, 5, True)
+    slopes = torch.tensor([0.5, 0.25, 0.1, 0.0], device="cuda")
+    o, lse = fa.flash_attention_forward(q, k, v, exact_first_rows=True, splits=3, alibi_slopes=slopes)
+    fa.flash_attention_backward(q, k, v, o, lse, do, alibi_slopes=slopes)
+    assert len(fa._plans) == 2
+    for entry in fa._plans.values():
+        kind = fa.FaFwdParams if len(entry[0]) == ctypes.sizeof(fa.FaFwdParams) else fa.FaBwdParams
+        block = kind.from_buffer_copy(entry[0])
+        assert [n for n, t in kind._fields_ if t is ctypes.c_void_p and getattr(block, n)] == []
+
+
 def test_backward_with_an_entry_when_memory_is_short(fa, monkeypatch):
     """Room for the gradients and the small workspace, or for the kept entry's workspace alone: the call takes the smaller
     workspace, as it does without an entry.  (The limit is counted here; the device has memory enough.)"""
