@@ -340,8 +340,10 @@ Launch launch_of(const fa_fwd_params *p, int compute_units)
     fa_mask_bounds(s_max, p->is_causal, p->window_size_left, p->window_size_right, &L, &R);
     Launch l;
     l.decode = decode_problem(p, R == 0, effective_splits(p));
-    // (the streaming hint from where K and V do not stay in the 256 MB memory-side cache: measured beside the kernel)
-    l.streaming = l.decode && (double)p->B * hk * sk * p->d * 4.0 > 128e6;
+    // (the streaming hint from where the K and V that are read -- under a left window the last S + L keys -- do not stay in
+    // the 256 MB memory-side cache: measured beside the kernel)
+    const long long visible = (long long)p->S + L < sk ? (long long)p->S + L : sk;
+    l.streaming = l.decode && (double)p->B * hk * (double)visible * p->d * 4.0 > 128e6;
     // FA_SCHED_AUTO: with at most one item per resident workgroup there is nothing to schedule (and the
     // queue's counter round trips, 2.3 us each, would double the run time of a 7 us problem).  With fewer than
     // eight items per workgroup the fixed snake wins: it pairs every long item with a short one, knows its next

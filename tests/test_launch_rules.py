@@ -50,6 +50,15 @@ def test_decoding_grid_stays_below_2_to_the_32_threads(fa):
         assert n >= 1 and launch(fa, b, 8, 8, 1, 4096, 64, splits=n)[1] == 1
 
 
+def test_streaming_hint_counts_the_keys_that_are_read(fa):
+    """More than 128 MB of K and V, behind a left window only its keys: B16, 8 K/V heads, D 128 read 64 KB per key."""
+    def hint(Skv, wl):
+        return launch(fa, 16, 32, 8, 2, Skv, 128, wl=wl, splits=4)[1:]
+    assert hint(1953, -1) == (1, 0) and hint(1954, -1) == (1, 1)
+    for Skv in (8192, 200000):
+        assert hint(Skv, 128) == (1, 0) and hint(Skv, 1951) == (1, 0) and hint(Skv, 1952) == (1, 1) and hint(Skv, -1) == (1, 1)
+
+
 def test_grid_of_the_merge_of_key_splits(tmp_path):
     """tests/c/check_combine_grid.c: every row covered, fewer than 2^32 threads."""
     exe = str(tmp_path / "check_combine_grid")
