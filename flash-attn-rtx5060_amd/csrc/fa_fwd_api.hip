@@ -307,6 +307,16 @@ long long base_items(const fa_fwd_params *p)
     if (pack > 1) return (long long)p->B * (p->N / pack);
     return fa_sched_num_items(p->B, p->N, p->S, p->d, p->is_causal, p->window_size_left, p->window_size_right);
 }
+// Key tiles that a work item visits at most: those of the keys from its first row's left bound to its last row's right one
+int block_tiles(const fa_fwd_params *p)
+{
+    const long long sk = p->S_kv > 0 ? p->S_kv : p->S;
+    const int s_max = sk > p->S ? (int)sk : p->S, block_rows = 32 * waves_of(p), rows = p->S < block_rows ? p->S : block_rows;
+    int L, R;
+    fa_mask_bounds(s_max, p->is_causal, p->window_size_left, p->window_size_right, &L, &R);
+    const long long keys = (long long)L + rows + R, tiles = (keys + kBlockKeysHost - 2) / kBlockKeysHost + 1;
+    return tiles < key_tiles(p) ? (int)tiles : key_tiles(p);
+}
 int effective_splits(const fa_fwd_params *p)
 {
     if (p->split_num <= 1) return 1;
@@ -391,12 +401,15 @@ int fa_fwd_suggest_splits(const fa_fwd_params *p)
     // work items without splits against the workgroups the device keeps resident; split until the device is
     // filled once (the items of such a problem are all alike, so one full round has no tail; measured against
     // filling it twice: 98 against 106 us on B16 H32/8 S1 S_kv8192, 53 against 61 us on B8 H32/8 S4 S_kv8192,
-    // 370 against 361 us on B4 H32 S1 S_kv32768), with at least four key tiles (256 keys) per split
+    // 370 against 361 us on B4 H32 S1 S_kv32768), with at least four key tiles (256 keys) per split -- of the tiles that
+    // a block visits: behind a left window splits beyond these write empty partial results for the merge to read (causal
+    // bf16 D128, window, us: B1 H8 S64 S_kv 32768 128 1 split 11.4, 64: 20.2; B1 H16/4 S1000 S_kv 9000 D64 256 1: 13.4, 4: 20.5;
+    // B1 H32 S300 S_kv 4000 512 2: 23.6, 6: 33.2; B1 H4 S128 S_kv 32768 D64 4096 16: 15.7, 128: 19.1)
     const long long items = base_items(p);
     const long long resident = (long long)kComputeUnits * (waves_of(p) == 8 ? 1 : 2);
     if (items >= resident) return 1;
     long long n = (resident + items - 1) / items;
-    const long long cap = key_tiles(p) / 4;
+    const long long cap = block_tiles(p) / 4;
     if (n > cap) n = cap;
     return n < 1 ? 1 : (int)n;
 }
