@@ -400,7 +400,7 @@ __global__ void __launch_bounds__(256) fa_combine_splits(const FaKernelArgs a)
         }
     }
     if (!live) return;
-    const bool empty = !(l > 0.0f);
+    const bool empty = l == 0.0f;                 // (not where l is NaN, from a logsumexp of +inf: that row is NaN)
     acc *= empty ? 0.0f : 1.0f / l;
     const int bh = (int)(row / a.S), q = (int)(row - (long long)bh * a.S);
     const int bi = bh / a.H, hi = bh - bi * a.H;

@@ -61,3 +61,17 @@ def test_logsumexps_of_any_size(fa, B, H, Hk, S, Skv, D, sign):
         want = v[:, :, :1].repeat_interleave(H // Hk, 1).expand_as(got).float()
         assert bool(((got.float() - want).abs() <= 2.0 ** -10 * want.abs()).all())
         assert bool((lse == sign * 64.0 * D * 2.0 ** 95).all())
+
+
+@pytest.mark.parametrize("B,H,Hk,S,Skv,D", SHAPES)
+def test_logsumexps_that_overflow(fa, B, H, Hk, S, Skv, D):
+    """Scaled scores of -2.9e38, a number in fp32 but not once multiplied by log2(e): the probabilities are infinite, the
+    rows NaN without splits, and NaN, not an empty row, with them."""
+    import torch
+    q, k, v = _inputs(torch, B, H, Hk, S, Skv, D)
+    q.fill_(8.0)
+    k.fill_(-8.0)
+    for splits in (1, 3, 11):
+        got, lse = fa.flash_attention_forward(q, k, v, softmax_scale=2.9e38 / (64.0 * D), splits=splits)
+        torch.cuda.synchronize()
+        assert bool(torch.isnan(got).all()) and not bool(torch.isfinite(lse).any()) and not bool((lse == float("-inf")).any())
