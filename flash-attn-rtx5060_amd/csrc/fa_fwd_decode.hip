@@ -347,9 +347,10 @@ __global__ void __launch_bounds__(256) fa_combine_splits(const FaKernelArgs a)
     const int n = a.n_splits;
     const float *lse_row = a.lse_part + row, *o_row = a.o_part + row * D + 4 * t;
     const size_t o_step = (size_t)n_rows * D;
+    // (the choice in front of the product, so that sums of products stay fused, with one rounding each)
     auto weighted = [](f32x4 part, float w) __attribute__((always_inline)) {
         const f32x4 none = {0.0f, 0.0f, 0.0f, 0.0f};
-        return w > 0.0f ? part * w : none;
+        return (w > 0.0f ? part : none) * w;
     };
     // running reference point and sum of weights (logsumexps are scaled scores, of any size: kNoReference is one for raw
     // scores; from the lowest finite number the differences below are never NaN)
