@@ -395,22 +395,44 @@ unsigned long long fa_fwd_workspace_bytes(const fa_fwd_params *p)
     return (unsigned long long)n * p->B * p->N * p->S * (unsigned long long)(p->d + 1) * 4ull;
 }
 
+namespace {
+// The tile kernels, 128-row blocks that visit `tiles` key tiles: the count from 1 to `most` with the least estimated time
+int least_time_splits(const fa_fwd_params *p, int tiles, int most, double second_launch_us)
+{
+    const long long items = base_items(p);
+    const double tile_us = p->d == 64 ? 0.55 : 0.85, partial = (double)p->B * p->N * p->S * p->d * 8.0 / 5.2e6;
+    int best = 1;
+    double best_us = 0.0;
+    for (int n = 1; n == 1 || n <= most; ++n) {
+        const long long per_cu = (items * n + kComputeUnits - 1) / kComputeUnits;
+        double us = (double)per_cu * ((tiles + n - 1) / n * tile_us + 1.4) * (per_cu == 1 ? 1.4 : 1.0);
+        if (n > 1) us += second_launch_us + partial * n;
+        if (n == 1 || us < best_us) { best = n; best_us = us; }
+    }
+    return best;
+}
+}  // namespace
+
 int fa_fwd_suggest_splits(const fa_fwd_params *p)
 {
     if (!p || p->B <= 0 || p->N <= 0 || p->S <= 0) return 1;
     // work items without splits against the workgroups the device keeps resident; split until the device is
     // filled once (the items of such a problem are all alike, so one full round has no tail; measured against
     // filling it twice: 98 against 106 us on B16 H32/8 S1 S_kv8192, 53 against 61 us on B8 H32/8 S4 S_kv8192,
-    // 370 against 361 us on B4 H32 S1 S_kv32768), with at least four key tiles (256 keys) per split -- of the tiles that
-    // a block visits: behind a left window splits beyond these write empty partial results for the merge to read (causal
-    // bf16 D128, window, us: B1 H8 S64 S_kv 32768 128 1 split 11.4, 64: 20.2; B1 H16/4 S1000 S_kv 9000 D64 256 1: 13.4, 4: 20.5;
-    // B1 H32 S300 S_kv 4000 512 2: 23.6, 6: 33.2; B1 H4 S128 S_kv 32768 D64 4096 16: 15.7, 128: 19.1)
+    // 370 against 361 us on B4 H32 S1 S_kv32768), with at least four key tiles (256 keys) per split
     const long long items = base_items(p);
     const long long resident = (long long)kComputeUnits * (waves_of(p) == 8 ? 1 : 2);
     if (items >= resident) return 1;
     long long n = (resident + items - 1) / items;
-    const long long cap = block_tiles(p) / 4;
-    if (n > cap) n = cap;
+    if (n > key_tiles(p) / 4) n = key_tiles(p) / 4;
+    // A left window leaves a block a few of these tiles, and splits beyond them write empty partial results for the merge
+    // to read: no more than one per tile, and the tile kernels of 128-row blocks take the count with the least estimated
+    // time (fa_fwd_auto_splits; the second launch costs 3 us here, where the first one is short).
+    const int sk = p->S_kv > 0 ? p->S_kv : p->S, s_max = sk > p->S ? sk : p->S, tiles = block_tiles(p);
+    int L, R;
+    fa_mask_bounds(s_max, p->is_causal, p->window_size_left, p->window_size_right, &L, &R);
+    if (n > tiles) n = tiles;
+    if (L < s_max && waves_of(p) != 8 && !decode_problem(p, R == 0, 1)) n = least_time_splits(p, tiles, (int)n, 3.0);
     return n < 1 ? 1 : (int)n;
 }
 
@@ -434,17 +456,9 @@ int fa_fwd_auto_splits(const fa_fwd_params *p)
         const long long items = base_items(p);
         const int tiles = key_tiles(p);
         if (sk <= p->S || L < s_max || waves_of(p) == 8 || items >= 2 * kComputeUnits) return fa_fwd_suggest_splits(p);
-        const double tile_us = p->d == 64 ? 0.55 : 0.85, partial = (double)p->B * p->N * p->S * p->d * 8.0 / 5.2e6;
-        int best = 1;
-        double best_us = 0.0;
         // (at least three tiles a split, B2 H16/4 S91 S_kv 636 5: 19.1, 2: 18.6; at most four workgroups on every slot)
-        for (int n = 1; n == 1 || (3 * n <= tiles && items * n <= 8 * kComputeUnits); ++n) {
-            const long long per_cu = (items * n + kComputeUnits - 1) / kComputeUnits;
-            double us = (double)per_cu * ((tiles + n - 1) / n * tile_us + 1.4) * (per_cu == 1 ? 1.4 : 1.0);
-            if (n > 1) us += 4.6 + partial * n;
-            if (n == 1 || us < best_us) { best = n; best_us = us; }
-        }
-        return best;
+        const long long slots = 8 * kComputeUnits / items;
+        return least_time_splits(p, tiles, (int)(slots < tiles / 3 ? slots : tiles / 3), 4.6);
     }
     // The decoding kernel: the splits with the least estimated time.  The chip's bandwidth is shared by its CUs, so K and V
     // take as long as the CU with the most workgroups: (their bytes at 6.5 TB/s) * ceil(load) / load with load workgroups
