@@ -332,7 +332,19 @@ bool decode_problem(const fa_fwd_params *p, bool causal_type, int splits)
     const int hk = p->n_kv_heads > 0 ? p->n_kv_heads : p->N, sk = p->S_kv > 0 ? p->S_kv : p->S;
     if ((long long)p->B * hk * splits > kDecodeMostGroups) return false;
     if ((long long)(p->N / hk) * p->S > 32 || sk < p->S || fa_dropout_threshold(p->dropout_prob) != 0) return false;
-    return !(causal_type && sk - p->S < 32 && packed_group(p) == 1 && !p->exact_first_rows);
+    if (causal_type && sk - p->S < 32 && packed_group(p) == 1 && !p->exact_first_rows) return false;
+    // The decoding kernel's set-up and its merge of four waves' 32 rows at head dimension 128 cost as much as three key tiles:
+    // up to there, with four workgroups and more per compute unit and no mask or a group's rows packed into one block, the
+    // tile kernels are the faster ones.  bf16, decoding against tile kernel, us: B64 H16 S32 S_kv 64 17.9 / 12.8, S_kv 128
+    // 22.3 / 17.3, S_kv 192 25.8 / 22.1; B256 H16 S17 S_kv 64 53.6 / 37.7, S24 S_kv 128 72.0 / 62.6, S32 S_kv 64 ALiBi 64 / 42; B512
+    // H16 S32 S_kv 64 111 / 89, S_kv 96 123 / 130; B1024 H16/2 S4 S_kv 128 causal 42.8 / 35.2; and beyond: B48 H16 S32 S_kv 96
+    // 16.9 / 17.7, B256 H16 S32 S_kv 200 101 / 104, S16 S_kv 100 42.4 / 63.7, S32 S_kv 100 D64 34.7 / 50.1, S_kv 128 causal 77 / 142.
+    if (p->d == 128 && (long long)(p->N / hk) * p->S > 16 && sk <= 192 && (long long)p->B * hk >= 4 * kComputeUnits) {
+        int L, R;
+        fa_mask_bounds(sk, p->is_causal, p->window_size_left, p->window_size_right, &L, &R);
+        if ((L >= sk && R >= sk) || packed_group(p) > 1) return false;
+    }
+    return true;
 }
 // Workgroups of the tile kernels that a device keeps resident
 long long resident_groups(int compute_units, int waves) { return (long long)compute_units * (waves == 8 ? 1 : 2); }

@@ -20,6 +20,8 @@ CASES = [
     (1, 8, 8, 3, 700, 128, 0, True, 100, True, 11),        # more than eight partial results per row; ALiBi
     (2, 8, 2, 2, 4100, 64, 1, False, -1, True, "auto"),    # no mask: keys behind the last query, on both sides of it
     (1, 6, 3, 5, 64, 128, 0, True, 0, False, 1),           # every row sees one key
+    (64, 16, 16, 20, 70, 128, 1, False, -1, True, 1),      # short keys, many heads: left to the tile kernels
+    (128, 32, 8, 5, 104, 128, 0, True, 50, False, "auto"), # the same with a group's rows in one block
 ]
 
 

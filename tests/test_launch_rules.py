@@ -50,6 +50,19 @@ def test_decoding_grid_stays_below_2_to_the_32_threads(fa):
         assert n >= 1 and launch(fa, b, 8, 8, 1, 4096, 64, splits=n)[1] == 1
 
 
+def test_short_keys_and_many_heads_take_the_tile_kernels(fa):
+    """Head dimension 128, 17 to 32 rows, at most 192 keys, 1024 K/V heads and more, no mask or a packed block."""
+    for S, Skv in ((17, 17), (32, 64), (32, 192), (20, 129)):
+        assert launch(fa, 64, 16, 16, S, Skv, 128, causal=False)[1] == 0
+    assert launch(fa, 128, 64, 8, 4, 104, 128)[1] == 0 and launch(fa, 128, 64, 8, 4, 104, 128, causal=False)[1] == 0
+    assert launch(fa, 128, 64, 8, 4, 104, 128, wl=50)[1] == 0
+    for args in ((64, 16, 16, 16, 64, 128), (64, 16, 16, 32, 193, 128), (64, 16, 16, 32, 64, 64), (63, 16, 16, 32, 64, 128)):
+        assert launch(fa, *args, causal=False)[1] == 1
+    assert launch(fa, 64, 16, 16, 32, 128, 128)[1] == 1
+    p = fa.make_params(64, 16, 32, 128, causal=False, S_kv=64)
+    assert fa.lib().fa_fwd_auto_splits(ctypes.byref(p)) == 1
+
+
 def test_streaming_hint_counts_the_keys_that_are_read(fa):
     """More than 128 MB of K and V, behind a left window only its keys: B16, 8 K/V heads, D 128 read 64 KB per key."""
     def hint(Skv, wl):
