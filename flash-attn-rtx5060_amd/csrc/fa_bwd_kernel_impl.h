@@ -139,7 +139,7 @@ __device__ __forceinline__ void wait_vm_upto(int n)
 #define FA_WAIT_CASE(k) case k: wait_vm<k>(); break;
     FA_WAIT_CASE(0) FA_WAIT_CASE(1) FA_WAIT_CASE(2) FA_WAIT_CASE(3) FA_WAIT_CASE(4) FA_WAIT_CASE(5) FA_WAIT_CASE(6) FA_WAIT_CASE(7)
     FA_WAIT_CASE(8) FA_WAIT_CASE(9) FA_WAIT_CASE(10) FA_WAIT_CASE(11) FA_WAIT_CASE(12) FA_WAIT_CASE(13) FA_WAIT_CASE(14) FA_WAIT_CASE(15)
-    FA_WAIT_CASE(16) FA_WAIT_CASE(17) FA_WAIT_CASE(18)
+    FA_WAIT_CASE(16)
 #undef FA_WAIT_CASE
     default: wait_vm<0>(); break;
     }
@@ -395,6 +395,7 @@ template <bool BF16, int D, bool MASKED, int LAYOUT, bool ALIBI, bool DROPOUT, b
 __global__ void __launch_bounds__(kBwdWaves * 64, 2) fa_bwd_dkdv(const FaBwdArgs a)
 {
     constexpr bool STRIDES = LAYOUT >= 1, GENERAL = LAYOUT == 2, ONE_ITEM = STRIDES && D == 128 && !(WRITE_DS && FA_DS_LOOP);
+    static_assert(!SHARES || (WRITE_DS && !ONE_ITEM), "a share is several walks, one pass of the item loop each");
     static_assert(!WRITE_DS || LAYOUT <= 1 || (!ALIBI && !DROPOUT), "general lengths: dS blocks without ALiBi and dropout only");
     typedef Num<BF16> N;
     typedef TileReader<D> Reader;
@@ -878,7 +879,7 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_bwd_dq_from_ds(const FaBwdArgs 
     constexpr int WAVE_DS = 2 * kDsBlockBytes;                 // a wave's two blocks of a key tile
     constexpr int STAGEB = TILEB + NW * WAVE_DS, ROWS = 32 * NW;
     constexpr int AHEAD = NST - 1;                             // tiles are requested this many ahead
-    static_assert((AHEAD - 1) * (IPW + 4) <= 18, "more requests in flight than wait_vm_upto counts");
+    static_assert((AHEAD - 1) * (IPW + 4) <= 16, "more requests in flight than wait_vm_upto counts");
     extern __shared__ __attribute__((aligned(1024))) char smem[];
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)smem;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);

@@ -19,11 +19,13 @@
 //    read-only loop over 2 GB runs at 7.1 TB/s with it and at 6.2 without (512 MB: 7.0 against 6.1).  Here, with the
 //    hint against without: B4 H32 S_kv 32768 (2.1 GB) 329 against 369 us, B16 H32/8 S_kv 8192 (537 MB) 87 against 98,
 //    B1 H64/8 S_kv 32768 (134 MB) 33.5 against 35.5; but B8 H32/8 S_kv 2048 (67 MB, called again and again) 18.5 against 17.2.
-//  * Four waves per workgroup, four workgroups per CU (up to 16 rows: 128 registers): B4 H32 S_kv 32768 324 us = 6.6 TB/s;
-//    with eight waves 329, with sixteen 334.
+//  * Four waves per workgroup, four workgroups per CU (up to 16 rows: 128 registers): both launches of B4 H32 S_kv 32768
+//    324 us, with eight waves 329, with sixteen 334 (before the splits followed the load of the busiest CU, see
+//    fa_fwd_auto_splits; since then 308, of which this kernel 306 = 7.0 TB/s).
 //
-// Measured, both launches of a call, against the tile kernels with the same splits: B4 H32 S_kv 32768 324 us against
-// 367, B16 H32/8 S_kv 8192 87 against 97, B1 H32/8 S_kv 1003 8.1 (16 splits) against 16.
+// Measured, both launches of a call, against the tile kernels, each with the splits that "auto" takes for it: B4 H32 S_kv
+// 32768 308 us against 370, B16 H32/8 S_kv 8192 82.6 against 96.5, B1 H32/8 S_kv 1003 10.4 against 16.5 (with the call's host
+// time, two microseconds of the difference).
 #include "fa_fwd_kernel_impl.h"
 
 namespace {
