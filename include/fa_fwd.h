@@ -126,7 +126,8 @@ int fa_fwd_validate(const fa_fwd_params *p);
  * splits * B * N * S * (d + 1) * 4 bytes of fp32 partial outputs and logsumexps. */
 unsigned long long fa_fwd_workspace_bytes(const fa_fwd_params *p);
 /* A split count that fills the device for these shapes (1 when the problem has enough work items anyway), with at least
- * four key tiles of those that a block of queries visits for every split. */
+ * four key tiles for every split; behind a left window the count estimated to be fastest, at most one split per key tile
+ * that a block of queries visits. */
 int fa_fwd_suggest_splits(const fa_fwd_params *p);
 /* The split count with which this library is fastest: that of fa_fwd_suggest_splits, and where the decoding kernel
  * takes the problem (at most 32 query rows per K/V head) what suits that kernel, which splits short caches further and
