@@ -12,8 +12,10 @@ struct FaBwdTensor {
 struct FaBwdArgs {
     const uint16_t *Q, *K, *V, *O, *dO;
     const float *lse;                       // [B,H,S] contiguous, natural log, as the forward pass writes it
-    float *delta;                           // [B,H,S] scratch: sum_t dO*O per row, written by fa_bwd_dq
-    float *lse2;                            // [B,H,S] scratch: lse * log2(e), +inf for rows that saw no key
+    // scratch [B,H,S] each, written by fa_bwd_dq or fa_bwd_prepare for the key-owning kernel, whose accumulators start from
+    // them: -(sum_t dO*O) / drop_scale per row, and -lse / scale, -inf for rows that saw no key (P is then 0)
+    float *delta;
+    float *lse2;
     uint16_t *dQ, *dK, *dV;
     // Five-product form (reference layout only), or null: dS in blocks of 32 queries x 32 keys, 2 KiB each, block
     // (head bh, query block i, key block j) at (bh * fa_ds_blocks_per_head + fa_ds_block_index(i, j)) * 2 KiB

@@ -34,14 +34,13 @@
 #ifndef FA_DS_LOOP
 #define FA_DS_LOOP 1
 #endif
-#ifndef FA_PARK_DROP
-#define FA_PARK_DROP 3
-#endif
 namespace {
 
 constexpr int kBwdWaves = 8;            // 8 waves x 32 owned rows = 256 rows per workgroup, two waves per SIMD
 constexpr int kBwdStages = 3;           // LDS ring: with three stages one barrier per tile is enough
 constexpr float kLog2e = 1.44269504088896340736f;
+// K^T fragments that the key-owning kernel keeps in LDS (see there); the dropout words take the place of one
+constexpr int fa_bwd_parked(int D, bool dropout) { return D == 128 ? (dropout ? 6 : 7) : 0; }
 constexpr int kDsBlockBytes = 2048;     // one 32-query x 32-key block of dS in the storage type
 
 // Takes the word by value on purpose: __builtin_bit_cast applied directly to an element of a vector
@@ -156,6 +155,15 @@ __device__ __forceinline__ void dma_16_stream(const char *base, uint32_t voff, u
                  :: "s"(__builtin_amdgcn_readfirstlane(lds)), "v"(voff), "s"(ub) : "memory", "m0");
 }
 
+// the lane index, read from the hardware and tied to the place of the call: what follows from it is formed there instead of
+// once at the top and kept in registers
+__device__ __forceinline__ int lane_here()
+{
+    int ln = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+    asm volatile("" : "+v"(ln));
+    return ln;
+}
+
 __device__ __forceinline__ f32x16 zero16()
 {
     f32x16 z;
@@ -263,8 +271,8 @@ __global__ void __launch_bounds__(kBwdWaves * 64, 2) fa_bwd_dq(const FaBwdArgs a
         }
         delta += swap_halves(delta);
         if (row_ok && half == 0) {
-            a.delta[(size_t)bh * S + my_q] = delta;
-            a.lse2[(size_t)bh * S + my_q] = lse_l2;
+            a.delta[(size_t)bh * S + my_q] = -delta / a.drop_scale;
+            a.lse2[(size_t)bh * S + my_q] = (GENERAL && lse_raw == -INFINITY) ? -INFINITY : -lse_raw / a.scale;
         }
     }
     const float c = a.scale * kLog2e;
@@ -391,23 +399,27 @@ __global__ void __launch_bounds__(kBwdWaves * 64, 2) fa_bwd_dq(const FaBwdArgs a
 // WRITE_DS (regular lengths, no ALiBi): every 32-query x 32-key block of dS that a wave forms is also written to
 // a.ds_blocks, in the wave's operand order, for fa_bwd_dq_from_ds.
 // SHARES (with WRITE_DS): the walks cut into equal shares, see fa_bwd_layout.h.
-template <bool BF16, int D, bool MASKED, int LAYOUT, bool ALIBI, bool DROPOUT, bool WRITE_DS = false, bool SHARES = false>
-__global__ void __launch_bounds__(kBwdWaves * 64, 2) fa_bwd_dkdv(const FaBwdArgs a)
+template <bool BF16, int D, bool MASKED, int LAYOUT, bool ALIBI, bool DROPOUT, bool WRITE_DS = false, bool SHARES = false, int NW = kBwdWaves>
+__global__ void __launch_bounds__(NW * 64, 2) fa_bwd_dkdv(const FaBwdArgs a)
 {
     constexpr bool STRIDES = LAYOUT >= 1, GENERAL = LAYOUT == 2, ONE_ITEM = STRIDES && D == 128 && !(WRITE_DS && FA_DS_LOOP);
     static_assert(!SHARES || (WRITE_DS && !ONE_ITEM), "a share is several walks, one pass of the item loop each");
     static_assert(!WRITE_DS || LAYOUT <= 1 || (!ALIBI && !DROPOUT), "general lengths: dS blocks without ALiBi and dropout only");
     typedef Num<BF16> N;
     typedef TileReader<D> Reader;
-    typedef TileLoader<D> Loader;
+    typedef TileLoader<D, NW> Loader;
+    constexpr int BK = 32 * NW;                   // keys per workgroup
     constexpr int KS = Reader::KS, DB = Reader::DB, TILEB = Loader::TILEB, STAGEB = 2 * TILEB + 512, IPW = Loader::IPW;
+    // LDS reads run this many matrix instructions ahead (at head dimension 128 what the registers hold: three with less of K
+    // in LDS, or with fewer address registers and an instruction more per read, measured 1-4 % slower on every shape tried)
+    constexpr int PD = D == 64 ? 4 : DROPOUT ? 1 : 2;
     constexpr int NSTG = kBwdStages;                                  // LDS stages; pairs are requested NSTG - 1 ahead
     extern __shared__ __attribute__((aligned(1024))) char smem[];
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)smem;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int S = a.S, Sk = GENERAL ? a.Sk : a.S, off = GENERAL ? a.Sk - a.S : 0;
     const int G = STRIDES ? a.H / a.Hk : 1;
-    const int n_kblocks = (Sk + 255) / 256;
+    const int n_kblocks = (Sk + BK - 1) / BK;
     // one K/V head per XCD at a time; key block 0 is seen by the most queries and goes first
     // (work items as in fa_bwd_dq; the list here is ascending in the key block, which is longest first under a
     // causal mask: key block 0 is seen by every query)
@@ -449,7 +461,7 @@ __global__ void __launch_bounds__(kBwdWaves * 64, 2) fa_bwd_dkdv(const FaBwdArgs
         const size_t head_off = (size_t)bhk * S * D;
         Kh = a.K + head_off; Vh = a.V + head_off;
     }
-    const int k0 = kblock * 256, kw = k0 + wave * 32;
+    const int k0 = kblock * BK, kw = k0 + wave * 32;
     const bool active = kw < Sk;
     const int my_k = kw + l32;                     // this lane's key (masks, ALiBi)
     const int my_kc = active ? (GENERAL && my_k >= Sk ? Sk - 1 : my_k) : (GENERAL ? 0 : l32);     // row to load
@@ -466,14 +478,12 @@ __global__ void __launch_bounds__(kBwdWaves * 64, 2) fa_bwd_dkdv(const FaBwdArgs
     // j - R - off <= i <= j + L - off: the forward bounds with the two sides exchanged and shifted
     const int Lq = a.R + off, Rq = a.L - off;
     int t0, t1, my_lo = 1, my_hi = 0;
-    fa_tile_range(S, 64, Lq, Rq, k0, Sk - k0 < 256 ? Sk - k0 : 256, &t0, &t1);
+    fa_tile_range(S, 64, Lq, Rq, k0, Sk - k0 < BK ? Sk - k0 : BK, &t0, &t1);
     if (active) fa_tile_range(S, 64, Lq, Rq, kw, GENERAL && Sk - kw < 32 ? Sk - kw : 32, &my_lo, &my_hi);
 
     Reader rd; rd.init(lane, lds0);
     uint32_t stat_addr = lds0 + 2 * TILEB + 16 * half;       // this lane's logsumexp / delta words in the stage being read
-    // dropout: 128 bytes per wave behind the ring, through which keep bits drawn with the query on the lane (one
-    // Philox block covers sixteen keys of ONE query) reach the lanes that own the keys
-    const uint32_t drop_lds = lds0 + NSTG * STAGEB + wave * 128;
+    const uint32_t drop_lds = lds0 + NSTG * STAGEB + wave * 1024;       // dropout: 1 KB per wave behind the ring
     Loader ldq, ldg;
     if (!STRIDES || GENERAL) ldq.init(wave, lane, q_rs * 2);      // (general: only its ragged tiles go through these two)
     if (GENERAL) ldg.init(wave, lane, g_rs * 2);
@@ -532,126 +542,210 @@ __global__ void __launch_bounds__(kBwdWaves * 64, 2) fa_bwd_dkdv(const FaBwdArgs
     f32x16 dk[DB], dv[DB];
 #pragma unroll
     for (int db = 0; db < DB; ++db) { dk[db] = zero16(); dv[db] = zero16(); }
-    // WRITE_DS, head dimension 128: the kernel needs every register it can have (two waves per SIMD: 256), and a
-    // value the compiler spills to scratch memory inside the tile loop comes back behind a wait for ALL loads and
-    // stores in flight.  The last PARKED of the K^T and V^T fragments, which every half tile uses once, are kept in
-    // LDS instead (32 bytes per lane and fragment pair, written once per work item) and read like any A operand.
-    constexpr int PARKED = WRITE_DS && D == 128 ? (DROPOUT ? FA_PARK_DROP : ALIBI ? 2 : 1) : 0;
-    constexpr uint32_t kParkPlane = 16u * kBwdWaves * 64u;
-    const uint32_t park_lds = lds0 + NSTG * STAGEB + (DROPOUT ? kBwdWaves * 128 : 0);       // (behind the dropout words)
-    auto parked = [&](int which, int s) __attribute__((always_inline)) {
-        uint32_t ln = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
-        asm volatile("" : "+v"(ln));
-        const uint32_t addr = park_lds + 16u * ((uint32_t)wave * 64u + ln) + kParkPlane * (uint32_t)(2 * (s - (KS - PARKED)) + which);
-        return *(volatile __attribute__((address_space(3))) u32x4 *)(uintptr_t)addr;
+    // Head dimension 128: the kernel needs every register it can have (two waves per SIMD: 256), and a value the compiler
+    // spills to scratch memory inside the tile loop comes back behind a wait for ALL loads and stores in flight.  The last
+    // PARKED of the K^T fragments, which every half tile uses once, are kept in LDS instead (a plane of 16 bytes per lane
+    // each, written once per work item) and read like any A operand: K's, because dP, dS and P are not alive yet where they
+    // are used.  (One K and one V fragment, as before the reads ran ahead: spills of 80-360 bytes inside the loop.)
+    constexpr int PARKED = fa_bwd_parked(D, DROPOUT);
+    constexpr uint32_t kParkPlane = 16u * NW * 64u;
+    const uint32_t park_lds = lds0 + NSTG * STAGEB + (DROPOUT ? NW * 1024 : 0);       // (behind the dropout words)
+    const uint32_t park_addr = park_lds + 16u * ((uint32_t)wave * 64u + (uint32_t)lane);
+    auto parked = [&](int plane) __attribute__((always_inline)) {
+        return *(volatile __attribute__((address_space(3))) u32x4 *)(uintptr_t)(park_addr + kParkPlane * (uint32_t)plane);
     };
 
-    // 32 queries (block qb of the tile in the stage being read) against this wave's 32 keys
-    auto half_tile = [&](bool edge, float slope_l2, uint32_t bhq, int t, int qb) __attribute__((always_inline)) {
-        constexpr int q_tile = 0, g_tile = TILEB;
-        if (DROPOUT) {
-            // lane (l32, half) draws for query 32*qb + l32 of the tile the sixteen keys 8*g + 4*half + e of this
-            // wave's 32-key block and leaves them as a 16-bit mask (bit 4*g + e) in LDS word [half][l32]
-            const DropWords dw = dropout_words(a.seed_lo, a.seed_hi, bhq, (uint32_t)(t * 64 + 32 * qb + l32 + off), (uint32_t)(2 * (kw >> 5) + half));
-            uint32_t m = 0;
+    // Dropout decisions of the 32 x 32 block (query block qb of tile t, this wave's keys).  A Philox block covers sixteen
+    // keys of ONE query, and a lane here owns a key: lane (l32, half) draws for query 32 qb + l32 the sixteen bytes of the
+    // keys 8 g + 4 half + e (word g, byte e); the 4 x 4 bytes of four neighbouring lanes are transposed in registers, so that
+    // a word holds four queries of ONE key, and the words change lanes through 1 KB of LDS that belong to the wave.
+    // (Bound by the vector ALU: ten Philox rounds, then a comparison and a select per element for P and for dP.  With the bytes
+    // compared in front of the exchange and sixteen bits put together on both sides of it, p = 0.1: B16 H16 S512 D64 no mask
+    // 121 us, now 112; B16 H32 S1534 D128 causal 2036 / 1644; B4 H32 S1024 D128 no mask 404 / 273; all of the backward pass.)
+    auto draw = [&](uint32_t bhq, int t, int qb) __attribute__((always_inline)) {
+        const int ln = lane_here(), key = ln & 31, quarter = ln >> 5;
+        // (the seed's registers are tied to this place too: the ten rounds' keys would otherwise be kept in twenty registers)
+        uint32_t seed_lo = a.seed_lo, seed_hi = a.seed_hi;
+        asm volatile("" : "+s"(seed_lo), "+s"(seed_hi));
+        const DropWords dw = dropout_words(seed_lo, seed_hi, bhq, (uint32_t)(t * 64 + 32 * qb + key + off), (uint32_t)(2 * (kw >> 5) + quarter));
+        const uint32_t sel1 = (ln & 1) ? 0x03070105u : 0x06020400u, sel2 = (ln & 2) ? 0x03020706u : 0x05040100u;
+        u32x4 w;
 #pragma unroll
-            for (int r = 0; r < 16; ++r) m |= dropout_keep_byte(dw, r, a.drop_threshold) ? (1u << r) : 0u;
-            *(__attribute__((address_space(3))) uint16_t *)(drop_lds + (uint32_t)(half * 32 + l32) * 2u) = (uint16_t)m;
+        for (int g = 0; g < 4; ++g) {
+            uint32_t x = dw.w[g];
+            x = __builtin_amdgcn_perm((uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0xB1, 0xf, 0xf, true), x, sel1);
+            w[g] = __builtin_amdgcn_perm((uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0x4E, 0xf, 0xf, true), x, sel2);
         }
-        f32x16 sx = zero16();            // rows = queries, column (lane) = key
-#pragma unroll
-        for (int s = 0; s < KS; ++s) sx = N::mfma(rd.rows(q_tile, s, qb), s >= KS - PARKED ? parked(0, s) : kf[s], sx);      // S = Q K^T
-        const int first = t * 64 + 32 * qb + 4 * half;                      // query of accumulator row 0 on this lane
-        if (MASKED && edge) {            // wave-uniform; a masked score becomes -inf and its P exactly 0
-            int hi = my_k + Rq, lo = my_k - Lq - first;                      // visible: lo <= 8*(r/4) + r%4 <= hi
-            if (GENERAL && hi > S - 1) hi = S - 1;
-            hi -= first;
-#pragma unroll
-            for (int r = 0; r < 16; ++r)
-                if (8 * (r >> 2) + (r & 3) > hi || 8 * (r >> 2) + (r & 3) < lo) sx[r] = -INFINITY;
-        }
-        // accumulator row r is query 32*qb + 8*(r/4) + 4*half + r%4 of the tile
-        uint32_t keep = 0xffffu;         // bit r: the forward kept (query of row r, this lane's key)
-        if (DROPOUT) {
-            // this lane's key is key l32 of the block: drawn by the lanes of half (l32 / 4) % 2 as bit 4*(l32/8) + l32%4;
-            // the four queries 8*g + 4*half + 0..3 sit in four consecutive 16-bit words
-            const uint32_t src = drop_lds + (uint32_t)(((l32 >> 2) & 1) * 32 + 4 * half) * 2u, bit = (uint32_t)(4 * (l32 >> 3) + (l32 & 3));
-            keep = 0;
+        *(__attribute__((address_space(3))) u32x4 *)(uintptr_t)(drop_lds + 16u * (uint32_t)ln) = w;
+        __builtin_amdgcn_sched_barrier(0);
+    };
+
+    // A tile: its 64 queries, 32 (block qb) at a time, against this wave's 32 keys.  Per block four products: S = Q K^T, dP =
+    // dO V^T, dV^T += dO^T P, dK^T += Q^T dS, NF matrix instructions that each read one fragment of the tile from LDS.
+    // The fragments are read PD instructions ahead, across the blocks of the tile, and what the vector ALU does (P from S, dS
+    // from P and dP) is dealt in pairs of elements over the instructions behind the one that its inputs come from.
+    // (What bounds it: the dependent chain of a block on two waves per SIMD, then the power cap -- on zeros instead of unit
+    // normal values the 64-wide kernel takes 232 us instead of 353.  Left to the compiler every read was waited for at once.
+    // B2 H16 S4096 without a mask, D64 fp16 397 us before, 353 now; whole backward passes: B2 H32/8 S4096 D128 bf16 882 / 819,
+    // B2 H32 S8192 D128 3270 / 3010, B4 H16 S1000 D128 96 / 90, B8 H16 S1000 D64 100 / 93.)
+    auto whole_tile = [&](bool edge, float slope_l2, uint32_t bhq, int t) __attribute__((always_inline)) {
+        constexpr int q_tile = 0, g_tile = TILEB, NH = 2 * KS + 4 * DB, NF = 2 * NH;
+        u32x4 fr[NF], fb[NF];
+        auto fetch = [&](int n) __attribute__((always_inline)) {
+            const int qb = n / NH, i = n % NH;
+            if (i < KS) {
+                fr[n] = rd.rows(q_tile, i, qb);
+                if (i >= KS - PARKED) fb[n] = parked(i - (KS - PARKED));
+            } else if (i < 2 * KS) {
+                fr[n] = rd.rows(g_tile, i - KS, qb);
+            } else {
+                const int m = (i - 2 * KS) % (2 * DB);
+                fr[n] = rd.transposed(i < 2 * KS + 2 * DB ? g_tile : q_tile, 2 * qb + m / DB, m % DB);
+            }
+        };
+        f32x16 sx, dp;
+        // the accumulators of block qb start from what the row's exponent and row sum subtract: -lse / scale, -delta
+        auto start = [&](f32x16 &acc, int qb, uint32_t at) __attribute__((always_inline)) {
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
-                const u32x2 w = *(const __attribute__((address_space(3))) u32x2 *)(src + 16u * g);
-                const uint32_t w0 = w[0], w1 = w[1];
-                keep |= ((w0 >> bit) & 1u) << (4 * g) | ((w0 >> (16 + bit)) & 1u) << (4 * g + 1) |
-                        ((w1 >> bit) & 1u) << (4 * g + 2) | ((w1 >> (16 + bit)) & 1u) << (4 * g + 3);
+                const u32x4 w = lds_read_b128(stat_addr + at + (uint32_t)(32 * qb + 8 * g) * 4u);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[4 * g + e] = as_f32(w[e]);
             }
-        }
-        uint32_t pp[8];
+        };
+        start(sx, 0, 0);
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            const u32x4 lraw = lds_read_b128(stat_addr + (uint32_t)(32 * qb + 8 * g) * 4u);
-            float p[4], pd[4];
+        for (int n = 0; n < PD; ++n) fetch(n);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int r = 4 * g + e;
-                float x = __builtin_fmaf(sx[r], c, -as_f32(lraw[e]));
-                if (ALIBI) x = __builtin_fmaf(-slope_l2, __builtin_fabsf((float)(first + 8 * g + e + off - my_k)), x);
-                p[e] = __builtin_amdgcn_exp2f(x);
-                sx[r] = p[e];                    // keep P in fp32 for dS
-                pd[e] = DROPOUT ? (((keep >> r) & 1u) ? p[e] * a.drop_scale : 0.0f) : p[e];      // what multiplied V
+        for (int qb = 0; qb < 2; ++qb) {
+            if (DROPOUT) draw(bhq, t, qb);
+            const int n0 = qb * NH;
+#pragma unroll
+            for (int s = 0; s < KS; ++s) {                                   // S = Q K^T: rows = queries, column (lane) = key
+                const int n = n0 + s;
+                if (n + PD < NF) fetch(n + PD);
+                sx = N::mfma(fr[n], s >= KS - PARKED ? fb[n] : kf[s], sx);
+                if (s == KS - 2) { if (DROPOUT) dp = zero16(); else start(dp, qb, 256u); }
+                __builtin_amdgcn_sched_barrier(0);
             }
-            pp[2 * g] = N::pack2(pd[0], pd[1]);
-            pp[2 * g + 1] = N::pack2(pd[2], pd[3]);
-        }
+            const int first = t * 64 + 32 * qb + 4 * half;                      // query of accumulator row 0 on this lane
+            if (MASKED && edge) {            // wave-uniform; a masked score becomes -inf and its P exactly 0
+                int hi = my_k + Rq, lo = my_k - Lq - first;                      // visible: lo <= 8*(r/4) + r%4 <= hi
+                if (GENERAL && hi > S - 1) hi = S - 1;
+                hi -= first;
 #pragma unroll
-        for (int n = 0; n < 2 * DB; ++n) {                // dV^T += dO^T P
-            const int h2 = n / DB, db = n % DB;
-            const u32x4 bfrag = {pp[4 * h2], pp[4 * h2 + 1], pp[4 * h2 + 2], pp[4 * h2 + 3]};
-            dv[db] = N::mfma(rd.transposed(g_tile, 2 * qb + h2, db), bfrag, dv[db]);
-        }
-        f32x16 dp = zero16();
-#pragma unroll
-        for (int s = 0; s < KS; ++s) dp = N::mfma(rd.rows(g_tile, s, qb), s >= KS - PARKED ? parked(1, s) : vf[s], dp);      // dP = dO V^T
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            const u32x4 draw = lds_read_b128(stat_addr + 256u + (uint32_t)(32 * qb + 8 * g) * 4u);
-            float v[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                float dpr = dp[4 * g + e];
-                if (DROPOUT) dpr = ((keep >> (4 * g + e)) & 1u) ? dpr * a.drop_scale : 0.0f;
-                v[e] = sx[4 * g + e] * (dpr - as_f32(draw[e]));
+                for (int r = 0; r < 16; ++r)
+                    if (8 * (r >> 2) + (r & 3) > hi || 8 * (r >> 2) + (r & 3) < lo) sx[r] = -INFINITY;
             }
-            pp[2 * g] = N::pack2(v[0], v[1]);     // now dS, same operand order
-            pp[2 * g + 1] = N::pack2(v[2], v[3]);
-        }
-        if (WRITE_DS) {
-            // Block (32-query block 2t + qb, this wave's 32-key block) of dS, 2 KiB, as the registers hold it: this
-            // lane's key against the queries 8g + 4*half + 0..3, g = 0..3.  Two store instructions of 1 KiB each,
-            // lane l writing bytes 16 l .. 16 l + 15 of its KiB: queries of g = 0, 1 in the first, g = 2, 3 in the second.
-            // (bhq: the QUERY head, batch * H + head; the blocks of the query heads that share this K/V head are apart)
-            const long long block = (long long)(bhq - (uint32_t)(a.head0 * G)) * fa_ds_blocks_per_head(S) + fa_ds_block_index(S, 2 * t + qb, kw >> 5);
-            // (Inline assembly: the block's address stays in two scalar registers and the lane's offset in one
-            // vector register that lives for these two instructions only -- as a 64-bit vector address it cost
-            // the registers that made the compiler spill inside the tile loop, and every reload from scratch
-            // memory there waits for all tile loads in flight.  Streaming stores: the blocks are read once, by
-            // another kernel, and should not displace the walked tiles from L2.  The wait states cover the rule
-            // that a store of more than 8 bytes must not be followed at once by a write of its data registers.)
-            const uint64_t dst = (uint64_t)(reinterpret_cast<char *>(a.ds_blocks) + block * kDsBlockBytes);
-            const uint64_t ub = ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(dst >> 32)) << 32) |
-                                (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)dst);
-            const uint32_t voff = 16u * __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
-            u32x4 w0 = {pp[0], pp[1], pp[2], pp[3]}, w1 = {pp[4], pp[5], pp[6], pp[7]};
-            // (general lengths: a lane whose key lies past the end has worked on a copy of the last key; what the
-            // query-owning kernel multiplies with the padding rows of its last key tile must be zero)
-            if (GENERAL && my_k >= Sk) { w0 = u32x4{0, 0, 0, 0}; w1 = u32x4{0, 0, 0, 0}; }
-            asm volatile("global_store_dwordx4 %0, %1, %3 nt\n\tglobal_store_dwordx4 %0, %2, %3 offset:1024 nt\n\ts_nop 1"
-                         :: "v"(voff), "v"(w0), "v"(w1), "s"(ub) : "memory");
-        }
+            // accumulator row r is query 32*qb + 8*(r/4) + 4*half + r%4 of the tile
+            uint32_t kept[4];                // dropout: byte e of word g belongs to row 4 g + e
+            if (DROPOUT) {
+                const int ln = lane_here(), key = ln & 31;
+                const uint32_t src = drop_lds + (uint32_t)(((key >> 2) & 1) * 512 + (ln >> 5) * 64 + (key & 3) * 16 + (key >> 3) * 4);
 #pragma unroll
-        for (int n = 0; n < 2 * DB; ++n) {                // dK^T += Q^T dS
-            const int h2 = n / DB, db = n % DB;
-            const u32x4 bfrag = {pp[4 * h2], pp[4 * h2 + 1], pp[4 * h2 + 2], pp[4 * h2 + 3]};
-            dk[db] = N::mfma(rd.transposed(q_tile, 2 * qb + h2, db), bfrag, dk[db]);
+                for (int g = 0; g < 4; ++g) kept[g] = *(const __attribute__((address_space(3))) uint32_t *)(src + 128u * g);
+            }
+            auto keeps = [&](int r) __attribute__((always_inline)) { return ((kept[r >> 2] >> (8 * (r & 3))) & 255u) >= a.drop_threshold; };
+            uint32_t pp[8], ds[8];
+            // rows 2 i and 2 i + 1: P, kept in fp32 in sx for dS, and what multiplied V
+            auto p_pair = [&](int i) __attribute__((always_inline)) {
+                float pd[2];
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    const int r = 2 * i + e;
+                    float x = sx[r] * c;
+                    if (ALIBI) x = __builtin_fmaf(-slope_l2, __builtin_fabsf((float)(first + 8 * (r >> 2) + (r & 3) + off - my_k)), x);
+                    sx[r] = __builtin_amdgcn_exp2f(x);
+                    pd[e] = !DROPOUT || keeps(r) ? sx[r] : 0.0f;         // (the factor 1 / (1 - p): once, at the end)
+                }
+                pp[i] = N::pack2(pd[0], pd[1]);
+                asm volatile("" : "+v"(pp[i]));
+            };
+            f32x4 del;
+            auto ds_pair = [&](int i) __attribute__((always_inline)) {
+                float v[2];
+                if (DROPOUT && i % 2 == 0) {
+                    const u32x4 w = lds_read_b128(stat_addr + 256u + (uint32_t)(32 * qb + 4 * i) * 4u);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) del[e] = as_f32(w[e]);
+                }
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    const int r = 2 * i + e;
+                    float dpr = dp[r];
+                    if (DROPOUT) dpr = (keeps(r) ? dpr : 0.0f) + del[r & 3];       // (both in units of 1 / (1 - p))
+                    v[e] = sx[r] * dpr;
+                }
+                ds[i] = N::pack2(v[0], v[1]);     // dS, same operand order
+                asm volatile("" : "+v"(ds[i]));
+            };
+            // dP (KS instructions) with P pairs from its second on; dV (2 DB) with the P pairs that are left and, from its
+            // second on, dS pairs; dK with the rest.  A pair is ready in front of the instruction that reads it: the 16-query
+            // slice h2 of P or dS needs the pairs 4 h2 .. 4 h2 + 3.
+            constexpr int P_IN_DP = 6;
+            int np = 0, nd = 0;
+#pragma unroll
+            for (int s = 0; s < KS; ++s) {
+                const int n = n0 + KS + s;
+                if (n + PD < NF) fetch(n + PD);
+                dp = N::mfma(fr[n], vf[s], dp);
+                const int upto = s * P_IN_DP / (KS - 1);
+#pragma unroll
+                for (int i = np; i < upto; ++i) p_pair(i);
+                np = upto;
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int m = 0; m < 2 * DB; ++m) {                // dV^T += dO^T P
+                const int n = n0 + 2 * KS + m, h2 = m / DB;
+                if (n + PD < NF) fetch(n + PD);
+                const u32x4 bfrag = {pp[4 * h2], pp[4 * h2 + 1], pp[4 * h2 + 2], pp[4 * h2 + 3]};
+                dv[m % DB] = N::mfma(fr[n], bfrag, dv[m % DB]);
+                if (m == 0)
+#pragma unroll
+                    for (int i = np; i < 8; ++i) p_pair(i);
+                const int upto = m * 6 / (2 * DB - 1);
+#pragma unroll
+                for (int i = nd; i < upto; ++i) ds_pair(i);
+                nd = upto;
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int m = 0; m < 2 * DB; ++m) {                // dK^T += Q^T dS
+                const int n = n0 + 2 * KS + 2 * DB + m, h2 = m / DB;
+                if (n + PD < NF) fetch(n + PD);
+                const u32x4 bfrag = {ds[4 * h2], ds[4 * h2 + 1], ds[4 * h2 + 2], ds[4 * h2 + 3]};
+                dk[m % DB] = N::mfma(fr[n], bfrag, dk[m % DB]);
+                if (m == 0)
+#pragma unroll
+                    for (int i = nd; i < 8; ++i) ds_pair(i);
+                if (m == 1 && qb == 0) start(sx, 1, 0);       // (P has been used)
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if (WRITE_DS) {
+                // Block (32-query block 2t + qb, this wave's 32-key block) of dS, 2 KiB, as the registers hold it: this
+                // lane's key against the queries 8g + 4*half + 0..3, g = 0..3.  Two store instructions of 1 KiB each,
+                // lane l writing bytes 16 l .. 16 l + 15 of its KiB: queries of g = 0, 1 in the first, g = 2, 3 in the second.
+                // (bhq: the QUERY head, batch * H + head; the blocks of the query heads that share this K/V head are apart)
+                const long long block = (long long)(bhq - (uint32_t)(a.head0 * G)) * fa_ds_blocks_per_head(S) + fa_ds_block_index(S, 2 * t + qb, kw >> 5);
+                // (Inline assembly: the block's address stays in two scalar registers and the lane's offset in one
+                // vector register that lives for these two instructions only -- as a 64-bit vector address it cost
+                // the registers that made the compiler spill inside the tile loop, and every reload from scratch
+                // memory there waits for all tile loads in flight.  Streaming stores: the blocks are read once, by
+                // another kernel, and should not displace the walked tiles from L2.  The wait states cover the rule
+                // that a store of more than 8 bytes must not be followed at once by a write of its data registers.)
+                const uint64_t dst = (uint64_t)(reinterpret_cast<char *>(a.ds_blocks) + block * kDsBlockBytes);
+                const uint64_t ub = ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(dst >> 32)) << 32) |
+                                    (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)dst);
+                const uint32_t voff = 16u * __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+                u32x4 w0 = {ds[0], ds[1], ds[2], ds[3]}, w1 = {ds[4], ds[5], ds[6], ds[7]};
+                // (general lengths: a lane whose key lies past the end has worked on a copy of the last key; what the
+                // query-owning kernel multiplies with the padding rows of its last key tile must be zero)
+                if (GENERAL && my_k >= Sk) { w0 = u32x4{0, 0, 0, 0}; w1 = u32x4{0, 0, 0, 0}; }
+                asm volatile("global_store_dwordx4 %0, %1, %3 nt\n\tglobal_store_dwordx4 %0, %2, %3 offset:1024 nt\n\ts_nop 1"
+                             :: "v"(voff), "v"(w0), "v"(w1), "s"(ub) : "memory");
+            }
         }
     };
 
@@ -677,15 +771,10 @@ __global__ void __launch_bounds__(kBwdWaves * 64, 2) fa_bwd_dkdv(const FaBwdArgs
         wait_vm<0>();
 #pragma unroll
         for (int s = 0; s < KS; ++s) asm volatile("" : "+v"(kf[s]), "+v"(vf[s]));
-        if (PARKED > 0) {           // from here on the last fragments live in LDS, and their registers are free
-            // (one plane of 16 bytes per thread for every parked fragment: consecutive lanes, consecutive 16 bytes)
-            const uint32_t slot = park_lds + 16u * (uint32_t)(wave * 64 + lane);
+        // from here on the parked fragments live in LDS, and their registers are free
+        // (one plane of 16 bytes per thread for every parked fragment: consecutive lanes, consecutive 16 bytes)
 #pragma unroll
-            for (int i = 0; i < PARKED; ++i) {
-                *(__attribute__((address_space(3))) u32x4 *)(uintptr_t)(slot + kParkPlane * (2 * i)) = kf[KS - PARKED + i];
-                *(__attribute__((address_space(3))) u32x4 *)(uintptr_t)(slot + kParkPlane * (2 * i + 1)) = vf[KS - PARKED + i];
-            }
-        }
+        for (int i = 0; i < PARKED; ++i) *(__attribute__((address_space(3))) u32x4 *)(uintptr_t)(park_addr + kParkPlane * i) = kf[KS - PARKED + i];
         int stage = 0;
         // WRITE_DS: the dS stores this wave made in the last two iterations, and the pairs still to come.  The next
         // pair is then requested in front of an iteration's work instead of behind it.
@@ -715,8 +804,7 @@ __global__ void __launch_bounds__(kBwdWaves * 64, 2) fa_bwd_dkdv(const FaBwdArgs
                 if (my_lo <= t && t <= my_hi) {
                     const bool edge = MASKED && (fa_tile_class(64, Lq, Rq, kw, 32, t) == 1 || (GENERAL && (t + 1) * 64 > S));
                     const uint32_t bhq = (uint32_t)(b * a.H + hk * G + g);        // the head the forward keyed its dropout on
-                    half_tile(edge, slope_l2, bhq, t, 0);
-                    half_tile(edge, slope_l2, bhq, t, 1);
+                    whole_tile(edge, slope_l2, bhq, t);
                 }
                 if (!TOP && ig < G) issue_next(prev);
                 rd.advance(next == 0 ? -(NSTG - 1) * STAGEB : STAGEB);
@@ -764,10 +852,11 @@ __global__ void __launch_bounds__(kBwdWaves * 64, 2) fa_bwd_dkdv(const FaBwdArgs
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 u32x2 wk, wv;
-                wk[0] = N::pack2(dk[db][4 * g] * a.scale, dk[db][4 * g + 1] * a.scale);
-                wk[1] = N::pack2(dk[db][4 * g + 2] * a.scale, dk[db][4 * g + 3] * a.scale);
-                wv[0] = N::pack2(dv[db][4 * g], dv[db][4 * g + 1]);
-                wv[1] = N::pack2(dv[db][4 * g + 2], dv[db][4 * g + 3]);
+                const float ks = DROPOUT ? a.scale * a.drop_scale : a.scale, vs = DROPOUT ? a.drop_scale : 1.0f;
+                wk[0] = N::pack2(dk[db][4 * g] * ks, dk[db][4 * g + 1] * ks);
+                wk[1] = N::pack2(dk[db][4 * g + 2] * ks, dk[db][4 * g + 3] * ks);
+                wv[0] = N::pack2(dv[db][4 * g] * vs, dv[db][4 * g + 1] * vs);
+                wv[1] = N::pack2(dv[db][4 * g + 2] * vs, dv[db][4 * g + 3] * vs);
                 *reinterpret_cast<u32x2 *>(dKh + (size_t)key_e * dk_rs + 32 * db + 8 * g + 4 * half_e) = wk;
                 *reinterpret_cast<u32x2 *>(dVh + (size_t)key_e * dv_rs + 32 * db + 8 * g + 4 * half_e) = wv;
             }
@@ -813,9 +902,9 @@ __global__ void __launch_bounds__(256) fa_bwd_prepare(const FaBwdArgs a)
 #pragma unroll
     for (int m = 1; m < TPR; m <<= 1) sum += __shfl_xor(sum, m);
     if (live && threadIdx.x % TPR == 0) {
-        a.delta[row] = sum;
+        a.delta[row] = -sum / a.drop_scale;
         const float l = a.lse[row];
-        a.lse2[row] = l == -INFINITY ? INFINITY : l * kLog2e;
+        a.lse2[row] = l == -INFINITY ? -INFINITY : -l / a.scale;
     }
 }
 
@@ -850,7 +939,7 @@ __global__ void __launch_bounds__(256) fa_bwd_add_parts(const FaBwdArgs a, int n
     uint16_t *out = which == 0 ? (STRIDED ? head_ptr(a.dK, a.dk, b, hk) : a.dK + (size_t)bhk * S * D)
                                : (STRIDED ? head_ptr(a.dV, a.dv, b, hk) : a.dV + (size_t)bhk * S * D);
     const int rs = STRIDED ? (which == 0 ? a.dk.rs : a.dv.rs) : D, lane = (int)threadIdx.x % 64, key = kblock * 256 + wave * 32 + (lane & 31);
-    const float scale = which == 0 ? a.scale : 1.0f;
+    const float scale = (which == 0 ? a.scale : 1.0f) * a.drop_scale;      // (drop_scale is 1 without dropout)
     if (key >= S) return;
 #pragma unroll
     for (int n = 0; n < SLOTS; ++n) {
@@ -1000,13 +1089,14 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_bwd_dq_from_ds(const FaBwdArgs 
     }
     if (active && (!GENERAL || qw + l32 < S)) {
         const int my_q = qw + l32;
+        const float scale = a.scale * a.drop_scale;        // (the blocks hold dS in units of drop_scale, which is 1 without dropout)
 #pragma unroll
         for (int db = 0; db < DB; ++db)
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 u32x2 w;
-                w[0] = N::pack2(dq[db][4 * g] * a.scale, dq[db][4 * g + 1] * a.scale);
-                w[1] = N::pack2(dq[db][4 * g + 2] * a.scale, dq[db][4 * g + 3] * a.scale);
+                w[0] = N::pack2(dq[db][4 * g] * scale, dq[db][4 * g + 1] * scale);
+                w[1] = N::pack2(dq[db][4 * g + 2] * scale, dq[db][4 * g + 3] * scale);
                 *reinterpret_cast<u32x2 *>(dQh + (size_t)my_q * dq_rs + 32 * db + 8 * g + 4 * half) = w;
             }
     }
@@ -1021,8 +1111,15 @@ hipError_t launch_bwd(const FaBwdArgs &a_in, int compute_units, hipStream_t stre
     const int all_heads = a.B * a.Hk, group = a.Hk > 0 ? a.H / a.Hk : 1;
     a.head0 = 0;
     a.heads = all_heads;
-    const int smem_dq = kBwdStages * 2 * TILEB, smem_dkdv = kBwdStages * (2 * TILEB + 512) + (DROPOUT ? kBwdWaves * 128 : 0);
-    const int smem_dkdv_ds = smem_dkdv + (D == 128 ? (DROPOUT ? FA_PARK_DROP : ALIBI ? 2 : 1) * 32 * kBwdWaves * 64 : 0);      // + the parked fragments
+    const int smem_dq = kBwdStages * 2 * TILEB;
+    auto smem_kv = [](int waves) { return kBwdStages * (2 * TILEB + 512) + (DROPOUT ? waves * 1024 : 0) + fa_bwd_parked(D, DROPOUT) * 16 * waves * 64; };
+    const int smem_dkdv = smem_kv(kBwdWaves);
+    // The key-owning kernel of the five-product form, head dimension 64: four waves, 128 keys, two workgroups per CU, whose
+    // waves wait at barriers of their own.  Backward pass, four waves against eight: causal B8 H16 S1000 94 against 97 us, B4
+    // H16 S2048 150 / 153, window 700 B1 H32 S8192 249 / 254, no mask B16 H16 S512 96 / 100, without a mask and ALiBi B23 H32
+    // S256 90 / 95; B6 H32/8 S4096 1698 / 1670 and B32 H8 S300 45 / 42 the other way.
+    constexpr int NWK = D == 64 ? 4 : kBwdWaves, KEYS_K = 32 * NWK, GROUPS_K = kBwdWaves / NWK;
+    const int smem_dkdv_ds = smem_kv(NWK);
     auto kq = fa_bwd_dq<BF16, D, MASKED, LAYOUT, ALIBI, DROPOUT>;
     auto kkv = fa_bwd_dkdv<BF16, D, MASKED, LAYOUT, ALIBI, DROPOUT>;
     // the five-product form: regular lengths (the reference's layout or a strided one) with dropout or ALiBi, any
@@ -1041,12 +1138,12 @@ hipError_t launch_bwd(const FaBwdArgs &a_in, int compute_units, hipStream_t stre
         e = hipFuncSetAttribute(reinterpret_cast<const void *>(kkv), hipFuncAttributeMaxDynamicSharedMemorySize, smem_dkdv);
         if (e != hipSuccess) return e;
         if constexpr (FIVE) {
-            e = hipFuncSetAttribute(reinterpret_cast<const void *>(fa_bwd_dkdv<BF16, D, MASKED, FL, ALIBI, DROPOUT, true>),
+            e = hipFuncSetAttribute(reinterpret_cast<const void *>(fa_bwd_dkdv<BF16, D, MASKED, FL, ALIBI, DROPOUT, true, false, NWK>),
                                     hipFuncAttributeMaxDynamicSharedMemorySize, smem_dkdv_ds);
             if (e != hipSuccess) return e;
             if constexpr (CAN_SHARE) {
                 e = hipFuncSetAttribute(reinterpret_cast<const void *>(fa_bwd_dkdv<BF16, D, MASKED, FL, ALIBI, DROPOUT, true, true>),
-                                        hipFuncAttributeMaxDynamicSharedMemorySize, smem_dkdv_ds);
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, smem_dkdv);
                 if (e != hipSuccess) return e;
             }
             e = hipFuncSetAttribute(reinterpret_cast<const void *>(fa_bwd_dq_from_ds<BF16, D, MASKED, FL, 8, 3>),
@@ -1077,9 +1174,9 @@ hipError_t launch_bwd(const FaBwdArgs &a_in, int compute_units, hipStream_t stre
     // fragments in LDS and compiles with it without spilling, or with 12 bytes outside the tile loop.)
     const bool uneven_items = MASKED && fa_bwd_uneven(a.S, a.Sk, a.L, a.R);
     const bool uneven = (LAYOUT == 0 || D == 64) && uneven_items;
-    auto grid_if = [&](bool snake, long long items) {
-        const unsigned g = (unsigned)items;
-        return (snake && g > resident && g < 16u * resident) ? resident : g;
+    auto grid_if = [&](bool snake, long long items, unsigned groups_per_cu = 1u) {
+        const unsigned g = (unsigned)items, all = groups_per_cu * resident;
+        return (snake && g > all && g < 16u * all) ? all : g;
     };
     auto grid_for = [&](long long items) { return grid_if(uneven, items); };
     if constexpr (FIVE) {
@@ -1093,18 +1190,18 @@ hipError_t launch_bwd(const FaBwdArgs &a_in, int compute_units, hipStream_t stre
             for (int h0 = 0; h0 < all_heads; h0 += chunk) {
                 a.head0 = h0;
                 a.heads = all_heads - h0 < chunk ? all_heads - h0 : chunk;
-                const unsigned launch_k = grid_if(FA_DS_LOOP ? uneven_items : uneven, (long long)a.heads * ((a.Sk + 255) / 256));
+                const unsigned launch_k = grid_if(FA_DS_LOOP ? uneven_items : uneven, (long long)a.heads * ((a.Sk + KEYS_K - 1) / KEYS_K), GROUPS_K);
                 unsigned n_shares = 0;
                 if constexpr (CAN_SHARE) {
                     if (a.partials != nullptr) n_shares = (unsigned)fa_bwd_launch_shares(a.heads, group, a.S, a.R, a.L, a.walk_head, (int)resident, a.share_slots);
                     if (n_shares != 0) {
                         a.walk_total = a.heads * a.walk_head;
-                        hipLaunchKernelGGL((fa_bwd_dkdv<BF16, D, MASKED, FL, ALIBI, DROPOUT, true, true>), dim3(n_shares), dim3(kBwdWaves * 64), smem_dkdv_ds, stream, a);
+                        hipLaunchKernelGGL((fa_bwd_dkdv<BF16, D, MASKED, FL, ALIBI, DROPOUT, true, true>), dim3(n_shares), dim3(kBwdWaves * 64), smem_dkdv, stream, a);
                         hipLaunchKernelGGL((fa_bwd_add_parts<BF16, D, FL >= 1>), dim3((n_shares - 1) * 2 * kBwdWaves), dim3(256), 0, stream, a, (int)n_shares);
                     }
                 }
                 if (n_shares == 0)
-                    hipLaunchKernelGGL((fa_bwd_dkdv<BF16, D, MASKED, FL, ALIBI, DROPOUT, true>), dim3(launch_k), dim3(kBwdWaves * 64), smem_dkdv_ds, stream, a);
+                    hipLaunchKernelGGL((fa_bwd_dkdv<BF16, D, MASKED, FL, ALIBI, DROPOUT, true, false, NWK>), dim3(launch_k), dim3(NWK * 64), smem_dkdv_ds, stream, a);
                 // Fewer than two 256-query items per CU: 128-query ones, twice as many, and a deeper ring, since a CU that
                 // walks one item waits for the latency of its tiles.  Backward pass, causal, 128 against 256 queries: B2 H16
                 // S2048 D128 (256 items) 162 against 177 us, B1 H8 S2048 D128 88 against 97, B1 H4 S4096 D64 86 against 98, B1 H16
