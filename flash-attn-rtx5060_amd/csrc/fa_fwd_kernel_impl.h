@@ -27,9 +27,11 @@
 //    wave's own exp/max/convert work issues in the gaps (the reference runs
 //    QK, softmax and PV back to back, flash_forward.h:193-315).
 //  * exp2 with scale*log2(e) folded into one FMA, the rescale of O done only
-//    when a row maximum has grown by more than 2^8 (the reference recomputes
-//    the factor 4*d/8 times per tile, flash_forward.h:296-299), the -inf
-//    guard the reference lacks (softmax.h:55,83).
+//    when the reference point of a row's exponentials has fallen far behind
+//    (the reference recomputes the factor 4*d/8 times per tile,
+//    flash_forward.h:296-299): a row maximum is taken on masked tiles only,
+//    elsewhere the tile's row sums tell; the -inf guard the reference lacks
+//    (softmax.h:55,83).
 //  * Masks are evaluated per element only on tiles that straddle a mask edge,
 //    and tiles that are fully masked for a wave are skipped by that wave (the
 //    reference masks every tile, mask.h:10-84).
@@ -48,14 +50,9 @@
 #include "fa_kernel_args.h"
 #include "fa_sched.h"
 
-// The row maximum of a tile's scores is taken next to this many of the iteration's first matrix instructions
-// (0: in front of them).
 #ifndef FA_S1K
 #define FA_S1K 3
 #define FA_S1V 2
-#endif
-#ifndef FA_ROW_MAX_SLOTS
-#define FA_ROW_MAX_SLOTS 4
 #endif
 
 namespace {
@@ -74,6 +71,8 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 constexpr int kBlockKeys = 64;          // keys per K/V tile
 constexpr float kNoReference = -1.0e30f; // reference point of a row before its first visible score
 constexpr float kRescaleLog2 = 8.0f;    // rescale O only when a row max grew by > 2^8
+constexpr float kTileSum = 4096.0f;     // ... or when half a row's exponentials of one tile add up to more than this (P stays far
+                                        // below fp16's 65504; larger than 2^8 so that a reference taken from a few keys holds)
 
 template <bool BF16> struct Num;
 template <> struct Num<false> {
@@ -422,7 +421,17 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
     constexpr int NPV = 4 * DB;                   // V^T fragments per tile: (16-key slice, head-dim block)
     constexpr int NQK = 2 * KS;                   // K fragments per tile: (head-dim slice, 32-key block)
     constexpr int NF = NPV + NQK;                 // every fragment feeds one matrix instruction
-    constexpr int PD = 6;                         // LDS reads run this many fragments ahead
+    // The reference point of a row's exponentials follows its tiles' sums instead of their maxima (see steady): sixteen
+    // three-way maxima, a half swap and the move itself, about thirty of 160 vector instructions per wave and tile, leave the
+    // loop; the scores then stay in registers to the iteration's end.  Against the maxima, us: c2 (B4 H16 S2048 D64) 54.2 /
+    // 52.1, c3 (B2 H32 S8192 D128) 1039 / 1022, c5 15195 / 14842, B4 H32/8 S2000 D64 no mask 181.6 / 171.8, S8100 D128
+    // 545 / 532, chunk B2 H32/8 S1000 S_kv 9000 277 / 268; level for one to four tiles a row and for windows.  With ALiBi the
+    // 128-wide kernels have no registers for it (a training step of B5 H16 S2637 bf16 892 / 948), with dropout the words drawn
+    // for the tile have to stay as well (B16 H16 S512 D64 146.0 / 147.4): both keep the maxima.
+    constexpr bool BY_SUM = !ALIBI && !DROPOUT;
+    // LDS reads run this many fragments ahead (general 128-wide kernels: three, or the scores that stay are spilled; with
+    // four, 12 bytes, chunk_prefill's shape 54.8 us against 53.2)
+    constexpr int PD = GENERAL && D == 128 && BY_SUM ? 3 : 6;
     constexpr int LA = NST - 1;                   // K tiles are requested LA iterations before their first use
     constexpr int LAV = NSTV - 1;                 // V tiles likewise (NSTV V stages: as many as K stages, or one fewer)
     constexpr int STAGES = NST + NSTV;
@@ -847,21 +856,45 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
         // instructions, two rounds each, they measured 1-5 % slower: with dropout the iteration is bound by the
         // vector ALU, not by the matrix pipe it would be hiding behind.)
         if (DROPOUT) draw_dropout(tile);
-        // the fragments are in flight; the row maxima need no matrix instruction and cover their latency
-        if (MASKED && tile_class(tile) == 1) apply_mask(tile);
-        // The row maximum rides along with the first MAXG matrix instructions of PV(tile-1), which do not depend on
-        // it (a quarter of the 32 scores per lane each); the reference point moves behind the last of them, without
-        // a branch: a factor of exactly 1 where it stays.  The exponentials follow over the remaining instructions.
-        constexpr int MAXG = FA_ROW_MAX_SLOTS;
-        static_assert(MAXG == 0 || (16 % MAXG == 0 && MAXG < NPV), "row-maximum slots");
         bool moved = false;
-        float alpha = 1.0f, nmc = 0.0f, mx = 0.0f;
-        if (MAXG == 0) {
-            alpha = new_reference(row_max(), moved);
-            nmc = -m_run * cs;
+        float alpha = 1.0f;
+        if (MASKED && tile_class(tile) == 1) {
+            apply_mask(tile);
+            // (BY_SUM: under a window the first keys that a row sees may be these, and without a maximum the tile would be done
+            // twice: windows of 300 keys, B2 H16 S8100 D64 72.0 us without this, 69.5 with it.  At a left edge only: no faster)
+            if (BY_SUM) alpha = new_reference(row_max(), moved);
         }
+        // BY_SUM: no row maximum otherwise.  The exponentials are taken against the reference point as it stands, and a tile that
+        // should have moved it shows in its row sums, which are needed anyway (see behind the matrix instructions).
+        // Otherwise the row maximum rides along with the first MAXG matrix instructions of PV(tile-1), which do not depend
+        // on it (a quarter of the 32 scores per lane each); the reference point moves behind the last of them, without
+        // a branch: a factor of exactly 1 where it stays.  The exponentials follow over the remaining instructions.
+        constexpr int MAXG = BY_SUM ? 0 : 4;
+        static_assert(MAXG == 0 || (16 % MAXG == 0 && MAXG < NPV), "row-maximum slots");
+        float nmc = -m_run * cs, mx = 0.0f, t_a = 0.0f, t_b = 0.0f;
         uint32_t pn[16];                           // P(tile), becomes pk at the end
         f32x16 nx[2];                              // S^T(tile+1)
+        // pair e: elements (2e, 2e+1) of key block 0 for e < 8, of key block 1 for e >= 8.  The two empty asm statements pin
+        // the arithmetic between the surrounding matrix instructions (without them the compiler sinks all of it to the end
+        // of the iteration); the first goes through the subtrahend, which stays in one register, so it costs no move.
+        auto pair = [&](int e) __attribute__((always_inline)) {
+            const float x0 = e < 8 ? sx[0][2 * e] : sx[1][2 * (e - 8)];
+            const float x1 = e < 8 ? sx[0][2 * e + 1] : sx[1][2 * (e - 8) + 1];
+            asm volatile("" : "+v"(nmc));
+            const float e0 = __builtin_amdgcn_exp2f(__builtin_fmaf(x0, c, nmc));
+            const float e1 = __builtin_amdgcn_exp2f(__builtin_fmaf(x1, c, nmc));
+            uint32_t packed = N::pack2(dropped(e0, e >> 3, 2 * (e & 7)), dropped(e1, e >> 3, 2 * (e & 7) + 1));
+            if (BY_SUM) {
+                t_a = e == 0 ? e0 : t_a + e0;
+                t_b = e == 0 ? e1 : t_b + e1;
+                asm volatile("" : "+v"(packed), "+v"(t_a), "+v"(t_b));
+            } else {
+                l_a += e0;
+                l_b += e1;
+                asm volatile("" : "+v"(packed), "+v"(l_a), "+v"(l_b));
+            }
+            pn[e] = packed;
+        };
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int g = 0; g < NF; ++g) {
@@ -899,27 +932,29 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
             }
             // softmax work riding along: the 16 element pairs of this tile spread over the matrix instructions
             constexpr int PAIRS = 16;
-            const int p_begin = ((g - MAXG) * PAIRS) / (NF - MAXG), p_end = ((g - MAXG + 1) * PAIRS) / (NF - MAXG);
 #pragma unroll
-            for (int e = p_begin; e < p_end; ++e) {
-                // pair e: elements (2e, 2e+1) of key block 0 for e < 8, of key block 1 for e >= 8.  The two empty
-                // asm statements pin the arithmetic between the surrounding matrix instructions (without them the
-                // compiler sinks all of it to the end of the iteration); the first goes through the subtrahend,
-                // which stays in one register, so it costs no move.
-                const float x0 = e < 8 ? sx[0][2 * e] : sx[1][2 * (e - 8)];
-                const float x1 = e < 8 ? sx[0][2 * e + 1] : sx[1][2 * (e - 8) + 1];
-                asm volatile("" : "+v"(nmc));
-                const float e0 = __builtin_amdgcn_exp2f(__builtin_fmaf(x0, c, nmc));
-                const float e1 = __builtin_amdgcn_exp2f(__builtin_fmaf(x1, c, nmc));
-                l_a += e0;
-                l_b += e1;
-                uint32_t packed = N::pack2(dropped(e0, e >> 3, 2 * (e & 7)), dropped(e1, e >> 3, 2 * (e & 7) + 1));
-                asm volatile("" : "+v"(packed), "+v"(l_a), "+v"(l_b));
-                pn[e] = packed;
-            }
+            for (int e = ((g - MAXG) * PAIRS) / (NF - MAXG); e < ((g - MAXG + 1) * PAIRS) / (NF - MAXG); ++e) pair(e);
             __builtin_amdgcn_sched_barrier(0);
         }
         if (moved) scale_o(alpha);                 // rare; PV(tile-1) has been issued in full by now
+        if (BY_SUM) {
+            // A lane's sum beyond kTileSum, or a NaN: the reference point moves up to the tile's maximum and the tile's
+            // exponentials are taken again (P(tile) has not been used yet).
+            if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(t_a + t_b <= kTileSum)) != 0, 0)) {
+                mx = row_max();
+                const float m_new = mx > m_run ? mx : m_run;
+                alpha = __builtin_amdgcn_exp2f((m_run - m_new) * cs);
+                l_a *= alpha;
+                l_b *= alpha;
+                m_run = m_new;
+                nmc = -m_new * cs;
+                scale_o(alpha);
+#pragma unroll
+                for (int e = 0; e < 16; ++e) pair(e);
+            }
+            l_a += t_a;
+            l_b += t_b;
+        }
 #pragma unroll
         for (int i = 0; i < 16; ++i) pk[i] = pn[i];
         sx[0] = nx[0];

@@ -1,0 +1,85 @@
+"""The reference point of the forward kernels' exponentials where it has to move inside the tile loop: scores that grow
+along the keys by far more than one tile's sum may hold, rows whose first visible keys lie in their second tile, and NaN.
+
+Against the same attention in 64 bits.  Tolerances: P and O are rounded to the storage type once each, u = 2^-11 (fp16) or
+2^-8 (bf16) at most per value.  With growing scores a few keys carry a row, so O is as far off as two roundings of its
+largest terms: 4 u of the row's largest |V| for single values, 1.5 u in the 2-norm (about u expected)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    # B, H, Hk, S, D, dtype, causal, wl, bshd, growth per key (in units of the scaled score)
+    (1, 2, 2, 512, 64, "fp16", True, -1, False, 0.4),      # every tile moves the reference point
+    (1, 2, 2, 512, 128, "bf16", False, -1, False, 0.4),
+    (1, 2, 1, 512, 128, "fp16", True, -1, True, 0.15),     # some do; strided kernels
+    (1, 2, 2, 500, 64, "bf16", True, -1, False, 0.3),      # general kernels
+    (1, 2, 2, 500, 128, "fp16", False, -1, True, 0.3),
+    (2, 16, 16, 2048, 128, "fp16", True, -1, False, 0.2),  # eight-wave workgroups
+    (2, 64, 64, 1200, 64, "fp16", True, 96, False, 0.2),   # windows: the first keys of a row in its block's second tile
+    (1, 2, 2, 1024, 128, "fp16", True, 65, False, 0.1),
+    (1, 2, 2, 512, 64, "fp16", False, -1, False, -0.4),    # the first tile holds the maximum: nothing moves
+]
+
+
+def _inputs(B, H, Hk, S, D, dtype, growth, bshd, seed):
+    import torch
+    g = torch.Generator().manual_seed(seed)
+    dt = torch.bfloat16 if dtype == "bf16" else torch.float16
+    q, k, v = (torch.randn((B, n, S, D), generator=g) for n in (H, Hk, Hk))
+    q[..., 0] = 8.0
+    k[..., 0] = torch.arange(S) * (growth * D ** 0.5 / 8.0)          # score of key j: growth * j + noise
+    q, k, v = (x.to(dt) for x in (q, k, v))
+    dev = [x.cuda() for x in (q, k, v)]
+    if bshd:
+        dev = [x.transpose(1, 2).contiguous().transpose(1, 2) for x in dev]
+    return (q, k, v), dev
+
+
+def _exact(q, k, v, causal, wl):
+    import torch
+    B, H, S, D = q.shape
+    group = H // k.shape[1]
+    kk, vv = (x.double().repeat_interleave(group, dim=1) for x in (k, v))
+    s = q.double() @ kk.transpose(2, 3).contiguous() / D ** 0.5
+    i, j = torch.arange(S)[:, None], torch.arange(S)[None, :]
+    if causal:
+        s.masked_fill_(j > i, -np.inf)
+    if wl >= 0:
+        s.masked_fill_(j < i - wl, -np.inf)
+    return torch.softmax(s, dim=-1) @ vv, torch.logsumexp(s, dim=-1)
+
+
+@pytest.mark.parametrize("B,H,Hk,S,D,dtype,causal,wl,bshd,growth", CASES)
+def test_reference_point_moves(fa, B, H, Hk, S, D, dtype, causal, wl, bshd, growth):
+    import torch
+    (q, k, v), (dq, dk, dv) = _inputs(B, H, Hk, S, D, dtype, growth, bshd, 31 + S + D)
+    o, lse = fa.flash_attention_forward(dq, dk, dv, causal=causal, window_left=wl, exact_first_rows=True)
+    torch.cuda.synchronize()
+    heads = slice(0, 2 * (H // Hk)), slice(0, 2)                      # (the first and last batch's first heads are enough)
+    for b in {0, B - 1}:
+        want, want_lse = _exact(q[b:b + 1, heads[0]], k[b:b + 1, heads[1]], v[b:b + 1, heads[1]], causal, wl)
+        got = o[b:b + 1, heads[0]].cpu().double()
+        u = 2.0 ** -8 if dtype == "bf16" else 2.0 ** -11
+        assert bool(torch.isfinite(got).all())
+        assert float((got - want).norm() / want.norm()) <= 1.5 * u
+        assert float((got - want).abs().max()) <= 4 * u * float(v.abs().max())
+        # fp32 sums of products of |q k| up to the largest score, 2^-24 each of D terms at most
+        bound = 2.0 ** -24 * D * float(want_lse.abs().max()) + 1e-5
+        assert float((lse[b:b + 1, heads[0]].cpu().double() - want_lse).abs().max()) <= bound
+
+
+@pytest.mark.parametrize("S,D", [(512, 64), (512, 128), (500, 64), (500, 128)])
+def test_nan_key_reaches_only_the_rows_that_see_it(fa, S, D):
+    """A NaN in key 300 of a causal problem: rows from 300 on are NaN, the others what they are without it."""
+    import torch
+    _, (q, k, v) = _inputs(1, 2, 2, S, D, "fp16", 0.02, False, 77)
+    clean, clean_lse = fa.flash_attention_forward(q, k, v, causal=True)
+    k = k.clone()
+    k[:, :, 300, 5] = float("nan")
+    o, lse = fa.flash_attention_forward(q, k, v, causal=True)
+    torch.cuda.synchronize()
+    assert bool(torch.isnan(o[:, :, 300:]).all())
+    assert float((o[:, :, :300].float() - clean[:, :, :300].float()).norm() / clean[:, :, :300].float().norm()) <= 1.5 * 2.0 ** -11
+    assert float((lse[:, :, :300] - clean_lse[:, :, :300]).abs().max()) <= 1e-5
