@@ -1157,7 +1157,8 @@ hipError_t launch_bwd(const FaBwdArgs &a_in, int compute_units, hipStream_t stre
     constexpr bool FIVE = LAYOUT <= 1 || (!ALIBI && !DROPOUT);
     constexpr int FL = FIVE ? LAYOUT : 0;
     constexpr bool CAN_SHARE = FIVE && fa_bwd_can_share(D, DROPOUT);
-    // the query-owning kernel from dS blocks: 8 waves (256 queries) and three LDS stages, or 4 waves and four stages
+    // the query-owning kernel from dS blocks: 8 waves (256 queries) and three LDS stages, or 4 waves and four stages, or, at
+    // head dimension 64, 4 waves and three stages, two workgroups per CU
     auto smem_dq_ds = [](int waves, int stages) { return stages * (TILEB + waves * 2 * kDsBlockBytes); };
     // the LDS opt-in is per (instantiation, device) and is made once, not on every launch
     static std::atomic<unsigned long long> configured{0ull};
@@ -1176,9 +1177,16 @@ hipError_t launch_bwd(const FaBwdArgs &a_in, int compute_units, hipStream_t stre
                                         hipFuncAttributeMaxDynamicSharedMemorySize, smem_dkdv);
                 if (e != hipSuccess) return e;
             }
-            e = hipFuncSetAttribute(reinterpret_cast<const void *>(fa_bwd_dq_from_ds<BF16, D, MASKED, FL, 8, 3>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, smem_dq_ds(8, 3));
-            if (e != hipSuccess) return e;
+            if constexpr (D == 128 || MASKED) {
+                e = hipFuncSetAttribute(reinterpret_cast<const void *>(fa_bwd_dq_from_ds<BF16, D, MASKED, FL, 8, 3>),
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, smem_dq_ds(8, 3));
+                if (e != hipSuccess) return e;
+            }
+            if constexpr (D == 64) {
+                e = hipFuncSetAttribute(reinterpret_cast<const void *>(fa_bwd_dq_from_ds<BF16, D, MASKED, FL, 4, 3>),
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, smem_dq_ds(4, 3));
+                if (e != hipSuccess) return e;
+            }
             e = hipFuncSetAttribute(reinterpret_cast<const void *>(fa_bwd_dq_from_ds<BF16, D, MASKED, FL, 4, 4>),
                                     hipFuncAttributeMaxDynamicSharedMemorySize, smem_dq_ds(4, 4));
             if (e != hipSuccess) return e;
@@ -1240,7 +1248,16 @@ hipError_t launch_bwd(const FaBwdArgs &a_in, int compute_units, hipStream_t stre
                 if (items_q < 2LL * compute_units) {
                     const unsigned launch_q = grid_if(uneven_items, heads_q * ((a.S + 127) / 128));
                     hipLaunchKernelGGL((fa_bwd_dq_from_ds<BF16, D, MASKED, FL, 4, 4>), dim3(launch_q), dim3(4 * 64), smem_dq_ds(4, 4), stream, a);
-                } else {
+                } else if (D == 64 && !uneven_items) {
+                    // 64-wide and items alike: 128-query ones, two workgroups per CU that wait at barriers and for their first
+                    // tiles at different times.  Backward pass, 128 against 256 queries: no mask B16 H16 S512 96.5 / 101.4 us,
+                    // with dropout 113.8 / 117.7, B2 H16 S8192 2064 / 2080, window 700 B2 H32 S8192 501 / 508.  Causal items,
+                    // which K read twice as often and shorter pairs of the snake cost more: B4 H16 S2048 151.5 / 149.5,
+                    // B16 H16 S1024 196.0 / 194.6, B6 H32/8 S4096 1741 / 1730; B8 H32 S1024 189.0 / 193.4 the other way.
+                    if constexpr (D == 64)
+                        hipLaunchKernelGGL((fa_bwd_dq_from_ds<BF16, D, MASKED, FL, 4, 3>), dim3((unsigned)(heads_q * ((a.S + 127) / 128))), dim3(4 * 64),
+                                           smem_dq_ds(4, 3), stream, a);
+                } else if constexpr (D == 128 || MASKED) {
                     const unsigned launch_q = grid_if(uneven_items, items_q);
                     hipLaunchKernelGGL((fa_bwd_dq_from_ds<BF16, D, MASKED, FL, 8, 3>), dim3(launch_q), dim3(8 * 64), smem_dq_ds(8, 3), stream, a);
                 }

@@ -1,5 +1,5 @@
-"""The query-owning kernel over dS blocks in its two sizes (128 queries and a ring of four stages below two 256-query items
-per CU, 256 and three otherwise) at the edges of blocks, tiles and the ring, against torch autograd in fp64 on the CPU."""
+"""The query-owning kernel over dS blocks in its three sizes (128 queries and a ring of four stages below two 256-query items
+per CU, 128 and three at head dimension 64 with items alike, 256 and three otherwise) at the edges of blocks, tiles and the ring, against torch autograd in fp64 on the CPU."""
 import pytest
 
 from test_gpu_parity_bwd import check, grad_errors, torch_grads_f64
@@ -17,6 +17,9 @@ CASES = [
     (2, 130, 130, 510, 64, 0, True, -1, False),      # 520 items: 256-query blocks, ragged
     (2, 129, 43, 512, 128, 1, False, -1, True),      # 516 items, grouped heads
     (1, 255, 255, 511, 64, 0, True, -1, False),      # 510 items: 128-query blocks, as a snake over the CUs
+    (2, 256, 256, 128, 64, 1, False, -1, True),      # items alike: one 128-query block, as many tiles as requested ahead
+    (1, 512, 256, 129, 64, 0, False, -1, False),     # a second block of one query, three tiles, grouped heads
+    (1, 171, 171, 600, 64, 0, True, 70, True),       # a window: tiles outside a wave's range
 ]
 
 
