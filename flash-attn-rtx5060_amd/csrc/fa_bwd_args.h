@@ -13,7 +13,7 @@ struct FaBwdArgs {
     const uint16_t *Q, *K, *V, *O, *dO;
     const float *lse;                       // [B,H,S] contiguous, natural log, as the forward pass writes it
     // scratch [B,H,S] each, written by fa_bwd_dq or fa_bwd_prepare for the key-owning kernel, whose accumulators start from
-    // them: -(sum_t dO*O) / drop_scale per row, and -lse / scale, -inf for rows that saw no key (P is then 0)
+    // them: -(sum_t dO*O) / drop_scale per row, and (ln(drop_scale) - lse) / scale, -inf for rows that saw no key (P is then 0)
     float *delta;
     float *lse2;
     uint16_t *dQ, *dK, *dV;
@@ -40,7 +40,7 @@ struct FaBwdArgs {
     int L, R;                               // key j visible to the query at position p iff p - L <= j <= p + R
     float scale;
     unsigned drop_threshold;                // dropout: keep iff the key's byte >= threshold (p in units of 1/256); 0 = none
-    float drop_scale;                       // 256 / (256 - threshold)
+    float drop_scale, drop_log;             // 256 / (256 - threshold) and its natural logarithm; 1 and 0 without dropout
     unsigned seed_lo, seed_hi;
 };
 

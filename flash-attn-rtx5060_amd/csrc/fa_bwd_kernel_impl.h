@@ -272,7 +272,7 @@ __global__ void __launch_bounds__(kBwdWaves * 64, 2) fa_bwd_dq(const FaBwdArgs a
         delta += swap_halves(delta);
         if (row_ok && half == 0) {
             a.delta[(size_t)bh * S + my_q] = -delta / a.drop_scale;
-            a.lse2[(size_t)bh * S + my_q] = (GENERAL && lse_raw == -INFINITY) ? -INFINITY : -lse_raw / a.scale;
+            a.lse2[(size_t)bh * S + my_q] = (GENERAL && lse_raw == -INFINITY) ? -INFINITY : (a.drop_log - lse_raw) / a.scale;
         }
     }
     const float c = a.scale * kLog2e;
@@ -604,7 +604,10 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_bwd_dkdv(const FaBwdArgs a)
             }
         };
         f32x16 sx, dp;
-        // the accumulators of block qb start from what the row's exponent and row sum subtract: -lse / scale, -delta
+        // the accumulators of block qb start from what the row's exponent and row sum subtract: -lse / scale, -delta.  With
+        // dropout from (ln(1 / (1 - p)) - lse) / scale and -delta (1 - p): P then carries the factor 1 / (1 - p) that both dV
+        // and dS need before they are rounded to the storage type (a factor at the end would leave fp16's subnormal range
+        // 1 / (1 - p) times larger: dK and dQ at p = 0.9, dO of 1e-3, nine times as far off)
         auto start = [&](f32x16 &acc, int qb, uint32_t at) __attribute__((always_inline)) {
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
@@ -657,7 +660,7 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_bwd_dkdv(const FaBwdArgs a)
                     float x = sx[r] * c;
                     if (ALIBI) x = __builtin_fmaf(-slope_l2, __builtin_fabsf((float)(first + 8 * (r >> 2) + (r & 3) + off - my_k)), x);
                     sx[r] = __builtin_amdgcn_exp2f(x);
-                    pd[e] = !DROPOUT || keeps(r) ? sx[r] : 0.0f;         // (the factor 1 / (1 - p): once, at the end)
+                    pd[e] = !DROPOUT || keeps(r) ? sx[r] : 0.0f;
                 }
                 pp[i] = N::pack2(pd[0], pd[1]);
                 asm volatile("" : "+v"(pp[i]));
@@ -674,7 +677,7 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_bwd_dkdv(const FaBwdArgs a)
                 for (int e = 0; e < 2; ++e) {
                     const int r = 2 * i + e;
                     float dpr = dp[r];
-                    if (DROPOUT) dpr = (keeps(r) ? dpr : 0.0f) + del[r & 3];       // (both in units of 1 / (1 - p))
+                    if (DROPOUT) dpr = (keeps(r) ? dpr : 0.0f) + del[r & 3];       // (in units of 1 / (1 - p), the factor that P has)
                     v[e] = sx[r] * dpr;
                 }
                 ds[i] = N::pack2(v[0], v[1]);     // dS, same operand order
@@ -852,11 +855,10 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_bwd_dkdv(const FaBwdArgs a)
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 u32x2 wk, wv;
-                const float ks = DROPOUT ? a.scale * a.drop_scale : a.scale, vs = DROPOUT ? a.drop_scale : 1.0f;
-                wk[0] = N::pack2(dk[db][4 * g] * ks, dk[db][4 * g + 1] * ks);
-                wk[1] = N::pack2(dk[db][4 * g + 2] * ks, dk[db][4 * g + 3] * ks);
-                wv[0] = N::pack2(dv[db][4 * g] * vs, dv[db][4 * g + 1] * vs);
-                wv[1] = N::pack2(dv[db][4 * g + 2] * vs, dv[db][4 * g + 3] * vs);
+                wk[0] = N::pack2(dk[db][4 * g] * a.scale, dk[db][4 * g + 1] * a.scale);
+                wk[1] = N::pack2(dk[db][4 * g + 2] * a.scale, dk[db][4 * g + 3] * a.scale);
+                wv[0] = N::pack2(dv[db][4 * g], dv[db][4 * g + 1]);
+                wv[1] = N::pack2(dv[db][4 * g + 2], dv[db][4 * g + 3]);
                 *reinterpret_cast<u32x2 *>(dKh + (size_t)key_e * dk_rs + 32 * db + 8 * g + 4 * half_e) = wk;
                 *reinterpret_cast<u32x2 *>(dVh + (size_t)key_e * dv_rs + 32 * db + 8 * g + 4 * half_e) = wv;
             }
@@ -871,7 +873,7 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_bwd_dkdv(const FaBwdArgs a)
 // still has exactly one writer and the same inputs give the same bits.  The price is S*S_kv storage-type elements
 // per head written once and read once, so this kernel is bound by HBM bandwidth, not by the matrix cores.
 //
-// fa_bwd_prepare: delta_i = sum_t dO_it O_it and the logsumexp in exp2 units, which fa_bwd_dkdv fetches per
+// fa_bwd_prepare: delta_i = sum_t dO_it O_it and the logsumexp, in the units that FaBwdArgs states, which fa_bwd_dkdv fetches per
 // query tile (fa_bwd_dq writes them in the seven-product form).
 // Bound by HBM: O and dO read once.  A workgroup takes kPrepareRows rows per thread of one head: the head is found once, by
 // scalar arithmetic (one row per thread found it with two 64-bit divisions each), and a thread has the loads of all its rows
@@ -933,7 +935,7 @@ __global__ void __launch_bounds__(256) fa_bwd_prepare(const FaBwdArgs a)
     }
     if (writes) {
         a.delta[row0 + mine] = -delta / a.drop_scale;
-        a.lse2[row0 + mine] = l == -INFINITY ? -INFINITY : -l / a.scale;
+        a.lse2[row0 + mine] = l == -INFINITY ? -INFINITY : (a.drop_log - l) / a.scale;
     }
     }
 }
@@ -969,7 +971,7 @@ __global__ void __launch_bounds__(256) fa_bwd_add_parts(const FaBwdArgs a, int n
     uint16_t *out = which == 0 ? (STRIDED ? head_ptr(a.dK, a.dk, b, hk) : a.dK + (size_t)bhk * S * D)
                                : (STRIDED ? head_ptr(a.dV, a.dv, b, hk) : a.dV + (size_t)bhk * S * D);
     const int rs = STRIDED ? (which == 0 ? a.dk.rs : a.dv.rs) : D, lane = (int)threadIdx.x % 64, key = kblock * 256 + wave * 32 + (lane & 31);
-    const float scale = (which == 0 ? a.scale : 1.0f) * a.drop_scale;      // (drop_scale is 1 without dropout)
+    const float scale = which == 0 ? a.scale : 1.0f;
     if (key >= S) return;
 #pragma unroll
     for (int n = 0; n < SLOTS; ++n) {
@@ -1119,14 +1121,13 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_bwd_dq_from_ds(const FaBwdArgs 
     }
     if (active && (!GENERAL || qw + l32 < S)) {
         const int my_q = qw + l32;
-        const float scale = a.scale * a.drop_scale;        // (the blocks hold dS in units of drop_scale, which is 1 without dropout)
 #pragma unroll
         for (int db = 0; db < DB; ++db)
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 u32x2 w;
-                w[0] = N::pack2(dq[db][4 * g] * scale, dq[db][4 * g + 1] * scale);
-                w[1] = N::pack2(dq[db][4 * g + 2] * scale, dq[db][4 * g + 3] * scale);
+                w[0] = N::pack2(dq[db][4 * g] * a.scale, dq[db][4 * g + 1] * a.scale);
+                w[1] = N::pack2(dq[db][4 * g + 2] * a.scale, dq[db][4 * g + 3] * a.scale);
                 *reinterpret_cast<u32x2 *>(dQh + (size_t)my_q * dq_rs + 32 * db + 8 * g + 4 * half) = w;
             }
     }

@@ -1016,6 +1016,7 @@ int fa_bwd_shared(const fa_bwd_params *p, void *partials, unsigned long long par
     a.scale = p->softmax_scale;
     a.drop_threshold = (unsigned)fa_dropout_threshold(p->dropout_prob);
     a.drop_scale = 256.0f / (256.0f - (float)a.drop_threshold);
+    a.drop_log = logf(a.drop_scale);
     a.seed_lo = (unsigned)(p->seed & 0xffffffffull);
     a.seed_hi = (unsigned)(p->seed >> 32);
     const int masked = (general || a.L < far || a.R < far) ? 1 : 0;
