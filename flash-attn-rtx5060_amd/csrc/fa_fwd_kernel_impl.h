@@ -29,9 +29,9 @@
 //  * exp2 with scale*log2(e) folded into one FMA, the rescale of O done only
 //    when the reference point of a row's exponentials has fallen far behind
 //    (the reference recomputes the factor 4*d/8 times per tile,
-//    flash_forward.h:296-299): a row maximum is taken on masked tiles only,
-//    elsewhere the tile's row sums tell; the -inf guard the reference lacks
-//    (softmax.h:55,83).
+//    flash_forward.h:296-299): a row maximum is taken on masked tiles and in
+//    items whose scores have proved sharp, elsewhere the tile's row sums tell;
+//    the -inf guard the reference lacks (softmax.h:55,83).
 //  * Masks are evaluated per element only on tiles that straddle a mask edge,
 //    and tiles that are fully masked for a wave are skipped by that wave (the
 //    reference masks every tile, mask.h:10-84).
@@ -71,8 +71,10 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 constexpr int kBlockKeys = 64;          // keys per K/V tile
 constexpr float kNoReference = -1.0e30f; // reference point of a row before its first visible score
 constexpr float kRescaleLog2 = 8.0f;    // rescale O only when a row max grew by > 2^8
-constexpr float kTileSum = 4096.0f;     // ... or when half a row's exponentials of one tile add up to more than this (P stays far
-                                        // below fp16's 65504; larger than 2^8 so that a reference taken from a few keys holds)
+// ... or, in the loop that takes no maxima (see steady), by > 2^14 (P stays below fp16's 65504): then half a row's exponentials of
+// one tile add up to more than kTileSum, which lies below 2^14 by more than their rounding
+constexpr float kLagLog2 = 14.0f, kTileSum = 15000.0f;
+constexpr int kFewTiles = 8;                // items of at most this many tiles take maxima from their start
 
 template <bool BF16> struct Num;
 template <> struct Num<false> {
@@ -422,12 +424,17 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
     constexpr int NQK = 2 * KS;                   // K fragments per tile: (head-dim slice, 32-key block)
     constexpr int NF = NPV + NQK;                 // every fragment feeds one matrix instruction
     // The reference point of a row's exponentials follows its tiles' sums instead of their maxima (see steady): sixteen
-    // three-way maxima, a half swap and the move itself, about thirty of 160 vector instructions per wave and tile, leave the
-    // loop; the scores then stay in registers to the iteration's end.  Against the maxima, us: c2 (B4 H16 S2048 D64) 54.2 /
-    // 52.1, c3 (B2 H32 S8192 D128) 1039 / 1022, c5 15195 / 14842, B4 H32/8 S2000 D64 no mask 181.6 / 171.8, S8100 D128
-    // 545 / 532, chunk B2 H32/8 S1000 S_kv 9000 277 / 268; level for one to four tiles a row and for windows.  With ALiBi the
-    // 128-wide kernels have no registers for it (a training step of B5 H16 S2637 bf16 892 / 948), with dropout the words drawn
-    // for the tile have to stay as well (B16 H16 S512 D64 146.0 / 147.4): both keep the maxima.
+    // three-way maxima, a half swap and the move itself, about thirty of the 140 vector instructions that the general 64-wide
+    // kernel's iteration has with maxima, leave the loop; the scores then stay in registers to the iteration's end.  A tile
+    // that the sums find too large is done again, which costs half an iteration: where scores are sharp (a standard deviation of
+    // eight) that happens to some row of a wave in most tiles, so from the first such tile on the rest of the item takes maxima,
+    // in a loop of its own, and so do items of few tiles.  Maxima throughout / sums alone / both loops, us, inputs of unit
+    // variance: B4 H16 S2048 D64 53.1 / 51.2 / 51.3, B2 H32 S8192 D128 1018 / 997 / 999, B4 H32/8 S2000 D64 no mask 175.5 /
+    // 166.4 / 167.5, B1 H32 S8100 D128 522 / 510 / 509, windows of 300 keys B2 H16 S8100 D64 69.5 / 69.2 / 70.2, B8 H16 S1000
+    // D64 38.8 / 37.9 / 39.0; Q eight times as large, in the same order: 54.1 / 59.2 / 56.5, 1001 / 1017 / 1009, 176 / 191 / 180,
+    // 509 / 515 / 511, 70.8 / 76.1 / 71.5, 40.3 / 44.7 / 41.3; sixteen times: 54.0 / 64.9 / 54.8.  With ALiBi the 128-wide
+    // kernels have no registers for it (a training step of B5 H16 S2637 bf16 892 / 948), with dropout the words drawn for the
+    // tile have to stay as well (B16 H16 S512 D64 146.0 / 147.4): both keep the maxima.
     constexpr bool BY_SUM = !ALIBI && !DROPOUT;
     // LDS reads run this many fragments ahead (general 128-wide kernels: three, or the scores that stay are spilled; with
     // four, 12 bytes, chunk_prefill's shape 54.8 us against 53.2)
@@ -687,6 +694,7 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
     // finite value far below every score: the first finite row maximum moves it, with a factor exp2(-huge) = 0
     // for the empty accumulators, and no place needs a test for -inf.)
     float m_run = kNoReference, l_a = 0.0f, l_b = 0.0f;
+    bool sharp = t1 - t0 < kFewTiles;      // BY_SUM: the rest of the item takes row maxima (see steady)
     // The tile scores stay raw dot products and the softmax scale is folded into the exponent (exp2(s*c - m*c)).
     // ALiBi (mask.h:21-26 subtracts slope*|i-j| from the scaled score) enters through the matrix instruction's
     // accumulator: the first product of a key block starts from -(slope/scale)*|i-j| instead of from zero, two
@@ -749,9 +757,14 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
     };
     // the decision to move the reference point; returns the factor by which everything accumulated so far has to
     // be multiplied (1 when the reference point stays)
+    // whether a row with maximum mx moves its reference point (from kNoReference every finite maximum does; BY_SUM: by the
+    // exponent as the elements have it)
+    auto grows = [&](float mx) __attribute__((always_inline)) {
+        return BY_SUM ? __builtin_fmaf(mx, cs, -m_run * cs) > kLagLog2 : mx > m_run + thresh;
+    };
     auto new_reference = [&](float mx, bool &moved) __attribute__((always_inline)) {
         float alpha = 1.0f;
-        const bool grow = mx > m_run + thresh;      // (from kNoReference every finite maximum grows)
+        const bool grow = grows(mx);
         moved = __builtin_amdgcn_ballot_w64(grow) != 0;
         if (moved) {
             const float m_new = grow ? mx : m_run;
@@ -840,7 +853,8 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
     };
 
     // ---- the steady-state iteration: PV(tile-1) from V stage VST, softmax(tile), QK(tile+1) from K stage KST
-    auto steady = [&](auto KST, auto VST, int vstage_rt, int tile) __attribute__((always_inline)) {
+    auto steady = [&](auto KST, auto VST, auto MAXIMA, int vstage_rt, int tile) __attribute__((always_inline)) {
+        constexpr bool BY_MAX = decltype(MAXIMA)::value != 0;
         constexpr uint32_t ks = decltype(KST)::value * TILEB;
         // (with as many V stages as K stages the V stage is a compile-time value like the K stage; with one fewer
         // the two cycle with different periods, and the V stage is a run-time offset added to the lanes' addresses)
@@ -860,16 +874,16 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
         float alpha = 1.0f;
         if (MASKED && tile_class(tile) == 1) {
             apply_mask(tile);
-            // (BY_SUM: under a window the first keys that a row sees may be these, and without a maximum the tile would be done
+            // (Without maxima: under a window the first keys that a row sees may be these, and without a maximum the tile would be done
             // twice: windows of 300 keys, B2 H16 S8100 D64 72.0 us without this, 69.5 with it.  At a left edge only: no faster)
-            if (BY_SUM) alpha = new_reference(row_max(), moved);
+            if (!BY_MAX) alpha = new_reference(row_max(), moved);
         }
-        // BY_SUM: no row maximum otherwise.  The exponentials are taken against the reference point as it stands, and a tile that
-        // should have moved it shows in its row sums, which are needed anyway (see behind the matrix instructions).
-        // Otherwise the row maximum rides along with the first MAXG matrix instructions of PV(tile-1), which do not depend
+        // Not BY_MAX: no row maximum otherwise.  The exponentials are taken against the reference point as it stands, and a tile
+        // that should have moved it shows in its row sums, which are needed anyway (see behind the matrix instructions).
+        // BY_MAX: the row maximum rides along with the first MAXG matrix instructions of PV(tile-1), which do not depend
         // on it (a quarter of the 32 scores per lane each); the reference point moves behind the last of them, without
         // a branch: a factor of exactly 1 where it stays.  The exponentials follow over the remaining instructions.
-        constexpr int MAXG = BY_SUM ? 0 : 4;
+        constexpr int MAXG = BY_MAX ? 4 : 0;
         static_assert(MAXG == 0 || (16 % MAXG == 0 && MAXG < NPV), "row-maximum slots");
         float nmc = -m_run * cs, mx = 0.0f, t_a = 0.0f, t_b = 0.0f;
         uint32_t pn[16];                           // P(tile), becomes pk at the end
@@ -915,7 +929,7 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
                 for (int r = g * PER + (g == 0 ? 1 : 0); r < (g + 1) * PER; ++r) mx = fmaxf(fmaxf(mx, sx[0][r]), sx[1][r]);
                 if (g == MAXG - 1) {
                     mx = max_of_halves(mx);
-                    const bool grow = mx > m_run + thresh;      // (from kNoReference every finite maximum grows)
+                    const bool grow = grows(mx);
                     moved = __builtin_amdgcn_ballot_w64(grow) != 0;
                     const float m_new = grow ? mx : m_run;
                     alpha = __builtin_amdgcn_exp2f((m_run - m_new) * cs);
@@ -938,19 +952,25 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
         }
         if (moved) scale_o(alpha);                 // rare; PV(tile-1) has been issued in full by now
         if (BY_SUM) {
-            // A lane's sum beyond kTileSum, or a NaN: the reference point moves up to the tile's maximum and the tile's
-            // exponentials are taken again (P(tile) has not been used yet).
-            if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(t_a + t_b <= kTileSum)) != 0, 0)) {
+            // A lane's sum beyond kTileSum, or a NaN: the reference points of the rows whose maximum asks for it move up to it, and
+            // the tile's exponentials are taken again (P(tile) has not been used yet).  A row moves by its own maximum alone, by
+            // the rule that a tile with maxima follows too: what it gives does not depend on the rows it shares a wave with, nor
+            // on which of the two loops its tiles went through.
+            if (!BY_MAX && __builtin_expect(__builtin_amdgcn_ballot_w64(!(t_a + t_b <= kTileSum)) != 0, 0)) {
                 mx = row_max();
-                const float m_new = mx > m_run ? mx : m_run;
-                alpha = __builtin_amdgcn_exp2f((m_run - m_new) * cs);
-                l_a *= alpha;
-                l_b *= alpha;
-                m_run = m_new;
-                nmc = -m_new * cs;
-                scale_o(alpha);
+                const bool grow = __builtin_fmaf(mx, c, nmc) > kLagLog2;
+                if (__builtin_amdgcn_ballot_w64(grow) != 0) {
+                    const float m_new = grow ? mx : m_run;
+                    alpha = __builtin_amdgcn_exp2f((m_run - m_new) * cs);
+                    l_a *= alpha;
+                    l_b *= alpha;
+                    m_run = m_new;
+                    nmc = -m_new * cs;
+                    scale_o(alpha);
+                    sharp = true;
 #pragma unroll
-                for (int e = 0; e < 16; ++e) pair(e);
+                    for (int e = 0; e < 16; ++e) pair(e);
+                }
             }
             l_a += t_a;
             l_b += t_b;
@@ -1047,7 +1067,7 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
         FA_RING_CHECK(i, j3, v_read, 3);
         finish_iteration(more_k, more_v, tv > t1);
     };
-    auto steady_iteration = [&](auto J3, int i, int jv) __attribute__((always_inline)) {
+    auto steady_iteration = [&](auto J3, auto MAXIMA, int i, int jv) __attribute__((always_inline)) {
         constexpr int j3 = decltype(J3)::value;
         constexpr int jm1 = (j3 + NST - 1) % NST, jm2 = (j3 + 2 * NST - 2) % NST, jm3 = (j3 + 3 * NST - 3) % NST;
         const int tk = i + 1 + LA, tv = i - 1 + LAV;
@@ -1062,7 +1082,7 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
 #endif
         if (NSTV == NST && more_v) issue_v(tv, v_fill);
         FA_RING_CHECK(i, j3, v_read, 1);
-        steady(IntC<j3>{}, IntC<jm2>{}, v_read, i);
+        steady(IntC<j3>{}, IntC<jm2>{}, MAXIMA, v_read, i);
         FA_RING_CHECK(i, j3, v_read, 5);
         finish_iteration(more_k, more_v, false);
     };
@@ -1082,17 +1102,24 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
         generic_iteration(i, j3, jv);
         advance();
     }
-    if (j3 == 1 && whole(i)) { steady_iteration(IntC<1>{}, i, jv); advance(); ++i; }
-    if (NST >= 3 && j3 == 2 && whole(i)) { steady_iteration(IntC<2 % NST>{}, i, jv); advance(); ++i; }
-    for (; j3 == 0 && whole(i) && whole(i + NST - 1); i += NST) {
-        steady_iteration(IntC<0>{}, i, jv);
+    // (single iterations in the general kernels take the maxima: 0-1 % faster than without, elsewhere 0-1 % slower)
+    typedef IntC<BY_SUM ? 0 : 1> Usual;
+    typedef IntC<BY_SUM && !GENERAL ? 0 : 1> Single;
+    if (j3 == 1 && whole(i)) { steady_iteration(IntC<1>{}, Single{}, i, jv); advance(); ++i; }
+    if (NST >= 3 && j3 == 2 && whole(i)) { steady_iteration(IntC<2 % NST>{}, Single{}, i, jv); advance(); ++i; }
+    auto turn = [&](auto MAXIMA) __attribute__((always_inline)) {
+        steady_iteration(IntC<0>{}, MAXIMA, i, jv);
         advance();
-        steady_iteration(IntC<1>{}, i + 1, jv);
+        steady_iteration(IntC<1>{}, MAXIMA, i + 1, jv);
         advance();
-        if (NST >= 3) { steady_iteration(IntC<2 % NST>{}, i + 2, jv); advance(); }
-    }
-    if (j3 == 0 && whole(i)) { steady_iteration(IntC<0>{}, i, jv); advance(); ++i; }
-    if (NST >= 3 && j3 == 1 && whole(i)) { steady_iteration(IntC<1>{}, i, jv); advance(); ++i; }
+        if (NST >= 3) { steady_iteration(IntC<2 % NST>{}, MAXIMA, i + 2, jv); advance(); }
+        i += NST;
+    };
+    while (!(BY_SUM && sharp) && j3 == 0 && whole(i) && whole(i + NST - 1)) turn(Usual{});
+    if (BY_SUM)                           // what is left once a tile had to be done again
+        while (j3 == 0 && whole(i) && whole(i + NST - 1)) turn(IntC<1>{});
+    if (j3 == 0 && whole(i)) { steady_iteration(IntC<0>{}, Single{}, i, jv); advance(); ++i; }
+    if (NST >= 3 && j3 == 1 && whole(i)) { steady_iteration(IntC<1>{}, Single{}, i, jv); advance(); ++i; }
     for (; i < t1; ++i) {                 // drain, up to the last two iterations
         generic_iteration(i, j3, jv);
         advance();
