@@ -411,8 +411,13 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_bwd_dkdv(const FaBwdArgs a)
     constexpr int BK = 32 * NW;                   // keys per workgroup
     constexpr int KS = Reader::KS, DB = Reader::DB, TILEB = Loader::TILEB, STAGEB = 2 * TILEB + 512, IPW = Loader::IPW;
     // LDS reads run this many matrix instructions ahead (at head dimension 128 what the registers hold: three with less of K
-    // in LDS, or with fewer address registers and an instruction more per read, measured 1-4 % slower on every shape tried)
-    constexpr int PD = D == 64 ? 4 : DROPOUT ? 1 : 2;
+    // in LDS, or with fewer address registers and an instruction more per read, measured 1-4 % slower on every shape tried).
+    // Masked walks with ALiBi, and masked shares in the reference's layout, hold one: with two they reload spilled values in
+    // every tile or walk, behind a wait for all loads and stores in flight.  Backward pass, causal, two ahead / one, us: ALiBi
+    // B2 H16 S4096 424 / 396, B4 H16 S2048 250 / 232, B1 H8 S2048 stored [B,S,H,D] (shares) 92.6 / 86.2, B1 H32/4 S2048 149.7 /
+    // 144.9 (B2 H32/8 S4096 840 / 853 the other way); without ALiBi, shares, B1 H8 S2048 87.0 / 86.0, B1 H16 S1024 66.4 / 64.2.
+    constexpr bool TIGHT = WRITE_DS && MASKED && (ALIBI || (LAYOUT == 0 && SHARES));
+    constexpr int PD = D == 64 ? 4 : DROPOUT || TIGHT ? 1 : 2;
     constexpr int NSTG = kBwdStages;                                  // LDS stages; pairs are requested NSTG - 1 ahead
     extern __shared__ __attribute__((aligned(1024))) char smem[];
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)smem;
@@ -546,7 +551,8 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_bwd_dkdv(const FaBwdArgs a)
     // spills to scratch memory inside the tile loop comes back behind a wait for ALL loads and stores in flight.  The last
     // PARKED of the K^T fragments, which every half tile uses once, are kept in LDS instead (a plane of 16 bytes per lane
     // each, written once per work item) and read like any A operand: K's, because dP, dS and P are not alive yet where they
-    // are used.  (One K and one V fragment, as before the reads ran ahead: spills of 80-360 bytes inside the loop.)
+    // are used.  (One K and one V fragment, as before the reads ran ahead: spills of 80-360 bytes inside the loop.  What is
+    // left of spills: see PD.)
     constexpr int PARKED = fa_bwd_parked(D, DROPOUT);
     constexpr uint32_t kParkPlane = 16u * NW * 64u;
     const uint32_t park_lds = lds0 + NSTG * STAGEB + (DROPOUT ? NW * 1024 : 0);       // (behind the dropout words)
@@ -1209,8 +1215,8 @@ hipError_t launch_bwd(const FaBwdArgs &a_in, int compute_units, hipStream_t stre
     // (The 128-wide strided and general instantiations are launched one workgroup per item only: with the item loop
     // around them they spill ten times as much, and a reload inside the tile loop waits for every tile load in
     // flight: c3's shape stored [B,S,H,D] 4.1 ms against 3.8.  The 64-wide ones have the registers for the loop.)
-    // (The kernels of the five-product form have the loop in every layout: the key-owning one keeps K^T / V^T
-    // fragments in LDS and compiles with it without spilling, or with 12 bytes outside the tile loop.)
+    // (The kernels of the five-product form have the loop in every layout: the key-owning one keeps K^T fragments in LDS and
+    // spills at most 24 bytes with it, 84 with dropout, which are touched per item or walked head and not per tile.)
     const bool uneven_items = MASKED && fa_bwd_uneven(a.S, a.Sk, a.L, a.R);
     const bool uneven = (LAYOUT == 0 || D == 64) && uneven_items;
     auto grid_if = [&](bool snake, long long items, unsigned groups_per_cu = 1u) {
