@@ -31,9 +31,6 @@
 #include "fa_bwd_args.h"
 #include "fa_bwd_layout.h"
 
-#ifndef FA_DS_LOOP
-#define FA_DS_LOOP 1
-#endif
 namespace {
 
 constexpr int kBwdWaves = 8;            // 8 waves x 32 owned rows = 256 rows per workgroup, two waves per SIMD
@@ -199,7 +196,7 @@ __device__ __forceinline__ uint16_t *head_ptr(uint16_t *p, const FaBwdTensor &t,
 template <bool BF16, int D, bool MASKED, int LAYOUT, bool ALIBI, bool DROPOUT>
 __global__ void __launch_bounds__(kBwdWaves * 64, 2) fa_bwd_dq(const FaBwdArgs a)
 {
-    constexpr bool STRIDES = LAYOUT >= 1, GENERAL = LAYOUT == 2, ONE_ITEM = STRIDES && D == 128;
+    constexpr bool STRIDES = LAYOUT >= 1, GENERAL = LAYOUT == 2, ONE_ITEM = STRIDES && D == 128 && !(DROPOUT && MASKED && !GENERAL);
     static_assert(LAYOUT >= 0 && LAYOUT <= 2, "0 the reference's layout, 1 strided, 2 general");
     static_assert(!GENERAL || MASKED, "the general instantiations always carry the mask code (ragged tiles need it)");
 
@@ -399,10 +396,12 @@ __global__ void __launch_bounds__(kBwdWaves * 64, 2) fa_bwd_dq(const FaBwdArgs a
 // WRITE_DS (regular lengths, no ALiBi): every 32-query x 32-key block of dS that a wave forms is also written to
 // a.ds_blocks, in the wave's operand order, for fa_bwd_dq_from_ds.
 // SHARES (with WRITE_DS): the walks cut into equal shares, see fa_bwd_layout.h.
-template <bool BF16, int D, bool MASKED, int LAYOUT, bool ALIBI, bool DROPOUT, bool WRITE_DS = false, bool SHARES = false, int NW = kBwdWaves>
+// ONE_ITEM: no loop around the work item (see launch_bwd).
+template <bool BF16, int D, bool MASKED, int LAYOUT, bool ALIBI, bool DROPOUT, bool WRITE_DS = false, bool SHARES = false, int NW = kBwdWaves,
+          bool ONE_ITEM = LAYOUT >= 1 && D == 128 && !WRITE_DS>
 __global__ void __launch_bounds__(NW * 64, 2) fa_bwd_dkdv(const FaBwdArgs a)
 {
-    constexpr bool STRIDES = LAYOUT >= 1, GENERAL = LAYOUT == 2, ONE_ITEM = STRIDES && D == 128 && !(WRITE_DS && FA_DS_LOOP);
+    constexpr bool STRIDES = LAYOUT >= 1, GENERAL = LAYOUT == 2;
     static_assert(!SHARES || (WRITE_DS && !ONE_ITEM), "a share is several walks, one pass of the item loop each");
     static_assert(!WRITE_DS || LAYOUT <= 1 || (!ALIBI && !DROPOUT), "general lengths: dS blocks without ALiBi and dropout only");
     typedef Num<BF16> N;
@@ -1157,6 +1156,7 @@ hipError_t launch_bwd(const FaBwdArgs &a_in, int compute_units, hipStream_t stre
     // S256 90 / 95; B6 H32/8 S4096 1698 / 1670 and B32 H8 S300 45 / 42 the other way.
     constexpr int NWK = D == 64 ? 4 : kBwdWaves, KEYS_K = 32 * NWK, GROUPS_K = kBwdWaves / NWK;
     const int smem_dkdv_ds = smem_kv(NWK);
+    constexpr bool EITHER = LAYOUT == 1 && D == 128 && DROPOUT && MASKED;        // the key-owning kernel is built with the item loop and without
     auto kq = fa_bwd_dq<BF16, D, MASKED, LAYOUT, ALIBI, DROPOUT>;
     auto kkv = fa_bwd_dkdv<BF16, D, MASKED, LAYOUT, ALIBI, DROPOUT>;
     // the five-product form: regular lengths (the reference's layout or a strided one) with dropout or ALiBi, any
@@ -1175,6 +1175,11 @@ hipError_t launch_bwd(const FaBwdArgs &a_in, int compute_units, hipStream_t stre
         if (e != hipSuccess) return e;
         e = hipFuncSetAttribute(reinterpret_cast<const void *>(kkv), hipFuncAttributeMaxDynamicSharedMemorySize, smem_dkdv);
         if (e != hipSuccess) return e;
+        if constexpr (EITHER) {
+            e = hipFuncSetAttribute(reinterpret_cast<const void *>(fa_bwd_dkdv<BF16, D, MASKED, LAYOUT, ALIBI, DROPOUT, false, false, kBwdWaves, false>),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, smem_dkdv);
+            if (e != hipSuccess) return e;
+        }
         if constexpr (FIVE) {
             e = hipFuncSetAttribute(reinterpret_cast<const void *>(fa_bwd_dkdv<BF16, D, MASKED, FL, ALIBI, DROPOUT, true, false, NWK>),
                                     hipFuncAttributeMaxDynamicSharedMemorySize, smem_dkdv_ds);
@@ -1214,11 +1219,15 @@ hipError_t launch_bwd(const FaBwdArgs &a_in, int compute_units, hipStream_t stre
     // items are alike as well)
     // (The 128-wide strided and general instantiations are launched one workgroup per item only: with the item loop
     // around them they spill ten times as much, and a reload inside the tile loop waits for every tile load in
-    // flight: c3's shape stored [B,S,H,D] 4.1 ms against 3.8.  The 64-wide ones have the registers for the loop.)
+    // flight: c3's shape stored [B,S,H,D] 4.1 ms against 3.8.  The 64-wide ones have the registers for the loop, and the
+    // strided ones with dropout, which serve the reference's layout too, spill outside the tile loop only: with the loop where
+    // the grid is a snake, without it elsewhere.  Seven products, p = 0.1, one item per workgroup / snake, us: causal B4 H16
+    // S2048 D128 424 / 310, B1 H32 S4096 740 / 562, B8 H32 S512 151 / 134; with the loop where it is not needed B1 H16 S1024
+    // 115 / 120, window 1000 B1 H32 S8192 646 / 671.)
     // (The kernels of the five-product form have the loop in every layout: the key-owning one keeps K^T fragments in LDS and
     // spills at most 24 bytes with it, 84 with dropout, which are touched per item or walked head and not per tile.)
     const bool uneven_items = MASKED && fa_bwd_uneven(a.S, a.Sk, a.L, a.R);
-    const bool uneven = (LAYOUT == 0 || D == 64) && uneven_items;
+    const bool uneven = (LAYOUT == 0 || D == 64 || EITHER) && uneven_items;
     auto grid_if = [&](bool snake, long long items, unsigned groups_per_cu = 1u) {
         const unsigned g = (unsigned)items, all = groups_per_cu * resident;
         return (snake && g > all && g < 16u * all) ? all : g;
@@ -1234,7 +1243,7 @@ hipError_t launch_bwd(const FaBwdArgs &a_in, int compute_units, hipStream_t stre
             for (int h0 = 0; h0 < all_heads; h0 += chunk) {
                 a.head0 = h0;
                 a.heads = all_heads - h0 < chunk ? all_heads - h0 : chunk;
-                const unsigned launch_k = grid_if(FA_DS_LOOP ? uneven_items : uneven, (long long)a.heads * ((a.Sk + KEYS_K - 1) / KEYS_K), GROUPS_K);
+                const unsigned launch_k = grid_if(uneven_items, (long long)a.heads * ((a.Sk + KEYS_K - 1) / KEYS_K), GROUPS_K);
                 unsigned n_shares = 0;
                 if constexpr (CAN_SHARE) {
                     if (a.partials != nullptr) n_shares = (unsigned)fa_bwd_launch_shares(a.heads, group, a.S, a.R, a.L, a.walk_head, (int)resident, a.share_slots);
@@ -1275,6 +1284,12 @@ hipError_t launch_bwd(const FaBwdArgs &a_in, int compute_units, hipStream_t stre
     const unsigned launch_q = grid_for((long long)a.B * a.H * ((a.S + 255) / 256));
     const unsigned launch_k = grid_for((long long)a.B * a.Hk * ((a.Sk + 255) / 256));
     hipLaunchKernelGGL(kq, dim3(launch_q), dim3(kBwdWaves * 64), smem_dq, stream, a);
+    if constexpr (EITHER) {
+        if ((long long)launch_k < (long long)a.B * a.Hk * ((a.Sk + 255) / 256)) {
+            hipLaunchKernelGGL((fa_bwd_dkdv<BF16, D, MASKED, LAYOUT, ALIBI, DROPOUT, false, false, kBwdWaves, false>), dim3(launch_k), dim3(kBwdWaves * 64), smem_dkdv, stream, a);
+            return hipGetLastError();
+        }
+    }
     hipLaunchKernelGGL(kkv, dim3(launch_k), dim3(kBwdWaves * 64), smem_dkdv, stream, a);
     return hipGetLastError();
 }
