@@ -9,11 +9,13 @@ struct FaBwdTensor {
     int rs;
 };
 
+constexpr float kTinyScale = 0x1p-100f, kTinyScaleKeys = 0x1p-40f;      // see key_scale
+
 struct FaBwdArgs {
     const uint16_t *Q, *K, *V, *O, *dO;
     const float *lse;                       // [B,H,S] contiguous, natural log, as the forward pass writes it
     // scratch [B,H,S] each, written by fa_bwd_dq or fa_bwd_prepare for the key-owning kernel, whose accumulators start from
-    // them: -(sum_t dO*O) / drop_scale per row, and (ln(drop_scale) - lse) / scale, -inf for rows that saw no key (P is then 0)
+    // them: -(sum_t dO*O) / drop_scale per row, and (ln(drop_scale) - lse) / key_scale, -inf for rows that saw no key (P is then 0)
     float *delta;
     float *lse2;
     uint16_t *dQ, *dK, *dV;
@@ -39,6 +41,10 @@ struct FaBwdArgs {
     int S, Sk;                              // queries, keys; query i sits at key position i + Sk - S
     int L, R;                               // key j visible to the query at position p iff p - L <= j <= p + R
     float scale;
+    // The scale that the key-owning kernel forms its scores with: `scale`, and where that is so small that lse / scale would leave
+    // fp32's range, 1 / kTinyScaleKeys times as much, with that kernel's copy of K kTinyScaleKeys times as large (a power of
+    // two: exact in bf16; what it takes from fp16 and from bf16's smallest values is scores of below 2^-50)
+    float key_scale;
     unsigned drop_threshold;                // dropout: keep iff the key's byte >= threshold (p in units of 1/256); 0 = none
     float drop_scale, drop_log;             // 256 / (256 - threshold) and its natural logarithm; 1 and 0 without dropout
     unsigned seed_lo, seed_hi;

@@ -269,7 +269,7 @@ __global__ void __launch_bounds__(kBwdWaves * 64, 2) fa_bwd_dq(const FaBwdArgs a
         delta += swap_halves(delta);
         if (row_ok && half == 0) {
             a.delta[(size_t)bh * S + my_q] = -delta / a.drop_scale;
-            a.lse2[(size_t)bh * S + my_q] = (GENERAL && lse_raw == -INFINITY) ? -INFINITY : (a.drop_log - lse_raw) / a.scale;
+            a.lse2[(size_t)bh * S + my_q] = (GENERAL && lse_raw == -INFINITY) ? -INFINITY : (a.drop_log - lse_raw) / a.key_scale;
         }
     }
     const float c = a.scale * kLog2e;
@@ -476,7 +476,7 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_bwd_dkdv(const FaBwdArgs a)
         kf[s] = *reinterpret_cast<const u32x4 *>(Kh + (size_t)my_kc * k_rs + 16 * s + 8 * half);
         vf[s] = *reinterpret_cast<const u32x4 *>(Vh + (size_t)my_kc * v_rs + 16 * s + 8 * half);
     }
-    const float c = a.scale * kLog2e;
+    const float c = a.key_scale * kLog2e;
 
     // the query tiles that see these keys: the query at index i (position i + off) sees key j iff
     // j - R - off <= i <= j + L - off: the forward bounds with the two sides exchanged and shifted
@@ -779,6 +779,15 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_bwd_dkdv(const FaBwdArgs a)
         wait_vm<0>();
 #pragma unroll
         for (int s = 0; s < KS; ++s) asm volatile("" : "+v"(kf[s]), "+v"(vf[s]));
+        if (__builtin_expect(a.key_scale != a.scale, 0)) {         // (see FaBwdArgs)
+#pragma unroll
+            for (int s = 0; s < KS; ++s)
+#pragma unroll
+                for (int w = 0; w < 4; ++w) {
+                    const uint32_t two = kf[s][w];
+                    kf[s][w] = N::pack2(storage_to_f32<BF16>((uint16_t)(two & 0xffffu)) * kTinyScaleKeys, storage_to_f32<BF16>((uint16_t)(two >> 16)) * kTinyScaleKeys);
+                }
+        }
         // from here on the parked fragments live in LDS, and their registers are free
         // (one plane of 16 bytes per thread for every parked fragment: consecutive lanes, consecutive 16 bytes)
 #pragma unroll
@@ -940,7 +949,7 @@ __global__ void __launch_bounds__(256) fa_bwd_prepare(const FaBwdArgs a)
     }
     if (writes) {
         a.delta[row0 + mine] = -delta / a.drop_scale;
-        a.lse2[row0 + mine] = l == -INFINITY ? -INFINITY : (a.drop_log - l) / a.scale;
+        a.lse2[row0 + mine] = l == -INFINITY ? -INFINITY : (a.drop_log - l) / a.key_scale;
     }
     }
 }

@@ -1014,6 +1014,7 @@ int fa_bwd_shared(const fa_bwd_params *p, void *partials, unsigned long long par
     fa_mask_bounds(far, p->is_causal, p->window_size_left, p->window_size_right, &a.L, &a.R);
     if (a.partials != nullptr) a.walk_head = walk_pairs_per_head(a.S, a.H / a.Hk, a.L, a.R);
     a.scale = p->softmax_scale;
+    a.key_scale = a.scale < kTinyScale ? a.scale / kTinyScaleKeys : a.scale;
     a.drop_threshold = (unsigned)fa_dropout_threshold(p->dropout_prob);
     a.drop_scale = 256.0f / (256.0f - (float)a.drop_threshold);
     a.drop_log = logf(a.drop_scale);
