@@ -776,10 +776,13 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_bwd_dkdv(const FaBwdArgs a)
         if (STRIDES) walk_head(first_g);
         issue_next(0);
         if (SHARES ? pairs_left > 1 : ig < G) issue_next(1);
+        // (read while K and V are on their way, not behind the wait for them)
+        uint32_t tiny_scale = __builtin_bit_cast(uint32_t, a.key_scale) ^ __builtin_bit_cast(uint32_t, a.scale);
+        asm volatile("" : "+s"(tiny_scale));
         wait_vm<0>();
 #pragma unroll
         for (int s = 0; s < KS; ++s) asm volatile("" : "+v"(kf[s]), "+v"(vf[s]));
-        if (__builtin_expect(a.key_scale != a.scale, 0)) {         // (see FaBwdArgs)
+        if (__builtin_expect(tiny_scale != 0, 0)) {         // (see FaBwdArgs)
 #pragma unroll
             for (int s = 0; s < KS; ++s)
 #pragma unroll
