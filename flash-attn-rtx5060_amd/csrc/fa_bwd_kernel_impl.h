@@ -1258,7 +1258,7 @@ hipError_t launch_bwd(const FaBwdArgs &a_in, int compute_units, hipStream_t stre
                 const unsigned launch_k = grid_if(uneven_items, (long long)a.heads * ((a.Sk + KEYS_K - 1) / KEYS_K), GROUPS_K);
                 unsigned n_shares = 0;
                 if constexpr (CAN_SHARE) {
-                    if (a.partials != nullptr) n_shares = (unsigned)fa_bwd_launch_shares(a.heads, group, a.S, a.R, a.L, a.walk_head, (int)resident, a.share_slots);
+                    if (a.partials != nullptr) n_shares = (unsigned)fa_bwd_launch_shares(D, a.heads, group, a.S, a.R, a.L, a.walk_head, (int)resident, a.share_slots);
                     if (n_shares != 0) {
                         a.walk_total = a.heads * a.walk_head;
                         hipLaunchKernelGGL((fa_bwd_dkdv<BF16, D, MASKED, FL, ALIBI, DROPOUT, true, true>), dim3(n_shares), dim3(kBwdWaves * 64), smem_dkdv, stream, a);

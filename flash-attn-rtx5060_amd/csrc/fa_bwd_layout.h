@@ -69,12 +69,13 @@ FA_LAYOUT_HD long long fa_ds_block_index(int S, int qb, int kb)
 // (head by head, from the last tile down).  Under a causal mask block 0 walks all tiles and the last block four of
 // them; a problem with few key blocks leaves CUs idle.  The walks of all blocks, block by block and head by head, are
 // therefore laid end to end and cut into shares that differ by at most one pair (no more shares than pairs).
-FA_LAYOUT_HD int fa_bwd_walk_tiles(int S, int Sk, int Lq, int Rq, int kblock)
+FA_LAYOUT_HD int fa_bwd_tiles_of_keys(int S, int Sk, int Lq, int Rq, int first, int keys)
 {
     int lo, hi;
-    fa_tile_range(S, 64, Lq, Rq, kblock * 256, Sk - kblock * 256 < 256 ? Sk - kblock * 256 : 256, &lo, &hi);
+    fa_tile_range(S, 64, Lq, Rq, first, Sk - first < keys ? Sk - first : keys, &lo, &hi);
     return hi - lo + 1;
 }
+FA_LAYOUT_HD int fa_bwd_walk_tiles(int S, int Sk, int Lq, int Rq, int kblock) { return fa_bwd_tiles_of_keys(S, Sk, Lq, Rq, kblock * 256, 256); }
 // Share of workgroup `block`: with workgroups dealt round robin over the eight XCDs, each XCD gets consecutive shares
 // (a head or two of the list: what runs there at a time reads the same tiles).  `shares` is a multiple of eight.
 FA_LAYOUT_HD int fa_bwd_share_of(int block, int shares) { return (block & 7) * (shares >> 3) + (block >> 3); }
@@ -113,46 +114,65 @@ FA_LAYOUT_HD int fa_bwd_uneven(int S, int Sk, int L, int R) { return (L < S + Sk
 // 32 : 4.5 102 against 157, B1 H16 S1024 16 : 2.5 77 against 93, B2 H8 S512 8 : 2 51 against 59, without a mask B1 H40 S2048
 // 64 : 40 330 against 370; and not cut: B1 H32 S2048 32 : 18 195 against 184, B6 H8 S2048 36 : 27 266 against 233, without a
 // mask B2 H16 S512 D64 8 : 2 47 against 44.
-FA_LAYOUT_HD int fa_bwd_shares(int heads, int G, int S, int Lq, int Rq, int walk_head, int compute_units)
+// Head dimension 64: an uncut launch has items of 128 keys, two workgroups to a compute unit, so the longest is counted in
+// pairs of 128 keys.  In units of a share's pair of 256, a workgroup that has its compute unit to itself takes 4/5 for one and
+// two side by side 11/20 each; a cut costs 15 (256 shares; less with fewer).  Backward pass, fp16, longest : share, cut against
+// whole, us: causal B1 H8 S2048 32 : 4.5 57 / 62, B1 H32/8 S2048 128 : 18 100 / 191, B1 H12 S3000 47 : 14 96 / 105, no mask B1 H4
+// S8192 128 : 64 265 / 277; and not cut: causal B1 H16 S1024 16 : 2.5 43 / 37.5, B4 H8 S1024 16 : 5 49 / 40, B2 H8 S512 8 : 2 30 /
+// 24, B5 H8 S4096 130 : 85 399 / 368, window 4000 B2 H8 S16000 260 : 229 994 / 877, no mask B1 H16 S2048 32 : 16 81 / 74.
+FA_LAYOUT_HD long long fa_bwd_item_load(long long at, long long g, long long items, int snake, int heads, int n_kblocks, int keys, int G, int S, int Lq, int Rq)
 {
-    const int n_kblocks = (S + 255) / 256;
-    const long long total = (long long)heads * walk_head, items = (long long)heads * n_kblocks;
+    long long sum = 0;
+    for (long long pass = 0; pass * g < items; ++pass) {
+        const long long item = pass * g + (snake && (pass & 1) ? g - 1 - at : at);
+        if (item >= items) continue;
+        int head, kblock;
+        fa_item_decode(item, heads, n_kblocks, 0, &head, &kblock);
+        sum += (long long)G * fa_bwd_tiles_of_keys(S, S, Lq, Rq, kblock * keys, keys);
+    }
+    return sum;
+}
+FA_LAYOUT_HD int fa_bwd_shares(int D, int heads, int G, int S, int Lq, int Rq, int walk_head, int compute_units)
+{
+    const int keys = D == 64 ? 128 : 256, n_kblocks = (S + keys - 1) / keys;
+    const long long total = (long long)heads * walk_head, items = (long long)heads * n_kblocks, slots = (long long)compute_units * (256 / keys);
     if (walk_head <= 0 || total > 0x3fffffffLL) return 0;
     long long shares = total / 2 / 8 * 8;          // at least two pairs each
     if (shares > compute_units) shares = compute_units / 8 * 8;
     if (shares < 8) return 0;
-    const int snake = fa_bwd_uneven(S, S, Rq, Lq) && items < 16LL * compute_units;
-    const long long g = items < compute_units ? items : compute_units;
-    long long worst = 0;
+    const int snake = fa_bwd_uneven(S, S, Rq, Lq) && items < 16 * slots;
+    const long long g = items < slots ? items : slots;
+    long long worst = 0, worst_two = 0;            // of one workgroup, of the two of a compute unit
     for (int probe = 0; probe < 8; ++probe) {
         const long long at = probe == 7 ? (items - 1) % g : probe * (g - 1) / 6;
-        long long sum = 0;
-        for (long long pass = 0; pass * g < items; ++pass) {
-            const long long item = pass * g + (snake && (pass & 1) ? g - 1 - at : at);
-            if (item >= items) continue;
-            int head, kblock;
-            fa_item_decode(item, heads, n_kblocks, 0, &head, &kblock);
-            sum += (long long)G * fa_bwd_walk_tiles(S, S, Lq, Rq, kblock);
+        const long long one = fa_bwd_item_load(at, g, items, snake, heads, n_kblocks, keys, G, S, Lq, Rq);
+        if (one > worst) worst = one;
+        if (D == 64 && at + compute_units < g) {
+            const long long two = one + fa_bwd_item_load(at + compute_units, g, items, snake, heads, n_kblocks, keys, G, S, Lq, Rq);
+            if (two > worst_two) worst_two = two;
         }
-        if (sum > worst) worst = sum;
+    }
+    if (D == 64) {
+        const long long sixtieths = 48 * worst > 33 * worst_two ? 48 * worst : 33 * worst_two;
+        return sixtieths > 80 * total / shares + 900 * shares / 256 ? (int)shares : 0;
     }
     return 3 * worst > 4 * (total / shares) + 9 + 18 * shares / 256 ? (int)shares : 0;
 }
 // The buffer of the parts is sized on the host without a device, for FA_BWD_SHARE_UNITS compute units (a whole MI355X):
 // the shares of the larger of the launches over a whole chunk of K/V heads and over the `rest` that is left (0: none).
 #define FA_BWD_SHARE_UNITS 256
-FA_LAYOUT_HD int fa_bwd_share_slots(int chunk, int rest, int G, int S, int Lq, int Rq, int walk_head)
+FA_LAYOUT_HD int fa_bwd_share_slots(int D, int chunk, int rest, int G, int S, int Lq, int Rq, int walk_head)
 {
-    const int whole = fa_bwd_shares(chunk, G, S, Lq, Rq, walk_head, FA_BWD_SHARE_UNITS);
-    const int last = rest > 0 ? fa_bwd_shares(rest, G, S, Lq, Rq, walk_head, FA_BWD_SHARE_UNITS) : 0;
+    const int whole = fa_bwd_shares(D, chunk, G, S, Lq, Rq, walk_head, FA_BWD_SHARE_UNITS);
+    const int last = rest > 0 ? fa_bwd_shares(D, rest, G, S, Lq, Rq, walk_head, FA_BWD_SHARE_UNITS) : 0;
     return whole > last ? whole : last;
 }
 // The shares of one launch: by the compute units of the device it runs on, which may cut what FA_BWD_SHARE_UNITS would
 // leave whole (a partition with 32 units: S 512, causal, chunks of 264 heads and a rest of 2, 32 shares where the buffer
 // holds 8), and none when the buffer has fewer slots than that.
-FA_LAYOUT_HD int fa_bwd_launch_shares(int heads, int G, int S, int Lq, int Rq, int walk_head, int compute_units, int slots)
+FA_LAYOUT_HD int fa_bwd_launch_shares(int D, int heads, int G, int S, int Lq, int Rq, int walk_head, int compute_units, int slots)
 {
-    const int shares = fa_bwd_shares(heads, G, S, Lq, Rq, walk_head, compute_units);
+    const int shares = fa_bwd_shares(D, heads, G, S, Lq, Rq, walk_head, compute_units);
     return shares <= slots ? shares : 0;
 }
 

@@ -942,7 +942,7 @@ unsigned long long fa_bwd_share_bytes(const fa_bwd_params *p)
     const int per_head = walk_pairs_per_head(p->S, G, L, R);
     // the launches: whole chunks and a smaller last one
     const int rest = (int)(kv_heads_total(p) % heads);
-    const int slots = fa_bwd_share_slots(heads, rest, G, p->S, R, L, per_head);
+    const int slots = fa_bwd_share_slots(p->d, heads, rest, G, p->S, R, L, per_head);
     return (unsigned long long)slots * bytes_per_share(p);
 }
 

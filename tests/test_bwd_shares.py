@@ -45,6 +45,11 @@ def test_share_bytes_and_refusals(fa):
     assert need == 256 * 2 * 2 * 256 * 128 * 4
     assert L.fa_bwd_share_bytes(ctypes.byref(fa.make_bwd_params(**{**ok, "S": 128, "n_kv_heads": 16}))) == 0          # nothing to cut
     assert L.fa_bwd_share_bytes(ctypes.byref(fa.make_bwd_params(**{**ok, "S_kv": 2048}))) == 0      # no five-product form
+    # head dimension 64, where the uncut launch has items of 128 keys, two workgroups to a compute unit: a longest walk of 16 pairs
+    # of 128 keys each against shares of 2.5 or 5 pairs is not worth a cut, walks of 128 are
+    for B, N, Nk, S, cut in ((1, 16, 16, 1024, 0), (4, 8, 8, 1024, 0), (5, 8, 8, 4096, 0), (1, 8, 8, 2048, 256), (1, 32, 8, 2048, 256)):
+        q = fa.make_bwd_params(**{**ok, "B": B, "N": N, "n_kv_heads": Nk, "S": S, "d": 64, "causal": True, "workspace_bytes": 1 << 40})
+        assert L.fa_bwd_share_bytes(ctypes.byref(q)) == cut * 2 * 2 * 256 * 64 * 4
     assert L.fa_bwd_shared(ctypes.byref(p), 0xB008, need, None) == fa.FA_ERR_WORKSPACE              # alignment
     assert L.fa_bwd_shared(ctypes.byref(p), 0xB000, need - 1, None) == fa.FA_ERR_WORKSPACE
 
