@@ -898,7 +898,7 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_bwd_dkdv(const FaBwdArgs a)
 // pass there 862 / 857 us, B16 H16 S1024 D64 196.7 / 194.6, B4 H16 S2048 D64 152.3 / 149.5, B1 H32 S2048 D128 148.5 / 147.0.
 // ---------------------------------------------------------------------------------------------------------
 constexpr int kPrepareRows = 4;               // rows per thread
-constexpr long long kPrepareGrid = 1 << 16;   // workgroups of a launch at most (a launch holds below 2^32 threads); they walk what is beyond
+constexpr long long kPrepareGrid = 1 << 16;   // workgroups of a launch at most (far below the 2^32 threads a launch may hold); they walk what is beyond
 constexpr int fa_bwd_prepare_rows(int D) { return kPrepareRows * (256 / (D / 8)); }       // rows per workgroup
 template <bool BF16, int D, bool STRIDED>
 __global__ void __launch_bounds__(256) fa_bwd_prepare(const FaBwdArgs a)
@@ -953,6 +953,43 @@ __global__ void __launch_bounds__(256) fa_bwd_prepare(const FaBwdArgs a)
     if (writes) {
         a.delta[row0 + mine] = -delta / a.drop_scale;
         a.lse2[row0 + mine] = l == -INFINITY ? -INFINITY : (a.drop_log - l) / a.key_scale;
+    }
+    }
+}
+
+// The same for sequences of at most a quarter of such a workgroup's rows, whose heads would leave most of its threads without a
+// row: rows of all heads one behind the other, one per group of threads.  us, a piece of one head per workgroup / this: D64
+// B512 H16 S16 12.2 / 7.6, B2048 H16 S1 35.9 / 4.8, D128 B1024 H16 S8 21.9 / 13.5; B256 H32 S33 28.2 / 30.5, and at D64 B128 H16
+// S64 the backward pass 50.8 / 51.3.
+template <bool BF16, int D, bool STRIDED>
+__global__ void __launch_bounds__(256) fa_bwd_prepare_short(const FaBwdArgs a)
+{
+    constexpr int TPR = D / 8;                    // threads per row, 16 bytes each
+    const long long n_rows = (long long)a.B * a.H * a.S;
+    const int c = (int)threadIdx.x % TPR * 8;
+    for (long long first = (long long)blockIdx.x * (256 / TPR); first < n_rows; first += (long long)gridDim.x * (256 / TPR)) {
+    const long long row = first + (int)threadIdx.x / TPR, r = row < n_rows ? row : n_rows - 1;
+    const uint16_t *o_row = a.O + r * D, *g_row = a.dO + r * D;
+    if (STRIDED) {                                // row r of the [B,H,S] order, wherever the tensors keep it
+        const long long bh = r / a.S;
+        const int i = (int)(r - bh * a.S), b = (int)(bh / a.H), h = (int)(bh - (long long)b * a.H);
+        o_row = head_ptr(a.O, a.o, b, h) + (long long)i * a.o.rs;
+        g_row = head_ptr(a.dO, a.dO_, b, h) + (long long)i * a.dO_.rs;
+    }
+    const u32x4 o = *reinterpret_cast<const u32x4 *>(o_row + c), g = *reinterpret_cast<const u32x4 *>(g_row + c);
+    float sum = 0.0f;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+        const uint32_t ow = o[w], gw = g[w];
+        sum += storage_to_f32<BF16>((uint16_t)(ow & 0xffffu)) * storage_to_f32<BF16>((uint16_t)(gw & 0xffffu));
+        sum += storage_to_f32<BF16>((uint16_t)(ow >> 16)) * storage_to_f32<BF16>((uint16_t)(gw >> 16));
+    }
+#pragma unroll
+    for (int m = 1; m < TPR; m <<= 1) sum += __shfl_xor(sum, m);
+    if (row < n_rows && c == 0) {
+        const float l = a.lse[row];
+        a.delta[row] = -sum / a.drop_scale;
+        a.lse2[row] = l == -INFINITY ? -INFINITY : (a.drop_log - l) / a.key_scale;
     }
     }
 }
@@ -1249,8 +1286,12 @@ hipError_t launch_bwd(const FaBwdArgs &a_in, int compute_units, hipStream_t stre
         if (a.ds_blocks != nullptr) {
             // delta and the rescaled logsumexp, for all heads at once; then, for as many heads at a time as the
             // workspace holds dS blocks for: dK, dV and the dS blocks; dQ from the blocks
-            const long long prepare_blocks = (long long)a.B * a.H * ((a.S + fa_bwd_prepare_rows(D) - 1) / fa_bwd_prepare_rows(D));
-            hipLaunchKernelGGL((fa_bwd_prepare<BF16, D, FL >= 1>), dim3((unsigned)(prepare_blocks < kPrepareGrid ? prepare_blocks : kPrepareGrid)), dim3(256), 0, stream, a);
+            constexpr int rows = fa_bwd_prepare_rows(D), short_rows = 256 / (D / 8);       // rows of a workgroup
+            const bool short_heads = 4 * a.S <= rows;
+            const long long prepare_blocks = short_heads ? ((long long)a.B * a.H * a.S + short_rows - 1) / short_rows : (long long)a.B * a.H * ((a.S + rows - 1) / rows);
+            const dim3 prepare_grid((unsigned)(prepare_blocks < kPrepareGrid ? prepare_blocks : kPrepareGrid));
+            if (short_heads) hipLaunchKernelGGL((fa_bwd_prepare_short<BF16, D, FL >= 1>), prepare_grid, dim3(256), 0, stream, a);
+            else hipLaunchKernelGGL((fa_bwd_prepare<BF16, D, FL >= 1>), prepare_grid, dim3(256), 0, stream, a);
             const int chunk = a.ds_heads > 0 && a.ds_heads < all_heads ? a.ds_heads : all_heads;
             for (int h0 = 0; h0 < all_heads; h0 += chunk) {
                 a.head0 = h0;
