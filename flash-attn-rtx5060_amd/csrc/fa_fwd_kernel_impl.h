@@ -70,10 +70,11 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kBlockKeys = 64;          // keys per K/V tile
 constexpr float kNoReference = -1.0e30f; // reference point of a row before its first visible score
-constexpr float kRescaleLog2 = 8.0f;    // rescale O only when a row max grew by > 2^8
-// ... or, in the loop that takes no maxima (see steady), by > 2^14 (P stays below fp16's 65504): then half a row's exponentials of
-// one tile add up to more than kTileSum, which lies below 2^14 by more than their rounding
-constexpr float kLagLog2 = 14.0f, kTileSum = 15000.0f;
+// rescale O only when a row max grew by > 2^8.  (The further a reference point may lag behind, the more of the rows that one key
+// carries have a weight that is rounded instead of exactly 1: with 2^14, fp16 scores of a standard deviation of 16, O was 7 %
+// further off.)
+constexpr float kRescaleLog2 = 8.0f;
+constexpr float kTileSum = 240.0f;      // a row whose maximum grew so has half a tile's exponentials that add up to more than this
 constexpr int kFewTiles = 8;                // items of at most this many tiles take maxima from their start
 
 template <bool BF16> struct Num;
@@ -426,15 +427,15 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
     // The reference point of a row's exponentials follows its tiles' sums instead of their maxima (see steady): sixteen
     // three-way maxima, a half swap and the move itself, about thirty of the 140 vector instructions that the general 64-wide
     // kernel's iteration has with maxima, leave the loop; the scores then stay in registers to the iteration's end.  A tile
-    // that the sums find too large is done again, which costs half an iteration: where scores are sharp (a standard deviation of
-    // eight) that happens to some row of a wave in most tiles, so from the first such tile on the rest of the item takes maxima,
-    // in a loop of its own, and so do items of few tiles.  Maxima throughout / sums alone / both loops, us, inputs of unit
-    // variance: B4 H16 S2048 D64 53.1 / 51.2 / 51.3, B2 H32 S8192 D128 1018 / 997 / 999, B4 H32/8 S2000 D64 no mask 175.5 /
-    // 166.4 / 167.5, B1 H32 S8100 D128 522 / 510 / 509, windows of 300 keys B2 H16 S8100 D64 69.5 / 69.2 / 70.2, B8 H16 S1000
-    // D64 38.8 / 37.9 / 39.0; Q eight times as large, in the same order: 54.1 / 59.2 / 56.5, 1001 / 1017 / 1009, 176 / 191 / 180,
-    // 509 / 515 / 511, 70.8 / 76.1 / 71.5, 40.3 / 44.7 / 41.3; sixteen times: 54.0 / 64.9 / 54.8.  With ALiBi the 128-wide
-    // kernels have no registers for it (a training step of B5 H16 S2637 bf16 892 / 948), with dropout the words drawn for the
-    // tile have to stay as well (B16 H16 S512 D64 146.0 / 147.4): both keep the maxima.
+    // that the sums find too large is done again, which costs half an iteration: where scores are sharp that happens to some row
+    // of a wave in most tiles, so from the first such tile on the rest of the item takes maxima, in a loop of its own, and so do
+    // items of few tiles.  Maxima throughout / sums alone / both loops, us, inputs of unit variance: B4 H16 S2048 D64 53.8 / 51.9
+    // / 52.2, B2 H32 S8192 D128 1028 / 1008 / 1011, B4 H32/8 S2000 D64 no mask 175.8 / 166.7 / 167.5, B1 H32 S8100 D128 522 /
+    // 509 / 508, windows of 300 keys B2 H16 S8100 D64 69.7 / 69.4 / 70.3, B8 H16 S1000 D64 38.8 / 38.2 / 39.0; Q four times as
+    // large, in the same order: 55.2 / 54.0 / 57.2, 1060 / 1038 / 1069, 180 / 174 / 185, 533 / 520 / 535, 70.9 / 72.4 / 71.6, 39.9
+    // / 39.6 / 41.3; eight times: 54.8 / 59.5 / 56.5, 1025 / 1039 / 1031, 177 / 190 / 181, 514 / 522 / 516, 71.1 / 76.1 / 71.6,
+    // 40.4 / 44.7 / 41.3.  With ALiBi the 128-wide kernels have no registers for it (a training step of B5 H16 S2637 bf16 892 /
+    // 948), with dropout the words drawn for the tile have to stay as well (B16 H16 S512 D64 146.0 / 147.4): both keep the maxima.
     constexpr bool BY_SUM = !ALIBI && !DROPOUT;
     // LDS reads run this many fragments ahead (general 128-wide kernels: three, or the scores that stay are spilled; with
     // four, 12 bytes, chunk_prefill's shape 54.8 us against 53.2)
@@ -760,7 +761,7 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
     // whether a row with maximum mx moves its reference point (from kNoReference every finite maximum does; BY_SUM: by the
     // exponent as the elements have it)
     auto grows = [&](float mx) __attribute__((always_inline)) {
-        return BY_SUM ? __builtin_fmaf(mx, cs, -m_run * cs) > kLagLog2 : mx > m_run + thresh;
+        return BY_SUM ? __builtin_fmaf(mx, cs, -m_run * cs) > kRescaleLog2 : mx > m_run + thresh;
     };
     auto new_reference = [&](float mx, bool &moved) __attribute__((always_inline)) {
         float alpha = 1.0f;
@@ -958,7 +959,8 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
             // on which of the two loops its tiles went through.
             if (!BY_MAX && __builtin_expect(__builtin_amdgcn_ballot_w64(!(t_a + t_b <= kTileSum)) != 0, 0)) {
                 mx = row_max();
-                const bool grow = __builtin_fmaf(mx, c, nmc) > kLagLog2;
+                const bool grow = __builtin_fmaf(mx, c, nmc) > kRescaleLog2;
+                sharp = true;
                 if (__builtin_amdgcn_ballot_w64(grow) != 0) {
                     const float m_new = grow ? mx : m_run;
                     alpha = __builtin_amdgcn_exp2f((m_run - m_new) * cs);
@@ -967,7 +969,6 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
                     m_run = m_new;
                     nmc = -m_new * cs;
                     scale_o(alpha);
-                    sharp = true;
 #pragma unroll
                     for (int e = 0; e < 16; ++e) pair(e);
                 }
@@ -1102,11 +1103,10 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
         generic_iteration(i, j3, jv);
         advance();
     }
-    // (single iterations in the general kernels take the maxima: 0-1 % faster than without, elsewhere 0-1 % slower)
+    // (single iterations take the maxima: without them 0.5 % faster for B4 H16 S2048 D64, 3 % slower for sharp B16 H16 S512 D128)
     typedef IntC<BY_SUM ? 0 : 1> Usual;
-    typedef IntC<BY_SUM && !GENERAL ? 0 : 1> Single;
-    if (j3 == 1 && whole(i)) { steady_iteration(IntC<1>{}, Single{}, i, jv); advance(); ++i; }
-    if (NST >= 3 && j3 == 2 && whole(i)) { steady_iteration(IntC<2 % NST>{}, Single{}, i, jv); advance(); ++i; }
+    if (j3 == 1 && whole(i)) { steady_iteration(IntC<1>{}, IntC<1>{}, i, jv); advance(); ++i; }
+    if (NST >= 3 && j3 == 2 && whole(i)) { steady_iteration(IntC<2 % NST>{}, IntC<1>{}, i, jv); advance(); ++i; }
     auto turn = [&](auto MAXIMA) __attribute__((always_inline)) {
         steady_iteration(IntC<0>{}, MAXIMA, i, jv);
         advance();
@@ -1118,8 +1118,8 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
     while (!(BY_SUM && sharp) && j3 == 0 && whole(i) && whole(i + NST - 1)) turn(Usual{});
     if (BY_SUM)                           // what is left once a tile had to be done again
         while (j3 == 0 && whole(i) && whole(i + NST - 1)) turn(IntC<1>{});
-    if (j3 == 0 && whole(i)) { steady_iteration(IntC<0>{}, Single{}, i, jv); advance(); ++i; }
-    if (NST >= 3 && j3 == 1 && whole(i)) { steady_iteration(IntC<1>{}, Single{}, i, jv); advance(); ++i; }
+    if (j3 == 0 && whole(i)) { steady_iteration(IntC<0>{}, IntC<1>{}, i, jv); advance(); ++i; }
+    if (NST >= 3 && j3 == 1 && whole(i)) { steady_iteration(IntC<1>{}, IntC<1>{}, i, jv); advance(); ++i; }
     for (; i < t1; ++i) {                 // drain, up to the last two iterations
         generic_iteration(i, j3, jv);
         advance();
