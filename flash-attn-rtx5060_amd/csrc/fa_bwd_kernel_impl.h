@@ -9,7 +9,7 @@
 //   dQ = scale * dS K,   dK = scale * dS^T Q
 //
 // Two kernels: fa_bwd_dq (a workgroup owns 256 queries and walks the key tiles; it also writes delta and the
-// rescaled logsumexp for the second kernel) and fa_bwd_dkdv (a workgroup owns 256 keys of one K/V head and walks
+// rescaled logsumexp for the second kernel) and fa_bwd_dkdv (a workgroup owns 256 or 128 keys of one K/V head and walks
 // the query tiles of the query heads that share it); no atomics, every output element has one writer, results
 // are the same bits from run to run.
 // Template flags: LAYOUT 0 = contiguous [B,H,S,D] with S a multiple of 128 and as many keys; 1 (strided) = the
@@ -388,12 +388,13 @@ __global__ void __launch_bounds__(kBwdWaves * 64, 2) fa_bwd_dq(const FaBwdArgs a
 }
 
 // ---------------------------------------------------------------------------------------------------------
-// dK, dV: a workgroup owns 256 keys of one K/V head (lane = key), walks the query tiles that see them, for each
+// dK, dV: a workgroup owns 32 NW keys of one K/V head (256, or 128 in the five-product form's uncut launches at head dimension
+// 64; lane = key), walks the query tiles that see them, for each
 // of the query heads that share the K/V head.
 // LDS stage: Q (row-wise for S = Q K^T, transposed for dK^T += Q^T dS), dO (row-wise for dP = dO V^T, transposed
-// for dV^T += dO^T P), 64 rescaled logsumexps, 64 deltas.
+// for dV^T += dO^T P), the 64 words each that the accumulators of S and dP start from (FaBwdArgs).
 // ---------------------------------------------------------------------------------------------------------
-// WRITE_DS (regular lengths, no ALiBi): every 32-query x 32-key block of dS that a wave forms is also written to
+// WRITE_DS (the five-product form): every 32-query x 32-key block of dS that a wave forms is also written to
 // a.ds_blocks, in the wave's operand order, for fa_bwd_dq_from_ds.
 // SHARES (with WRITE_DS): the walks cut into equal shares, see fa_bwd_layout.h.
 // ONE_ITEM: no loop around the work item (see launch_bwd).
