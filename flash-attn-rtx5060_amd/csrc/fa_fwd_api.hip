@@ -348,6 +348,25 @@ bool decode_problem(const fa_fwd_params *p, bool causal_type, int splits)
 }
 // Workgroups of the tile kernels that a device keeps resident
 long long resident_groups(int compute_units, int waves) { return (long long)compute_units * (waves == 8 ? 1 : 2); }
+// Rows in the verifier's arithmetic in workgroups of their own (FaKernelArgs.first_parts), in launches of one workgroup per item:
+// whether the launch has such rows in items that could leave them, and into how many parts per head they go, 0 to leave them in
+// the items.  Behind a tile loop the path is a chain of latencies, 4 us for eight rows and 8 to 15 for 32, which short items
+// cannot hide; beside the items it costs slots.  As many parts as fit next to the items into the slots that a device has at a
+// time, times two (head dimension 64, where the path is shorter: times 7/4), since the first blocks of a head are short
+// themselves.  Causal, us, in the items / apart: B1 H4 S256 D64 14.1 / 8.7, B4 H32 S128 D128 bf16 30.3 / 16.4, B5 H16 S284 D128
+// 23.2 / 14.4, B1 H32 S512 D128 20.3 / 15.2, B1 H384 S128 D64 19.4 / 17.7, B1 H256 S256 D128 31.4 / 29.2; further parts, H512 S100
+// D64 21.6 / 21.9, H128 S500 D64 22.1 / 22.5, and at four times the slots H200 S256 D64 15.9 (two) / 21.6.
+bool first_rows_apart(const FaKernelArgs &a, int masked)
+{
+    const int pos_off = a.Sk - a.S;
+    return masked != 0 && a.R == 0 && pos_off >= 0 && pos_off < 32 && a.n_splits == 1 && a.pack == 1 && !a.exact_first_rows;
+}
+int first_rows_parts(long long items, long long heads, int d, long long resident)
+{
+    int parts = 8;
+    while (parts > 0 && items + parts * heads > (d == 128 ? 8 : 7) * resident / 4) parts /= 2;
+    return parts;
+}
 // How a call reaches the device: by the decoding kernel, whose workgroups (one per K/V head and key split) the hardware
 // hands out, with the streaming hint or without; else the schedule of the tile kernels' work items.
 struct Launch {
@@ -635,6 +654,8 @@ int forward(const fa_fwd_params *p, void *workspace, const FaDeviceState *ds, vo
     a.seed_lo = (unsigned)(p->seed & 0xffffffffull);
     a.seed_hi = (unsigned)(p->seed >> 32);
     a.exact_first_rows = p->exact_first_rows != 0;
+    a.first_parts = 0;
+    if (launch.sched == FA_SCHED_DISPATCH && first_rows_apart(a, masked)) a.first_parts = first_rows_parts(a.n_items, a.BH, p->d, resident_groups(ds->compute_units, waves));
 #ifdef FA_CHECK_RING
     a.ring_check = ds->ring_check;
 #endif

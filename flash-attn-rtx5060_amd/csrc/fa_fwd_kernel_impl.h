@@ -401,6 +401,36 @@ __device__ __forceinline__ void faithful_first_rows(const uint16_t *Qh, const ui
     __syncthreads();
 }
 
+// Workgroup `at` of the grid's second row (FaKernelArgs.first_parts): part at / BH of the first rows of list head at % BH.
+template <bool BF16, int D, bool ALIBI, bool GENERAL, bool DROPOUT, bool STRIDED>
+__device__ __forceinline__ void first_rows_item(const FaKernelArgs &a, unsigned at, uint32_t lds)
+{
+    const int part = (int)(at / (unsigned)a.BH), list_bh = (int)(at - (unsigned)part * (unsigned)a.BH);
+    const int pos_off = GENERAL ? a.Sk - a.S : 0;
+    const int f_rows = kFaithfulRows - pos_off < a.S ? kFaithfulRows - pos_off : a.S, per = kFaithfulRows / a.first_parts;
+    const int r0 = part * per, r1 = r0 + per < f_rows ? r0 + per : f_rows;
+    if (part >= a.first_parts || r0 >= r1) return;
+    constexpr bool STRIDES = GENERAL || STRIDED;
+    int bh = list_bh;
+    const uint16_t *Qh, *Kh, *Vh;
+    uint16_t *Oh;
+    if (STRIDES) {
+        int hi, hk;
+        const int bi = fa_strided_heads(list_bh, a.H, a.Hk, &hi, &hk);
+        bh = bi * a.H + hi;
+        Qh = a.Q + (size_t)bi * a.q_bs + (size_t)hi * a.q_hs;
+        Kh = a.K + (size_t)bi * a.k_bs + (size_t)hk * a.k_hs;
+        Vh = a.V + (size_t)bi * a.v_bs + (size_t)hk * a.v_hs;
+        Oh = a.O + (size_t)bi * a.o_bs + (size_t)hi * a.o_hs;
+    } else {
+        const size_t off = (size_t)bh * a.S * D;
+        Qh = a.Q + off; Kh = a.K + off; Vh = a.V + off; Oh = a.O + off;
+    }
+    faithful_first_rows<BF16, D>(Qh, Kh, Vh, Oh, nullptr, a.lse != nullptr ? a.lse + (size_t)bh * a.S : nullptr, r0, r1, pos_off, a.L, a.scale,
+                                 ALIBI ? a.alibi[bh % a.H] : 0.0f, STRIDES ? a.q_rs : D, STRIDES ? a.k_rs : D, STRIDES ? a.v_rs : D,
+                                 STRIDES ? a.o_rs : D, DROPOUT ? a.drop_threshold : 0u, a.drop_scale, a.seed_lo, a.seed_hi, (uint32_t)bh, lds);
+}
+
 // ---------------------------------------------------------------------------
 // The kernel.  NW waves per workgroup, 32 query rows per wave, NST LDS stages
 // per tensor.  Every wave runs ONE instruction stream per key tile; tiles are
@@ -458,6 +488,13 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int half = lane >> 5, l32 = lane & 31, l16 = lane & 15;
+
+    // (told by the grid's second dimension, which costs no argument: a test of the arguments here waits for them a trip to
+    // memory ahead of the others, 0.3 to 0.45 us of every launch)
+    if (MASKED && blockIdx.y != 0) {
+        first_rows_item<BF16, D, ALIBI, GENERAL, DROPOUT, STRIDED>(a, blockIdx.x, lds0);
+        return;
+    }
 
     // Work items.  Without a queue the grid is static: one workgroup per item (a single pass), or a resident
     // grid that walks the longest-first list as a snake (pass 0 forwards, pass 1 backwards, ...), pairing
@@ -1158,7 +1195,8 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
     // 521.  The general 4-wave kernels keep two LDS stages per tensor: with three for K their 128-wide instantiations
     // spill 24-40 bytes and measure 3-5 % slower.)
     const bool dealt = !GENERAL || (n_splits == 1 && pos_off == 0 && a.n_qblocks >= 2);
-    if (!dealt) fr1 = f_rows;
+    if (MASKED && a.first_parts > 0) {      // (workgroups of their own)
+    } else if (!dealt) fr1 = f_rows;
     else if (first_rows_on) {
         // (a resident grid without a queue walks the list as a snake: a workgroup's items come in pairs of block k
         // and block n - 1 - k, and parts on the lower half of the blocks give every pair exactly one)
@@ -1310,7 +1348,8 @@ hipError_t launch(const FaKernelArgs &a, unsigned grid, hipStream_t stream, bool
         configured.fetch_or(dev_bit, std::memory_order_relaxed);
     }
     if (configure_only) return hipSuccess;
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(NW * 64), smem, stream, a);
+    const unsigned first = (unsigned)(a.BH * a.first_parts);      // (at most twice the resident workgroups)
+    hipLaunchKernelGGL(kern, dim3(grid > first ? grid : first, first > 0 ? 2 : 1), dim3(NW * 64), smem, stream, a);
     return hipGetLastError();
 }
 
