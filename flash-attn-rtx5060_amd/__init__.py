@@ -23,6 +23,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "lib", "libfa_fwd_gfx950.so")
 HOST_LIB_PATH = os.path.join(_HERE, "lib", "libfa_host.so")
 HARNESS_PATH = os.path.join(_HERE, "bin", "fa_harness")
+TORCH_LIB_PATH = os.path.join(_HERE, "lib", "_fa_torch.so")
 
 FA_OK = 0
 FA_ERR_NULL_POINTER = -1
@@ -175,6 +176,26 @@ def lib():
     return _lib
 
 
+_native_module = None
+
+
+def _native():
+    """The binding's native part (csrc/fa_torch.cpp); raises if it has not been built (no fallback)."""
+    global _native_module
+    if _native_module is None:
+        import importlib.util
+        if not os.path.exists(TORCH_LIB_PATH):
+            raise RuntimeError(f"{TORCH_LIB_PATH} is missing: run `make -C {_HERE}` (hipcc, gfx950) first")
+        L = lib()
+        spec = importlib.util.spec_from_file_location("_fa_torch", TORCH_LIB_PATH)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        module.set_up(*(ctypes.cast(f, ctypes.c_void_p).value for f in (L.fa_fwd, L.fa_fwd_split_static, L.fa_bwd_shared)),
+                      _first_forward, _first_backward)
+        _native_module = module
+    return _native_module
+
+
 def host_lib():
     """Host-side helper library (seeded input generator, host/fa_inputs.h)."""
     global _host
@@ -259,6 +280,7 @@ _plans = {}
 _PLANS_MAX = 1024
 _PLAIN = frozenset((int, float, bool, str, type(None)))
 _WHOLE = frozenset((int, bool))            # (a float is refused for these, and 1.0 would find the entry of 1)
+_SEEDS = (1 << 64) - 1                     # (a seed is 64 bits; ctypes takes any whole number's low ones)
 _torch_module = None
 
 
@@ -278,6 +300,19 @@ def _raw_stream(torch, t):
 
 def _slopes_key(alibi_slopes):
     return None if alibi_slopes is None else (alibi_slopes.shape, alibi_slopes.stride(), alibi_slopes.dtype, alibi_slopes.device)
+
+
+def _forward_key(q, k, v, softmax_scale, causal, window_left, window_right, return_lse, sched, dropout_prob, splits, exact_first_rows, static_scratch,
+                 alibi_slopes):
+    return (q.shape, q.stride(), q.dtype, q.device, k.shape, k.stride(), k.dtype, k.device, v.shape, v.stride(), v.dtype, v.device,
+            softmax_scale, causal, window_left, window_right, return_lse, sched, dropout_prob, splits, exact_first_rows, static_scratch,
+            _slopes_key(alibi_slopes))
+
+
+def _backward_key(q, k, v, o, lse, do, softmax_scale, causal, window_left, window_right, alibi_slopes, dropout_prob):
+    return (q.shape, q.stride(), q.dtype, q.device, k.shape, k.stride(), k.dtype, k.device, v.shape, v.stride(), v.dtype, v.device,
+            o.shape, o.stride(), o.dtype, o.device, do.shape, do.stride(), do.dtype, do.device, lse.shape, lse.stride(), lse.dtype, lse.device,
+            softmax_scale, causal, window_left, window_right, dropout_prob, _slopes_key(alibi_slopes))
 
 
 def _keep_plan(key, p, *rest):
@@ -307,24 +342,11 @@ def flash_attention_forward(q, k, v, softmax_scale=None, causal=False, window_le
     if (out is None and lse is None and {type(window_left), type(window_right), type(sched), type(seed)} <= _WHOLE and
             {type(softmax_scale), type(causal), type(return_lse), type(dropout_prob), type(splits), type(exact_first_rows),
              type(static_scratch)} <= _PLAIN):
-        key = (q.shape, q.stride(), q.dtype, q.device, k.shape, k.stride(), k.dtype, k.device, v.shape, v.stride(), v.dtype, v.device,
-               softmax_scale, causal, window_left, window_right, return_lse, sched, dropout_prob, splits, exact_first_rows,
-               static_scratch, _slopes_key(alibi_slopes))
+        key = _forward_key(q, k, v, softmax_scale, causal, window_left, window_right, return_lse, sched, dropout_prob, splits, exact_first_rows,
+                           static_scratch, alibi_slopes)
         plan = _plans.get(key)
         if plan is not None:
-            block, lse_shape, need, entry = plan
-            p = FaFwdParams.from_buffer_copy(block)
-            out = torch.empty_like(q)
-            p.Q, p.K, p.V, p.O, p.seed = q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), seed
-            if return_lse:
-                lse = torch.empty(lse_shape, dtype=torch.float32, device=q.device)
-                p.L = lse.data_ptr()
-            if alibi_slopes is not None:
-                p.alibi_slopes_ptr = alibi_slopes.data_ptr()
-            if need:
-                workspace = torch.empty(need, dtype=torch.uint8, device=q.device)   # stream-ordered: freed after the launch
-                p.workspace = workspace.data_ptr()
-            st = entry(ctypes.byref(p), _raw_stream(torch, q))
+            st, out, lse = _native().forward_planned(plan[0], q, k, v, alibi_slopes, seed & _SEEDS, bool(return_lse), plan[1], bool(static_scratch))
             if st != FA_OK:
                 raise FaError(st, lib().fa_last_device_error().decode() if st == FA_ERR_DEVICE else "")
             return (out, lse) if return_lse else out
@@ -373,7 +395,7 @@ def flash_attention_forward(q, k, v, softmax_scale=None, causal=False, window_le
     if st != FA_OK:
         raise FaError(st, lib().fa_last_device_error().decode() if st == FA_ERR_DEVICE else "")
     if key is not None and q is given[0] and k is given[1] and v is given[2]:         # (no dense copy was needed)
-        _keep_plan(key, p, (B, N, S), 0 if workspace is None else p.workspace_bytes, entry)
+        _keep_plan(key, p, 0 if workspace is None else p.workspace_bytes)
     return (out, lse) if return_lse else out
 
 
@@ -416,9 +438,7 @@ def flash_attention_backward(q, k, v, o, lse, do, softmax_scale=None, causal=Fal
     key = None
     if (type(five_products) is str and five_products == "auto" and not poison_workspace and workspace_limit is None and
             {type(window_left), type(window_right), type(seed)} <= _WHOLE and {type(softmax_scale), type(causal), type(dropout_prob)} <= _PLAIN):
-        key = (q.shape, q.stride(), q.dtype, q.device, k.shape, k.stride(), k.dtype, k.device, v.shape, v.stride(), v.dtype, v.device,
-               o.shape, o.stride(), o.dtype, o.device, do.shape, do.stride(), do.dtype, do.device, lse.shape, lse.stride(), lse.dtype, lse.device,
-               softmax_scale, causal, window_left, window_right, dropout_prob, _slopes_key(alibi_slopes))
+        key = _backward_key(q, k, v, o, lse, do, softmax_scale, causal, window_left, window_right, alibi_slopes, dropout_prob)
         plan = _plans.get(key)
         workspace = None
         if plan is not None:
@@ -526,7 +546,27 @@ def flash_attention_backward(q, k, v, o, lse, do, softmax_scale=None, causal=Fal
     return dq, dk, dv
 
 
+def _first_forward(q, k, v, options):
+    """A differentiable call's forward pass where the native part has no plan for it yet: O, the logsumexp, and the plan's
+    parameter block where the call may be repeated from one."""
+    scale, causal, window_left, window_right, slopes, dropout, seed = options
+    # exact products in every row: the logsumexp must be the one fa_bwd recomputes P from
+    o, lse = flash_attention_forward(q, k, v, scale, causal, window_left, window_right, alibi_slopes=slopes, dropout_prob=dropout, seed=seed,
+                                     exact_first_rows=True)
+    plan = _plans.get(_forward_key(q, k, v, scale, causal, window_left, window_right, True, FA_SCHED_AUTO, dropout, 1, True, False, slopes))
+    return o, lse, None if plan is None else plan[0]
+
+
+def _first_backward(q, k, v, o, lse, do, options):
+    scale, causal, window_left, window_right, slopes, dropout, seed = options
+    kw = dict(softmax_scale=scale, causal=causal, window_left=window_left, window_right=window_right, alibi_slopes=slopes, dropout_prob=dropout)
+    return flash_attention_backward(q, k, v, o, lse, do, seed=seed, **kw) + (_plans.get(_backward_key(q, k, v, o, lse, do, **kw)),)
+
+
 _autograd_function = None
+_plain_tensors = None
+_NUMBERS = frozenset((int, float, bool))
+_INTS = range(-(1 << 31), 1 << 31)
 
 
 def flash_attention(q, k, v, softmax_scale=None, causal=False, window_left=-1, window_right=-1, alibi_slopes=None,
@@ -534,8 +574,20 @@ def flash_attention(q, k, v, softmax_scale=None, causal=False, window_left=-1, w
     """Differentiable attention for PyTorch callers: fa_fwd in the forward pass, fa_bwd in the backward pass
     (which replays the dropout decisions from ``seed``; nothing but O and the logsumexp is saved).  Shapes and
     layouts as in flash_attention_forward.  Plumbing only: both passes are the library's kernels."""
-    global _autograd_function
+    global _autograd_function, _plain_tensors
     import torch
+    if _plain_tensors is None:
+        _plain_tensors = frozenset((torch.Tensor, torch.nn.Parameter))
+    # Plain tensors on the GPU with plain numbers for options: an autograd function in C++, which is a third of the host time.
+    # What it cannot take -- transforms of torch.func, forward-mode gradients, tracing and compiling, tensor subclasses -- and
+    # what is refused goes through the one in Python.
+    if ({type(q), type(k), type(v)} <= _plain_tensors and q.is_cuda and k.is_cuda and v.is_cuda and type(seed) in _WHOLE and 0 <= seed <= _SEEDS and
+            {type(window_left), type(window_right)} <= _WHOLE and window_left in _INTS and window_right in _INTS and
+            (softmax_scale is None or type(softmax_scale) in _NUMBERS) and type(causal) in _NUMBERS and type(dropout_prob) in _NUMBERS and
+            (alibi_slopes is None or type(alibi_slopes) in _plain_tensors) and not torch.compiler.is_compiling() and
+            torch.autograd.forward_ad._current_level < 0 and not torch._C._are_functorch_transforms_active() and
+            torch._C._get_tracing_state() is None):
+        return _native().attention(q, k, v, softmax_scale, bool(causal), window_left, window_right, alibi_slopes, dropout_prob, seed)
     if _autograd_function is None:
         class _FlashAttention(torch.autograd.Function):
             @staticmethod
