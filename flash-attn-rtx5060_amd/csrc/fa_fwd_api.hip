@@ -101,7 +101,7 @@ int waves_of(const fa_fwd_params *p)
 
 thread_local char g_last_error[256] = "";
 
-std::atomic<unsigned> g_capture_ticket[kFaMaxDevices];     // captured queue launches so far, per device
+std::atomic<unsigned> g_capture_ticket[kFaMaxDevices], g_merge_ticket[kFaMaxDevices];     // captured launches with counters so far, per device
 // Eager launches: which stream owns which counter set of a device.  A stream is named by its handle AND the id
 // the runtime gave it at creation (hipStreamGetId): a handle value can come back for a new stream after the old
 // one was destroyed, while the old stream's last launch may still be running on its counters; the id never does.
@@ -120,7 +120,7 @@ bool stream_id(hipStream_t stream, unsigned long long *id)
     *id = 0;
     return fn == nullptr || fn(stream, id) == hipSuccess;
 }
-SlotOwner g_slot_owner[kFaMaxDevices][kFaEagerQueueSlots];
+SlotOwner g_slot_owner[kFaMaxDevices][kFaEagerQueueSlots], g_merge_owner[kFaMaxDevices][kFaEagerMergeSlots];
 
 // A counter set for one FA_SCHED_QUEUE launch, or null when none can be given safely (the caller then walks the
 // list with the fixed snake: same results, no counters).  Eager launches: a set belongs to a stream -- launches on
@@ -131,32 +131,50 @@ SlotOwner g_slot_owner[kFaMaxDevices][kFaEagerQueueSlots];
 // every replay of that graph, and a replay may run next to anything: every captured launch gets a set of its own
 // from the remaining 240, for good, and when those are used up captured launches get none.  No two launches that
 // can run at the same time ever share counters.
-unsigned *work_queue_for_launch(const FaDeviceState *ds, hipStream_t stream)
+// (Likewise the sets of the decoding kernel's merges: 64 for streams, 192 for captured launches; what gets none has its key
+// splits merged by a second launch.)  Returns the set's number, or -1.
+int counter_set_for_launch(SlotOwner *owners, int eager, int all, std::atomic<unsigned> *captured, hipStream_t stream)
 {
-    if (stream == hipStreamPerThread) return nullptr;
+    if (stream == hipStreamPerThread) return -1;
     hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
     const bool capturing = stream != nullptr && stream != hipStreamLegacy && hipStreamIsCapturing(stream, &status) == hipSuccess &&
                            status == hipStreamCaptureStatusActive;
     if (capturing) {
-        const unsigned n = g_capture_ticket[fa_launch_device()].fetch_add(1u, std::memory_order_relaxed);
-        if (n >= (unsigned)(kFaQueueSlots - kFaEagerQueueSlots)) return nullptr;
-        return ds->queues + 16u * ((unsigned)kFaEagerQueueSlots + n);
+        const unsigned n = captured->load(std::memory_order_relaxed) < (unsigned)(all - eager) ? captured->fetch_add(1u, std::memory_order_relaxed) : ~0u;
+        return n < (unsigned)(all - eager) ? eager + (int)n : -1;
     }
     // (the two names of the legacy default stream are one stream)
     const bool legacy = stream == nullptr || stream == hipStreamLegacy;
     const uintptr_t handle = legacy ? (uintptr_t)1 : reinterpret_cast<uintptr_t>(stream);
     unsigned long long id = 0;
-    if (!legacy && !stream_id(stream, &id)) return nullptr;
+    if (!legacy && !stream_id(stream, &id)) return -1;
     std::lock_guard<std::mutex> lock(g_slot_mutex);
-    SlotOwner *owners = g_slot_owner[fa_launch_device()];
     int free_slot = -1;
-    for (int i = 0; i < kFaEagerQueueSlots; ++i) {
-        if (owners[i].handle == handle && owners[i].id == id) return ds->queues + 16u * (unsigned)i;
+    for (int i = 0; i < eager; ++i) {
+        if (owners[i].handle == handle && owners[i].id == id) return i;
         if (owners[i].handle == 0 && free_slot < 0) free_slot = i;
     }
-    if (free_slot < 0) return nullptr;
-    owners[free_slot] = SlotOwner{handle, id};
-    return ds->queues + 16u * (unsigned)free_slot;
+    if (free_slot >= 0) owners[free_slot] = SlotOwner{handle, id};
+    return free_slot;
+}
+unsigned *work_queue_for_launch(const FaDeviceState *ds, hipStream_t stream)
+{
+    const int dev = fa_launch_device(), set = counter_set_for_launch(g_slot_owner[dev], kFaEagerQueueSlots, kFaQueueSlots, &g_capture_ticket[dev], stream);
+    return set < 0 ? nullptr : ds->queues + 16u * (unsigned)set;
+}
+unsigned *merge_counters_for_launch(const FaDeviceState *ds, hipStream_t stream)
+{
+    const int dev = fa_launch_device(), set = counter_set_for_launch(g_merge_owner[dev], kFaEagerMergeSlots, kFaMergeSlots, &g_merge_ticket[dev], stream);
+    return set < 0 ? nullptr : ds->merges + (size_t)(kFaMergeHeads * kFaMergeStride) * (unsigned)set;
+}
+// Whether the decoding kernel merges a call's key splits itself: a counter per K/V head, and at most the 32 KB of parts a head
+// that one workgroup's threads load at once, eight of 16 bytes each.  On the device the two are level there (beside the
+// kernel); the launch that goes is 2.5 us of a short call's host time.  128 KB: B4 H32/8 S8 S_kv 2000, 13.4 us merged by a
+// second launch, 16.3 inside; 360 KB, B1 H8 S30 S_kv 3000, 12.2 and 21.4.  Calls that read more than 64 MB of K and V, 10 us, hide a
+// launch's host time and keep the second one: B16 H32/8 S_kv 8192 (537 MB) 82.6, inside 83.1.
+bool merge_inside(long long kv_heads, long long rows, long long keys, int d, int splits)
+{
+    return kv_heads <= kFaMergeHeads && (double)kv_heads * (double)keys * d * 4.0 <= 64e6 && rows * d * 4 * splits <= 32 << 10;
 }
 
 int device_fail(hipError_t e, const char *what)
@@ -621,14 +639,18 @@ int forward(const fa_fwd_params *p, void *workspace, const FaDeviceState *ds, vo
     a.scale_log2e = p->softmax_scale * 1.44269504088896340736f;
     a.n_items = (long long)(a.BH / a.pack) * a.n_qblocks * a.n_splits;
 
+    a.merge = nullptr;
     const Launch launch = launch_of(p, ds->compute_units);
     auto launch_decode = [&]() {
         a.pack = p->N / a.Hk;
         const long long heads = (long long)p->B * a.Hk;
         a.n_items = heads * a.n_splits;
+        a.merge = nullptr;
+        if (a.n_splits > 1 && merge_inside(heads, (long long)a.pack * p->S, (long long)p->S + a.L < a.Sk ? (long long)p->S + a.L : a.Sk, p->d, a.n_splits))
+            a.merge = merge_counters_for_launch(ds, static_cast<hipStream_t>(stream));
         hipError_t e = fa_launch_forward_decode(a, p->dtype == FA_DTYPE_BF16, p->d, a.pack * p->S, launch.streaming ? 1 : 0, static_cast<hipStream_t>(stream));
         if (e != hipSuccess) return device_fail(e, "decode launch");
-        if (a.n_splits > 1) {
+        if (a.n_splits > 1 && a.merge == nullptr) {
             e = fa_launch_combine_splits(a, p->dtype == FA_DTYPE_BF16, p->d, static_cast<hipStream_t>(stream));
             if (e != hipSuccess) return device_fail(e, "combine launch");
         }
@@ -744,10 +766,12 @@ int fa_reset_work_queues(void)
     e = hipDeviceSynchronize();
     if (e != hipSuccess) return device_fail(e, "synchronize");
     e = hipMemset(ds->queues, 0, (size_t)kFaQueueSlots * 16 * sizeof(unsigned));
+    if (e == hipSuccess) e = hipMemset(ds->merges, 0, sizeof(unsigned) * kFaMergeSlots * kFaMergeHeads * kFaMergeStride);
     if (e != hipSuccess) return device_fail(e, "work queue reset");
     // (nothing is in flight after the synchronisation: streams may claim their sets anew)
     std::lock_guard<std::mutex> lock(g_slot_mutex);
     for (int i = 0; i < kFaEagerQueueSlots; ++i) g_slot_owner[fa_launch_device()][i] = SlotOwner{0, 0};
+    for (int i = 0; i < kFaEagerMergeSlots; ++i) g_merge_owner[fa_launch_device()][i] = SlotOwner{0, 0};
     return FA_OK;
 }
 
@@ -766,9 +790,12 @@ int fa_release_work_queue(void *stream_handle)
     e = hipStreamSynchronize(stream);
     if (e != hipSuccess) return device_fail(e, "synchronize");
     std::lock_guard<std::mutex> lock(g_slot_mutex);
-    SlotOwner *owners = g_slot_owner[fa_launch_device()];
-    for (int i = 0; i < kFaEagerQueueSlots; ++i)
-        if (owners[i].handle == handle && owners[i].id == id) owners[i] = SlotOwner{0, 0};
+    auto release = [&](SlotOwner *owners, int n) {
+        for (int i = 0; i < n; ++i)
+            if (owners[i].handle == handle && owners[i].id == id) owners[i] = SlotOwner{0, 0};
+    };
+    release(g_slot_owner[fa_launch_device()], kFaEagerQueueSlots);
+    release(g_merge_owner[fa_launch_device()], kFaEagerMergeSlots);
     return FA_OK;
 }
 

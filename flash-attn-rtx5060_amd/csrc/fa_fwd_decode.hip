@@ -61,6 +61,75 @@ __device__ __forceinline__ int lane_again()
     return ln;
 }
 
+// ---- what merges the parts of a row's key splits (fa_combine_splits, and the decoding kernel's own merge)
+// A part of weight zero is left out, not multiplied: what it holds may be infinite.
+// (the choice in front of the product, so that sums of products stay fused, with one rounding each)
+__device__ __forceinline__ f32x4 merge_weighted(f32x4 part, float w)
+{
+    const f32x4 none = {0.0f, 0.0f, 0.0f, 0.0f};
+    return (w > 0.0f ? part : none) * w;
+}
+struct MergeSum {
+    // running reference point and sum of weights (logsumexps are scaled scores, of any size: kNoReference is one for raw
+    // scores; from the lowest finite number the differences below are never NaN)
+    float m = -__FLT_MAX__, l = 0.0f;
+    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+};
+typedef unsigned long long u64x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void part_store(float *p, f32x4 v)
+{
+    const u64x2 w = __builtin_bit_cast(u64x2, v);
+    __hip_atomic_store(reinterpret_cast<unsigned long long *>(p), w[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(reinterpret_cast<unsigned long long *>(p) + 1, w[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// The parts of a row's four elements, eight at a time, of group `group` of `groups` that take eight in turn.  AGENT: parts that
+// other workgroups of this launch have stored at the device's scope.
+template <bool AGENT>
+__device__ __forceinline__ void merge_parts(MergeSum &sum, const float *lse_row, const float *o_row, size_t lse_step, size_t o_step, int n, int group, int groups)
+{
+    constexpr int BATCH = 8;
+    for (int s0 = BATCH * group; s0 < n; s0 += BATCH * groups) {
+        float lse[BATCH];
+        f32x4 o[BATCH];
+#pragma unroll
+        for (int u = 0; u < BATCH; ++u) {
+            const int s = s0 + u < n ? s0 + u : n - 1;
+            if (AGENT) {
+                lse[u] = __hip_atomic_load(&lse_row[(size_t)s * lse_step], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                asm volatile("global_load_dwordx4 %0, %1, off sc1" : "=v"(o[u]) : "v"(o_row + (size_t)s * o_step) : "memory");
+            } else {
+                lse[u] = lse_row[(size_t)s * lse_step];
+                o[u] = *reinterpret_cast<const f32x4 *>(o_row + (size_t)s * o_step);
+            }
+        }
+        if (AGENT)
+            asm volatile("s_waitcnt vmcnt(0)" : "+v"(o[0]), "+v"(o[1]), "+v"(o[2]), "+v"(o[3]), "+v"(o[4]), "+v"(o[5]), "+v"(o[6]), "+v"(o[7]) :: "memory");
+        float mx = sum.m;
+#pragma unroll
+        for (int u = 0; u < BATCH; ++u) {
+            if (s0 + u >= n) lse[u] = -INFINITY;
+            mx = fmaxf(mx, lse[u]);
+        }
+        const float alpha = __expf(sum.m - mx);
+        sum.acc = merge_weighted(sum.acc, alpha);
+        sum.l *= alpha;
+        sum.m = mx;
+#pragma unroll
+        for (int u = 0; u < BATCH; ++u) {
+            const float w = __expf(lse[u] - mx);
+            sum.acc += merge_weighted(o[u], w);
+            sum.l += w;
+        }
+    }
+}
+__device__ __forceinline__ void merge_two(MergeSum &a, const MergeSum &b)
+{
+    const float m = fmaxf(a.m, b.m), wa = __expf(a.m - m), wb = __expf(b.m - m);
+    a.acc = merge_weighted(a.acc, wa) + merge_weighted(b.acc, wb);
+    a.l = a.l * wa + b.l * wb;
+    a.m = m;
+}
+
 // NB: 16-row blocks of queries (R <= 16 * NB rows); NW: waves per workgroup; NT: K and V with the streaming hint
 template <bool BF16, int D, int NB, int NW, bool ALIBI, bool NT>
 __global__ void __launch_bounds__(NW * 64, NB == 1 ? 4 : 2) fa_fwd_decode(const FaKernelArgs a)
@@ -314,8 +383,13 @@ __global__ void __launch_bounds__(NW * 64, NB == 1 ? 4 : 2) fa_fwd_decode(const 
             acc *= empty ? 0.0f : 1.0f / l_all;
             const float lse = empty ? -INFINITY : m_all * a.scale + __builtin_logf(l_all);
             if (n_splits > 1) {
-                *reinterpret_cast<f32x4 *>(a.o_part + (part + row) * D + 4 * c) = acc;
-                if (c == 0) a.lse_part[part + row] = lse;
+                if (a.merge != nullptr) {         // (for a workgroup that may run on another XCD, see below)
+                    part_store(a.o_part + (part + row) * D + 4 * c, acc);
+                    if (c == 0) __hip_atomic_store(&a.lse_part[part + row], lse, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                } else {
+                    *reinterpret_cast<f32x4 *>(a.o_part + (part + row) * D + 4 * c) = acc;
+                    if (c == 0) a.lse_part[part + row] = lse;
+                }
             } else {
                 const int rh = row / S;
                 u32x2 w2;
@@ -324,6 +398,61 @@ __global__ void __launch_bounds__(NW * 64, NB == 1 ? 4 : 2) fa_fwd_decode(const 
                 *reinterpret_cast<u32x2 *>(a.O + (size_t)b * a.o_bs + (size_t)(h0 + rh) * a.o_hs + (size_t)(row - rh * S) * a.o_rs + 4 * c) = w2;
                 if (a.lse != nullptr && c == 0) a.lse[(size_t)bh * S + row] = lse;
             }
+        }
+    }
+    if (n_splits == 1 || a.merge == nullptr) return;
+
+    // ---- the head's splits merged by the workgroup that finishes the last of them, in the order of the splits.  Parts are
+    // stored and loaded at the device's scope, past the L2 of the XCD, so a store that has been acknowledged is seen from
+    // every XCD, and no cache has to be written back: a workgroup waits for its stores, counts itself, and who counts last
+    // finds all parts.
+    // (Bound by latency: three trips to memory, against a launch, its gap and two trips.  GPU time of a call by two launches /
+    // this: B1 H32/8 S_kv 1003 bf16 8.1 / 7.9 us, B2 H32 S_kv 1155 11.9 / 11.3, B4 H32/8 S_kv 1616 9.2 / 8.6, B1 H8/1 S_kv 2000 8.4 /
+    // 8.6; with the host's part the first takes 9.9 / 7.4.)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    volatile __attribute__((address_space(3))) unsigned *arrived = (volatile __attribute__((address_space(3))) unsigned *)(uintptr_t)lds_stat;
+    if (tid_e == 0) *arrived = atomicAdd(&a.merge[item * kFaMergeStride], 1u);
+    __syncthreads();
+    if (*arrived != (unsigned)n_splits - 1u) return;
+    if (tid_e == 0) __hip_atomic_store(&a.merge[item * kFaMergeStride], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    constexpr int TPR = D / 4, ALL = NW * 64;
+    // groups of threads that share the splits, as many as there are threads for, up to eight; their sums meet in LDS
+    int groups = 1;
+    while (groups < 8 && R * TPR * groups * 2 <= ALL && groups * 8 < n_splits) groups *= 2;
+    const size_t n_rows = (size_t)a.BH * S;
+    const int pairs = R * TPR;
+    for (int first = 0; first < pairs * groups; first += ALL) {
+        const int at = first + tid_e, group = groups > 1 ? at / pairs : 0, pair = at - group * pairs;
+        const bool live = group < groups && pair < pairs;
+        const int row = live ? pair / TPR : R - 1, t = live ? pair - row * TPR : 0;
+        const size_t grow = (size_t)bh * S + row;
+        MergeSum sum;
+        if (live) merge_parts<true>(sum, a.lse_part + grow, a.o_part + grow * D + 4 * t, n_rows, n_rows * D, n_splits, group, groups);
+        if (groups > 1) {                         // (then all pairs are in this one pass)
+            const uint32_t mine = lds0 + (uint32_t)tid_e * 16u, scalars = lds0 + ALL * 16u + (uint32_t)tid_e * 8u;
+            *(lds_f32x4 *)(uintptr_t)mine = sum.acc;
+            *(lds_f32 *)(uintptr_t)scalars = sum.m;
+            *(lds_f32 *)(uintptr_t)(scalars + 4u) = sum.l;
+            __syncthreads();
+            if (live && group == 0)
+                for (int g = 1; g < groups; ++g) {
+                    MergeSum other;
+                    other.acc = *(const lds_f32x4 *)(uintptr_t)(mine + (uint32_t)(g * pairs) * 16u);
+                    other.m = *(const lds_f32 *)(uintptr_t)(scalars + (uint32_t)(g * pairs) * 8u);
+                    other.l = *(const lds_f32 *)(uintptr_t)(scalars + (uint32_t)(g * pairs) * 8u + 4u);
+                    merge_two(sum, other);
+                }
+        }
+        if (live && group == 0) {
+            const bool empty = sum.l == 0.0f;
+            const f32x4 acc = sum.acc * (empty ? 0.0f : 1.0f / sum.l);
+            const int rh = row / S;
+            u32x2 w2;
+            w2[0] = N::pack2(acc[0], acc[1]);
+            w2[1] = N::pack2(acc[2], acc[3]);
+            *reinterpret_cast<u32x2 *>(a.O + (size_t)b * a.o_bs + (size_t)(h0 + rh) * a.o_hs + (size_t)(row - rh * S) * a.o_rs + 4 * t) = w2;
+            if (a.lse != nullptr && t == 0) a.lse[grow] = empty ? -INFINITY : sum.m + __logf(sum.l);
         }
     }
 }
@@ -340,50 +469,15 @@ __global__ void __launch_bounds__(256) fa_combine_splits(const FaKernelArgs a)
 {
     constexpr int TPR = D / 4;                    // threads per (row, group)
     constexpr int ROWS = 256 / (TPR * GROUPS);    // rows per workgroup
-    constexpr int BATCH = 8;
     const int t = threadIdx.x % TPR, group = threadIdx.x / TPR % GROUPS, r = threadIdx.x / (TPR * GROUPS);
     const long long n_rows = (long long)a.BH * a.S;
     long long row = (long long)blockIdx.x * ROWS + r;
     const bool live = row < n_rows;
     if (!live) row = n_rows - 1;
-    const int n = a.n_splits;
-    const float *lse_row = a.lse_part + row, *o_row = a.o_part + row * D + 4 * t;
-    const size_t o_step = (size_t)n_rows * D;
-    // (the choice in front of the product, so that sums of products stay fused, with one rounding each)
-    auto weighted = [](f32x4 part, float w) __attribute__((always_inline)) {
-        const f32x4 none = {0.0f, 0.0f, 0.0f, 0.0f};
-        return (w > 0.0f ? part : none) * w;
-    };
-    // running reference point and sum of weights (logsumexps are scaled scores, of any size: kNoReference is one for raw
-    // scores; from the lowest finite number the differences below are never NaN)
-    float m = -__FLT_MAX__, l = 0.0f;
-    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int s0 = BATCH * group; s0 < n; s0 += BATCH * GROUPS) {
-        float lse[BATCH];
-        f32x4 o[BATCH];
-#pragma unroll
-        for (int u = 0; u < BATCH; ++u) {
-            const int s = s0 + u < n ? s0 + u : n - 1;
-            lse[u] = lse_row[(size_t)s * n_rows];
-            o[u] = *reinterpret_cast<const f32x4 *>(o_row + (size_t)s * o_step);
-        }
-        float mx = m;
-#pragma unroll
-        for (int u = 0; u < BATCH; ++u) {
-            if (s0 + u >= n) lse[u] = -INFINITY;
-            mx = fmaxf(mx, lse[u]);
-        }
-        const float alpha = __expf(m - mx);
-        acc = weighted(acc, alpha);
-        l *= alpha;
-        m = mx;
-#pragma unroll
-        for (int u = 0; u < BATCH; ++u) {
-            const float w = __expf(lse[u] - mx);
-            acc += weighted(o[u], w);
-            l += w;
-        }
-    }
+    MergeSum sum;
+    merge_parts<false>(sum, a.lse_part + row, a.o_part + row * D + 4 * t, (size_t)n_rows, (size_t)n_rows * D, a.n_splits, group, GROUPS);
+    float m = sum.m, l = sum.l;
+    f32x4 acc = sum.acc;
     if (GROUPS > 1) {
         __shared__ float sm[GROUPS * ROWS], sl[GROUPS * ROWS];
         __shared__ f32x4 so[256];
@@ -398,7 +492,7 @@ __global__ void __launch_bounds__(256) fa_combine_splits(const FaKernelArgs a)
 #pragma unroll
         for (int i = 0; i < GROUPS; ++i) {
             const float w = __expf(sm[r * GROUPS + i] - m);
-            acc += weighted(so[(r * GROUPS + i) * TPR + t], w);
+            acc += merge_weighted(so[(r * GROUPS + i) * TPR + t], w);
             l += sl[r * GROUPS + i] * w;
         }
     }

@@ -10,6 +10,7 @@
 // (work_queue_for_launch in fa_fwd_api.hip): a set per stream for eager launches, a set of its own for every
 // captured launch.
 static __device__ __align__(256) unsigned g_work_queues[kFaQueueSlots][16];
+static __device__ __align__(256) unsigned g_merge_counters[kFaMergeSlots][kFaMergeHeads * kFaMergeStride];
 
 // Scratch of fa_fwd_split_static: the fp32 partial outputs and logsumexps of a launch with key splits, for
 // callers that may not allocate a workspace.  Every device holds its own copy for the life of the process.
@@ -40,9 +41,11 @@ hipError_t fa_device_state(const FaDeviceState **state)
             FaDeviceState st = {};
             e = hipGetSymbolAddress(reinterpret_cast<void **>(&st.queues), HIP_SYMBOL(g_work_queues));
             if (e != hipSuccess) return e;
+            e = hipGetSymbolAddress(reinterpret_cast<void **>(&st.merges), HIP_SYMBOL(g_merge_counters));
+            if (e != hipSuccess) return e;
             e = hipGetSymbolAddress(reinterpret_cast<void **>(&st.scratch), HIP_SYMBOL(g_split_scratch));
             if (e != hipSuccess) return e;
-            if (st.queues == nullptr || st.scratch == nullptr) return hipErrorInvalidSymbol;
+            if (st.queues == nullptr || st.merges == nullptr || st.scratch == nullptr) return hipErrorInvalidSymbol;
 #ifdef FA_CHECK_RING
             e = hipGetSymbolAddress(reinterpret_cast<void **>(&st.ring_check), HIP_SYMBOL(g_ring_check));
             if (e != hipSuccess) return e;

@@ -44,6 +44,9 @@ struct FaKernelArgs {
     int exact_first_rows;      // 1: no row is recomputed in the reference verifier's rounded-product arithmetic
     int first_parts;           // > 0: the rows that are (of every head) belong to workgroups of their own, this many per head
                                //      (1, 2, 4 or 8) in the second row of the grid, and the list's items leave them alone
+    // --- decoding kernel
+    unsigned *merge;           // null (fa_combine_splits merges the key splits), or a zero per (batch, K/V head), kFaMergeStride words apart: the workgroup
+                               //      that finishes a head's last split merges them and leaves a zero
 #ifdef FA_CHECK_RING
     // checking build only: [0] comparisons made, [1] LDS bytes that were not the tile the iteration expected
     unsigned long long *ring_check;

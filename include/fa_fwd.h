@@ -176,7 +176,10 @@ unsigned long long fa_fwd_static_scratch_bytes(void);
  * process, after which captured launches use the fixed order as well.  No two launches that can run at the same
  * time share counters.  A launch that was killed half-way (device reset, process signal) leaves its set dirty:
  * fa_reset_work_queues() waits for the device, zeroes all sets of the current device and forgets which stream
- * owned which.  Never call it while launches are being captured. */
+ * owned which.  Never call it while launches are being captured.
+ * Short decoding calls with key splits (fa_fwd with split_num > 1, few query rows) count the splits of a head in sets of the
+ * same kind, which the same rules and the same two calls govern: 64 sets for streams, 192 for captured launches; a launch
+ * without a set merges its splits by a second kernel. */
 int fa_reset_work_queues(void);
 int fa_release_work_queue(void *stream);
 
