@@ -35,6 +35,8 @@ hipError_t fa_launch_forward_dropout_regular(const FaKernelArgs &a, int bf16, in
 hipError_t fa_launch_forward_decode(const FaKernelArgs &a, int bf16, int D, int rows, int streaming, hipStream_t stream,
                                     bool configure_only = false);
 hipError_t fa_configure_forward_decode();
+hipError_t fa_launch_forward_small(const FaKernelArgs &a, int bf16, int D, int waves, hipStream_t stream, bool configure_only = false);
+hipError_t fa_configure_forward_small();
 hipError_t fa_launch_combine_splits(const FaKernelArgs &a, int bf16, int D, hipStream_t stream);
 hipError_t fa_launch_backward(const FaBwdArgs &a, int bf16, int D, int masked, int general, int alibi, int compute_units,
                               hipStream_t stream, bool configure_only = false);
@@ -374,10 +376,10 @@ long long resident_groups(int compute_units, int waves) { return (long long)comp
 // themselves.  Causal, us, in the items / apart: B1 H4 S256 D64 14.1 / 8.7, B4 H32 S128 D128 bf16 30.3 / 16.4, B5 H16 S284 D128
 // 23.2 / 14.4, B1 H32 S512 D128 20.3 / 15.2, B1 H384 S128 D64 19.4 / 17.7, B1 H256 S256 D128 31.4 / 29.2; further parts, H512 S100
 // D64 21.6 / 21.9, H128 S500 D64 22.1 / 22.5, and at four times the slots H200 S256 D64 15.9 (two) / 21.6.
-bool first_rows_apart(const FaKernelArgs &a, int masked)
+bool first_rows_few_keys(const fa_fwd_params *p, int R)
 {
-    const int pos_off = a.Sk - a.S;
-    return masked != 0 && a.R == 0 && pos_off >= 0 && pos_off < 32 && a.n_splits == 1 && a.pack == 1 && !a.exact_first_rows;
+    const int pos_off = (p->S_kv > 0 ? p->S_kv : p->S) - p->S;
+    return R == 0 && pos_off >= 0 && pos_off < 32 && packed_group(p) == 1 && !p->exact_first_rows;
 }
 int first_rows_parts(long long items, long long heads, int d, long long resident)
 {
@@ -389,8 +391,46 @@ int first_rows_parts(long long items, long long heads, int d, long long resident
 // hands out, with the streaming hint or without; else the schedule of the tile kernels' work items.
 struct Launch {
     bool decode, streaming;
+    int small_waves, first_parts;      // the kernel of 32-row blocks: waves per workgroup (0: not taken), parts of the first rows
     int sched;
 };
+// The kernel of 32-row blocks whose waves share the keys (fa_fwd_small.hip).  The key tiles, in its own units, that a block visits
+// at most; whether a problem is small enough for it, and with how many waves.
+int small_tiles(const fa_fwd_params *p)
+{
+    const long long sk = p->S_kv > 0 ? p->S_kv : p->S, keys_per_tile = p->d == 64 ? 64 : 32;
+    const int s_max = sk > p->S ? (int)sk : p->S;
+    int L, R;
+    fa_mask_bounds(s_max, p->is_causal, p->window_size_left, p->window_size_right, &L, &R);
+    const long long seen = ((long long)L + 32 + R + keys_per_tile - 2) / keys_per_tile + 1, all = (sk + keys_per_tile - 1) / keys_per_tile;
+    return (int)(seen < all ? seen : all);
+}
+// At most the workgroups that a device holds at a time, two per compute unit; twice as many where a causal walk of at least
+// 2048 queries makes the tile kernels wait for their longest blocks.  GPU time, tile kernels / this, us: no mask H16 S1024 D64 (512
+// workgroups) 14.2 / 10.5, H8 S2048 D128 (512) 34.1 / 27.9, H64 S256 D128 (512) 9.5 / 9.4, H32 S1024 D64 (1024) 15.4 / 18.9; causal
+// H8 S4096 D128 (1024) 68.6 / 56.1, H16 S2048 D64 (1024) 26.9 / 22.0, H32 S1024 D64 (1024) 16.9 / 17.3, H16 S4096 D128 (2048) 101 /
+// 107.  Two key tiles and more than a workgroup per unit: H128 S128 D64 5.5 / 5.7.  First rows in fewer parts than eight (four at
+// head dimension 64, or where all are resident) would be what the call waits for: causal H64 S256 D64 8.7 / 10.9, H48 S256 D128
+// 10.9 / 13.7, H24 S512 D128 14.7 / 12.1.  Eight waves: no mask H4 S2048 D64 12.7 (four) / 11.1, D128 22.0 / 17.3, H8 S1024 D64 8.1 / 7.9,
+// causal 8.4 / 9.4.
+int small_waves_for(const fa_fwd_params *p, int compute_units, int *first_parts)
+{
+    const int sk = p->S_kv > 0 ? p->S_kv : p->S, s_max = sk > p->S ? sk : p->S;
+    const long long heads = (long long)p->B * p->N, items = heads * ((p->S + 31) / 32), slots = 2LL * compute_units;
+    *first_parts = 0;
+    if (effective_splits(p) != 1 || fa_dropout_threshold(p->dropout_prob) != 0) return 0;
+    int L, R;
+    fa_mask_bounds(s_max, p->is_causal, p->window_size_left, p->window_size_right, &L, &R);
+    const bool uneven = R == 0 && L >= s_max && sk == p->S && p->S >= 2048;
+    if (items > (uneven ? 2 : 1) * slots || (items > compute_units && sk <= 128 && p->S % 128 == 0)) return 0;
+    if (first_rows_few_keys(p, R)) {              // (in workgroups of their own, or the problem stays with the tile kernels)
+        const long long most = (uneven ? 2 : 1) * slots + slots / 4;
+        const int parts = items + 8 * heads <= most ? 8 : 4;
+        if (parts == 4 && items + 4 * heads > (p->d == 64 ? most : slots)) return 0;
+        *first_parts = parts;
+    }
+    return items <= compute_units && small_tiles(p) >= 24 ? 8 : 4;
+}
 Launch launch_of(const fa_fwd_params *p, int compute_units)
 {
     const int sk = p->S_kv > 0 ? p->S_kv : p->S, hk = p->n_kv_heads > 0 ? p->n_kv_heads : p->N;
@@ -399,6 +439,8 @@ Launch launch_of(const fa_fwd_params *p, int compute_units)
     fa_mask_bounds(s_max, p->is_causal, p->window_size_left, p->window_size_right, &L, &R);
     Launch l;
     l.decode = decode_problem(p, R == 0, effective_splits(p));
+    l.first_parts = 0;
+    l.small_waves = l.decode ? 0 : small_waves_for(p, compute_units, &l.first_parts);      // (whatever the schedule: the same bits)
     // (the streaming hint from where the K and V that are read -- under a left window the last S + L keys -- do not stay in
     // the 256 MB memory-side cache: measured beside the kernel)
     const long long visible = (long long)p->S + L < sk ? (long long)p->S + L : sk;
@@ -445,20 +487,41 @@ unsigned long long fa_fwd_workspace_bytes(const fa_fwd_params *p)
 }
 
 namespace {
-// The tile kernels, 128-row blocks that visit `tiles` key tiles: the count from 1 to `most` with the least estimated time
+// The tile kernels' estimated time of a call with n splits, us: 128-row blocks that visit `tiles` key tiles
+double tile_kernels_us(const fa_fwd_params *p, int tiles, long long n, double second_launch_us)
+{
+    const double tile_us = p->d == 64 ? 0.55 : 0.85, partial = (double)p->B * p->N * p->S * p->d * 8.0 / 5.2e6;
+    const long long per_cu = (base_items(p) * n + kComputeUnits - 1) / kComputeUnits;
+    const double us = (double)per_cu * ((tiles + n - 1) / n * tile_us + 1.4) * (per_cu == 1 ? 1.4 : 1.0);
+    return n > 1 ? us + second_launch_us + partial * (double)n : us;
+}
+// the count from 1 to `most` with the least of it
 int least_time_splits(const fa_fwd_params *p, int tiles, int most, double second_launch_us)
 {
-    const long long items = base_items(p);
-    const double tile_us = p->d == 64 ? 0.55 : 0.85, partial = (double)p->B * p->N * p->S * p->d * 8.0 / 5.2e6;
     int best = 1;
     double best_us = 0.0;
     for (int n = 1; n == 1 || n <= most; ++n) {
-        const long long per_cu = (items * n + kComputeUnits - 1) / kComputeUnits;
-        double us = (double)per_cu * ((tiles + n - 1) / n * tile_us + 1.4) * (per_cu == 1 ? 1.4 : 1.0);
-        if (n > 1) us += second_launch_us + partial * n;
+        const double us = tile_kernels_us(p, tiles, n, second_launch_us);
         if (n == 1 || us < best_us) { best = n; best_us = us; }
     }
     return best;
+}
+// The 32-row kernel's estimated time of a call, us, or -1 where it does not take it: the tiles of its longest block in turns of
+// its waves, and what lies beside them, for four waves with one and with two workgroups on a compute unit and for eight (within
+// 10 % of 24 calls without a mask of 4 to 64 heads and 256 to 4096 keys).  Causal [B,S,H,D], split tile kernels / this, us: H32 S256
+// S_kv 1231 D128 23.0 / 13.2, D64 17.7 / 9.3, H8 S512 S_kv 2000 D128 24.2 / 15.8, H64 S128 S_kv 400 D64 12.9 / 6.0; left where they
+// were: H16 S64 S_kv 4000 D128 17.5 / 25.9, H32 S500 S_kv 4596 D128 56 / 58, H4 S100 S_kv 20000 D64 17.2 / 66.
+double small_kernel_us(const fa_fwd_params *p)
+{
+    fa_fwd_params whole = *p;
+    whole.split_num = 1;
+    int first_parts;
+    const int waves = small_waves_for(&whole, kComputeUnits, &first_parts);
+    if (waves == 0) return -1.0;
+    const double turns = (small_tiles(p) + waves - 1) / waves;
+    const bool alone = (long long)p->B * p->N * ((p->S + 31) / 32) <= kComputeUnits;
+    if (p->d == 64) return waves == 8 ? 4.7 + 1.6 * turns : alone ? 3.5 + 1.15 * turns : 4.1 + 1.65 * turns;
+    return waves == 8 ? 6.0 + 1.4 * turns : alone ? 4.8 + 1.07 * turns : 7.0 + 1.3 * turns;
 }
 }  // namespace
 
@@ -507,7 +570,10 @@ int fa_fwd_auto_splits(const fa_fwd_params *p)
         if (sk <= p->S || L < s_max || waves_of(p) == 8 || items >= 2 * kComputeUnits) return fa_fwd_suggest_splits(p);
         // (at least three tiles a split, B2 H16/4 S91 S_kv 636 5: 19.1, 2: 18.6; at most four workgroups on every slot)
         const long long slots = 8 * kComputeUnits / items;
-        return least_time_splits(p, tiles, (int)(slots < tiles / 3 ? slots : tiles / 3), 4.6);
+        const int n = least_time_splits(p, tiles, (int)(slots < tiles / 3 ? slots : tiles / 3), 4.6);
+        // (no split where the kernel of 32-row blocks, whose waves split the keys among them, is estimated to be as fast)
+        const double whole = small_kernel_us(p);
+        return whole >= 0.0 && whole <= tile_kernels_us(p, tiles, n, 4.6) ? 1 : n;
     }
     // The decoding kernel: the splits with the least estimated time.  The chip's bandwidth is shared by its CUs, so K and V
     // take as long as the CU with the most workgroups: (their bytes at 6.5 TB/s) * ceil(load) / load with load workgroups
@@ -659,6 +725,18 @@ int forward(const fa_fwd_params *p, void *workspace, const FaDeviceState *ds, vo
 #ifndef FA_CHECK_RING
     if (launch.decode) return launch_decode();      // (before a work queue is asked for: this kernel uses none)
 #endif      // (the checking build runs the tile kernels, whose ring it checks, on these problems as well, in front)
+    a.exact_first_rows = p->exact_first_rows != 0;
+    auto launch_small = [&]() {
+        a.pack = 1;
+        a.n_qblocks = (p->S + 31) / 32;
+        a.n_items = (long long)a.BH * a.n_qblocks;
+        a.first_parts = launch.first_parts;
+        const hipError_t e = fa_launch_forward_small(a, p->dtype == FA_DTYPE_BF16, p->d, launch.small_waves, static_cast<hipStream_t>(stream));
+        return e != hipSuccess ? device_fail(e, "small launch") : (int)FA_OK;
+    };
+#ifndef FA_CHECK_RING
+    if (launch.small_waves > 0) return launch_small();      // (the checking build: as with the decoding kernel)
+#endif
     // Dispatch mode launches one workgroup per item, in list order; the hardware hands them to CUs as these
     // free up, which is a longest-first greedy schedule.  Persistent mode launches one resident set of
     // workgroups that walk the list themselves.
@@ -675,9 +753,9 @@ int forward(const fa_fwd_params *p, void *workspace, const FaDeviceState *ds, vo
     a.drop_scale = 256.0f / (256.0f - (float)a.drop_threshold);
     a.seed_lo = (unsigned)(p->seed & 0xffffffffull);
     a.seed_hi = (unsigned)(p->seed >> 32);
-    a.exact_first_rows = p->exact_first_rows != 0;
     a.first_parts = 0;
-    if (launch.sched == FA_SCHED_DISPATCH && first_rows_apart(a, masked)) a.first_parts = first_rows_parts(a.n_items, a.BH, p->d, resident_groups(ds->compute_units, waves));
+    if (launch.sched == FA_SCHED_DISPATCH && a.n_splits == 1 && first_rows_few_keys(p, a.R))
+        a.first_parts = first_rows_parts(a.n_items, a.BH, p->d, resident_groups(ds->compute_units, waves));
 #ifdef FA_CHECK_RING
     a.ring_check = ds->ring_check;
 #endif
@@ -692,6 +770,7 @@ int forward(const fa_fwd_params *p, void *workspace, const FaDeviceState *ds, vo
     }
 #ifdef FA_CHECK_RING
     if (launch.decode) return launch_decode();
+    if (launch.small_waves > 0) return launch_small();
 #endif
     return FA_OK;
 }
@@ -704,7 +783,7 @@ int fa_init(void)
     if (e != hipSuccess) return device_fail(e, "device set-up");
     // everything a first launch would otherwise do besides the launch itself: after this call no entry point makes
     // a HIP call on this device that is not a stream operation (which is what a stream capture needs)
-    hipError_t (*const configure[])() = {fa_configure_forward_contiguous, fa_configure_forward_strided, fa_configure_forward_general, fa_configure_forward_decode,
+    hipError_t (*const configure[])() = {fa_configure_forward_contiguous, fa_configure_forward_strided, fa_configure_forward_general, fa_configure_forward_decode, fa_configure_forward_small,
                                          fa_configure_forward_dropout, fa_configure_forward_dropout_regular, fa_configure_backward, fa_configure_backward_dropout,
                                          fa_configure_backward_strided, fa_configure_backward_dropout_regular, fa_configure_backward_alibi_regular};
     for (auto fn : configure) {

@@ -8,12 +8,14 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
 @pytest.mark.parametrize("H,Hk,S,S_kv,D,bshd,kw", [
-    (4, 4, 1, 1, 64, False, {}), (4, 4, 3, 3, 128, False, {}), (4, 2, 31, 31, 64, True, {}), (3, 3, 33, 33, 128, True, {}),
-    (4, 4, 128, 128, 64, False, {}), (8, 2, 256, 256, 128, True, {}), (4, 4, 300, 300, 64, False, dict(window_left=5)),
-    (4, 4, 384, 384, 128, False, dict(window_left=40)), (5, 5, 100, 131, 64, False, {}), (4, 4, 9, 40, 128, True, {}),
-    (300, 300, 128, 128, 64, False, {}), (200, 100, 256, 256, 128, False, {}),             # fewer parts: four, two, one
-    (500, 500, 100, 100, 128, False, {}), (8, 8, 256, 256, 64, True, dict(dropout_prob=0.3, seed=5)),
-    (4, 4, 200, 200, 128, False, dict(dropout_prob=0.3, seed=5)), (8, 4, 128, 128, 64, False, "slopes"), (8, 8, 170, 170, 128, True, "slopes")])
+    # (two batch entries; more 32-row blocks than the kernel for small problems takes)
+    (140, 140, 33, 33, 64, False, {}), (140, 70, 33, 33, 128, True, {}), (100, 100, 128, 128, 64, False, {}), (100, 25, 128, 128, 128, True, {}),
+    (40, 10, 256, 256, 128, True, {}), (30, 30, 300, 300, 64, False, dict(window_left=5)), (25, 25, 384, 384, 128, False, dict(window_left=40)),
+    (70, 70, 100, 131, 64, False, {}), (140, 140, 40, 60, 128, True, {}),
+    (8, 8, 256, 256, 64, True, dict(dropout_prob=0.3, seed=5)), (4, 4, 200, 200, 128, False, dict(dropout_prob=0.3, seed=5)),
+    (4, 4, 1, 1, 64, False, dict(dropout_prob=0.3, seed=5)), (4, 2, 31, 31, 64, True, dict(dropout_prob=0.3, seed=5)), (4, 4, 9, 40, 128, True, dict(dropout_prob=0.3, seed=5)),
+    (100, 50, 128, 128, 64, False, "slopes"), (50, 50, 170, 170, 128, True, "slopes"),
+    (300, 300, 128, 128, 64, False, {}), (500, 500, 100, 100, 128, False, {})])             # (none apart)
 def test_rows_apart_are_the_bits_of_rows_in_items(fa, dtype, H, Hk, S, S_kv, D, bshd, kw):
     import torch
     g = torch.Generator(device="cuda").manual_seed(S + H)
