@@ -221,189 +221,229 @@ template <bool BF16> __device__ __forceinline__ uint16_t f32_to_storage(float x)
     if (BF16) return __builtin_bit_cast(uint16_t, (__bf16)x);
     return __builtin_bit_cast(uint16_t, (_Float16)x);
 }
-// Two storage-type products a.lo * b.lo and a.hi * b.hi of packed storage-type values, each rounded once to the
-// storage type (round to nearest even) and widened to fp32: the reference's half x half -> half product
-// (main.cu:193,259).  fp16: v_pk_mul_f16 rounds exactly so; the empty asm keeps the compiler from contracting
-// the product with the addition that follows into one fused operation, which would skip the rounding.
+// s0 += a.lo * b.lo and s1 += a.hi * b.hi (or both, the low one first, to one sum) of packed storage-type values, every product rounded
+// once to the storage type (round to nearest even) and widened to fp32: the reference's half x half -> half product
+// (main.cu:193,259).  fp16: v_pk_mul_f16 rounds exactly so, and the rounded pair goes into the sums through v_fma_mix_f32
+// (x * 1.0 + sum with the half-precision operand widened on the way: the same bits as a conversion followed by an addition, in one
+// instruction instead of two).  One block of assembly, or the compiler puts a wait state behind each.
 // bf16: the fp32 product of two bf16 values is exact, then one rounding.
-template <bool BF16> __device__ __forceinline__ f32x2 storage_product2(uint32_t a, uint32_t b)
+template <bool BF16> __device__ __forceinline__ void add_storage_products(uint32_t a, uint32_t b, float &s0, float &s1)
 {
     if (!BF16) {
-        f16x2 pr = __builtin_bit_cast(f16x2, a) * __builtin_bit_cast(f16x2, b);
-        uint32_t bits = __builtin_bit_cast(uint32_t, pr);
-        asm volatile("" : "+v"(bits));
-        pr = __builtin_bit_cast(f16x2, bits);
-        return f32x2{(float)pr[0], (float)pr[1]};
+        uint32_t pr;
+        asm("v_pk_mul_f16 %2, %3, %4\n\t"
+            "v_fma_mix_f32 %0, %2, 1.0, %0 op_sel:[0,0,0] op_sel_hi:[1,0,0]\n\t"
+            "v_fma_mix_f32 %1, %2, 1.0, %1 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "+v"(s0), "+v"(s1), "=&v"(pr) : "v"(a), "v"(b));
+        return;
     }
     const f32x2 exact = {__builtin_bit_cast(float, a << 16) * __builtin_bit_cast(float, b << 16),
                          __builtin_bit_cast(float, a & 0xffff0000u) * __builtin_bit_cast(float, b & 0xffff0000u)};
     const uint32_t r = __builtin_bit_cast(uint32_t, __builtin_convertvector(exact, bf16x2));
-    return f32x2{__builtin_bit_cast(float, r << 16), __builtin_bit_cast(float, r & 0xffff0000u)};
+    s0 += __builtin_bit_cast(float, r << 16);
+    s1 += __builtin_bit_cast(float, r & 0xffff0000u);
 }
-
-// s0 += a.lo * b.lo and s1 += a.hi * b.hi with every product rounded to the storage type first (s0 and s1 may be
-// the same sum: the low product is then added before the high one).  fp16: the rounded pair from v_pk_mul_f16 goes
-// into the fp32 sums through v_fma_mix_f32 (x * 1.0 + sum with the half-precision operand widened on the way:
-// the same bits as a conversion followed by an addition, in one instruction instead of two).
-template <bool BF16> __device__ __forceinline__ void add_storage_products(uint32_t a, uint32_t b, float &s0, float &s1)
+template <bool BF16> __device__ __forceinline__ void add_storage_products(uint32_t a, uint32_t b, float &sum)
 {
     if (!BF16) {
-        f16x2 pr = __builtin_bit_cast(f16x2, a) * __builtin_bit_cast(f16x2, b);
-        uint32_t bits = __builtin_bit_cast(uint32_t, pr);
-        asm("v_fma_mix_f32 %0, %1, 1.0, %0 op_sel:[0,0,0] op_sel_hi:[1,0,0]" : "+v"(s0) : "v"(bits));
-        asm("v_fma_mix_f32 %0, %1, 1.0, %0 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "+v"(s1) : "v"(bits));
+        uint32_t pr;
+        asm("v_pk_mul_f16 %1, %2, %3\n\t"
+            "v_fma_mix_f32 %0, %1, 1.0, %0 op_sel:[0,0,0] op_sel_hi:[1,0,0]\n\t"
+            "v_fma_mix_f32 %0, %1, 1.0, %0 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "+v"(sum), "=&v"(pr) : "v"(a), "v"(b));
         return;
     }
-    const f32x2 pr = storage_product2<BF16>(a, b);
-    s0 += pr[0];
-    s1 += pr[1];
+    add_storage_products<BF16>(a, b, sum, sum);
 }
 
-// Queries row0..row1-1 of a head (query i at key position i + pos_off, all positions below 32) against keys
-// 0..31.  The 32 x D blocks of Q, K and V (the rows needed) are staged in LDS once (K with its 16-byte chunks
-// XOR-swizzled by the row, so that 32 lanes reading one chunk of 32 different rows do not collide), everything
-// else runs from there.  LDS use: 3 * 32 * D * 2 + 2 * 4096 + 128 bytes.
-template <bool BF16, int D>
-__device__ __forceinline__ void faithful_first_rows(const uint16_t *Qh, const uint16_t *Kh, const uint16_t *Vh, uint16_t *Oh,
-                                    float *o32 /* null, or [rows][D] fp32 to write instead of Oh */,
-                                    float *lse_h, int row0, int row1 /* queries row0..row1-1 */,
-                                    int pos_off /* query i sits at key position i + pos_off */,
-                                    int L, float scale, float slope,
-                                    int q_rs, int k_rs, int v_rs, int o_rs /* row strides in elements */,
-                                    uint32_t drop_threshold, float drop_scale, uint32_t seed_lo, uint32_t seed_hi, uint32_t bh,
-                                    uint32_t lds /* LDS byte address of the work area */)
+// maximum over the 32 lanes of a half-wave, in all of them
+__device__ __forceinline__ float max_of_32(float x)
 {
-    constexpr int R = kFaithfulRows, CPR = D / 8;
-    // (LDS-typed pointers: through generic ones every access would be a flat instruction)
-    typedef __attribute__((address_space(3))) uint16_t lds_u16;
-    typedef __attribute__((address_space(3))) float lds_f32;
-    typedef __attribute__((address_space(3))) uint32_t lds_u32;
-    typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
-    lds_u16 *Qs = (lds_u16 *)(uintptr_t)lds, *Ks = Qs + R * D, *Vs = Ks + R * D;
-    lds_f32 *sc = (lds_f32 *)(Vs + R * D), *ex = sc + R * R, *rsum = ex + R * R;
-    lds_u32 *pbits = (lds_u32 *)ex;                         // after the softmax: p as two copies of its storage bits
-    const int tid = threadIdx.x, nthr = blockDim.x;
-    const int nrows = row1 - row0;
-    const int nkeys = row1 + pos_off;                       // keys 0..nkeys-1 are the ones any of these queries sees
-    for (int idx = tid; idx < R * CPR; idx += nthr) {
-        const int row = idx / CPR, c = idx % CPR;
-        if (row >= row0 && row < row1)
-            *(lds_u32x4 *)(Qs + row * D + 8 * c) = *reinterpret_cast<const u32x4 *>(Qh + (size_t)row * q_rs + 8 * c);
-        if (row < nkeys) {
-            *(lds_u32x4 *)(Ks + row * D + 8 * (c ^ (row & (CPR - 1)))) = *reinterpret_cast<const u32x4 *>(Kh + (size_t)row * k_rs + 8 * c);
-            *(lds_u32x4 *)(Vs + row * D + 8 * c) = *reinterpret_cast<const u32x4 *>(Vh + (size_t)row * v_rs + 8 * c);
+    x = fmaxf(x, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0xB1, 0xf, 0xf, true)));       // lanes 1 0 3 2
+    x = fmaxf(x, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0x4E, 0xf, 0xf, true)));       // lanes 2 3 0 1
+    x = fmaxf(x, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0x141, 0xf, 0xf, true)));      // mirror of eight
+    x = fmaxf(x, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0x140, 0xf, 0xf, true)));      // mirror of sixteen
+    return fmaxf(x, __shfl_xor(x, 16));
+}
+
+// Queries row0..row1-1 of a head (query i at key position i + pos_off, all positions below 32) against keys 0..31, by all waves of
+// a workgroup.  The rows of Q, K and V are requested by request() and put in LDS by finish() (K with its 16-byte chunks XOR-swizzled
+// by the row, so that 32 lanes reading one chunk of 32 rows do not collide); then a half-wave has a row, a lane one of its 32 keys, and
+// at last D / 32 of its output elements, and what the lanes of a row exchange goes through LDS of the wave's own.
+// Bound by latency: a trip to memory, then chains of additions in the verifier's order.  So the rows are requested in front of the
+// epilogue (behind it they would wait for its stores), two barriers of the workgroup are all, and a wave runs a row from its scores to
+// its output alone.  Against requests behind the epilogue and a pass over the workgroup's threads per step, six barriers between them:
+// causal B8 H16 S512 D64 18.1 against 19.6 us, D128 26.3 against 28.9, S1024 34.0 against 35.4 and 52.0 against 53.0, S1000 D128 57.5
+// against 59.4 (without the part, exact_first_rows, 16.5, 23.5, 32.1, 49.2 and 54.4).  Without the LDS, each lane reading its
+// key from memory: 18.5, 31.2, 34.3, 56.5, 59.2 -- thirty-two cache lines per load.
+template <bool BF16, int D, int NW> struct FirstRows {
+    static constexpr int R = kFaithfulRows, CPR = D / 8, COLS = D / 32, WORDS = COLS / 2, N = (R * CPR + NW * 64 - 1) / (NW * 64);
+    static constexpr int LDS_BYTES = 3 * R * D * 2 + NW * 512;
+    static_assert(R == 32, "a half-wave per row");
+    const uint16_t *Qh, *Kh, *Vh;
+    int row0, row1 /* queries row0..row1-1 */, pos_off /* query i sits at key position i + pos_off */;
+    int q_rs, k_rs, v_rs /* row strides in elements: at most 2^24 */, wave;
+    u32x4 qw[N], kw[N], vw[N];
+
+    // (the lane index is taken from the hardware and tied to its place: see the epilogue)
+    static __device__ __forceinline__ int lane_here()
+    {
+        int ln = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+        asm volatile("" : "+v"(ln));
+        return ln;
+    }
+    __device__ __forceinline__ void request()
+    {
+        const int t = wave * 64 + lane_here(), last = row1 + pos_off - 1;        // (the last key that any of these queries sees)
+#pragma unroll
+        for (int n = 0; n < N; ++n) {
+            const int idx = t + n * NW * 64, row = (idx / CPR) & (R - 1), k_row = row < last ? row : last;
+            const int q_row = row < row0 ? row0 : row < row1 ? row : row1 - 1;
+            const uint32_t col = (uint32_t)(16 * (idx % CPR));
+            qw[n] = *reinterpret_cast<const u32x4 *>(reinterpret_cast<const char *>(Qh) + ((uint32_t)(q_row * (2 * q_rs)) + col));
+            kw[n] = *reinterpret_cast<const u32x4 *>(reinterpret_cast<const char *>(Kh) + ((uint32_t)(k_row * (2 * k_rs)) + col));
+            vw[n] = *reinterpret_cast<const u32x4 *>(reinterpret_cast<const char *>(Vh) + ((uint32_t)(k_row * (2 * v_rs)) + col));
         }
     }
-    __syncthreads();
-    // scores (main.cu:189-197), masked entries -inf (main.cu:210-229); query i at position p sees keys p-L..p
-    for (int idx = tid; idx < nrows * R; idx += nthr) {
-        const int i = row0 + idx / R, j = idx % R, p = i + pos_off;
-        float s = -INFINITY;
-        if (j <= p && p - j <= L) {
+    // `lds`: LDS byte address of LDS_BYTES that no wave uses any more
+    __device__ __forceinline__ void finish(uint16_t *Oh, float *o32 /* null, or [rows][D] fp32 to write instead of Oh */, float *lse_h, int o_rs,
+                                           int L, float scale, float slope, uint32_t drop_threshold, float drop_scale, uint32_t seed_lo, uint32_t seed_hi,
+                                           uint32_t bh, uint32_t lds)
+    {
+        typedef __attribute__((address_space(3))) uint32_t lds_u32;
+        typedef __attribute__((address_space(3))) float lds_f32;
+        typedef __attribute__((address_space(3))) u32x2 lds_u32x2;
+        typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
+        const int ln = lane_here(), half = ln >> 5, j = ln & 31, last = row1 + pos_off - 1;
+        const uint32_t lds_k = lds + (uint32_t)(R * D * 2), lds_v = lds_k + (uint32_t)(R * D * 2);
+        const uint32_t e_at = lds_v + (uint32_t)(R * D * 2 + wave * 512 + half * 128), p_at = e_at + 256u;
+#pragma unroll
+        for (int n = 0; n < N; ++n) {
+            const int idx = wave * 64 + ln + n * NW * 64, row = idx / CPR, c = idx % CPR;
+            if (R * CPR % (NW * 64) != 0 && row >= R) break;
+            *(lds_u32x4 *)(uintptr_t)(lds + (uint32_t)(row * (2 * D) + 16 * c)) = qw[n];
+            *(lds_u32x4 *)(uintptr_t)(lds_k + (uint32_t)(row * (2 * D) + 16 * (c ^ (row & (CPR - 1))))) = kw[n];
+            *(lds_u32x4 *)(uintptr_t)(lds_v + (uint32_t)(row * (2 * D) + 16 * c)) = vw[n];
+        }
+        phase_barrier();
+        for (int r = row0 + wave; r < row1; r += 2 * NW) {
+            const bool live = half == 0 || r + NW < row1;
+            const int i = live ? r + half * NW : r, p = i + pos_off;         // (a row that is none repeats the first)
+            // scores (main.cu:189-197), masked entries -inf (main.cu:210-229); query i at position p sees keys p-L..p
+            const lds_u32x4 *q_lds = (const lds_u32x4 *)(uintptr_t)(lds + (uint32_t)(i * (2 * D)));
+            const uint32_t k_lds = lds_k + (uint32_t)(j * (2 * D));
             float sum = 0.0f;
-            // (the operands are read four chunks at a time, ahead of the additions that have to wait for each other)
+            // (tied four chunks at a time: left to the compiler, the rounded products are formed ahead of the additions and spilled)
 #pragma unroll
             for (int c0 = 0; c0 < CPR; c0 += 4) {
                 u32x4 qa[4], kb[4];
 #pragma unroll
                 for (int c = 0; c < 4; ++c) {
-                    qa[c] = *(const lds_u32x4 *)(Qs + i * D + 8 * (c0 + c));
-                    kb[c] = *(const lds_u32x4 *)(Ks + j * D + 8 * ((c0 + c) ^ (j & (CPR - 1))));
+                    qa[c] = q_lds[c0 + c];
+                    kb[c] = *(const lds_u32x4 *)(uintptr_t)(k_lds + (uint32_t)(16 * ((c0 + c) ^ (j & (CPR - 1)))));
                 }
+                asm volatile("" : "+v"(sum));
 #pragma unroll
                 for (int c = 0; c < 4; ++c)
 #pragma unroll
-                    for (int w = 0; w < 4; ++w) {
-                        add_storage_products<BF16>(qa[c][w], kb[c][w], sum, sum);
+                    for (int w = 0; w < 4; ++w) add_storage_products<BF16>(qa[c][w], kb[c][w], sum);
+            }
+            float s = -INFINITY;
+            if (j <= p && p - j <= L) {
+                s = sum * scale;
+                // ALiBi as the verifier applies it (main.cu:200-207): a rounded product, then a rounded difference
+                if (slope != 0.0f) s = __fsub_rn(s, __fmul_rn(slope, (float)(p - j)));
+            }
+            // softmax of the row (main.cu:232-252): the maximum does not depend on the order it is taken in, the sum adds in index order
+            // (masked entries are +0: they change no bit of it)
+            const float mx = max_of_32(s), ex = s != -INFINITY ? expf(s - mx) : 0.0f;
+            *(lds_f32 *)(uintptr_t)(e_at + 4u * (uint32_t)j) = ex;
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            float rsum = 0.0f;
+#pragma unroll
+            for (int c = 0; c < R / 4; ++c) {
+                const u32x4 e = *(const lds_u32x4 *)(uintptr_t)(e_at + (uint32_t)(16 * c));
+#pragma unroll
+                for (int w = 0; w < 4; ++w) {
+                    const uint32_t bits = e[w];
+                    rsum += __builtin_bit_cast(float, bits);
+                }
+            }
+            if (lse_h != nullptr && live && j == 0) lse_h[i] = mx + logf(rsum);
+            // p rounded to the storage type (main.cu:259), two copies of its bits
+            float pj = 0.0f;
+            if (s != -INFINITY) {
+                pj = ex / rsum;
+                if (drop_threshold != 0u) {        // keys 0..31: one 32-key block, two Philox blocks per query
+                    const DropWords d = dropout_words(seed_lo, seed_hi, bh, (uint32_t)p, (uint32_t)((j >> 2) & 1));
+                    // (the word is picked with selects: indexed with a run-time value the four words would live in scratch memory)
+                    const int wi = j >> 3;
+                    const uint32_t word = wi == 0 ? d.w[0] : wi == 1 ? d.w[1] : wi == 2 ? d.w[2] : d.w[3];
+                    pj = ((word >> (8 * (j & 3))) & 255u) >= drop_threshold ? __fmul_rn(pj, drop_scale) : 0.0f;
+                }
+            }
+            const uint32_t bits = f32_to_storage<BF16>(pj);
+            *(lds_u32 *)(uintptr_t)(p_at + 4u * (uint32_t)j) = bits | (bits << 16);
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            // weighted sum (main.cu:255-263), keys in ascending order; masked keys add nothing (their p is +0, and their V, which may
+            // not be finite, is replaced by +0: no sum that starts at +0 is ever -0, and +0 leaves all others as they are)
+            const int lo = p - L > 0 ? p - L : 0;
+            const uint32_t seen = (0xffffffffu >> (31 - p)) & (0xffffffffu << lo), v_lds = lds_v + (uint32_t)(2 * COLS * j);
+            float o[COLS];
+#pragma unroll
+            for (int t = 0; t < COLS; ++t) o[t] = 0.0f;
+#pragma unroll
+            for (int c = 0; c < R / 8; ++c) {
+                if (8 * c > last) break;
+                uint32_t pw[8], vv[8][WORDS];
+#pragma unroll
+                for (int w = 0; w < 8; ++w) {
+                    const uint32_t v_at = v_lds + (uint32_t)((8 * c + w) * (2 * D));
+                    if (WORDS == 1) {
+                        vv[w][0] = *(const lds_u32 *)(uintptr_t)v_at;
+                    } else {
+                        const u32x2 two = *(const lds_u32x2 *)(uintptr_t)v_at;
+                        vv[w][0] = two[0];
+                        vv[w][WORDS - 1] = two[1];
                     }
+                }
+#pragma unroll
+                for (int w = 0; w < 2; ++w) {
+                    const u32x4 four = *(const lds_u32x4 *)(uintptr_t)(p_at + (uint32_t)(32 * c + 16 * w));
+#pragma unroll
+                    for (int x = 0; x < 4; ++x) pw[4 * w + x] = four[x];
+                }
+#pragma unroll
+                for (int t = 0; t < COLS; ++t) asm volatile("" : "+v"(o[t]));
+#pragma unroll
+                for (int w = 0; w < 8; ++w) {
+                    const uint32_t keep = (uint32_t)__builtin_amdgcn_sbfe((int)seen, 8 * c + w, 1);
+#pragma unroll
+                    for (int t = 0; t < WORDS; ++t) add_storage_products<BF16>(pw[w], vv[w][t] & keep, o[2 * t], o[2 * t + 1]);
+                }
             }
-            s = sum * scale;
-            // ALiBi as the verifier applies it (main.cu:200-207): a rounded product, then a rounded difference
-            if (slope != 0.0f) s = __fsub_rn(s, __fmul_rn(slope, (float)(p - j)));
-        }
-        sc[i * R + j] = s;
-    }
-    __syncthreads();
-    // softmax of each row (main.cu:232-252).  The row maximum does not depend on the order it is taken in and
-    // the exponentials are independent, so every thread does one element; only the row sum has to add in
-    // index order, and one thread per row does that.
-    for (int idx = tid; idx < nrows * R; idx += nthr) {
-        const int i = row0 + idx / R, e = i * R + idx % R;
-        const lds_f32 *row = sc + i * R;
-        float mx = -INFINITY;
+            if (live) {
+                uint32_t packed[WORDS];
 #pragma unroll
-        for (int j = 0; j < R; ++j) mx = fmaxf(mx, row[j]);
-        ex[e] = sc[e] != -INFINITY ? expf(sc[e] - mx) : 0.0f;
-    }
-    __syncthreads();
-    if (tid < nrows) {
-        const int i = row0 + tid;
-        const lds_f32 *row = ex + i * R;
-        float sum = 0.0f;
+                for (int t = 0; t < WORDS; ++t) packed[t] = Num<BF16>::pack2(o[2 * t], o[2 * t + 1]);
+                if (o32 != nullptr) {
 #pragma unroll
-        for (int j = 0; j < R; ++j) sum += row[j];          // masked entries are +0: they change no bit of the sum
-        rsum[i] = sum;
-        if (lse_h != nullptr) {
-            float mx = -INFINITY;
+                    for (int t = 0; t < WORDS; ++t) {
+                        o32[(size_t)i * D + COLS * j + 2 * t] = storage_to_f32<BF16>((uint16_t)(packed[t] & 0xffffu));
+                        o32[(size_t)i * D + COLS * j + 2 * t + 1] = storage_to_f32<BF16>((uint16_t)(packed[t] >> 16));
+                    }
+                } else {
 #pragma unroll
-            for (int j = 0; j < R; ++j) mx = fmaxf(mx, sc[i * R + j]);
-            lse_h[i] = mx + logf(sum);
-        }
-    }
-    __syncthreads();
-    // p rounded to the storage type (main.cu:259)
-    for (int idx = tid; idx < nrows * R; idx += nthr) {
-        const int i = row0 + idx / R, j = idx % R, e = i * R + j;
-        float pj = 0.0f;
-        if (sc[e] != -INFINITY) {
-            pj = ex[e] / rsum[i];
-            if (drop_threshold != 0u) {        // keys 0..31: one 32-key block, two Philox blocks per query
-                const DropWords d = dropout_words(seed_lo, seed_hi, bh, (uint32_t)(i + pos_off), (uint32_t)((j >> 2) & 1));
-                // (the word is picked with selects: indexed with a run-time value the four words would live in scratch memory)
-                const int wi = j >> 3;
-                const uint32_t word = wi == 0 ? d.w[0] : wi == 1 ? d.w[1] : wi == 2 ? d.w[2] : d.w[3];
-                pj = ((word >> (8 * (j & 3))) & 255u) >= drop_threshold ? __fmul_rn(pj, drop_scale) : 0.0f;
+                    for (int t = 0; t < WORDS; ++t) *reinterpret_cast<uint32_t *>(Oh + (size_t)i * o_rs + COLS * j + 2 * t) = packed[t];
+                }
             }
         }
-        const uint32_t bits = f32_to_storage<BF16>(pj);
-        pbits[e] = bits | (bits << 16);         // (each thread overwrites only the element it has just read)
     }
-    __syncthreads();
-    // weighted sum (main.cu:255-263), keys in ascending order; masked keys have p = 0 and add nothing.  A thread
-    // owns two neighbouring output elements of one row.
-    for (int idx = tid; idx < nrows * (D / 2); idx += nthr) {
-        const int i = row0 + idx / (D / 2), t2 = idx % (D / 2), p = i + pos_off;
-        const int lo = p - L > 0 ? p - L : 0;
-        float s0 = 0.0f, s1 = 0.0f;
-        // (all operands are read first, with a fixed trip count, and the additions follow in key order under a
-        // predicate: read one by one inside a loop from lo to p, every step waited for its own LDS round trip,
-        // 85 ns per key)
-        uint32_t pw[R], vw[R];
-#pragma unroll
-        for (int j = 0; j < R; ++j) {
-            pw[j] = pbits[i * R + j];
-            vw[j] = *(const lds_u32 *)(Vs + j * D + 2 * t2);        // (rows past the last key hold stale bytes: never used)
-        }
-#pragma unroll
-        for (int j = 0; j < R; ++j) {
-            if (j >= lo && j <= p) {
-                add_storage_products<BF16>(pw[j], vw[j], s0, s1);
-            }
-        }
-        const uint32_t packed = Num<BF16>::pack2(s0, s1);
-        if (o32 != nullptr) {
-            o32[(size_t)i * D + 2 * t2] = storage_to_f32<BF16>((uint16_t)(packed & 0xffffu));
-            o32[(size_t)i * D + 2 * t2 + 1] = storage_to_f32<BF16>((uint16_t)(packed >> 16));
-        } else {
-            *reinterpret_cast<uint32_t *>(Oh + (size_t)i * o_rs + 2 * t2) = packed;
-        }
-    }
-    __syncthreads();
-}
+};
 
 // Workgroup `at` of the grid's second row (FaKernelArgs.first_parts): part at / BH of the first rows of list head at % BH.
-template <bool BF16, int D, bool ALIBI, bool GENERAL, bool DROPOUT, bool STRIDED>
-__device__ __forceinline__ void first_rows_item(const FaKernelArgs &a, unsigned at, uint32_t lds)
+template <bool BF16, int D, bool ALIBI, bool GENERAL, bool DROPOUT, bool STRIDED, int NW>
+__device__ __forceinline__ void first_rows_item(const FaKernelArgs &a, unsigned at, int wave, uint32_t lds)
 {
     const int part = (int)(at / (unsigned)a.BH), list_bh = (int)(at - (unsigned)part * (unsigned)a.BH);
     const int pos_off = GENERAL ? a.Sk - a.S : 0;
@@ -426,9 +466,10 @@ __device__ __forceinline__ void first_rows_item(const FaKernelArgs &a, unsigned 
         const size_t off = (size_t)bh * a.S * D;
         Qh = a.Q + off; Kh = a.K + off; Vh = a.V + off; Oh = a.O + off;
     }
-    faithful_first_rows<BF16, D>(Qh, Kh, Vh, Oh, nullptr, a.lse != nullptr ? a.lse + (size_t)bh * a.S : nullptr, r0, r1, pos_off, a.L, a.scale,
-                                 ALIBI ? a.alibi[bh % a.H] : 0.0f, STRIDES ? a.q_rs : D, STRIDES ? a.k_rs : D, STRIDES ? a.v_rs : D,
-                                 STRIDES ? a.o_rs : D, DROPOUT ? a.drop_threshold : 0u, a.drop_scale, a.seed_lo, a.seed_hi, (uint32_t)bh, lds);
+    FirstRows<BF16, D, NW> first{Qh, Kh, Vh, r0, r1, pos_off, STRIDES ? a.q_rs : D, STRIDES ? a.k_rs : D, STRIDES ? a.v_rs : D, wave};
+    first.request();
+    first.finish(Oh, nullptr, a.lse != nullptr ? a.lse + (size_t)bh * a.S : nullptr, STRIDES ? a.o_rs : D, a.L, a.scale,
+                 ALIBI ? a.alibi[bh % a.H] : 0.0f, DROPOUT ? a.drop_threshold : 0u, a.drop_scale, a.seed_lo, a.seed_hi, (uint32_t)bh, lds);
 }
 
 // ---------------------------------------------------------------------------
@@ -475,7 +516,7 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
     constexpr int STAGES = NST + NSTV;
     // (the first-rows path works in LDS behind the K stages that the requests for the next item fill)
     static_assert(GENERAL || LA * TILEB + NW * 32 * ROWB <= STAGES * TILEB, "the epilogue's row blocks do not fit behind the requested stages");
-    static_assert(NST <= 3 && LA * TILEB + 3 * kFaithfulRows * D * 2 + 2 * 4096 + 128 <= STAGES * TILEB, "first-rows path does not fit behind the requested stages");
+    static_assert(NST <= 3 && LA * TILEB + FirstRows<BF16, D, NW>::LDS_BYTES <= STAGES * TILEB - 64, "first-rows path does not fit behind the requested stages");
     static_assert(NSTV == NST || (NSTV == NST - 1 && NSTV >= 2), "V stages: as many as K stages, or one fewer");
     constexpr uint32_t LDS_V = NST * TILEB;       // K stages first, then V stages
     static_assert(INSTR % NW == 0, "tile must divide over the waves");
@@ -492,7 +533,7 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
     // (told by the grid's second dimension, which costs no argument: a test of the arguments here waits for them a trip to
     // memory ahead of the others, 0.3 to 0.45 us of every launch)
     if (MASKED && blockIdx.y != 0) {
-        first_rows_item<BF16, D, ALIBI, GENERAL, DROPOUT, STRIDED>(a, blockIdx.x, lds0);
+        first_rows_item<BF16, D, ALIBI, GENERAL, DROPOUT, STRIDED, NW>(a, blockIdx.x, wave, lds0);
         return;
     }
 
@@ -1171,7 +1212,7 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
     }
 
     }   // any_tile
-    // rows 0..31 of a causal head are written by faithful_first_rows below instead (with key splits: in the
+    // rows 0..31 of a causal head are written by FirstRows below instead (with key splits: in the
     // split that holds their keys, the first one; the others see none of their keys and write empty partials)
     // (GENERAL: query i sits at key position i + pos_off, so the rows concerned are those with i + pos_off < 32
     // (with more queries than keys, pos_off < 0, the path is not taken);
@@ -1235,6 +1276,9 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
             qf[s] = *reinterpret_cast<const u32x4 *>(nQ + (size_t)nrow * q_rs + 16 * s + 8 * half);
         next_requested = true;
     }
+    // (what the first rows' part reads is requested in front of the epilogue: behind it, it would wait for the epilogue's stores)
+    FirstRows<BF16, D, NW> first{Qh, Kh, Vh, fr0, fr1, pos_off, q_rs, k_rs, v_rs, wave};
+    if (MASKED && fr1 > fr0) first.request();
     // With key splits the item writes fp32 partial results, (O normalised over its own keys, logsumexp of its
     // own keys), which fa_combine_splits merges.
     float *o_part = nullptr, *lse_part = nullptr;
@@ -1244,7 +1288,7 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
         lse_part = a.lse_part + part * S;
     }
     // ---- epilogue: O / l, logsumexp (the reference has none; flash_forward.h:318-327 only divides).  Not for a
-    // row past the end, nor for rows that faithful_first_rows writes below.
+    // row past the end, nor for rows that FirstRows writes below.
     const bool own_store = wave_live && row_ok && !(!GENERAL && faithful && wave == 0) && !(GENERAL && my_q < f_rows);
     if (own_store) {
         {
@@ -1316,11 +1360,13 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
             if (!(GENERAL && o_part != nullptr) && a.lse != nullptr && half == 0) a.lse[(size_t)bh * S + q] = lse_row;
         }
     }
-    if (!GENERAL && fr1 > fr0) __syncthreads();       // (the epilogue's LDS blocks have been read by their waves)
-    if (fr1 > fr0)    // the LDS behind the first LA K stages is free
-        faithful_first_rows<BF16, D>(Qh, Kh, Vh, Oh, o_part, o_part != nullptr ? lse_part : a.lse != nullptr ? a.lse + (size_t)bh * S : nullptr,
-                                     fr0, fr1, pos_off, a.L, a.scale, slope, q_rs, k_rs, v_rs, o_rs, DROPOUT ? a.drop_threshold : 0u, a.drop_scale,
-                                     a.seed_lo, a.seed_hi, (uint32_t)bh, lds0 + LA * TILEB);
+    // (The first rows' LDS lies behind the first LA K stages, which requests for the next item may be filling already, over the rows of
+    // the epilogue; what else goes there is requested behind the next item's first barrier.)
+    if (fr1 > fr0) {
+        if (!GENERAL) phase_barrier();
+        first.finish(Oh, o_part, o_part != nullptr ? lse_part : a.lse != nullptr ? a.lse + (size_t)bh * S : nullptr, o_rs, a.L, a.scale, slope,
+                     DROPOUT ? a.drop_threshold : 0u, a.drop_scale, a.seed_lo, a.seed_hi, (uint32_t)bh, lds0 + LA * TILEB);
+    }
     item = next_item;
     }   // next work item
     // the last workgroup to leave rewinds the queue for the next launch that uses it

@@ -36,13 +36,13 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_small(const FaKernelArgs a)
 
     extern __shared__ __attribute__((aligned(1024))) char smem[];
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)smem;
+    const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, l32 = lane & 31, l16 = lane & 15;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     if (blockIdx.y != 0) {
-        first_rows_item<BF16, D, ALIBI, true, false, false>(a, blockIdx.x, lds0);
+        first_rows_item<BF16, D, ALIBI, true, false, false, NW>(a, blockIdx.x, wave, lds0);
         return;
     }
     if ((long long)blockIdx.x >= a.n_items) return;       // (the grid is as wide as its wider row)
-    const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, l32 = lane & 31, l16 = lane & 15;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t lds_k = lds0 + wave * WAVEB, lds_v = lds_k + TILEB, lds_stat = lds0 + NW * WAVEB;
 
     int list_bh, qblock, hi, hk;
