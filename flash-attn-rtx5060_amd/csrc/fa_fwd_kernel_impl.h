@@ -157,6 +157,20 @@ __device__ __forceinline__ void dma_16(const char *base, uint32_t voff, uint32_t
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
                  :: "s"(__builtin_amdgcn_readfirstlane(lds)), "v"(voff), "s"(ub) : "memory", "m0");
 }
+// Reads a word of every cache line of a kernel's arguments (one struct of type ARGS), all in one trip.  A kernel reads its arguments
+// where it first needs them, in several places that each wait for the line they touch; behind this call they are in the scalar
+// cache.  (Causal B8 H16 S1024 D64 [B,S,H,D] 36.5 against 37.8 us without it, S500 19.0 against 19.4, S1000 38.1 against 38.5.)
+template <typename ARGS> __device__ __forceinline__ void fetch_args()
+{
+    typedef const __attribute__((address_space(4))) uint32_t *Words;
+    const Words w = (Words)__builtin_amdgcn_kernarg_segment_ptr();
+    constexpr int LINES = (int)(sizeof(ARGS) + 63) / 64;
+    static_assert(LINES <= 9 && sizeof(ARGS) % 4 == 0, "a line's word each");
+    auto word = [&](int line) __attribute__((always_inline)) { return w[line < LINES ? 16 * line : 0]; };
+    const uint32_t a = word(0), b = word(1), c = word(2), d = word(3), e = word(4), f = word(5), g = word(6), h = word(7), i = word(8);
+    asm volatile("" :: "s"(a), "s"(b), "s"(c), "s"(d), "s"(e), "s"(f), "s"(g), "s"(h), "s"(i));
+}
+
 __device__ __forceinline__ void phase_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 template <int V> struct IntC { static constexpr int value = V; };
@@ -481,7 +495,7 @@ __device__ __forceinline__ void first_rows_item(const FaKernelArgs &a, unsigned 
 template <int N> __device__ __forceinline__ void wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" :: "n"(N) : "memory"); }
 
 template <bool BF16, int D, bool MASKED, bool ALIBI, bool GENERAL, bool DROPOUT, int NW, int NST, bool STRIDED = false, int NSTV = NST>
-__global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArgs a)
+__global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArgs args)
 {
     constexpr int WR = 32;                        // query rows per wave
     constexpr int BR = WR * NW;                   // query rows per workgroup
@@ -517,12 +531,14 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
     // (the first-rows path works in LDS behind the K stages that the requests for the next item fill)
     static_assert(GENERAL || LA * TILEB + NW * 32 * ROWB <= STAGES * TILEB, "the epilogue's row blocks do not fit behind the requested stages");
     static_assert(NST <= 3 && LA * TILEB + FirstRows<BF16, D, NW>::LDS_BYTES <= STAGES * TILEB - 64, "first-rows path does not fit behind the requested stages");
+    constexpr bool TIED = !(GENERAL && DROPOUT && D == 128);      // (these spill a dozen vector registers with it)
     static_assert(NSTV == NST || (NSTV == NST - 1 && NSTV >= 2), "V stages: as many as K stages, or one fewer");
     constexpr uint32_t LDS_V = NST * TILEB;       // K stages first, then V stages
     static_assert(INSTR % NW == 0, "tile must divide over the waves");
     static_assert(NST >= 2 && NST * TILEB <= 65536, "stage offsets must fit the 16-bit LDS immediate");
     typedef Num<BF16> N;
 
+    if (TIED) fetch_args<FaKernelArgs>();
     extern __shared__ __attribute__((aligned(1024))) char smem[];
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)smem;
 
@@ -533,7 +549,7 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
     // (told by the grid's second dimension, which costs no argument: a test of the arguments here waits for them a trip to
     // memory ahead of the others, 0.3 to 0.45 us of every launch)
     if (MASKED && blockIdx.y != 0) {
-        first_rows_item<BF16, D, ALIBI, GENERAL, DROPOUT, STRIDED, NW>(a, blockIdx.x, wave, lds0);
+        first_rows_item<BF16, D, ALIBI, GENERAL, DROPOUT, STRIDED, NW>(args, blockIdx.x, wave, lds0);
         return;
     }
 
@@ -545,7 +561,7 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
     // greedy schedule without its workgroup launch gaps (about 10 us per item on this chip).
     const int G = (int)gridDim.x;
     unsigned xcd = 0;
-    if (a.queue != nullptr) {
+    if (args.queue != nullptr) {
         asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID)" : "=s"(xcd));
         xcd &= 7u;
     }
@@ -557,10 +573,10 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
     // bits, the host checks that).  Queue schedule: `ticket` is the value of the own XCD's counter when thread 0
     // has fetched it ahead of time, or kNoTicket.
     auto take_item = [&](int pass_no, unsigned ticket) __attribute__((always_inline)) -> int {
-        if (a.queue == nullptr) {
+        if (args.queue == nullptr) {
             const long long base = (long long)pass_no * G;
             const long long it = base + ((pass_no & 1) ? G - 1 - (int)blockIdx.x : (int)blockIdx.x);
-            return it < a.n_items ? (int)it : -1;     // (an odd pass may leave this workgroup out; the next is empty then)
+            return it < args.n_items ? (int)it : -1;     // (an odd pass may leave this workgroup out; the next is empty then)
         }
         if (tid == 0) {
             // own XCD's list first; when that is exhausted, help the others (this also makes the result
@@ -569,22 +585,24 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
             // updated: a workgroup that finds nothing left then pays for one read instead of eight updates in
             // a row, on counters that every other leaving workgroup updates at the same time.)
             unsigned found = 0xffffffffu;
-            if (ticket == kNoTicket) ticket = atomicAdd(&a.queue[xcd], 1u);
+            __attribute__((address_space(1))) unsigned *queue = (__attribute__((address_space(1))) unsigned *)args.queue;
+            asm volatile("" : "+s"(queue));      // (or its eight addresses are formed in front of the first item)
+            if (ticket == kNoTicket) ticket = __hip_atomic_fetch_add(&queue[xcd], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             const long long own = (long long)ticket * 8 + xcd;
-            if (own < a.n_items) found = (unsigned)own;
+            if (own < args.n_items) found = (unsigned)own;
             while (found == 0xffffffffu) {
                 unsigned cnt[8];
 #pragma unroll
                 for (unsigned xo = 1; xo < 8u; ++xo)
-                    cnt[xo] = __hip_atomic_load(&a.queue[(xcd + xo) & 7u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    cnt[xo] = __hip_atomic_load(&queue[(xcd + xo) & 7u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 unsigned pick = 8u;
 #pragma unroll
                 for (unsigned xo = 7; xo >= 1u; --xo)
-                    if ((long long)cnt[xo] * 8 + ((xcd + xo) & 7u) < a.n_items) pick = xo;
+                    if ((long long)cnt[xo] * 8 + ((xcd + xo) & 7u) < args.n_items) pick = xo;
                 if (pick == 8u) break;
                 const unsigned xq = (xcd + pick) & 7u;
-                const long long cand = (long long)atomicAdd(&a.queue[xq], 1u) * 8 + xq;
-                if (cand < a.n_items) found = (unsigned)cand;
+                const long long cand = (long long)__hip_atomic_fetch_add(&queue[xq], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) * 8 + xq;
+                if (cand < args.n_items) found = (unsigned)cand;
             }
             *next_slot = found;
         }
@@ -601,6 +619,20 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
     bool next_requested = false;
     int item = take_item(0, kNoTicket);
     for (int pass = 0; item >= 0; ++pass) {
+    // (The arguments are read through a pointer that every pass ties anew, or everything that depends on them alone -- the
+    // divisions' reciprocals, conditions of the epilogue, ... -- is formed in front of the first item and parked in lanes of vector
+    // registers: 175 of them in the general 128-wide kernels, 72 with it, of the strided 64-wide ones 132 and 90, and 0.5 to 1 us of
+    // every launch.  Causal B8 H16 S1024 D64 [B,S,H,D] 35.3 against 38.0 us, with four K/V heads 35.5 against 37.5, S500 19.2 against
+    // 20.2, D128 ALiBi 31.3 against 32.1, S512 17.0 against 17.5, D128 29.3 against 29.5, B4 H16 S2048 53.0 against 53.6.  What the tile
+    // loops read is kept as it was.)
+    typedef const __attribute__((address_space(4))) FaKernelArgs KernelArgs;
+    KernelArgs *tied_args = (KernelArgs *)__builtin_amdgcn_kernarg_segment_ptr();
+    if (TIED) asm volatile("" : "+s"(tied_args));
+    auto arguments = [&]() __attribute__((always_inline)) -> auto & {
+        if constexpr (TIED) return *tied_args;
+        else return args;
+    };
+    auto &a = arguments();
     int bh, qblock;
     // (GENERAL with key splits: consecutive list positions are the splits of one (head, query block))
     const int n_splits = GENERAL ? a.n_splits : 1;
@@ -657,8 +689,8 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
         Oh = a.O + head_off;
         }
     }
-    const int q_rs = (GENERAL || STRIDED) ? a.q_rs : D, k_rs = (GENERAL || STRIDED) ? a.k_rs : D, v_rs = (GENERAL || STRIDED) ? a.v_rs : D,
-              o_rs = (GENERAL || STRIDED) ? a.o_rs : D;
+    const int q_rs = STRIDED ? args.q_rs : GENERAL ? a.q_rs : D, k_rs = STRIDED ? args.k_rs : GENERAL ? a.k_rs : D,
+              v_rs = STRIDED ? args.v_rs : GENERAL ? a.v_rs : D, o_rs = STRIDED ? args.o_rs : GENERAL ? a.o_rs : D;
 
     const int q0 = qblock * BR;
     const int qw = q0 + wave * WR;          // first query row of this wave
@@ -683,19 +715,19 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
     }
 
     // Q^T fragments: B operand, lane = (query l32, head-dim slice 8*half..+7 of each 16)
+    // (a wave without rows never uses its fragments and reads others: selects would put a branch in front of every load)
     if (!next_requested) {
+        const uint16_t *src = GENERAL ? Qh + (size_t)row_head * a.q_hs + (size_t)row_pos * q_rs
+                                      : Qh + (size_t)(wave_live ? my_q : q0 + l32) * q_rs;
 #pragma unroll
-        for (int s = 0; s < KS; ++s)
-            qf[s] = wave_live ? *reinterpret_cast<const u32x4 *>(
-                                    Qh + (GENERAL ? (size_t)row_head * a.q_hs : 0) + (size_t)row_pos * q_rs + 16 * s + 8 * half)
-                              : u32x4{0, 0, 0, 0};
+        for (int s = 0; s < KS; ++s) qf[s] = *reinterpret_cast<const u32x4 *>(src + 16 * s + 8 * half);
     }
 
     const int rows_in_block = pack > 1 ? S : S - q0 < BR ? S - q0 : BR;
     int t0, t1;                 // key tiles visited by the workgroup
-    fa_tile_range(Sk, kBlockKeys, a.L, a.R, block_pos0 + pos_off, rows_in_block, &t0, &t1);
+    fa_tile_range(Sk, kBlockKeys, args.L, args.R, block_pos0 + pos_off, rows_in_block, &t0, &t1);
     int my_lo = 1, my_hi = 0;   // key tiles with at least one visible pair for this wave (contiguous)
-    if (wave_live) fa_tile_range(Sk, kBlockKeys, a.L, a.R, wave_pos0 + pos_off, wave_npos, &my_lo, &my_hi);
+    if (wave_live) fa_tile_range(Sk, kBlockKeys, args.L, args.R, wave_pos0 + pos_off, wave_npos, &my_lo, &my_hi);
     if (n_splits > 1) {         // this item's share of the key tiles that the block visits; may leave nothing
         // (of the block's own range, not of all keys: under a window most shares of the whole cache hold nothing that the
         // block sees, and one or two did all the work.  Causal bf16 [B,S,H,D], shares of all keys against these, us: window
@@ -743,23 +775,27 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
     auto issue_k_from = [&](const uint16_t *k_head, int tile, int stage) __attribute__((always_inline)) {
         const char *src = reinterpret_cast<const char *>(k_head) + (size_t)tile * (kBlockKeys * 2) * k_rs;
         const bool ragged = GENERAL && (tile + 1) * kBlockKeys > Sk;
+        uint32_t to = lds0 + (uint32_t)(wave * 1024);
+        if (TIED) asm volatile("" : "+s"(to));             // (or the stages' addresses are all formed in front of the loop)
 #pragma unroll
         for (int i = 0; i < IPW; ++i)
-            dma_16(src, ragged ? ragged_source(tile, i, k_rs, true) : gk[i], lds0 + stage * TILEB + (i * NW + wave) * 1024);
+            dma_16(src, ragged ? ragged_source(tile, i, k_rs, true) : gk[i], to + stage * TILEB + i * NW * 1024);
     };
     auto issue_k = [&](int tile, int stage) __attribute__((always_inline)) { issue_k_from(Kh, tile, stage); };
     auto issue_v_from = [&](const uint16_t *v_head, int tile, int stage) __attribute__((always_inline)) {
         const char *src = reinterpret_cast<const char *>(v_head) + (size_t)tile * (kBlockKeys * 2) * v_rs;
         const bool ragged = GENERAL && (tile + 1) * kBlockKeys > Sk;
+        uint32_t to = lds0 + (uint32_t)(wave * 1024);
+        if (TIED) asm volatile("" : "+s"(to));             // (or the stages' addresses are all formed in front of the loop)
 #pragma unroll
         for (int i = 0; i < IPW; ++i)
-            dma_16(src, ragged ? ragged_source(tile, i, v_rs, false) : gv[i], lds0 + LDS_V + stage * TILEB + (i * NW + wave) * 1024);
+            dma_16(src, ragged ? ragged_source(tile, i, v_rs, false) : gv[i], to + LDS_V + stage * TILEB + i * NW * 1024);
     };
     auto issue_v = [&](int tile, int stage) __attribute__((always_inline)) { issue_v_from(Vh, tile, stage); };
     // skip / edge / free classification of a key tile for this wave (GENERAL: a tile that reaches past the
     // end of the sequence is an edge tile)
     auto tile_class = [&](int tile) __attribute__((always_inline)) {
-        int cls = fa_tile_class(kBlockKeys, a.L, a.R, wave_pos0 + pos_off, wave_npos, tile);
+        int cls = fa_tile_class(kBlockKeys, args.L, args.R, wave_pos0 + pos_off, wave_npos, tile);
         if (GENERAL && cls == 2 && (tile + 1) * kBlockKeys > Sk) cls = 1;
         return cls;
     };
@@ -802,13 +838,13 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
         const int kb0 = tile * kBlockKeys + 4 * half;
         const int q = row_pos + pos_off;
         // last visible key of this query (GENERAL: the sequence may end inside the tile)
-        const int j_hi = (GENERAL && q + a.R > Sk - 1) ? Sk - 1 : q + a.R;
+        const int j_hi = (GENERAL && q + args.R > Sk - 1) ? Sk - 1 : q + args.R;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             const int j0 = kb0 + 8 * (r >> 2) + (r & 3);
             const int j1 = j0 + 32;
-            if (j0 > j_hi || j0 < q - a.L) sx[0][r] = -INFINITY;
-            if (j1 > j_hi || j1 < q - a.L) sx[1][r] = -INFINITY;
+            if (j0 > j_hi || j0 < q - args.L) sx[0][r] = -INFINITY;
+            if (j1 > j_hi || j1 < q - args.L) sx[1][r] = -INFINITY;
         }
     };
     // the initial accumulator of key block `blk` of `tile`
@@ -816,7 +852,7 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
         // signed distance of this lane's query to the lane's first key of the block: exact in fp32
         const float base = (float)(row_pos + pos_off - (tile * kBlockKeys + 32 * blk + 4 * half));
         f32x16 v;
-        if (MASKED && a.R == 0) {
+        if (MASKED && args.R == 0) {
             // no visible key lies behind its query: the distance is base - k without the absolute value (the
             // elements for which that is wrong are masked), one fused multiply-add with the key offset as a literal
             const float at_base = base * neg_slope_raw;
@@ -1228,7 +1264,7 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
     // (GENERAL: query i sits at key position i + pos_off, so the rows concerned are those with i + pos_off < 32
     // (with more queries than keys, pos_off < 0, the path is not taken);
     // fa_fwd_params.exact_first_rows switches the path off)
-    const bool first_rows_on = MASKED && a.R == 0 && pos_off >= 0 && pos_off < kFaithfulRows && split == 0 && pack == 1 && !a.exact_first_rows;
+    const bool first_rows_on = MASKED && args.R == 0 && pos_off >= 0 && pos_off < kFaithfulRows && split == 0 && pack == 1 && !a.exact_first_rows;
     const bool faithful = first_rows_on && q0 == 0;         // this item's own rows 0..31 are not stored by the epilogue
     const int f_rows = !faithful ? 0 : !GENERAL ? kFaithfulRows : (kFaithfulRows - pos_off < S ? kFaithfulRows - pos_off : S);
     // Which of those rows THIS item recomputes.  General layouts: the item with the head's first block, all of
@@ -1275,7 +1311,7 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
             nQ = a.Q + noff; nK = a.K + noff; nV = a.V + noff;
         }
         const int nq0 = nqb * BR;
-        fa_tile_range(S, kBlockKeys, a.L, a.R, nq0, S - nq0 < BR ? S - nq0 : BR, &nt0, &nt1);
+        fa_tile_range(S, kBlockKeys, args.L, args.R, nq0, S - nq0 < BR ? S - nq0 : BR, &nt0, &nt1);
         // (every LDS stage is free: the last iteration ended with a barrier)
         issue_k_from(nK, nt0, 0);
         if (LA > 1 && nt0 + 1 <= nt1) issue_k_from(nK, nt0 + 1, 1);
@@ -1375,17 +1411,17 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
     // the epilogue; what else goes there is requested behind the next item's first barrier.)
     if (fr1 > fr0) {
         if (!GENERAL) phase_barrier();
-        first.finish(Oh, o_part, o_part != nullptr ? lse_part : a.lse != nullptr ? a.lse + (size_t)bh * S : nullptr, o_rs, a.L, a.scale, slope,
+        first.finish(Oh, o_part, o_part != nullptr ? lse_part : a.lse != nullptr ? a.lse + (size_t)bh * S : nullptr, o_rs, args.L, a.scale, slope,
                      DROPOUT ? a.drop_threshold : 0u, a.drop_scale, a.seed_lo, a.seed_hi, (uint32_t)bh, lds0 + LA * TILEB);
     }
     item = next_item;
     }   // next work item
     // the last workgroup to leave rewinds the queue for the next launch that uses it
-    if (a.queue != nullptr && tid == 0) {
+    if (args.queue != nullptr && tid == 0) {
         __threadfence();
-        if (atomicAdd(&a.queue[8], 1u) == (unsigned)G - 1u) {
+        if (atomicAdd(&args.queue[8], 1u) == (unsigned)G - 1u) {
 #pragma unroll
-            for (int x = 0; x < 9; ++x) a.queue[x] = 0u;
+            for (int x = 0; x < 9; ++x) args.queue[x] = 0u;
         }
     }
 }
