@@ -568,12 +568,18 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_bwd_dkdv(const FaBwdArgs a)
     // (Bound by the vector ALU: ten Philox rounds, then a comparison and a select per element for P and for dP.  With the bytes
     // compared in front of the exchange and sixteen bits put together on both sides of it, p = 0.1: B16 H16 S512 D64 no mask
     // 121 us, now 112; B16 H32 S1534 D128 causal 2036 / 1644; B4 H32 S1024 D128 no mask 404 / 273; all of the backward pass.)
+    // (Head dimension 64: what the draws of a head have in common is kept in four registers; the 128-wide kernels have none left.
+    // With it against all twenty products per draw: B16 H16 S512 D64 no mask, forward and backward, 138.5 against 140.1 us, B4 H16 S2048
+    // 244.4 / 247.1, B8 H16 S1000 161.2 / 163.9.)
+    DropAhead ahead = {0, 0, 0, 0, 0};
+    uint32_t ahead_of = 0xffffffffu;
     auto draw = [&](uint32_t bhq, int t, int qb) __attribute__((always_inline)) {
         const int ln = lane_here(), key = ln & 31, quarter = ln >> 5;
         // (the seed's registers are tied to this place too: the ten rounds' keys would otherwise be kept in twenty registers)
         uint32_t seed_lo = a.seed_lo, seed_hi = a.seed_hi;
         asm volatile("" : "+s"(seed_lo), "+s"(seed_hi));
-        const DropWords dw = dropout_words(seed_lo, seed_hi, bhq, (uint32_t)(t * 64 + 32 * qb + key + off), (uint32_t)(2 * (kw >> 5) + quarter));
+        const uint32_t query = (uint32_t)(t * 64 + 32 * qb + key + off);
+        const DropWords dw = D == 64 ? dropout_words(ahead, seed_lo, seed_hi, query) : dropout_words(seed_lo, seed_hi, bhq, query, (uint32_t)(2 * (kw >> 5) + quarter));
         const uint32_t sel1 = (ln & 1) ? 0x03070105u : 0x06020400u, sel2 = (ln & 2) ? 0x03020706u : 0x05040100u;
         u32x4 w;
 #pragma unroll
@@ -825,6 +831,10 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_bwd_dkdv(const FaBwdArgs a)
                 if (my_lo <= t && t <= my_hi) {
                     const bool edge = MASKED && (fa_tile_class(64, Lq, Rq, kw, 32, t) == 1 || (GENERAL && (t + 1) * 64 > S));
                     const uint32_t bhq = (uint32_t)(b * a.H + hk * G + g);        // the head the forward keyed its dropout on
+                    if (DROPOUT && D == 64 && bhq != ahead_of) {
+                        ahead = dropout_ahead(a.seed_lo, a.seed_hi, bhq, (uint32_t)(2 * (kw >> 5) + half));
+                        ahead_of = bhq;
+                    }
                     whole_tile(edge, slope_l2, bhq, t);
                 }
                 if (!TOP && ig < G) issue_next(prev);

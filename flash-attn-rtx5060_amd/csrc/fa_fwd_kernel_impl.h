@@ -204,20 +204,45 @@ constexpr int kFaithfulRows = 32;
 //   byte index = 4 * ((j % 32) / 8) + j % 4, bytes numbered from the low byte of output word 0
 // ---------------------------------------------------------------------------
 struct DropWords { uint32_t w[4]; };
-__device__ __forceinline__ DropWords dropout_words(uint32_t seed_lo, uint32_t seed_hi, uint32_t bh, uint32_t i, uint32_t group)
+constexpr uint32_t kPhilox0 = 0xD2511F53u, kPhilox1 = 0xCD9E8D57u, kPhiloxKey0 = 0x9E3779B9u, kPhiloxKey1 = 0xBB67AE85u;
+template <int FROM> __device__ __forceinline__ void dropout_rounds(uint32_t &c0, uint32_t &c1, uint32_t &c2, uint32_t &c3, uint32_t k0, uint32_t k1)
 {
-    uint32_t c0 = group, c1 = i, c2 = bh, c3 = 0x44524F50u, k0 = seed_lo, k1 = seed_hi;
 #pragma unroll
-    for (int round = 0; round < 10; ++round) {
+    for (int round = FROM; round < 10; ++round) {
         // (one 32 x 32 -> 64-bit multiply-add instruction per product instead of a high and a low multiply, each
         // of which runs at a quarter of the vector ALU's rate)
-        const uint64_t p0 = (uint64_t)0xD2511F53u * (uint64_t)c0, p1 = (uint64_t)0xCD9E8D57u * (uint64_t)c2;
+        const uint64_t p0 = (uint64_t)kPhilox0 * (uint64_t)c0, p1 = (uint64_t)kPhilox1 * (uint64_t)c2;
         const uint32_t h0 = (uint32_t)(p0 >> 32), l0 = (uint32_t)p0, h1 = (uint32_t)(p1 >> 32), l1 = (uint32_t)p1;
         // (the two three-way exclusive ors as one v_bitop3_b32 each, truth table 0x96; left to the compiler they
         // are two v_xor_b32 each)
         c0 = __builtin_amdgcn_bitop3_b32(h1, c1, k0, 0x96); c1 = l1; c2 = __builtin_amdgcn_bitop3_b32(h0, c3, k1, 0x96); c3 = l0;
-        k0 += 0x9E3779B9u; k1 += 0xBB67AE85u;
+        k0 += kPhiloxKey0; k1 += kPhiloxKey1;
     }
+}
+__device__ __forceinline__ DropWords dropout_words(uint32_t seed_lo, uint32_t seed_hi, uint32_t bh, uint32_t i, uint32_t group)
+{
+    uint32_t c0 = group, c1 = i, c2 = bh, c3 = 0x44524F50u, k0 = seed_lo, k1 = seed_hi;
+    dropout_rounds<0>(c0, c1, c2, c3, k0, k1);
+    return DropWords{{c0, c1, c2, c3}};
+}
+// The same words for a group of keys and a head that stay while the queries change: what does not depend on the query, four of the
+// first three rounds' six products among it, is formed once (DropAhead), three of twenty products fewer per draw than the compiler
+// leaves (it hoists the head's first one).
+struct DropAhead { uint32_t x0, x1, x2, x3, x4; };
+__device__ __forceinline__ DropAhead dropout_ahead(uint32_t seed_lo, uint32_t seed_hi, uint32_t bh, uint32_t group)
+{
+    const uint64_t p0 = (uint64_t)kPhilox0 * (uint64_t)group, p1 = (uint64_t)kPhilox1 * (uint64_t)bh;
+    const uint64_t p1b = (uint64_t)kPhilox1 * (uint64_t)((uint32_t)(p0 >> 32) ^ 0x44524F50u ^ seed_hi);
+    const uint64_t p0c = (uint64_t)kPhilox0 * (uint64_t)((uint32_t)(p1b >> 32) ^ (uint32_t)p1 ^ (seed_lo + kPhiloxKey0));
+    return DropAhead{(uint32_t)(p1 >> 32) ^ seed_lo, (uint32_t)p0 ^ (seed_hi + kPhiloxKey1), (uint32_t)p1b ^ (seed_lo + 2u * kPhiloxKey0),
+                     (uint32_t)(p0c >> 32) ^ (seed_hi + 2u * kPhiloxKey1), (uint32_t)p0c};
+}
+__device__ __forceinline__ DropWords dropout_words(const DropAhead &ahead, uint32_t seed_lo, uint32_t seed_hi, uint32_t i)
+{
+    const uint64_t p0 = (uint64_t)kPhilox0 * (uint64_t)(ahead.x0 ^ i);                                // of the second round
+    const uint64_t p1 = (uint64_t)kPhilox1 * (uint64_t)((uint32_t)(p0 >> 32) ^ ahead.x1);             // of the third
+    uint32_t c0 = (uint32_t)(p1 >> 32) ^ ahead.x2, c1 = (uint32_t)p1, c2 = (uint32_t)p0 ^ ahead.x3, c3 = ahead.x4;
+    dropout_rounds<3>(c0, c1, c2, c3, seed_lo + 3u * kPhiloxKey0, seed_hi + 3u * kPhiloxKey1);
     return DropWords{{c0, c1, c2, c3}};
 }
 __device__ __forceinline__ bool dropout_keep_byte(const DropWords &d, int r, uint32_t threshold)
@@ -531,7 +556,7 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
     // (the first-rows path works in LDS behind the K stages that the requests for the next item fill)
     static_assert(GENERAL || LA * TILEB + NW * 32 * ROWB <= STAGES * TILEB, "the epilogue's row blocks do not fit behind the requested stages");
     static_assert(NST <= 3 && LA * TILEB + FirstRows<BF16, D, NW>::LDS_BYTES <= STAGES * TILEB - 64, "first-rows path does not fit behind the requested stages");
-    constexpr bool TIED = !(GENERAL && DROPOUT && D == 128);      // (these spill a dozen vector registers with it)
+    constexpr bool TIED = !(GENERAL && DROPOUT && D == 128) || (MASKED && ALIBI);      // (the others spill a dozen vector registers with it, these spill them without)
     static_assert(NSTV == NST || (NSTV == NST - 1 && NSTV >= 2), "V stages: as many as K stages, or one fewer");
     constexpr uint32_t LDS_V = NST * TILEB;       // K stages first, then V stages
     static_assert(INSTR % NW == 0, "tile must divide over the waves");
@@ -623,8 +648,8 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
     // divisions' reciprocals, conditions of the epilogue, ... -- is formed in front of the first item and parked in lanes of vector
     // registers: 175 of them in the general 128-wide kernels, 72 with it, of the strided 64-wide ones 132 and 90, and 0.5 to 1 us of
     // every launch.  Causal B8 H16 S1024 D64 [B,S,H,D] 35.3 against 38.0 us, with four K/V heads 35.5 against 37.5, S500 19.2 against
-    // 20.2, D128 ALiBi 31.3 against 32.1, S512 17.0 against 17.5, D128 29.3 against 29.5, B4 H16 S2048 53.0 against 53.6.  What the tile
-    // loops read is kept as it was.)
+    // 20.2, D128 ALiBi 31.3 against 32.1, S512 17.0 against 17.5, D128 29.3 against 29.5, B4 H16 S2048 53.0 against 53.6.  In
+    // launches of more items it costs nothing.)
     typedef const __attribute__((address_space(4))) FaKernelArgs KernelArgs;
     KernelArgs *tied_args = (KernelArgs *)__builtin_amdgcn_kernarg_segment_ptr();
     if (TIED) asm volatile("" : "+s"(tied_args));
@@ -633,6 +658,8 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
         else return args;
     };
     auto &a = arguments();
+    // (what the tile loop reads of them is kept for the launch, or it is read again there and waits with the LDS reads)
+    const int win_L = GENERAL && DROPOUT && D == 128 ? a.L : args.L, win_R = GENERAL && DROPOUT && D == 128 ? a.R : args.R;
     int bh, qblock;
     // (GENERAL with key splits: consecutive list positions are the splits of one (head, query block))
     const int n_splits = GENERAL ? a.n_splits : 1;
@@ -725,9 +752,9 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
 
     const int rows_in_block = pack > 1 ? S : S - q0 < BR ? S - q0 : BR;
     int t0, t1;                 // key tiles visited by the workgroup
-    fa_tile_range(Sk, kBlockKeys, args.L, args.R, block_pos0 + pos_off, rows_in_block, &t0, &t1);
+    fa_tile_range(Sk, kBlockKeys, win_L, win_R, block_pos0 + pos_off, rows_in_block, &t0, &t1);
     int my_lo = 1, my_hi = 0;   // key tiles with at least one visible pair for this wave (contiguous)
-    if (wave_live) fa_tile_range(Sk, kBlockKeys, args.L, args.R, wave_pos0 + pos_off, wave_npos, &my_lo, &my_hi);
+    if (wave_live) fa_tile_range(Sk, kBlockKeys, win_L, win_R, wave_pos0 + pos_off, wave_npos, &my_lo, &my_hi);
     if (n_splits > 1) {         // this item's share of the key tiles that the block visits; may leave nothing
         // (of the block's own range, not of all keys: under a window most shares of the whole cache hold nothing that the
         // block sees, and one or two did all the work.  Causal bf16 [B,S,H,D], shares of all keys against these, us: window
@@ -795,7 +822,7 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
     // skip / edge / free classification of a key tile for this wave (GENERAL: a tile that reaches past the
     // end of the sequence is an edge tile)
     auto tile_class = [&](int tile) __attribute__((always_inline)) {
-        int cls = fa_tile_class(kBlockKeys, args.L, args.R, wave_pos0 + pos_off, wave_npos, tile);
+        int cls = fa_tile_class(kBlockKeys, win_L, win_R, wave_pos0 + pos_off, wave_npos, tile);
         if (GENERAL && cls == 2 && (tile + 1) * kBlockKeys > Sk) cls = 1;
         return cls;
     };
@@ -838,13 +865,13 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
         const int kb0 = tile * kBlockKeys + 4 * half;
         const int q = row_pos + pos_off;
         // last visible key of this query (GENERAL: the sequence may end inside the tile)
-        const int j_hi = (GENERAL && q + args.R > Sk - 1) ? Sk - 1 : q + args.R;
+        const int j_hi = (GENERAL && q + win_R > Sk - 1) ? Sk - 1 : q + win_R;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             const int j0 = kb0 + 8 * (r >> 2) + (r & 3);
             const int j1 = j0 + 32;
-            if (j0 > j_hi || j0 < q - args.L) sx[0][r] = -INFINITY;
-            if (j1 > j_hi || j1 < q - args.L) sx[1][r] = -INFINITY;
+            if (j0 > j_hi || j0 < q - win_L) sx[0][r] = -INFINITY;
+            if (j1 > j_hi || j1 < q - win_L) sx[1][r] = -INFINITY;
         }
     };
     // the initial accumulator of key block `blk` of `tile`
@@ -852,7 +879,7 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
         // signed distance of this lane's query to the lane's first key of the block: exact in fp32
         const float base = (float)(row_pos + pos_off - (tile * kBlockKeys + 32 * blk + 4 * half));
         f32x16 v;
-        if (MASKED && args.R == 0) {
+        if (MASKED && win_R == 0) {
             // no visible key lies behind its query: the distance is base - k without the absolute value (the
             // elements for which that is wrong are masked), one fused multiply-add with the key offset as a literal
             const float at_base = base * neg_slope_raw;
@@ -939,14 +966,14 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
     auto draw_dropout = [&](int tile) __attribute__((always_inline)) {
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb)
-            dw[kb] = dropout_words(a.seed_lo, a.seed_hi, (uint32_t)(bh + (GENERAL ? row_head : 0)),
+            dw[kb] = dropout_words(args.seed_lo, args.seed_hi, (uint32_t)(bh + (GENERAL ? row_head : 0)),
                                    (uint32_t)(row_pos + pos_off), (uint32_t)(2 * (2 * tile + kb) + half));
     };
     auto dropped = [&](float e, int kb, int r) __attribute__((always_inline)) {
         if (!DROPOUT) return e;
         // (a kept probability's factor 1 / (1 - p) is the same for all of them: it multiplies the row once, in the
         // epilogue, instead of 32 elements per lane and tile here)
-        return dropout_keep_byte(dw[kb], r, a.drop_threshold) ? e : 0.0f;
+        return dropout_keep_byte(dw[kb], r, args.drop_threshold) ? e : 0.0f;
     };
     auto softmax_plain = [&](int tile) __attribute__((always_inline)) {
         if (DROPOUT) draw_dropout(tile);
@@ -1264,7 +1291,7 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
     // (GENERAL: query i sits at key position i + pos_off, so the rows concerned are those with i + pos_off < 32
     // (with more queries than keys, pos_off < 0, the path is not taken);
     // fa_fwd_params.exact_first_rows switches the path off)
-    const bool first_rows_on = MASKED && args.R == 0 && pos_off >= 0 && pos_off < kFaithfulRows && split == 0 && pack == 1 && !a.exact_first_rows;
+    const bool first_rows_on = MASKED && win_R == 0 && pos_off >= 0 && pos_off < kFaithfulRows && split == 0 && pack == 1 && !a.exact_first_rows;
     const bool faithful = first_rows_on && q0 == 0;         // this item's own rows 0..31 are not stored by the epilogue
     const int f_rows = !faithful ? 0 : !GENERAL ? kFaithfulRows : (kFaithfulRows - pos_off < S ? kFaithfulRows - pos_off : S);
     // Which of those rows THIS item recomputes.  General layouts: the item with the head's first block, all of
@@ -1311,7 +1338,7 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
             nQ = a.Q + noff; nK = a.K + noff; nV = a.V + noff;
         }
         const int nq0 = nqb * BR;
-        fa_tile_range(S, kBlockKeys, args.L, args.R, nq0, S - nq0 < BR ? S - nq0 : BR, &nt0, &nt1);
+        fa_tile_range(S, kBlockKeys, win_L, win_R, nq0, S - nq0 < BR ? S - nq0 : BR, &nt0, &nt1);
         // (every LDS stage is free: the last iteration ended with a barrier)
         issue_k_from(nK, nt0, 0);
         if (LA > 1 && nt0 + 1 <= nt1) issue_k_from(nK, nt0 + 1, 1);
@@ -1411,7 +1438,7 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
     // the epilogue; what else goes there is requested behind the next item's first barrier.)
     if (fr1 > fr0) {
         if (!GENERAL) phase_barrier();
-        first.finish(Oh, o_part, o_part != nullptr ? lse_part : a.lse != nullptr ? a.lse + (size_t)bh * S : nullptr, o_rs, args.L, a.scale, slope,
+        first.finish(Oh, o_part, o_part != nullptr ? lse_part : a.lse != nullptr ? a.lse + (size_t)bh * S : nullptr, o_rs, win_L, a.scale, slope,
                      DROPOUT ? a.drop_threshold : 0u, a.drop_scale, a.seed_lo, a.seed_hi, (uint32_t)bh, lds0 + LA * TILEB);
     }
     item = next_item;
