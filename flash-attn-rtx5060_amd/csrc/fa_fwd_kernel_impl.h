@@ -553,9 +553,15 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
     constexpr int LA = NST - 1;                   // K tiles are requested LA iterations before their first use
     constexpr int LAV = NSTV - 1;                 // V tiles likewise (NSTV V stages: as many as K stages, or one fewer)
     constexpr int STAGES = NST + NSTV;
-    // (the first-rows path works in LDS behind the K stages that the requests for the next item fill)
     static_assert(GENERAL || LA * TILEB + NW * 32 * ROWB <= STAGES * TILEB, "the epilogue's row blocks do not fit behind the requested stages");
-    static_assert(NST <= 3 && LA * TILEB + FirstRows<BF16, D, NW>::LDS_BYTES <= STAGES * TILEB - 64, "first-rows path does not fit behind the requested stages");
+    // The epilogue writes whole rows, through LDS.  (Not the general 64-wide kernels: B8 H16 S1000 36.5 us with it, 36.7 without, S500
+    // 18.6 / 19.1, but B16 H16 S200 17.3 / 17.1, with ALiBi 18.0 / 17.6, B8 H16 S300 13.3 / 13.0.)
+    constexpr bool BY_ROWS = GENERAL && D == 128;
+    // The first rows' LDS: behind the K stages that the requests for the next item fill, over the rows of the epilogue.  The general kernels
+    // request nothing that early: where they write whole rows theirs begins with the stages, the epilogue's rows follow it.
+    constexpr int FIRST_AT = BY_ROWS ? 0 : LA * TILEB, ROWS_AT = BY_ROWS ? FirstRows<BF16, D, NW>::LDS_BYTES : LA * TILEB;
+    static_assert(NST <= 3 && FIRST_AT + FirstRows<BF16, D, NW>::LDS_BYTES <= STAGES * TILEB - 64, "first-rows path does not fit behind the requested stages");
+    static_assert(!BY_ROWS || (ROWS_AT >= LA * TILEB && ROWS_AT + NW * 4096 <= STAGES * TILEB - 64), "the epilogue's rows do not fit behind the requested stages");
     constexpr bool TIED = !(GENERAL && DROPOUT && D == 128) || (MASKED && ALIBI);      // (the others spill a dozen vector registers with it, these spill them without)
     static_assert(NSTV == NST || (NSTV == NST - 1 && NSTV >= 2), "V stages: as many as K stages, or one fewer");
     constexpr uint32_t LDS_V = NST * TILEB;       // K stages first, then V stages
@@ -1363,7 +1369,70 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
     }
     // ---- epilogue: O / l, logsumexp (the reference has none; flash_forward.h:318-327 only divides).  Not for a
     // row past the end, nor for rows that FirstRows writes below.
-    const bool own_store = wave_live && row_ok && !(!GENERAL && faithful && wave == 0) && !(GENERAL && my_q < f_rows);
+    if (BY_ROWS && wave_live) {
+        // The general kernels' rows likewise, 128 bytes of each at a time: from the registers, an instruction would touch 32 rows with 16
+        // bytes each (32 of fp32 partial results).  Causal B8 H16 S1000 D128 52.8 against 55.1 us, S500 27.2 / 28.3, with ALiBi 29.3 /
+        // 31.5, B2 H16 S4000 133.2 / 136.5, 500 queries on 4596 keys with four splits 51.6 / 52.6.
+        typedef __attribute__((address_space(3))) u32x2 lds_u32x2;
+        typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
+        int lane_e = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));       // (see below)
+        asm volatile("" : "+v"(lane_e));
+        const int l32_e = lane_e & 31, half_e = lane_e >> 5, chunk = lane_e & 7;
+        const uint32_t obase = lds0 + ROWS_AT + wave * 4096;
+        const float l_half = l_a + l_b;
+        const float l_tot = l_half + swap_halves(l_half);
+        const bool empty = !(l_tot > 0.0f);                 // this row saw no key (here)
+        const float inv = empty ? 0.0f : (DROPOUT ? a.drop_scale : 1.0f) / l_tot;
+        float *lse_rows = o_part != nullptr ? lse_part : a.lse != nullptr ? a.lse + (size_t)bh * S : nullptr;
+        const int my_row = qw + l32_e;
+        if (lse_rows != nullptr && half_e == 0 && my_row < n_rows && my_row >= f_rows)
+            lse_rows[my_row] = empty ? -INFINITY : m_run * a.scale + __builtin_logf(l_tot);
+        auto fence = [&]() __attribute__((always_inline)) {
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        };
+        // row i of the eight that a store instruction writes, 16 bytes a lane
+        auto stored = [&](int i, auto to) __attribute__((always_inline)) {
+            const int row = 8 * i + (lane_e >> 3), q = qw + row;
+            const u32x4 w = *(const lds_u32x4 *)(uintptr_t)(obase + row * 128 + ((chunk ^ (row & 7)) << 4));
+            if (q < n_rows && q >= f_rows) *reinterpret_cast<u32x4 *>(to(q)) = w;
+        };
+        if (o_part != nullptr) {
+#pragma unroll
+            for (int db = 0; db < DB; ++db) {
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    const f32x4 w = {o[db][4 * g] * inv, o[db][4 * g + 1] * inv, o[db][4 * g + 2] * inv, o[db][4 * g + 3] * inv};
+                    *(lds_u32x4 *)(uintptr_t)(obase + l32_e * 128 + (((2 * g + half_e) ^ (l32_e & 7)) << 4)) = __builtin_bit_cast(u32x4, w);
+                }
+                fence();
+#pragma unroll
+                for (int i = 0; i < 4; ++i) stored(i, [&](int q) { return o_part + (size_t)q * D + 32 * db + 4 * chunk; });
+                fence();
+            }
+        } else {
+#pragma unroll
+            for (int part = 0; part < D / 64; ++part) {
+#pragma unroll
+                for (int c = 0; c < 8; ++c) {
+                    const int db = 2 * part + c / 4, g = c % 4;
+                    u32x2 w;
+                    w[0] = N::pack2(o[db][4 * g] * inv, o[db][4 * g + 1] * inv);
+                    w[1] = N::pack2(o[db][4 * g + 2] * inv, o[db][4 * g + 3] * inv);
+                    *(lds_u32x2 *)(uintptr_t)(obase + l32_e * 128 + ((c ^ (l32_e & 7)) << 4) + 8 * half_e) = w;
+                }
+                fence();
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    stored(i, [&](int q) {
+                        const int head = pack > 1 ? q / S : 0;
+                        return Oh + (size_t)head * a.o_hs + (size_t)(q - head * S) * o_rs + 64 * part + 8 * chunk;
+                    });
+                fence();
+            }
+        }
+    }
+    const bool own_store = !BY_ROWS && wave_live && row_ok && !(!GENERAL && faithful && wave == 0) && !(GENERAL && my_q < f_rows);
     if (own_store) {
         {
             // the row's index in its head's [S, ...] output, counted from head `bh` (packed groups: row_head
@@ -1399,7 +1468,7 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
                 int lane_e = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
                 asm volatile("" : "+v"(lane_e));
                 const int l32_e = lane_e & 31, half_e = lane_e >> 5;
-                const uint32_t obase = lds0 + LA * TILEB + wave * (32 * ROWB);
+                const uint32_t obase = lds0 + ROWS_AT + wave * (32 * ROWB);
 #pragma unroll
                 for (int db = 0; db < DB; ++db)
 #pragma unroll
@@ -1434,12 +1503,13 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
             if (!(GENERAL && o_part != nullptr) && a.lse != nullptr && half == 0) a.lse[(size_t)bh * S + q] = lse_row;
         }
     }
-    // (The first rows' LDS lies behind the first LA K stages, which requests for the next item may be filling already, over the rows of
-    // the epilogue; what else goes there is requested behind the next item's first barrier.)
+    // (No other wave uses FIRST_AT's LDS behind these barriers, or in the general kernels in front of them: what the next item requests
+    // behind the first LA K stages it requests behind its first barrier.)
     if (fr1 > fr0) {
         if (!GENERAL) phase_barrier();
         first.finish(Oh, o_part, o_part != nullptr ? lse_part : a.lse != nullptr ? a.lse + (size_t)bh * S : nullptr, o_rs, win_L, a.scale, slope,
-                     DROPOUT ? a.drop_threshold : 0u, a.drop_scale, a.seed_lo, a.seed_hi, (uint32_t)bh, lds0 + LA * TILEB);
+                     DROPOUT ? a.drop_threshold : 0u, a.drop_scale, a.seed_lo, a.seed_hi, (uint32_t)bh, lds0 + FIRST_AT);
+        if (BY_ROWS) phase_barrier();       // (the next item's first K tile goes over it)
     }
     item = next_item;
     }   // next work item
