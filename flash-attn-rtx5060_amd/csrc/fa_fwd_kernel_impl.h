@@ -562,7 +562,8 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
     constexpr int FIRST_AT = BY_ROWS ? 0 : LA * TILEB, ROWS_AT = BY_ROWS ? FirstRows<BF16, D, NW>::LDS_BYTES : LA * TILEB;
     static_assert(NST <= 3 && FIRST_AT + FirstRows<BF16, D, NW>::LDS_BYTES <= STAGES * TILEB - 64, "first-rows path does not fit behind the requested stages");
     static_assert(!BY_ROWS || (ROWS_AT >= LA * TILEB && ROWS_AT + NW * 4096 <= STAGES * TILEB - 64), "the epilogue's rows do not fit behind the requested stages");
-    constexpr bool TIED = !(GENERAL && DROPOUT && D == 128) || (MASKED && ALIBI);      // (the others spill a dozen vector registers with it, these spill them without)
+    // (see the item loop; the kernels left out spill a dozen vector registers with it, those with ALiBi and a mask without it)
+    constexpr bool TIED = !(GENERAL && DROPOUT && D == 128) || (MASKED && ALIBI);
     static_assert(NSTV == NST || (NSTV == NST - 1 && NSTV >= 2), "V stages: as many as K stages, or one fewer");
     constexpr uint32_t LDS_V = NST * TILEB;       // K stages first, then V stages
     static_assert(INSTR % NW == 0, "tile must divide over the waves");
