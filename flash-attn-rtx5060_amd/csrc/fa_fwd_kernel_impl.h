@@ -1293,12 +1293,17 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
     }
 
     }   // any_tile
+    // (tied once more, or what depends on them alone behind the tile loop is formed in front of it: causal B4 H16 S2048 D64 52.4 against
+    // 53.0 us, B8 H16 S1024 34.5 / 35.3, S512 16.7 / 17.0.  Not the general kernels: D64 without a mask B8 H16 S1000 48.6 / 49.3, but
+    // B16 H16 S200 12.9 / 12.4, D128 S500 28.1 / 27.9)
+    if (TIED && !GENERAL) asm volatile("" : "+s"(tied_args));
+    auto &late = arguments();
     // rows 0..31 of a causal head are written by FirstRows below instead (with key splits: in the
     // split that holds their keys, the first one; the others see none of their keys and write empty partials)
     // (GENERAL: query i sits at key position i + pos_off, so the rows concerned are those with i + pos_off < 32
     // (with more queries than keys, pos_off < 0, the path is not taken);
     // fa_fwd_params.exact_first_rows switches the path off)
-    const bool first_rows_on = MASKED && win_R == 0 && pos_off >= 0 && pos_off < kFaithfulRows && split == 0 && pack == 1 && !a.exact_first_rows;
+    const bool first_rows_on = MASKED && win_R == 0 && pos_off >= 0 && pos_off < kFaithfulRows && split == 0 && pack == 1 && !late.exact_first_rows;
     const bool faithful = first_rows_on && q0 == 0;         // this item's own rows 0..31 are not stored by the epilogue
     const int f_rows = !faithful ? 0 : !GENERAL ? kFaithfulRows : (kFaithfulRows - pos_off < S ? kFaithfulRows - pos_off : S);
     // Which of those rows THIS item recomputes.  General layouts: the item with the head's first block, all of
@@ -1316,15 +1321,15 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
     // (causal B8 H32 S1000 D64 445 against 382 TFLOP/s, B16 H16 S500 D128 341 against 296, B4 H16 S2047 D64 573 against
     // 521.  The general 4-wave kernels keep two LDS stages per tensor: with three for K their 128-wide instantiations
     // spill 24-40 bytes and measure 3-5 % slower.)
-    const bool dealt = !GENERAL || (n_splits == 1 && pos_off == 0 && a.n_qblocks >= 2);
-    if (MASKED && a.first_parts > 0) {      // (workgroups of their own)
+    const bool dealt = !GENERAL || (n_splits == 1 && pos_off == 0 && late.n_qblocks >= 2);
+    if (MASKED && late.first_parts > 0) {      // (workgroups of their own)
     } else if (!dealt) fr1 = f_rows;
     else if (first_rows_on) {
         // (a resident grid without a queue walks the list as a snake: a workgroup's items come in pairs of block k
         // and block n - 1 - k, and parts on the lower half of the blocks give every pair exactly one)
-        const bool snake = a.queue == nullptr && (long long)gridDim.x < a.n_items;
-        const int parts = snake ? (a.n_qblocks >= 16 ? 8 : a.n_qblocks >= 8 ? 4 : a.n_qblocks >= 4 ? 2 : 1)
-                                : (a.n_qblocks >= 4 ? 4 : a.n_qblocks >= 2 ? 2 : 1);
+        const bool snake = late.queue == nullptr && (long long)gridDim.x < late.n_items;
+        const int parts = snake ? (late.n_qblocks >= 16 ? 8 : late.n_qblocks >= 8 ? 4 : late.n_qblocks >= 4 ? 2 : 1)
+                                : (late.n_qblocks >= 4 ? 4 : late.n_qblocks >= 2 ? 2 : 1);
         if (qblock < parts) { fr0 = qblock * (kFaithfulRows / parts); fr1 = fr0 + kFaithfulRows / parts; }
     }
     // ---- the next work item, and the first requests for it
@@ -1332,17 +1337,17 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
     // (the first-rows path below works in the LDS behind the K stages that are filled here)
     if (!GENERAL && next_item >= 0) {
         int nbh, nqb, nt0, nt1;
-        fa_item_decode(next_item, a.BH, a.n_qblocks, a.descending, &nbh, &nqb);
+        fa_item_decode(next_item, late.BH, late.n_qblocks, late.descending, &nbh, &nqb);
         const uint16_t *nQ, *nK, *nV;
         if (STRIDED) {
             int nhi, nhk;
-            const int nbi = fa_strided_heads(nbh, a.H, a.Hk, &nhi, &nhk);
-            nQ = a.Q + (size_t)nbi * a.q_bs + (size_t)nhi * a.q_hs;
-            nK = a.K + (size_t)nbi * a.k_bs + (size_t)nhk * a.k_hs;
-            nV = a.V + (size_t)nbi * a.v_bs + (size_t)nhk * a.v_hs;
+            const int nbi = fa_strided_heads(nbh, late.H, late.Hk, &nhi, &nhk);
+            nQ = late.Q + (size_t)nbi * late.q_bs + (size_t)nhi * late.q_hs;
+            nK = late.K + (size_t)nbi * late.k_bs + (size_t)nhk * late.k_hs;
+            nV = late.V + (size_t)nbi * late.v_bs + (size_t)nhk * late.v_hs;
         } else {
             const size_t noff = (size_t)nbh * S * D;
-            nQ = a.Q + noff; nK = a.K + noff; nV = a.V + noff;
+            nQ = late.Q + noff; nK = late.K + noff; nV = late.V + noff;
         }
         const int nq0 = nqb * BR;
         fa_tile_range(S, kBlockKeys, win_L, win_R, nq0, S - nq0 < BR ? S - nq0 : BR, &nt0, &nt1);
@@ -1364,9 +1369,9 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
     // own keys), which fa_combine_splits merges.
     float *o_part = nullptr, *lse_part = nullptr;
     if (GENERAL && n_splits > 1) {
-        const size_t part = (size_t)split * a.BH + bh;       // (row_head rows further for the heads of a packed group)
-        o_part = a.o_part + part * S * D;
-        lse_part = a.lse_part + part * S;
+        const size_t part = (size_t)split * late.BH + bh;       // (row_head rows further for the heads of a packed group)
+        o_part = late.o_part + part * S * D;
+        lse_part = late.lse_part + part * S;
     }
     // ---- epilogue: O / l, logsumexp (the reference has none; flash_forward.h:318-327 only divides).  Not for a
     // row past the end, nor for rows that FirstRows writes below.
@@ -1383,11 +1388,11 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
         const float l_half = l_a + l_b;
         const float l_tot = l_half + swap_halves(l_half);
         const bool empty = !(l_tot > 0.0f);                 // this row saw no key (here)
-        const float inv = empty ? 0.0f : (DROPOUT ? a.drop_scale : 1.0f) / l_tot;
-        float *lse_rows = o_part != nullptr ? lse_part : a.lse != nullptr ? a.lse + (size_t)bh * S : nullptr;
+        const float inv = empty ? 0.0f : (DROPOUT ? late.drop_scale : 1.0f) / l_tot;
+        float *lse_rows = o_part != nullptr ? lse_part : late.lse != nullptr ? late.lse + (size_t)bh * S : nullptr;
         const int my_row = qw + l32_e;
         if (lse_rows != nullptr && half_e == 0 && my_row < n_rows && my_row >= f_rows)
-            lse_rows[my_row] = empty ? -INFINITY : m_run * a.scale + __builtin_logf(l_tot);
+            lse_rows[my_row] = empty ? -INFINITY : m_run * late.scale + __builtin_logf(l_tot);
         auto fence = [&]() __attribute__((always_inline)) {
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
             __builtin_amdgcn_wave_barrier();
@@ -1427,7 +1432,7 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
                 for (int i = 0; i < 4; ++i)
                     stored(i, [&](int q) {
                         const int head = pack > 1 ? q / S : 0;
-                        return Oh + (size_t)head * a.o_hs + (size_t)(q - head * S) * o_rs + 64 * part + 8 * chunk;
+                        return Oh + (size_t)head * late.o_hs + (size_t)(q - head * S) * o_rs + 64 * part + 8 * chunk;
                     });
                 fence();
             }
@@ -1442,9 +1447,9 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
             const float l_half = l_a + l_b;
             const float l_tot = l_half + swap_halves(l_half);
             const bool empty = GENERAL && !(l_tot > 0.0f);         // this row saw no key (here)
-            const float inv = empty ? 0.0f : (DROPOUT ? a.drop_scale : 1.0f) / l_tot;
+            const float inv = empty ? 0.0f : (DROPOUT ? late.drop_scale : 1.0f) / l_tot;
             const float lse_row = empty ? -INFINITY
-                                        : m_run * a.scale + __builtin_logf(l_tot);
+                                        : m_run * late.scale + __builtin_logf(l_tot);
             if (GENERAL && o_part != nullptr) {
 #pragma unroll
                 for (int db = 0; db < DB; ++db)
@@ -1497,19 +1502,19 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
                     u32x2 w;
                     w[0] = N::pack2(o[db][4 * g] * inv, o[db][4 * g + 1] * inv);
                     w[1] = N::pack2(o[db][4 * g + 2] * inv, o[db][4 * g + 3] * inv);
-                    *reinterpret_cast<u32x2 *>(Oh + (GENERAL ? (size_t)row_head * a.o_hs + (size_t)row_pos * o_rs : (size_t)q * o_rs) +
+                    *reinterpret_cast<u32x2 *>(Oh + (GENERAL ? (size_t)row_head * late.o_hs + (size_t)row_pos * o_rs : (size_t)q * o_rs) +
                                                32 * db + 8 * g + 4 * half) = w;
                 }
             }
-            if (!(GENERAL && o_part != nullptr) && a.lse != nullptr && half == 0) a.lse[(size_t)bh * S + q] = lse_row;
+            if (!(GENERAL && o_part != nullptr) && late.lse != nullptr && half == 0) late.lse[(size_t)bh * S + q] = lse_row;
         }
     }
     // (No other wave uses FIRST_AT's LDS behind these barriers, or in the general kernels in front of them: what the next item requests
     // behind the first LA K stages it requests behind its first barrier.)
     if (fr1 > fr0) {
         if (!GENERAL) phase_barrier();
-        first.finish(Oh, o_part, o_part != nullptr ? lse_part : a.lse != nullptr ? a.lse + (size_t)bh * S : nullptr, o_rs, win_L, a.scale, slope,
-                     DROPOUT ? a.drop_threshold : 0u, a.drop_scale, a.seed_lo, a.seed_hi, (uint32_t)bh, lds0 + FIRST_AT);
+        first.finish(Oh, o_part, o_part != nullptr ? lse_part : late.lse != nullptr ? late.lse + (size_t)bh * S : nullptr, o_rs, win_L, late.scale, slope,
+                     DROPOUT ? late.drop_threshold : 0u, late.drop_scale, late.seed_lo, late.seed_hi, (uint32_t)bh, lds0 + FIRST_AT);
         if (BY_ROWS) phase_barrier();       // (the next item's first K tile goes over it)
     }
     item = next_item;
