@@ -207,7 +207,9 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_small(const FaKernelArgs a)
             x += *(const lds_f32x4 *)(uintptr_t)(base + (uint32_t)(((2 * c) ^ (row & 7)) << 4));
             y += *(const lds_f32x4 *)(uintptr_t)(base + (uint32_t)(((2 * c + 1) ^ (row & 7)) << 4));
         }
-        const bool empty = !(l > 0.0f);           // this row sees no key
+        // (a row that sees no key; not where l is NaN, that row is NaN.  With the regular kernels' lengths every row sees one: a sum of
+        // zero is one of scores that are all -inf, and 0 / 0 says so)
+        const bool empty = l == 0.0f && !(Sk == S && S % 128 == 0);
         const float inv = empty ? 0.0f : 1.0f / l;
         const u32x4 w4 = {N::pack2(x[0] * inv, x[1] * inv), N::pack2(x[2] * inv, x[3] * inv), N::pack2(y[0] * inv, y[1] * inv), N::pack2(y[2] * inv, y[3] * inv)};
         *reinterpret_cast<u32x4 *>(a.O + (size_t)bi * a.o_bs + (size_t)hi * a.o_hs + (size_t)q * a.o_rs + 8 * c) = w4;

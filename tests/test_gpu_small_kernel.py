@@ -62,6 +62,36 @@ def test_values_that_are_not_finite(fa):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("S", [256, 300])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("bshd", [False, True])
+def test_logsumexp_of_rows_that_are_not_finite(fa, S, D, bshd):
+    """A NaN in a key or a query: the logsumexp of the rows that see it is NaN, as their O is -- -inf says that a row saw no key -- and the
+    other rows keep their bits.  A row all of whose scores are -inf has seen keys: NaN where the lengths are the regular kernels' (0 / 0,
+    as they have it), while the general ones give 0."""
+    import torch
+    q, k, v = _inputs(torch, S + D, 4, 4, S, S, D, bshd, "float16")
+    clean, clean_lse = fa.flash_attention_forward(q, k, v, causal=True, exact_first_rows=True)
+    k2, q2 = k.clone(memory_format=torch.preserve_format), q.clone(memory_format=torch.preserve_format)
+    k2[0, 1, 200, 3] = float("nan")
+    q2[0, 2, 100, 5] = float("nan")
+    for want_lse in (True, False):
+        r = fa.flash_attention_forward(q2, k2, v, causal=True, exact_first_rows=True, return_lse=want_lse)
+        o, lse = r if want_lse else (r, None)
+        nan = torch.zeros((1, 4, S), dtype=torch.bool, device="cuda")
+        nan[0, 1, 200:] = True
+        nan[0, 2, 100] = True
+        assert bool(o[nan].isnan().all()) and torch.equal(o[~nan], clean[~nan])
+        if want_lse:
+            assert bool(lse[nan].isnan().all()) and torch.equal(lse[~nan], clean_lse[~nan])
+    q.abs_().clamp_(min=0.1)
+    k[0, 1] = float("-inf")
+    o, lse = fa.flash_attention_forward(q, k, v, causal=True, exact_first_rows=True)
+    assert bool((lse[0, 1] == float("-inf")).all()) and bool(o[0, [0, 2, 3]].isfinite().all())
+    assert bool(o[0, 1].isnan().all() if S % 128 == 0 else (o[0, 1] == 0).all())
+
+
+@pytest.mark.gpu
 def test_sharp_scores(fa):
     """Scores of a standard deviation of 16: reference points far apart between the waves of a block."""
     import torch
