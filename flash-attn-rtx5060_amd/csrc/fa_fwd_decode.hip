@@ -379,7 +379,7 @@ __global__ void __launch_bounds__(NW * 64, NB == 1 ? 4 : 2) fa_fwd_decode(const 
                 l_all += *(const lds_f32 *)(uintptr_t)(lds_stat + (uint32_t)((w * 16 * NB + row) * 8 + 4)) * __builtin_amdgcn_exp2f((mw[w] - m_all) * cs);
                 acc += *(const lds_f32x4 *)(uintptr_t)(lds0 + (uint32_t)(w * (16 * D * 4) + q * (D * 4) + ((c ^ q) << 4)));
             }
-            const bool empty = !(l_all > 0.0f);   // no key of this row in this share
+            const bool empty = l_all == 0.0f;     // no key of this row in this share (a NaN is one's: as -inf, the merge would drop it)
             acc *= empty ? 0.0f : 1.0f / l_all;
             const float lse = empty ? -INFINITY : m_all * a.scale + __builtin_logf(l_all);
             if (n_splits > 1) {

@@ -1387,7 +1387,7 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
         const uint32_t obase = lds0 + ROWS_AT + wave * 4096;
         const float l_half = l_a + l_b;
         const float l_tot = l_half + swap_halves(l_half);
-        const bool empty = !(l_tot > 0.0f);                 // this row saw no key (here)
+        const bool empty = l_tot == 0.0f;                   // this row saw no key (here); a NaN row has seen one, and is NaN
         const float inv = empty ? 0.0f : (DROPOUT ? late.drop_scale : 1.0f) / l_tot;
         float *lse_rows = o_part != nullptr ? lse_part : late.lse != nullptr ? late.lse + (size_t)bh * S : nullptr;
         const int my_row = qw + l32_e;
@@ -1446,7 +1446,7 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
             const int q = GENERAL ? row_head * S + row_pos : my_q;
             const float l_half = l_a + l_b;
             const float l_tot = l_half + swap_halves(l_half);
-            const bool empty = GENERAL && !(l_tot > 0.0f);         // this row saw no key (here)
+            const bool empty = GENERAL && l_tot == 0.0f;           // this row saw no key (here)
             const float inv = empty ? 0.0f : (DROPOUT ? late.drop_scale : 1.0f) / l_tot;
             const float lse_row = empty ? -INFINITY
                                         : m_run * late.scale + __builtin_logf(l_tot);

@@ -75,3 +75,20 @@ def test_logsumexps_that_overflow(fa, B, H, Hk, S, Skv, D):
         got, lse = fa.flash_attention_forward(q, k, v, softmax_scale=2.9e38 / (64.0 * D), splits=splits)
         torch.cuda.synchronize()
         assert bool(torch.isnan(got).all()) and not bool(torch.isfinite(lse).any()) and not bool((lse == float("-inf")).any())
+
+
+@pytest.mark.parametrize("splits", [1, 3, 8, 11])
+@pytest.mark.parametrize("B,H,Hk,S,Skv,D", SHAPES + [(8, 16, 4, 200, 704, 64), (8, 16, 16, 200, 704, 128)])       # (128-row blocks without splits too)
+def test_a_nan_is_not_lost(fa, B, H, Hk, S, Skv, D, splits):
+    """A NaN in the last key of one head, in one split: that head's rows, which all see it, and their logsumexps are NaN however the
+    keys are split; the other heads keep their bits."""
+    import torch
+    q, k, v = _inputs(torch, B, H, Hk, S, Skv, D)
+    want, lse_want = fa.flash_attention_forward(q, k, v, splits=splits)
+    k[0, 0, -1, 5] = float("nan")
+    got, lse = fa.flash_attention_forward(q, k, v, splits=splits)
+    torch.cuda.synchronize()
+    group = H // Hk
+    assert bool(torch.isnan(got[0, :group]).all()) and bool(torch.isnan(lse[0, :group]).all())
+    for a, b in ((got, want), (lse, lse_want)):
+        assert torch.equal(a[0, group:], b[0, group:]) and torch.equal(a[1:], b[1:])
