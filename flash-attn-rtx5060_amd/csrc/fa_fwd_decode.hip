@@ -122,12 +122,11 @@ __device__ __forceinline__ void merge_parts(MergeSum &sum, const float *lse_row,
         }
     }
 }
-__device__ __forceinline__ void merge_two(MergeSum &a, const MergeSum &b)
+// A group's sum added to those of the groups in front of it; w: its weight against the largest reference point of all groups
+__device__ __forceinline__ void merge_group(f32x4 &acc, float &l, f32x4 group_acc, float group_l, float w)
 {
-    const float m = fmaxf(a.m, b.m), wa = __expf(a.m - m), wb = __expf(b.m - m);
-    a.acc = merge_weighted(a.acc, wa) + merge_weighted(b.acc, wb);
-    a.l = a.l * wa + b.l * wb;
-    a.m = m;
+    acc += merge_weighted(group_acc, w);
+    l += group_l * w;
 }
 
 // NB: 16-row blocks of queries (R <= 16 * NB rows); NW: waves per workgroup; NT: K and V with the streaming hint
@@ -416,44 +415,49 @@ __global__ void __launch_bounds__(NW * 64, NB == 1 ? 4 : 2) fa_fwd_decode(const 
     __syncthreads();
     if (*arrived != (unsigned)n_splits - 1u) return;
     if (tid_e == 0) __hip_atomic_store(&a.merge[item * kFaMergeStride], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    // fa_combine_splits' groups of splits, its batches and its order of sums, so that a call's bits do not depend on which of the two
+    // merges it; here a group is whichever threads get to it (of its eight groups, those behind the last split add nothing).
+    // (9 splits and more have at most 32 KB of parts, 2048 / splits output places of four elements: 455 sums at most.)
     constexpr int TPR = D / 4, ALL = NW * 64;
-    // groups of threads that share the splits, as many as there are threads for, up to eight; their sums meet in LDS
-    int groups = 1;
-    while (groups < 8 && R * TPR * groups * 2 <= ALL && groups * 8 < n_splits) groups *= 2;
     const size_t n_rows = (size_t)a.BH * S;
-    const int pairs = R * TPR;
-    for (int first = 0; first < pairs * groups; first += ALL) {
-        const int at = first + tid_e, group = groups > 1 ? at / pairs : 0, pair = at - group * pairs;
-        const bool live = group < groups && pair < pairs;
-        const int row = live ? pair / TPR : R - 1, t = live ? pair - row * TPR : 0;
+    const int pairs = R * TPR, all_groups = fa_combine_groups((long long)n_rows, D, n_splits);
+    const int groups = all_groups == 1 ? 1 : n_splits < 8 * all_groups ? (n_splits + 7) / 8 : all_groups, sums = pairs * groups;
+    auto write = [&](int pair, f32x4 acc, float m, float l) __attribute__((always_inline)) {
+        const int row = pair / TPR, t = pair - row * TPR, rh = row / S;
+        const bool empty = l == 0.0f;
+        acc *= empty ? 0.0f : 1.0f / l;
+        u32x2 w2;
+        w2[0] = N::pack2(acc[0], acc[1]);
+        w2[1] = N::pack2(acc[2], acc[3]);
+        *reinterpret_cast<u32x2 *>(a.O + (size_t)b * a.o_bs + (size_t)(h0 + rh) * a.o_hs + (size_t)(row - rh * S) * a.o_rs + 4 * t) = w2;
+        if (a.lse != nullptr && t == 0) a.lse[(size_t)bh * S + row] = empty ? -INFINITY : m + __logf(l);
+    };
+    const uint32_t lds_scalars = lds0 + (uint32_t)sums * 16u;
+    for (int at = tid_e; at < sums; at += ALL) {
+        const int group = groups > 1 ? at / pairs : 0, pair = at - group * pairs, row = pair / TPR, t = pair - row * TPR;
         const size_t grow = (size_t)bh * S + row;
         MergeSum sum;
-        if (live) merge_parts<true>(sum, a.lse_part + grow, a.o_part + grow * D + 4 * t, n_rows, n_rows * D, n_splits, group, groups);
-        if (groups > 1) {                         // (then all pairs are in this one pass)
-            const uint32_t mine = lds0 + (uint32_t)tid_e * 16u, scalars = lds0 + ALL * 16u + (uint32_t)tid_e * 8u;
-            *(lds_f32x4 *)(uintptr_t)mine = sum.acc;
-            *(lds_f32 *)(uintptr_t)scalars = sum.m;
-            *(lds_f32 *)(uintptr_t)(scalars + 4u) = sum.l;
-            __syncthreads();
-            if (live && group == 0)
-                for (int g = 1; g < groups; ++g) {
-                    MergeSum other;
-                    other.acc = *(const lds_f32x4 *)(uintptr_t)(mine + (uint32_t)(g * pairs) * 16u);
-                    other.m = *(const lds_f32 *)(uintptr_t)(scalars + (uint32_t)(g * pairs) * 8u);
-                    other.l = *(const lds_f32 *)(uintptr_t)(scalars + (uint32_t)(g * pairs) * 8u + 4u);
-                    merge_two(sum, other);
-                }
+        merge_parts<true>(sum, a.lse_part + grow, a.o_part + grow * D + 4 * t, n_rows, n_rows * D, n_splits, group, all_groups);
+        if (groups == 1) {
+            write(pair, sum.acc, sum.m, sum.l);
+        } else {
+            *(lds_f32x4 *)(uintptr_t)(lds0 + (uint32_t)at * 16u) = sum.acc;
+            *(lds_f32 *)(uintptr_t)(lds_scalars + (uint32_t)at * 8u) = sum.m;
+            *(lds_f32 *)(uintptr_t)(lds_scalars + (uint32_t)at * 8u + 4u) = sum.l;
         }
-        if (live && group == 0) {
-            const bool empty = sum.l == 0.0f;
-            const f32x4 acc = sum.acc * (empty ? 0.0f : 1.0f / sum.l);
-            const int rh = row / S;
-            u32x2 w2;
-            w2[0] = N::pack2(acc[0], acc[1]);
-            w2[1] = N::pack2(acc[2], acc[3]);
-            *reinterpret_cast<u32x2 *>(a.O + (size_t)b * a.o_bs + (size_t)(h0 + rh) * a.o_hs + (size_t)(row - rh * S) * a.o_rs + 4 * t) = w2;
-            if (a.lse != nullptr && t == 0) a.lse[grow] = empty ? -INFINITY : sum.m + __logf(sum.l);
+    }
+    if (groups == 1) return;
+    __syncthreads();
+    for (int pair = tid_e; pair < pairs; pair += ALL) {
+        float m = -__FLT_MAX__, l = 0.0f;
+        f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+        for (int g = 0; g < groups; ++g) m = fmaxf(m, *(const lds_f32 *)(uintptr_t)(lds_scalars + (uint32_t)(g * pairs + pair) * 8u));
+        for (int g = 0; g < groups; ++g) {
+            const uint32_t scalars = lds_scalars + (uint32_t)(g * pairs + pair) * 8u;
+            merge_group(acc, l, *(const lds_f32x4 *)(uintptr_t)(lds0 + (uint32_t)(g * pairs + pair) * 16u), *(const lds_f32 *)(uintptr_t)(scalars + 4u),
+                        __expf(*(const lds_f32 *)(uintptr_t)scalars - m));
         }
+        write(pair, acc, m, l);
     }
 }
 
@@ -491,9 +495,7 @@ __global__ void __launch_bounds__(256) fa_combine_splits(const FaKernelArgs a)
         acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int i = 0; i < GROUPS; ++i) {
-            const float w = __expf(sm[r * GROUPS + i] - m);
-            acc += merge_weighted(so[(r * GROUPS + i) * TPR + t], w);
-            l += sl[r * GROUPS + i] * w;
+            merge_group(acc, l, so[(r * GROUPS + i) * TPR + t], sl[r * GROUPS + i], __expf(sm[r * GROUPS + i] - m));
         }
     }
     if (!live) return;

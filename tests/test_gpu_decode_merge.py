@@ -34,6 +34,32 @@ def test_splits_merged_inside(fa, dtype, B, H, Hk, S, Sk, D, splits, window):
     assert float((lse - lse_ref).abs().max()) <= 1e-4
 
 
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("B,H,Hk,S,Sk,D,splits", [
+    (1, 8, 2, 1, 1003, 128, 7), (2, 4, 4, 2, 2000, 64, 8), (1, 14, 2, 1, 1200, 128, 9), (1, 10, 2, 1, 2000, 128, 12), (2, 9, 1, 1, 2000, 64, 14),
+    (1, 8, 2, 1, 2100, 128, 16), (1, 6, 2, 1, 4000, 128, 20), (1, 2, 1, 3, 4000, 64, 20), (3, 7, 7, 1, 2200, 64, 17), (1, 1, 1, 1, 5000, 128, 63),
+    (1, 2, 1, 1, 9000, 64, 60), (2, 1, 1, 1, 9000, 64, 66), (1, 1, 1, 1, 9000, 64, 128)])
+def test_bits_do_not_depend_on_which_kernel_merges(fa, dtype, B, H, Hk, S, Sk, D, splits):
+    """The same call with a counter set, its splits merged in the decoding kernel, and without one (hipStreamPerThread has none), merged
+    by the second kernel: one batch of parts, several that threads take in turn, and up to eight groups of them."""
+    import ctypes
+    import torch
+    q, k, v = _inputs(torch, Sk + splits, B, H, Hk, S, Sk, D, dtype)
+    results = []
+    for stream in (torch.cuda.current_stream().cuda_stream, 2):
+        o, lse = torch.full_like(q, float("nan")), torch.full((B, H, S), float("nan"), device="cuda")
+        p = fa.make_params(B, H, S, D, q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr(), causal=True, n_kv_heads=0 if Hk == H else Hk,
+                           S_kv=Sk, split_num=splits, dtype=fa.FA_DTYPE_BF16 if dtype == "bfloat16" else fa.FA_DTYPE_F16)
+        workspace = torch.empty(fa.lib().fa_fwd_workspace_bytes(ctypes.byref(p)), dtype=torch.uint8, device="cuda")
+        p.workspace, p.workspace_bytes = workspace.data_ptr(), workspace.numel()
+        torch.cuda.synchronize()
+        assert fa.lib().fa_fwd(ctypes.byref(p), ctypes.c_void_p(stream)) == fa.FA_OK
+        torch.cuda.synchronize()
+        assert not o.isnan().any() and not lse.isnan().any()
+        results.append((o.view(torch.int16), lse.view(torch.int32)))
+    assert torch.equal(results[0][0], results[1][0]) and torch.equal(results[0][1], results[1][1])
+
+
 def test_streams_and_graphs(fa):
     """More streams than there are sets, launches of all of them in flight together, and a graph of more launches than there are
     sets for captured ones: every result is the first one's."""
