@@ -169,14 +169,18 @@ unsigned *merge_counters_for_launch(const FaDeviceState *ds, hipStream_t stream)
     const int dev = fa_launch_device(), set = counter_set_for_launch(g_merge_owner[dev], kFaEagerMergeSlots, kFaMergeSlots, &g_merge_ticket[dev], stream);
     return set < 0 ? nullptr : ds->merges + (size_t)(kFaMergeHeads * kFaMergeStride) * (unsigned)set;
 }
-// Whether the decoding kernel merges a call's key splits itself: a counter per K/V head, and at most the 32 KB of parts a head
-// that one workgroup's threads load at once, eight of 16 bytes each.  On the device the two are level there (beside the
-// kernel); the launch that goes is 2.5 us of a short call's host time.  128 KB: B4 H32/8 S8 S_kv 2000, 13.4 us merged by a
-// second launch, 16.3 inside; 360 KB, B1 H8 S30 S_kv 3000, 12.2 and 21.4.  Calls that read more than 64 MB of K and V, 10 us, hide a
-// launch's host time and keep the second one: B16 H32/8 S_kv 8192 (537 MB) 82.6, inside 83.1.
+// Whether the decoding kernel merges a call's key splits itself: a counter per K/V head, at most the 32 KB of parts a head
+// that one workgroup's threads load at once, eight of 16 bytes each, and one pass of its 256 threads, four elements of the head's rows
+// each.  So the device is level or faster too, and the launch that goes is 1.5 to 2.5 us of a short call's host time; a second pass
+// costs the device more than the second launch.  Graphs, second launch / inside, us (a library's place in memory alone moves
+// them by 1.5 %): 8 K/V heads, 4 rows, D128, S_kv 1003 8.39 / 7.88; 64 heads, 1 row, S_kv 1000 10.08 / 9.38; 2 heads, 8 rows, D64,
+// S_kv 3000 8.25 / 7.87; the least work, one row of one head, D64, S_kv 2000, 7.95 / 8.14 (called one by one 12.1 / 7.9).  Two passes: 1
+// head, 16 rows, D128, S_kv 900 9.20 / 10.05, 32 rows, D64, S_kv 1000 9.60 / 10.39; four: 32 rows, D128, S_kv 500 11.25 / 14.22.  128 KB
+// of parts: B4 H32/8 S8 S_kv 2000 13.4 / 16.3.  Calls that read more than 64 MB of K and V, 10 us, hide a launch's host time and
+// keep the second one: B16 H32/8 S_kv 8192 (537 MB) 82.6, inside 83.1.
 bool merge_inside(long long kv_heads, long long rows, long long keys, int d, int splits)
 {
-    return kv_heads <= kFaMergeHeads && (double)kv_heads * (double)keys * d * 4.0 <= 64e6 && rows * d * 4 * splits <= 32 << 10;
+    return kv_heads <= kFaMergeHeads && rows * d <= 4 * 256 && (double)kv_heads * (double)keys * d * 4.0 <= 64e6 && rows * d * 4 * splits <= 32 << 10;
 }
 
 int device_fail(hipError_t e, const char *what)

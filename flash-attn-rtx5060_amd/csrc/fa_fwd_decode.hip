@@ -417,7 +417,7 @@ __global__ void __launch_bounds__(NW * 64, NB == 1 ? 4 : 2) fa_fwd_decode(const 
     if (tid_e == 0) __hip_atomic_store(&a.merge[item * kFaMergeStride], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     // fa_combine_splits' groups of splits, its batches and its order of sums, so that a call's bits do not depend on which of the two
     // merges it; here a group is whichever threads get to it (of its eight groups, those behind the last split add nothing).
-    // (9 splits and more have at most 32 KB of parts, 2048 / splits output places of four elements: 455 sums at most.)
+    // (At most 256 output places of four elements; from 9 splits on at most 32 KB of parts, so 2048 / splits of them and 455 sums.)
     constexpr int TPR = D / 4, ALL = NW * 64;
     const size_t n_rows = (size_t)a.BH * S;
     const int pairs = R * TPR, all_groups = fa_combine_groups((long long)n_rows, D, n_splits);
