@@ -22,6 +22,8 @@ struct FaKernelArgs {
     int R;
     float scale;         // softmax scale
     float scale_log2e;   // softmax scale * log2(e)
+    int first_parts;     // masked instantiations, > 0: the rows in the reference verifier's arithmetic (of every head) belong to workgroups of
+                         // their own, this many per head (1, 2, 4 or 8) in the second row of the grid, and the list's items leave them alone
     long long n_items;   // work items: BH * n_qblocks
     unsigned *queue;     // null, or 9 counters of a work queue: next list position per XCD [0..7], finished workgroups [8]
     // --- used by the GENERAL and STRIDED instantiations only (strides in elements; the head dimension is contiguous)
@@ -42,8 +44,6 @@ struct FaKernelArgs {
     unsigned seed_lo, seed_hi;
     // --- masked instantiations
     int exact_first_rows;      // 1: no row is recomputed in the reference verifier's rounded-product arithmetic
-    int first_parts;           // > 0: the rows that are (of every head) belong to workgroups of their own, this many per head
-                               //      (1, 2, 4 or 8) in the second row of the grid, and the list's items leave them alone
     // --- decoding kernel
     unsigned *merge;           // null (fa_combine_splits merges the key splits), or a zero per (batch, K/V head), kFaMergeStride words apart: the workgroup
                                //      that finishes a head's last split merges them and leaves a zero
@@ -52,5 +52,11 @@ struct FaKernelArgs {
     unsigned long long *ring_check;
 #endif
 };
+#ifndef FA_CHECK_RING
+// The grid's size lies behind the arguments, and kernels that ask for it read it with them: in another cache line than the last of
+// them it is a line more to wait for.  (256 bytes of arguments against 248, [B,S,H,D], one token, bf16, us: B8 H32/4 S_kv 303 D128 7.48
+// / 7.39, called one by one 7.56 / 7.31, B1 H32/8 S_kv 1003 7.98 / 7.81, B32 H32 S_kv 200 D64 12.98 / 12.78.)
+static_assert(sizeof(FaKernelArgs) % 64 != 0, "the grid's size lies in a cache line of its own");
+#endif
 
 #endif
