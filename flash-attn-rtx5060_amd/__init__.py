@@ -282,12 +282,14 @@ _PLAIN = frozenset((int, float, bool, str, type(None)))
 _WHOLE = frozenset((int, bool))            # (a float is refused for these, and 1.0 would find the entry of 1)
 _SEEDS = (1 << 64) - 1                     # (a seed is 64 bits; ctypes takes any whole number's low ones)
 _torch_module = None
+_plain_tensors = None
 
 
 def _torch():
-    global _torch_module
+    global _torch_module, _plain_tensors
     if _torch_module is None:
         import torch
+        _plain_tensors = frozenset((torch.Tensor, torch.nn.Parameter))
         _torch_module = torch
     return _torch_module
 
@@ -346,7 +348,8 @@ def flash_attention_forward(q, k, v, softmax_scale=None, causal=False, window_le
                            static_scratch, alibi_slopes)
         plan = _plans.get(key)
         if plan is not None:
-            st, out, lse = _native().forward_planned(plan[0], q, k, v, alibi_slopes, seed & _SEEDS, bool(return_lse), plan[1], bool(static_scratch))
+            out = None if type(q) in _plain_tensors else torch.empty_like(q)         # (of q's class)
+            st, out, lse = _native().forward_planned(plan[0], q, k, v, alibi_slopes, seed & _SEEDS, bool(return_lse), plan[1], bool(static_scratch), out)
             if st != FA_OK:
                 raise FaError(st, lib().fa_last_device_error().decode() if st == FA_ERR_DEVICE else "")
             return (out, lse) if return_lse else out
@@ -564,7 +567,6 @@ def _first_backward(q, k, v, o, lse, do, options):
 
 
 _autograd_function = None
-_plain_tensors = None
 _NUMBERS = frozenset((int, float, bool))
 _INTS = range(-(1 << 31), 1 << 31)
 
@@ -574,10 +576,8 @@ def flash_attention(q, k, v, softmax_scale=None, causal=False, window_left=-1, w
     """Differentiable attention for PyTorch callers: fa_fwd in the forward pass, fa_bwd in the backward pass
     (which replays the dropout decisions from ``seed``; nothing but O and the logsumexp is saved).  Shapes and
     layouts as in flash_attention_forward.  Plumbing only: both passes are the library's kernels."""
-    global _autograd_function, _plain_tensors
-    import torch
-    if _plain_tensors is None:
-        _plain_tensors = frozenset((torch.Tensor, torch.nn.Parameter))
+    global _autograd_function
+    torch = _torch()
     # Plain tensors on the GPU with plain numbers for options: an autograd function in C++, which is a third of the host time.
     # What it cannot take -- transforms of torch.func, forward-mode gradients, tracing and compiling, tensor subclasses -- and
     # what is refused goes through the one in Python.

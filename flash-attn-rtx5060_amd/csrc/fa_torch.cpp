@@ -37,16 +37,17 @@ PyObject *g_first_forward = nullptr, *g_first_backward = nullptr;
 void *raw_stream(const Tensor &t) { return c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(t.device().index()).stream(); }
 Tensor bytes_like(const Tensor &t, int64_t n) { return at::empty({n}, t.options().dtype(at::kByte)); }
 
-// flash_attention_forward with its plan at hand: the status, O and the logsumexp (or None).
+// flash_attention_forward with its plan at hand: the status, O and the logsumexp (or None).  `given`: the tensor for O where q is of a
+// subclass (made in Python, whose empty_like returns one of that class).
 std::tuple<int, Tensor, c10::optional<Tensor>> forward_planned(const std::string &block, const Tensor &q, const Tensor &k, const Tensor &v,
                                                                const c10::optional<Tensor> &slopes, unsigned long long seed, bool want_lse,
-                                                               int64_t workspace_bytes, bool static_scratch)
+                                                               int64_t workspace_bytes, bool static_scratch, const c10::optional<Tensor> &given)
 {
     py::gil_scoped_release release;
     fa_fwd_params p;
     TORCH_CHECK(block.size() == sizeof(p), "not a forward plan");
     std::memcpy(&p, block.data(), sizeof(p));
-    Tensor out = at::empty_like(q);
+    Tensor out = given ? *given : at::empty_like(q);
     c10::optional<Tensor> lse;
     p.Q = q.data_ptr(); p.K = k.data_ptr(); p.V = v.data_ptr(); p.O = out.data_ptr();
     p.seed = seed;

@@ -77,6 +77,22 @@ def test_hooks_graphs_and_refusals(fa):
         torch.func.vmap(lambda x: fa.flash_attention(x, k, v))(torch.stack([q, q]))
 
 
+def test_a_subclass_of_the_query_is_the_class_of_the_output(fa):
+    """The first call of a combination, the ones from its plan, and those whose plan a plain tensor has made."""
+    import torch
+
+    class Sub(torch.Tensor):
+        pass
+    for n, plain_first in ((232, False), (248, True)):
+        q, k, v, _ = (t.detach() for t in _inputs(torch, 8, n, 64, 4, 4, False, torch.float16))
+        calls = [q, q] if plain_first else []
+        for x in calls + [q.as_subclass(Sub)] * 3 + [torch.nn.Parameter(q)]:
+            o, lse = fa.flash_attention_forward(x, k, v)
+            assert type(o) is (Sub if type(x) is Sub else torch.Tensor) and type(lse) is torch.Tensor
+            assert type(fa.flash_attention_forward(x, k.as_subclass(Sub), v, return_lse=False)) is type(o)
+            assert type(fa.flash_attention(x, k, v)) is type(o)
+
+
 def test_other_streams_and_threads(fa):
     import threading
     import torch
