@@ -393,6 +393,8 @@ def flash_attention_forward(q, k, v, softmax_scale=None, causal=False, window_le
         if need and not static_scratch:
             workspace = torch.empty(need, dtype=torch.uint8, device=q.device)   # stream-ordered: freed after the launch
             p.workspace, p.workspace_bytes = workspace.data_ptr(), need
+    if key is not None:
+        _native()                       # (the next call of this combination needs it: what is missing is said now)
     entry = lib().fa_fwd_split_static if static_scratch else lib().fa_fwd
     st = entry(ctypes.byref(p), _raw_stream(torch, q))
     if st != FA_OK:

@@ -133,3 +133,14 @@ def test_what_was_refused_stays_refused(fa):
     shifted = torch.empty(q.numel() + 8, dtype=q.dtype, device="cuda")[1:1 + q.numel()].view(q.shape)      # 2 bytes off
     with pytest.raises(fa.FaError):
         fa.flash_attention_forward(shifted, k, v, causal=True, window_left=1, seed=1)
+
+
+def test_a_missing_native_part_is_said_on_the_first_call(fa, monkeypatch):
+    import torch
+    q = torch.randn((1, 2, 72, 64), device="cuda").half()
+    monkeypatch.setattr(fa, "_native_module", None)
+    monkeypatch.setattr(fa, "TORCH_LIB_PATH", "/nowhere/_fa_torch.so")
+    with pytest.raises(RuntimeError, match="is missing"):
+        fa.flash_attention_forward(q, q, q, causal=True)
+    monkeypatch.undo()
+    fa.flash_attention_forward(q, q, q, causal=True)
