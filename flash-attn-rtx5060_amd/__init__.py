@@ -589,7 +589,8 @@ def flash_attention(q, k, v, softmax_scale=None, causal=False, window_left=-1, w
             (alibi_slopes is None or type(alibi_slopes) in _plain_tensors) and not torch.compiler.is_compiling() and
             torch.autograd.forward_ad._current_level < 0 and not torch._C._are_functorch_transforms_active() and
             torch._C._get_tracing_state() is None):
-        return _native().attention(q, k, v, softmax_scale, bool(causal), window_left, window_right, alibi_slopes, dropout_prob, seed)
+        return _native().attention(q, k, v, None if softmax_scale is None else float(softmax_scale), bool(causal), window_left, window_right,
+                                   alibi_slopes, float(dropout_prob), seed)
     if _autograd_function is None:
         class _FlashAttention(torch.autograd.Function):
             @staticmethod

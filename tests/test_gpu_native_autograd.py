@@ -63,6 +63,9 @@ def test_hooks_graphs_and_refusals(fa):
         fa.flash_attention(q, k, v, window_left=1.0)
     with pytest.raises(fa.FaError):
         fa.flash_attention(q, k, v, softmax_scale=-1.0)
+    for too_large in (dict(softmax_scale=10 ** 400), dict(dropout_prob=10 ** 400)):
+        with pytest.raises(OverflowError):
+            fa.flash_attention(q, k, v, **too_large)
     fa.flash_attention(q, k, v, softmax_scale=0.5)
     shifted = torch.empty(q.numel() + 8, dtype=q.dtype, device="cuda")[1:1 + q.numel()].view(q.shape)       # 2 bytes off, a known combination
     with pytest.raises(fa.FaError):
