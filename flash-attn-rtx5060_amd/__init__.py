@@ -49,7 +49,7 @@ EXPORTED_SYMBOLS = (
     "fa_fwd_validate", "fa_fwd", "fa_init", "fa_fwd_split_static", "fa_fwd_static_scratch_bytes",
     "fa_reset_work_queues", "fa_release_work_queue", "run_flash_attention", "fa_strerror", "fa_last_device_error",
     "fa_sched_block_rows", "fa_sched_block_keys", "fa_sched_num_items", "fa_sched_item",
-    "fa_sched_heads", "fa_sched_launch", "fa_sched_tile_range", "fa_sched_classify", "fa_count_pairs", "fa_algorithmic_flops",
+    "fa_sched_heads", "fa_sched_launch", "fa_sched_small", "fa_sched_tile_range", "fa_sched_classify", "fa_count_pairs", "fa_algorithmic_flops",
     "fa_dropout_threshold", "fa_dropout_keep", "fa_fwd_workspace_bytes", "fa_fwd_suggest_splits", "fa_fwd_auto_splits",
     "fa_bwd_validate", "fa_bwd", "fa_bwd_workspace_bytes", "fa_bwd_fast_workspace_bytes", "fa_bwd_min_fast_workspace_bytes",
     "fa_bwd_share_bytes", "fa_bwd_shared", "fa_bwd_algorithmic_flops",
@@ -147,6 +147,7 @@ def lib():
                                                          ctypes.POINTER(ctypes.c_int)]
         L.fa_sched_heads.argtypes = [ctypes.c_int] * 3 + [ctypes.POINTER(ctypes.c_int)] * 3
         L.fa_sched_launch.argtypes = [ctypes.POINTER(FaFwdParams), ctypes.c_int] + [ctypes.POINTER(ctypes.c_int)] * 2
+        L.fa_sched_small.argtypes = [ctypes.POINTER(FaFwdParams), ctypes.c_int, ctypes.POINTER(ctypes.c_int)]
         L.fa_sched_tile_range.restype = None
         L.fa_sched_tile_range.argtypes = [ctypes.c_int] * 7 + [ctypes.POINTER(ctypes.c_int)] * 2
         L.fa_sched_classify.argtypes = [ctypes.c_int] * 7

@@ -392,11 +392,12 @@ int first_rows_parts(long long items, long long heads, int d, long long resident
     return parts;
 }
 // How a call reaches the device: by the decoding kernel, whose workgroups (one per K/V head and key split) the hardware
-// hands out, with the streaming hint or without; else the schedule of the tile kernels' work items.
+// hands out, with the streaming hint or without; by the kernel of 32-row blocks, which it hands out too, with small_waves waves each
+// (0: not by it) and small_parts for FaKernelArgs.first_parts; else the schedule of the tile kernels' work items and theirs.
 struct Launch {
     bool decode, streaming;
-    int small_waves, first_parts;      // the kernel of 32-row blocks: waves per workgroup (0: not taken), parts of the first rows
-    int sched;
+    int small_waves, small_parts;
+    int sched, first_parts;
 };
 // The kernel of 32-row blocks whose waves share the keys (fa_fwd_small.hip).  The key tiles, in its own units, that a block visits
 // at most; whether a problem is small enough for it, and with how many waves.
@@ -443,8 +444,8 @@ Launch launch_of(const fa_fwd_params *p, int compute_units)
     fa_mask_bounds(s_max, p->is_causal, p->window_size_left, p->window_size_right, &L, &R);
     Launch l;
     l.decode = decode_problem(p, R == 0, effective_splits(p));
-    l.first_parts = 0;
-    l.small_waves = l.decode ? 0 : small_waves_for(p, compute_units, &l.first_parts);      // (whatever the schedule: the same bits)
+    l.small_parts = 0;
+    l.small_waves = l.decode ? 0 : small_waves_for(p, compute_units, &l.small_parts);      // (whatever the schedule: the same bits)
     // (the streaming hint from where the K and V that are read -- under a left window the last S + L keys -- do not stay in
     // the 256 MB memory-side cache: measured beside the kernel)
     const long long visible = (long long)p->S + L < sk ? (long long)p->S + L : sk;
@@ -462,12 +463,14 @@ Launch launch_of(const fa_fwd_params *p, int compute_units)
     // Items that are all alike (no mask, or a window of at most half the length: all but the first few query blocks
     // of a head see the same number of tiles) need no balancing either, and the fixed order saves them the
     // counters' barriers: c4 766 against 748 TFLOP/s, c3's shape without a mask 1101 against 1096.
+    const long long blocks = pack > 1 ? 1 : (p->S + 32 * waves - 1) / (32 * waves);
+    const long long items = (long long)p->B * p->N / pack * blocks * effective_splits(p), resident = resident_groups(compute_units, waves);
     if (l.sched == FA_SCHED_AUTO) {
-        const long long blocks = pack > 1 ? 1 : (p->S + 32 * waves - 1) / (32 * waves);
-        const long long items = (long long)p->B * p->N / pack * blocks * effective_splits(p), resident = resident_groups(compute_units, waves);
         const bool alike = !(L < s_max || R < s_max) || 2LL * L <= (long long)p->S;
         l.sched = items <= resident ? FA_SCHED_DISPATCH : (items < 8 * resident || alike) ? FA_SCHED_PERSISTENT : FA_SCHED_QUEUE;
     }
+    const bool apart = l.sched == FA_SCHED_DISPATCH && effective_splits(p) == 1 && first_rows_few_keys(p, R);
+    l.first_parts = apart ? first_rows_parts(items, (long long)p->B * p->N, p->d, resident) : 0;
     return l;
 }
 }  // namespace
@@ -479,7 +482,16 @@ int fa_sched_launch(const fa_fwd_params *p, int compute_units, int *decoding, in
     const Launch l = launch_of(p, compute_units);
     if (decoding) *decoding = l.decode;
     if (streaming) *streaming = l.streaming;
-    return l.decode ? FA_SCHED_DISPATCH : l.sched;
+    return l.decode || l.small_waves > 0 ? FA_SCHED_DISPATCH : l.sched;
+}
+
+int fa_sched_small(const fa_fwd_params *p, int compute_units, int *first_parts)
+{
+    const int st = fa_fwd_validate(p);
+    if (st != FA_OK) return st;
+    const Launch l = launch_of(p, compute_units);
+    if (first_parts) *first_parts = l.decode ? 0 : l.small_waves > 0 ? l.small_parts : l.first_parts;
+    return l.small_waves;
 }
 
 unsigned long long fa_fwd_workspace_bytes(const fa_fwd_params *p)
@@ -734,7 +746,7 @@ int forward(const fa_fwd_params *p, void *workspace, const FaDeviceState *ds, vo
         a.pack = 1;
         a.n_qblocks = (p->S + 31) / 32;
         a.n_items = (long long)a.BH * a.n_qblocks;
-        a.first_parts = launch.first_parts;
+        a.first_parts = launch.small_parts;
         const hipError_t e = fa_launch_forward_small(a, p->dtype == FA_DTYPE_BF16, p->d, launch.small_waves, static_cast<hipStream_t>(stream));
         return e != hipSuccess ? device_fail(e, "small launch") : (int)FA_OK;
     };
@@ -757,9 +769,7 @@ int forward(const fa_fwd_params *p, void *workspace, const FaDeviceState *ds, vo
     a.drop_scale = 256.0f / (256.0f - (float)a.drop_threshold);
     a.seed_lo = (unsigned)(p->seed & 0xffffffffull);
     a.seed_hi = (unsigned)(p->seed >> 32);
-    a.first_parts = 0;
-    if (launch.sched == FA_SCHED_DISPATCH && a.n_splits == 1 && first_rows_few_keys(p, a.R))
-        a.first_parts = first_rows_parts(a.n_items, a.BH, p->d, resident_groups(ds->compute_units, waves));
+    a.first_parts = launch.first_parts;
 #ifdef FA_CHECK_RING
     a.ring_check = ds->ring_check;
 #endif

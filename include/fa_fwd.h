@@ -91,7 +91,8 @@ typedef struct fa_fwd_params {
     /* --- beyond mykernelParamType --- */
     int dtype;                /* FA_DTYPE_F16 / FA_DTYPE_BF16                                 */
     int is_causal;            /* keys with j > i are masked (mask.h:27-38)                    */
-    int sched;                /* FA_SCHED_*; without effect where the decoding kernel runs (fa_sched_launch) */
+    int sched;                /* FA_SCHED_*; without effect where the decoding kernel runs (fa_sched_launch) or
+                                 the kernel of 32-row blocks (fa_sched_small)                            */
     /* --- layouts beyond the reference's contiguous [B,N,S,d] (main.cu:182); all zero = that layout --- */
     int n_kv_heads;           /* K/V heads per batch entry, 0 = N.  Must divide N: query head h reads K/V
                                  head h / (N / n_kv_heads) (grouped-query / multi-query attention)      */
@@ -179,7 +180,9 @@ unsigned long long fa_fwd_static_scratch_bytes(void);
  * owned which.  Never call it while launches are being captured.
  * Short decoding calls with key splits (fa_fwd with split_num > 1, few query rows) count the splits of a head in sets of the
  * same kind, which the same rules and the same two calls govern: 64 sets for streams, 192 for captured launches; a launch
- * without a set merges its splits by a second kernel. */
+ * without a set merges its splits by a second kernel, with the same bits.
+ * (A captured launch keeps its set wherever its graph goes: two executable graphs instantiated from one capture, or one
+ * child graph in two places, must not run at the same time.) */
 int fa_reset_work_queues(void);
 int fa_release_work_queue(void *stream);
 
@@ -222,7 +225,9 @@ const char *fa_last_device_error(void);
 /* ------------------------------------------------------------------ */
 /* Tile scheduler, host side.  Mirrors what the kernel computes, so the */
 /* schedule can be checked without a GPU.  Replaces Schedule<0,...>     */
-/* (flash_forward.h:22-65).                                             */
+/* (flash_forward.h:22-65).  The work items are the tile kernels'; a    */
+/* call that fa_sched_launch gives to the decoding kernel, or           */
+/* fa_sched_small to the kernel of 32-row blocks, has that one's.       */
 /* ------------------------------------------------------------------ */
 enum { FA_TILE_SKIP = 0, FA_TILE_PARTIAL = 1, FA_TILE_FULL = 2 };
 
@@ -244,8 +249,17 @@ int fa_sched_heads(int N, int n_kv_heads, int bh, int *batch, int *q_head, int *
 /* How a call with these parameters reaches a device of `compute_units`: the schedule of its work items
  * (FA_SCHED_DISPATCH, _PERSISTENT or _QUEUE), or a negative status for parameters that fa_fwd refuses.  *decoding
  * (may be NULL): the decoding kernel runs it, one workgroup per K/V head and key split that the hardware hands out
- * (FA_SCHED_DISPATCH), and *streaming: that kernel reads K and V with the non-temporal hint. */
+ * (FA_SCHED_DISPATCH), and *streaming: that kernel reads K and V with the non-temporal hint.  The kernel of 32-row blocks,
+ * see below, has its workgroups handed out by the hardware as well. */
 int fa_sched_launch(const fa_fwd_params *p, int compute_units, int *decoding, int *streaming);
+/* Problems whose 32-row blocks are resident together on a device of `compute_units` (no key splits, no dropout, not the decoding
+ * kernel's): the kernel whose workgroups have 32 query rows each and share the keys among their waves runs them, whatever
+ * `sched` says.  Returns its waves per workgroup, 4 or 8; 0 for a call that another kernel runs; a negative status for parameters
+ * that fa_fwd refuses.  *first_parts (may be NULL): the workgroups per head, beside those of the blocks, that have the rows
+ * in the reference verifier's arithmetic (see exact_first_rows), 0 where there are none; for the tile kernels too.
+ * Its waves' sums meet at the end, so a head's O and L can differ by a rounding from what the same head has in a call of more
+ * heads, which the tile kernels run.  Within either kind they do not depend on the call's other heads. */
+int fa_sched_small(const fa_fwd_params *p, int compute_units, int *first_parts);
 /* Key-tile range [*tile_lo, *tile_hi] (inclusive) visited for query rows
  * [q_begin, q_begin + rows).  Same clipping as flash_forward.h:52-61. */
 void fa_sched_tile_range(int S, int block_keys, int is_causal, int window_left,

@@ -25,8 +25,53 @@ def test_schedules_of_the_tile_kernels(fa):
     assert launch(fa, 4, 16, 16, 2048, 2048, 64)[:2] == (fa.FA_SCHED_PERSISTENT, 0)
     assert launch(fa, 2, 32, 32, 8192, 8192, 128)[:2] == (fa.FA_SCHED_QUEUE, 0)
     assert launch(fa, 2, 32, 32, 8192, 8192, 128, causal=False)[:2] == (fa.FA_SCHED_PERSISTENT, 0)
-    assert launch(fa, 1, 4, 4, 512, 512, 64, sched=fa.FA_SCHED_QUEUE)[0] == fa.FA_SCHED_QUEUE
+    assert launch(fa, 1, 40, 40, 512, 512, 64, sched=fa.FA_SCHED_QUEUE)[0] == fa.FA_SCHED_QUEUE
     assert launch(fa, 1, 4, 3, 512, 512, 64)[0] == fa.FA_ERR_LAYOUT
+
+
+def small(fa, B, H, S, Skv, D, causal=True, wl=-1, wr=-1, splits=1, sched=0, cus=CUS, Hk=None, dropout=0.0, exact=False):
+    """(waves of the kernel of 32-row blocks, parts of the first rows)"""
+    p = fa.make_params(B, H, S, D, 0x1000, 0x2000, 0x3000, 0x4000, causal=causal, window_left=wl, window_right=wr, n_kv_heads=Hk or 0, sched=sched,
+                       S_kv=0 if Skv == S else Skv, split_num=splits, workspace_ptr=0x5000, workspace_bytes=1 << 62, dropout_prob=dropout,
+                       exact_first_rows=exact)
+    parts = ctypes.c_int(-1)
+    waves = fa.lib().fa_sched_small(ctypes.byref(p), cus, ctypes.byref(parts))
+    if waves > 0:
+        assert fa.lib().fa_sched_launch(ctypes.byref(p), cus, None, None) == fa.FA_SCHED_DISPATCH
+    return waves, parts.value
+
+
+def test_line_between_32_row_blocks_and_the_tile_kernels(fa):
+    """Two blocks to a compute unit, four where a causal walk of 2048 queries and more is uneven; key splits, dropout, two key tiles on
+    most units; whatever schedule is named, on other devices too."""
+    for D in (64, 128):
+        assert [small(fa, 1, h, 320, 320, D, causal=False)[0] for h in (1, 51, 52)] == [4, 4, 0]                  # 510 and 520 blocks
+        assert [small(fa, 1, h, 500, 500, D, wl=100, exact=True)[0] for h in (32, 33)] == [4, 0]                   # 512 and 528
+        assert [small(fa, 1, h, 2048, 2048, D, exact=True)[0] for h in (4, 8, 16, 17)] == [8, 4, 4, 0]             # 256, 512, 1024 and 1088
+        assert [small(fa, 1, h, 2048, 2048, D, causal=False)[0] for h in (8, 9)] == [4, 0]
+        assert [small(fa, 1, h, 2048, 2048, D, wl=2000, exact=True)[0] for h in (8, 9)] == [4, 0]
+        assert [small(fa, 1, h, 128, 128, D, causal=False)[0] for h in (64, 65)] == [4, 0] and small(fa, 1, 100, 129, 129, D, causal=False)[0] == 4
+        assert small(fa, 1, 4, 256, 2000, D, splits=2)[0] == 0 and small(fa, 1, 4, 256, 256, D, dropout=0.1)[0] == 0
+        assert [small(fa, 1, 8, 256, 256, D, sched=n)[0] for n in range(4)] == [4] * 4
+        assert [small(fa, 1, 16, 320, 320, D, causal=False, cus=c)[0] for c in (64, 80)] == [0, 4]
+        # eight waves: at most a block to a compute unit, from 24 key tiles (64 keys each, 32 at head dimension 128) on
+        n = 24 * (64 if D == 64 else 32)
+        assert small(fa, 1, 4, 64, n - 1, D, causal=False)[0] == 8 and small(fa, 1, 4, 64, n - n // 24, D, causal=False)[0] == 4
+        assert small(fa, 1, 4, 200, 5000, D, wl=n)[0] == 8 and small(fa, 1, 4, 200, 5000, D, wl=n // 2)[0] == 4
+        assert small(fa, 1, 4, 1, 1000, D)[0] == 0 and small(fa, 1, 4, 8, 4, D, causal=False)[0] == 4              # (one is the decoding kernel's)
+    assert small(fa, 1, 4, 256, 256, 96)[0] == fa.FA_ERR_HEAD_DIM
+
+
+def test_parts_of_the_first_rows(fa):
+    """Eight per head beside 32-row blocks where a quarter of the slots more holds them, else four at head dimension 64 or where all are
+    resident, else the tile kernels; these in as many as fit into twice the slots (head dimension 64: 7/4); none where there are none."""
+    assert [small(fa, 1, h, 256, 256, 64) for h in (40, 41, 53, 54)] == [(4, 8), (4, 4), (4, 4), (0, 8)]
+    assert [small(fa, 1, h, 256, 256, 128) for h in (40, 41, 42, 43)] == [(4, 8), (4, 4), (4, 4), (0, 8)]
+    assert [small(fa, 1, h, 256, 256, 128)[1] for h in (100, 180, 256, 257)] == [8, 2, 2, 0]
+    assert small(fa, 1, 8, 2048, 2048, 64) == (4, 8) and small(fa, 1, 16, 2048, 2048, 64) == (4, 8) and small(fa, 1, 16, 4096, 4096, 64) == (0, 8)
+    assert small(fa, 1, 8, 256, 256, 64, exact=True) == (4, 0) and small(fa, 1, 8, 256, 288, 64) == (4, 0) and small(fa, 1, 8, 256, 287, 64) == (4, 8)
+    assert small(fa, 1, 8, 256, 256, 64, causal=False) == (4, 0) and small(fa, 1, 8, 256, 256, 64, causal=False, wr=0) == (4, 8)
+    assert small(fa, 1, 8, 256, 200, 64) == (4, 0) and small(fa, 1, 8, 10, 20, 64, Hk=1) == (4, 0)                 # (a group's rows in one block)
 
 
 @pytest.mark.parametrize("sched", [0, 1, 2, 3])
