@@ -32,3 +32,12 @@ def fa():
 def oracle():
     import oracle_binding
     return oracle_binding
+
+
+@pytest.fixture(params=["alone", "among_others"])
+def forward(request, fa):
+    """flash_attention_forward of a small problem as it is, which the kernel of 32-row blocks may run, and among copies of itself, which the
+    tile kernels do."""
+    import functools
+    from parity_util import forward_among_others
+    return fa.flash_attention_forward if request.param == "alone" else functools.partial(forward_among_others, fa)

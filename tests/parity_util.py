@@ -85,3 +85,46 @@ def numpy_keep_mask(seed, bh, S, threshold):
     byte = 4 * ((j % 32) // 8) + j % 4
     word = np.choose(byte // 4, w)
     return ((word >> (8 * (byte % 4)).astype(np.uint64)) & np.uint64(255)) >= np.uint64(threshold)
+
+
+def small_waves(fa, q, k, causal=False, window_left=-1, window_right=-1, splits=1, dropout_prob=0.0, exact_first_rows=False, sched=0, batches=1, **_):
+    """Waves of the kernel of 32-row blocks where it runs this call of `batches` times as many batch entries, 0 where another kernel does."""
+    B, H, S, D = q.shape
+    p = fa.make_params(B * batches, H, S, D, 0x1000, 0x2000, 0x3000, 0x4000, causal=causal, window_left=window_left, window_right=window_right,
+                       sched=sched, n_kv_heads=k.shape[1], S_kv=k.shape[2], dropout_prob=dropout_prob, split_num=splits, workspace_ptr=0x5000,
+                       workspace_bytes=1 << 62, exact_first_rows=exact_first_rows)
+    waves = fa.lib().fa_sched_small(p, 256, None)
+    assert waves >= 0, waves
+    return waves
+
+
+def copies_for_tiles(fa, q, k, **kw):
+    """How many copies of a problem's batch entries the tile kernels run: one where the call is theirs (or the decoding kernel's) as it is."""
+    n = 1
+    while small_waves(fa, q, k, batches=n, **kw):
+        n += 1
+    return n
+
+
+def among_others(t, copies):
+    """t's batch entries `copies` times, every entry stored as t stores it."""
+    import torch
+    if t.shape[0] > 1 and t.stride(0) == 0:
+        return t[:1].expand((copies * t.shape[0],) + t.shape[1:])
+    entry = t.stride(0) if t.shape[0] > 1 else (1 + sum((n - 1) * s for n, s in zip(t.shape[1:], t.stride()[1:])) + 7) // 8 * 8
+    many = torch.empty_strided((copies * t.shape[0],) + t.shape[1:], (entry,) + t.stride()[1:], dtype=t.dtype, device=t.device)
+    for n in range(copies):
+        many[n * t.shape[0]:(n + 1) * t.shape[0]].copy_(t)
+    return many
+
+
+def forward_among_others(fa, q, k, v, **kw):
+    """flash_attention_forward of a problem among as many copies of it as it takes to leave the kernel of 32-row blocks; the copies'
+    results are the same bits."""
+    import torch
+    copies, B = copies_for_tiles(fa, q, k, **kw), q.shape[0]
+    out = fa.flash_attention_forward(*(among_others(t, copies) if copies > 1 else t for t in (q, k, v)), **kw)
+    for r in out if isinstance(out, tuple) else (out,):
+        bits = r.contiguous().view(torch.int32 if r.dtype == torch.float32 else torch.int16)
+        assert copies == 1 or torch.equal(bits[:B], bits[-B:])
+    return tuple(r[:B] for r in out) if isinstance(out, tuple) else out[:B]

@@ -25,7 +25,7 @@ def ulp(x, dtype):
 
 
 @pytest.mark.parametrize("dtype", [0, 1])
-@pytest.mark.parametrize("shape,wl,seed,sched", [((2, 4, 256, 128), -1, 29, 0), ((1, 8, 384, 64), -1, 7, 0), ((1, 4, 256, 128), 9, 3, 0),
+@pytest.mark.parametrize("shape,wl,seed,sched", [((2, 4, 256, 128), -1, 29, 0), ((1, 8, 384, 64), -1, 7, 0), ((1, 4, 256, 128), 9, 3, 0), ((2, 80, 256, 128), 9, 3, 0),
                                                  ((2, 32, 1024, 128), -1, 29, 0),
                                                  # the path dealt in one, two and four parts, in workgroups of 128 and of 256
                                                  # rows, under every schedule (several passes over the resident grid included)
@@ -56,13 +56,13 @@ def test_first_rows_are_the_verifiers_bits(fa, oracle, dtype, shape, wl, seed, s
 
 @pytest.mark.parametrize("dtype", [0, 1])
 @pytest.mark.parametrize("S,S_kv", [(128, 131), (64, 80), (200, 231), (5, 36), (300, 301)])
-def test_first_rows_behind_a_few_earlier_keys(fa, oracle, dtype, S, S_kv):
+def test_first_rows_behind_a_few_earlier_keys(fa, oracle, forward, dtype, S, S_kv):
     """Queries at the end of a slightly longer key sequence (query i at position i + S_kv - S): the rows at
     positions below 32 still see few keys and still take the verifier's arithmetic."""
     H, D = 3, 128
     q_full, k, v = make_inputs(fa, (1, H, S_kv, D), dtype, 41 + S)
     q = np.ascontiguousarray(q_full[:, :, S_kv - S:, :])
-    o, lse = fa.flash_attention_forward(to_torch(q, dtype), to_torch(k, dtype), to_torch(v, dtype), causal=True)
+    o, lse = forward(to_torch(q, dtype), to_torch(k, dtype), to_torch(v, dtype), causal=True)
     rows = np.array([h * S_kv + r for h in range(H) for r in range(S_kv - S, S_kv)], dtype=np.int64)
     o_ref, lse_ref = oracle.rows(q_full, k, v, rows, dtype, None, True, -1, -1)
     got = oracle.to_f32(from_torch(o), dtype).reshape(-1, D)
@@ -78,15 +78,14 @@ def test_first_rows_behind_a_few_earlier_keys(fa, oracle, dtype, S, S_kv):
 @pytest.mark.parametrize("dtype", [0, 1])
 @pytest.mark.parametrize("causal,wl,wr", [(True, 0, -1), (True, 4, -1), (True, 15, -1), (False, 0, 0), (False, 4, 4),
                                           (False, 15, 15), (False, 15, 3)])
-def test_narrow_windows_documented_bound(fa, oracle, dtype, causal, wl, wr):
+def test_narrow_windows_documented_bound(fa, oracle, forward, dtype, causal, wl, wr):
     """Every row sees at most 31 keys.  Rows beyond the first 32 (and all rows of a two-sided window) accumulate
     exact products while the verifier rounds each one, and with so few keys an output can be several units
     large: the stated bound is the tolerance or one output ulp, whichever is larger, and the usual rel-L2."""
     shape = (1, 4, 512, 128)
     q, k, v = make_inputs(fa, shape, dtype, 77 + wl)
     o_ref, lse_ref = oracle.full(q, k, v, dtype, None, causal, wl, wr)
-    o, lse = fa.flash_attention_forward(to_torch(q, dtype), to_torch(k, dtype), to_torch(v, dtype),
-                                        causal=causal, window_left=wl, window_right=wr)
+    o, lse = forward(to_torch(q, dtype), to_torch(k, dtype), to_torch(v, dtype), causal=causal, window_left=wl, window_right=wr)
     ref = oracle.to_f32(o_ref, dtype)
     got = oracle.to_f32(from_torch(o), dtype)
     err = errors(got, ref, lse.cpu().numpy(), lse_ref)
@@ -98,7 +97,7 @@ def test_narrow_windows_documented_bound(fa, oracle, dtype, causal, wl, wr):
 
 
 @pytest.mark.parametrize("dtype", [0, 1])
-def test_exact_first_rows_against_fp64(fa, oracle, dtype):
+def test_exact_first_rows_against_fp64(fa, oracle, forward, dtype):
     """exact_first_rows = 1: no row takes the verifier's rounded products; the whole output, first rows
     included, is within the usual tolerance of exact attention, and the logsumexp of the
     first rows is the exact one (what fa_bwd recomputes P from)."""
@@ -107,8 +106,7 @@ def test_exact_first_rows_against_fp64(fa, oracle, dtype):
     q, k, v = make_inputs(fa, shape, dtype, 29)
     rows = np.arange(B * H * S, dtype=np.int64)
     o64, lse64 = oracle.rows_f64(q, k, v, rows, dtype, None, True, -1, -1)
-    o, lse = fa.flash_attention_forward(to_torch(q, dtype), to_torch(k, dtype), to_torch(v, dtype), causal=True,
-                                        exact_first_rows=True)
+    o, lse = forward(to_torch(q, dtype), to_torch(k, dtype), to_torch(v, dtype), causal=True, exact_first_rows=True)
     got = oracle.to_f32(from_torch(o), dtype).reshape(-1, D)
     # p rounded to the storage type before the second product, one rounding of the result
     err = errors(got, o64.astype(np.float32), lse.cpu().numpy().reshape(-1), lse64.astype(np.float32))
@@ -117,5 +115,5 @@ def test_exact_first_rows_against_fp64(fa, oracle, dtype):
     assert err["rel_l2"] <= (4e-4 if dtype == 0 else 3e-3)
     assert err["lse_abs"] <= 2e-5
     # and it differs from the default path where the verifier's rounding matters
-    o_default, _ = fa.flash_attention_forward(to_torch(q, dtype), to_torch(k, dtype), to_torch(v, dtype), causal=True)
+    o_default, _ = forward(to_torch(q, dtype), to_torch(k, dtype), to_torch(v, dtype), causal=True)
     assert np.count_nonzero(from_torch(o_default).reshape(-1, D)[:32] != from_torch(o).reshape(-1, D)[:32]) > 0

@@ -43,13 +43,13 @@ def slopes_for(kind, H):
 
 
 @pytest.mark.parametrize("shape,dtype,causal,wl,wr,kind", SMALL)
-def test_small_full_tensor_alibi(fa, oracle, shape, dtype, causal, wl, wr, kind):
+def test_small_full_tensor_alibi(fa, oracle, forward, shape, dtype, causal, wl, wr, kind):
     import torch
     slopes = slopes_for(kind, shape[1])
     q, k, v = make_inputs(fa, shape, dtype, seed=4321 + shape[2] + dtype)
     o_ref, lse_ref = oracle.full(q, k, v, dtype, None, causal, wl, wr, slopes)
-    o, lse = fa.flash_attention_forward(to_torch(q, dtype), to_torch(k, dtype), to_torch(v, dtype), causal=causal,
-                                        window_left=wl, window_right=wr, alibi_slopes=torch.from_numpy(slopes).cuda())
+    o, lse = forward(to_torch(q, dtype), to_torch(k, dtype), to_torch(v, dtype), causal=causal, window_left=wl, window_right=wr,
+                     alibi_slopes=torch.from_numpy(slopes).cuda())
     err = errors(oracle.to_f32(from_torch(o), dtype), oracle.to_f32(o_ref, dtype), lse.cpu().numpy(), lse_ref)
     print(shape, dtype, causal, wl, wr, kind, err)
     assert_within(err, dtype, f"alibi {kind} {shape} dtype={dtype} causal={causal} w=({wl},{wr})")
@@ -79,7 +79,7 @@ def test_benchmark_shapes_alibi(fa, oracle, name, shape, dtype, causal, wl, seed
     assert_within(err, dtype, f"alibi {name} sched={sched}")
 
 
-def test_alibi_closed_form_on_gpu(fa):
+def test_alibi_closed_form_on_gpu(forward):
     """Q = 0 leaves only the bias.  With V[j, t] = [j mod D == t] the output is O[i, t] = sum over visible keys
     j = t (mod D) of exp(-slope_h |i-j|) / Z_i, which numpy evaluates in fp64 without any oracle code; the
     logsumexp is log Z_i.  Size independent: run at S = 4096, all rows checked."""
@@ -95,7 +95,7 @@ def test_alibi_closed_form_on_gpu(fa):
     onehot = np.zeros((S, D))
     onehot[np.arange(S), np.arange(S) % D] = 1.0
     for causal in (False, True):
-        o, lse = fa.flash_attention_forward(q, k, v, causal=causal, alibi_slopes=torch.from_numpy(slopes).cuda())
+        o, lse = forward(q, k, v, causal=causal, alibi_slopes=torch.from_numpy(slopes).cuda())
         torch.cuda.synchronize()
         o, lse = o.float().cpu().numpy(), lse.cpu().numpy()
         for h in range(H):
@@ -110,15 +110,15 @@ def test_alibi_closed_form_on_gpu(fa):
             assert np.max(np.abs(lse[0, h] - (mx[:, 0] + np.log(Z[:, 0])))) <= 1e-3, (causal, h)
 
 
-def test_alibi_zero_slopes_equal_no_alibi(fa):
+def test_alibi_zero_slopes_equal_no_alibi(fa, forward):
     """All-zero slopes go through the biased kernel and must reproduce the unbiased result (the exponent is
     computed as s*c - m*c in one rounding there and in two here, hence a tolerance of one output ulp)."""
     import torch
     shape = (2, 4, 1024, 128)
     q, k, v = make_inputs(fa, shape, 0, seed=91)
     tq, tk, tv = (to_torch(x, 0) for x in (q, k, v))
-    o0, l0 = fa.flash_attention_forward(tq, tk, tv, causal=True)
-    o1, l1 = fa.flash_attention_forward(tq, tk, tv, causal=True, alibi_slopes=torch.zeros(4, device="cuda"))
+    o0, l0 = forward(tq, tk, tv, causal=True)
+    o1, l1 = forward(tq, tk, tv, causal=True, alibi_slopes=torch.zeros(4, device="cuda"))
     torch.cuda.synchronize()
     assert float((o0.float() - o1.float()).abs().max()) <= 1e-3
     assert float((l0 - l1).abs().max()) <= 1e-5

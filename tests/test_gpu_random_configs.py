@@ -37,7 +37,7 @@ def reference(q, k, v, do, causal, wl, wr, slopes, keep=None):
 
 
 @pytest.mark.parametrize("regular", [False, True], ids=["any_shape", "regular_lengths"])
-def test_random_configurations(fa, regular):
+def test_random_configurations(fa, forward, regular):
     """regular: lengths that are multiples of 128 with as many keys, no ALiBi, no dropout -- the problems that the
     strided kernels take when the storage is not the reference's or K/V heads are grouped; padded rows now and then."""
     import torch
@@ -80,7 +80,7 @@ def test_random_configurations(fa, regular):
             keep = torch.from_numpy(m.astype(np.float32) * grow).cuda()
         # exact products in every row (what the autograd wrapper uses): the comparison is with exact fp32
         # attention, not with the reference verifier's rounded products
-        o, lse = fa.flash_attention_forward(q, k, v, exact_first_rows=True, **kw)
+        o, lse = forward(q, k, v, exact_first_rows=True, **kw)
         dq, dk, dv = fa.flash_attention_backward(q, k, v, o, lse, do, **kw)
         torch.cuda.synchronize()
         o_ref, lse_ref, dq_ref, dk_ref, dv_ref, vis = reference(q, k, v, do, causal, wl, wr, slopes, keep)

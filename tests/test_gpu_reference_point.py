@@ -10,7 +10,8 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 CASES = [
-    # B, H, Hk, S, D, dtype, causal, wl, bshd, growth per key (in units of the scaled score)
+    # B, H, Hk, S, D, dtype, causal, wl, bshd, growth per key (in units of the scaled score); the kernels named are those that run the
+    # case, or copies of it where it is small
     (1, 2, 2, 512, 64, "fp16", True, -1, False, 0.4),      # every tile moves the reference point
     (1, 2, 2, 512, 128, "bf16", False, -1, False, 0.4),
     (1, 2, 1, 512, 128, "fp16", True, -1, True, 0.15),     # some do; strided kernels
@@ -52,10 +53,10 @@ def _exact(q, k, v, causal, wl):
 
 
 @pytest.mark.parametrize("B,H,Hk,S,D,dtype,causal,wl,bshd,growth", CASES)
-def test_reference_point_moves(fa, B, H, Hk, S, D, dtype, causal, wl, bshd, growth):
+def test_reference_point_moves(forward, B, H, Hk, S, D, dtype, causal, wl, bshd, growth):
     import torch
     (q, k, v), (dq, dk, dv) = _inputs(B, H, Hk, S, D, dtype, growth, bshd, 31 + S + D)
-    o, lse = fa.flash_attention_forward(dq, dk, dv, causal=causal, window_left=wl, exact_first_rows=True)
+    o, lse = forward(dq, dk, dv, causal=causal, window_left=wl, exact_first_rows=True)
     torch.cuda.synchronize()
     heads = slice(0, 2 * (H // Hk)), slice(0, 2)                      # (the first and last batch's first heads are enough)
     for b in {0, B - 1}:
@@ -71,14 +72,14 @@ def test_reference_point_moves(fa, B, H, Hk, S, D, dtype, causal, wl, bshd, grow
 
 
 @pytest.mark.parametrize("S,D", [(512, 64), (512, 128), (500, 64), (500, 128)])
-def test_nan_key_reaches_only_the_rows_that_see_it(fa, S, D):
+def test_nan_key_reaches_only_the_rows_that_see_it(forward, S, D):
     """A NaN in key 300 of a causal problem: rows from 300 on are NaN, the others what they are without it."""
     import torch
     _, (q, k, v) = _inputs(1, 2, 2, S, D, "fp16", 0.02, False, 77)
-    clean, clean_lse = fa.flash_attention_forward(q, k, v, causal=True)
+    clean, clean_lse = forward(q, k, v, causal=True)
     k = k.clone()
     k[:, :, 300, 5] = float("nan")
-    o, lse = fa.flash_attention_forward(q, k, v, causal=True)
+    o, lse = forward(q, k, v, causal=True)
     torch.cuda.synchronize()
     assert bool(torch.isnan(o[:, :, 300:]).all())
     assert torch.equal(o[:, :, :300], clean[:, :, :300])
@@ -95,7 +96,7 @@ def test_nan_key_reaches_only_the_rows_that_see_it(fa, S, D):
     (1, 8, 1, 40, 3000, 128, "fp16", True, -1, True, 1),               # rows of several heads in one wave
     (1, 8, 2, 200, 5000, 64, "bf16", True, -1, True, 4),               # key splits
 ])
-def test_rows_do_not_depend_on_each_other(fa, B, H, Hk, S, Sk, D, dtype, causal, wl, bshd, splits):
+def test_rows_do_not_depend_on_each_other(forward, B, H, Hk, S, Sk, D, dtype, causal, wl, bshd, splits):
     """A query forty times as large moves its own reference point in many tiles (and sends its wave through the loop that takes
     maxima); every other row keeps its bits."""
     import torch
@@ -105,13 +106,13 @@ def test_rows_do_not_depend_on_each_other(fa, B, H, Hk, S, Sk, D, dtype, causal,
     if bshd:
         q, k, v = (x.transpose(1, 2).contiguous().transpose(1, 2) for x in (q, k, v))
     kw = dict(causal=causal, window_left=wl, splits=splits, exact_first_rows=True)
-    clean, clean_lse = fa.flash_attention_forward(q, k, v, **kw)
+    clean, clean_lse = forward(q, k, v, **kw)
     large = torch.arange(S) % 32 == 13
     large_heads = torch.arange(H) % 2 == 0
     q2 = q.clone(memory_format=torch.preserve_format)
     rows = (large_heads[:, None] & large[None, :]).cuda()
     q2[:, rows] = q2[:, rows] * 40
-    o, lse = fa.flash_attention_forward(q2, k, v, **kw)
+    o, lse = forward(q2, k, v, **kw)
     torch.cuda.synchronize()
     assert not torch.equal(o[:, rows], clean[:, rows])
     assert torch.equal(o[:, ~rows], clean[:, ~rows])
@@ -119,7 +120,7 @@ def test_rows_do_not_depend_on_each_other(fa, B, H, Hk, S, Sk, D, dtype, causal,
 
 
 @pytest.mark.parametrize("S,D,dtype,sigma,bound", [(2048, 128, "fp16", 4.0, 2.70e-4), (2048, 64, "bf16", 8.0, 1.97e-3), (2000, 64, "fp16", 4.0, 2.70e-4)])
-def test_a_row_that_one_key_carries_has_its_weight_exact(fa, S, D, dtype, sigma, bound):
+def test_a_row_that_one_key_carries_has_its_weight_exact(forward, S, D, dtype, sigma, bound):
     """Sharp scores: the key that carries a row mostly has a weight of exactly 1, its own score being the reference point; a point
     that lags further behind rounds that weight too.  The bounds lie between the error of a point that lags by up to 2^8
     (2.60e-4 and 1.93e-3 of the outputs' norm against 64 bits) and by up to 2^12 (2.77e-4 and 1.98e-3)."""
@@ -128,6 +129,6 @@ def test_a_row_that_one_key_carries_has_its_weight_exact(fa, S, D, dtype, sigma,
     dt = torch.bfloat16 if dtype == "bf16" else torch.float16
     q, k, v = (torch.randn((1, 4, S, D), generator=g) for _ in range(3))
     q, k, v = (q * sigma).to(dt), k.to(dt), v.to(dt)
-    o, _ = fa.flash_attention_forward(q.cuda(), k.cuda(), v.cuda(), causal=True, exact_first_rows=True)
+    o, _ = forward(q.cuda(), k.cuda(), v.cuda(), causal=True, exact_first_rows=True)
     want, _ = _exact(q, k, v, True, -1)
     assert float((o.cpu().double() - want).norm() / want.norm()) <= bound

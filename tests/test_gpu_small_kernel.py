@@ -1,9 +1,10 @@
 """The kernel of 32-row blocks whose waves share the keys, against the tile kernels: the same heads once as a small problem and
 once among enough others that the tile kernels take the call.  Edges of its tiles (64 keys, 32 at head dimension 128), of its blocks
-and of what a wave gets; every mask; and the line of the rule, on the host and at both sides of it on the device."""
-import ctypes
-
+and of what a wave gets; every mask, with four waves and with eight; the first rows in eight parts and in four; and both sides of the
+rule's line (on the host: tests/test_launch_rules.py)."""
 import pytest
+
+from parity_util import small_waves
 
 
 def _inputs(torch, seed, heads, kv_heads, S, Sk, D, bshd, dtype):
@@ -21,7 +22,9 @@ def _inputs(torch, seed, heads, kv_heads, S, Sk, D, bshd, dtype):
     (300, 300, 128, 1, False, dict(window_left=33, window_right=7)), (500, 500, 64, 1, False, dict(causal=True, window_left=0)),
     (40, 700, 64, 1, False, dict(causal=True)), (50, 75, 128, 2, True, dict(causal=True)), (96, 1111, 128, 1, False, dict(causal=True)),
     (90, 40, 64, 1, False, dict(causal=True)), (70, 200, 128, 1, True, dict(window_left=10, window_right=3)), (1700, 1700, 64, 1, False, {}),
-    (130, 1900, 128, 1, True, {}), (200, 200, 64, 2, False, "slopes"), (150, 260, 128, 1, True, "slopes"), (128, 128, 64, 1, False, dict(softmax_scale=1.5, causal=True)),
+    (130, 1900, 128, 1, True, {}), (200, 200, 64, 2, False, "slopes"), (150, 260, 128, 1, True, "slopes"),
+    (70, 1600, 64, 1, False, "slopes"), (100, 900, 128, 2, True, "slopes"), (200, 3000, 64, 1, True, dict(causal=True, window_left=1700)),
+    (90, 2000, 128, 1, False, dict(window_left=500, window_right=400)), (128, 128, 64, 1, False, dict(softmax_scale=1.5, causal=True)),
     (200, 200, 128, 1, False, dict(causal=True, exact_first_rows=True))])
 def test_small_against_tile_kernels(fa, dtype, S, Sk, D, group, bshd, kw):
     import torch
@@ -32,6 +35,7 @@ def test_small_against_tile_kernels(fa, dtype, S, Sk, D, group, bshd, kw):
     many = [x.repeat(times, 1, 1, 1) if not bshd else x.transpose(1, 2).repeat(times, 1, 1, 1).transpose(1, 2) for x in (q, k, v)]
     if kw == "slopes":
         kw = dict(alibi_slopes=torch.tensor([0.5, -0.25, 0.1, 0.0], device="cuda"), causal=True)
+    assert small_waves(fa, q, k, **kw) > 0 and small_waves(fa, many[0], many[1], **kw) == 0
     out = torch.full_like(q, float("nan"))
     lse = torch.full((1, 4, S), float("nan"), device="cuda")
     fa.flash_attention_forward(q, k, v, out=out, lse=lse, **kw)
@@ -43,6 +47,27 @@ def test_small_against_tile_kernels(fa, dtype, S, Sk, D, group, bshd, kw):
     assert float((a - b).abs().max()) <= tol * max(1.0, float(b.abs().max())) and float((a - b).norm()) <= tol * float(b.norm())
     assert torch.equal(lse[0].isinf(), lse2[0].isinf())
     assert float((lse[0] - lse2[0]).nan_to_num(0.0, 0.0, 0.0).abs().max()) <= 1e-4 * max(1.0, float(lse2[0].nan_to_num(0.0, 0.0, 0.0).abs().max()))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,S,D,parts,kw", [(16, 1024, 64, 0, dict()), (51, 320, 128, 0, dict()), (8, 4096, 64, 8, dict(causal=True)), (16, 2048, 128, 8, dict(causal=True)),
+                                            (53, 256, 64, 4, dict(causal=True)), (42, 256, 128, 4, dict(causal=True))])
+def test_both_sides_of_the_line(fa, H, S, D, parts, kw):
+    """The most heads that the small kernel takes, and one more, with which the tile kernels do: the same heads agree."""
+    import ctypes
+    import torch
+    q, k, v = _inputs(torch, H + S, H + 1, H + 1, S, S, D, False, "float16")
+    p = fa.make_params(1, H, S, D, 0x1000, 0x2000, 0x3000, 0x4000, **kw)
+    got = ctypes.c_int(-1)
+    assert fa.lib().fa_sched_small(ctypes.byref(p), 256, ctypes.byref(got)) == 4 and got.value == parts and small_waves(fa, q, k, **kw) == 0
+    o, lse = fa.flash_attention_forward(q[:, :H], k[:, :H], v[:, :H], **kw)
+    o2, lse2 = fa.flash_attention_forward(q, k, v, **kw)
+    a, b = o.float(), o2[:, :H].float()
+    # (as above)
+    assert float((a - b).abs().max()) <= 2.0 ** -9 * max(1.0, float(b.abs().max())) and float((a - b).norm()) <= 2.0 ** -9 * float(b.norm())
+    assert float((lse - lse2[:, :H]).abs().max()) <= 1e-4 * max(1.0, float(lse2.abs().max()))
+    if parts:                     # (the first rows are the verifier's arithmetic in both)
+        assert torch.equal(o[:, :, :32], o2[:, :H, :32]) and torch.equal(lse[:, :, :32], lse2[:, :H, :32])
 
 
 @pytest.mark.gpu
