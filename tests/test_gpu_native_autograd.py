@@ -96,6 +96,36 @@ def test_a_subclass_of_the_query_is_the_class_of_the_output(fa):
             assert type(fa.flash_attention(x, k, v)) is type(o)
 
 
+@pytest.mark.filterwarnings("ignore::torch.jit.TracerWarning")
+def test_ways_that_stay_with_the_python_function(fa, monkeypatch):
+    """Forward mode, the transforms of torch.func and tracing never reach the function in C++ (which is made to fail here), compiled code
+    gives what eager code does."""
+    import torch
+    import torch.autograd.forward_ad as forward_ad
+    q, k, v, do = _inputs(torch, 9, 136, 64, 4, 4, False, torch.float16)
+    o = fa.flash_attention(q, k, v)
+    want = (o.detach(),) + torch.autograd.grad(o, (q, k, v), do)
+    compiled = torch.compile(lambda *t: fa.flash_attention(*t) * 1, backend="eager")(q, k, v)
+    got = (compiled.detach(),) + torch.autograd.grad(compiled, (q, k, v), do)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+    def native(*args):
+        raise AssertionError("the function in C++ was called")
+    monkeypatch.setattr(fa._native(), "attention", native)
+    p, k, v = q.detach(), k.detach(), v.detach()
+    with pytest.raises(AssertionError):
+        fa.flash_attention(p, k, v)
+    with pytest.raises(NotImplementedError), forward_ad.dual_level():
+        fa.flash_attention(forward_ad.make_dual(p, p), k, v)
+    for transformed in (lambda: torch.func.jvp(lambda x: fa.flash_attention(x, k, v), (p,), (p,)), lambda: torch.func.vjp(lambda x: fa.flash_attention(x, k, v), p),
+                        lambda: torch.func.vmap(lambda x: fa.flash_attention(x, k, v))(torch.stack([p, p]))):
+        with pytest.raises(RuntimeError, match="functorch"):
+            transformed()
+    traced = torch.jit.trace(lambda x: fa.flash_attention(x, k, v), (p,), check_trace=False)
+    assert traced(p).shape == p.shape
+    assert torch.equal(_python(torch, fa, p, k, v), want[0])
+
+
 def test_other_streams_and_threads(fa):
     import threading
     import torch
