@@ -414,7 +414,11 @@ int small_tiles(const fa_fwd_params *p)
 // 2048 queries makes the tile kernels wait for their longest blocks.  GPU time, tile kernels / this, us: no mask H16 S1024 D64 (512
 // workgroups) 14.2 / 10.5, H8 S2048 D128 (512) 34.1 / 27.9, H64 S256 D128 (512) 9.5 / 9.4, H32 S1024 D64 (1024) 15.4 / 18.9; causal
 // H8 S4096 D128 (1024) 68.6 / 56.1, H16 S2048 D64 (1024) 26.9 / 22.0, H32 S1024 D64 (1024) 16.9 / 17.3, H16 S4096 D128 (2048) 101 /
-// 107.  Two key tiles and more than a workgroup per unit: H128 S128 D64 5.5 / 5.7.  First rows in fewer parts than eight (four at
+// 107.  With more than a workgroup per unit the tile kernels keep what they do in one or two tiles at full width: 128 queries on as many
+// keys, no mask H72 to H128 D64 5.5 to 5.7 / 5.7 to 5.9, D128 7.2 to 7.5 / 7.7 to 8.1, causal H96 7.4 / 7.8 and 9.8 / 10.2; 64 keys that are a
+// whole tile without a mask, D128 H130 S64 6.4 / 7.1, H256 6.7 / 7.7, H110 S96 6.6 / 7.4, H33 S320 6.8 / 7.4, D64 H165 S40 4.9 / 5.4, H256 S64
+// 5.2 / 5.6, H170 S96 5.5 / 5.6, but H82 S100 5.4 / 5.35, H66 S160 5.6 / 5.4; with a mask 40 to the left D128 H165 S64 7.8 / 7.5, with 48 keys
+// 7.8 / 7.5, with 100 9.2 / 8.0, with 128 7.8 / 7.7.  First rows in fewer parts than eight (four at
 // head dimension 64, or where all are resident) would be what the call waits for: causal H64 S256 D64 8.7 / 10.9, H48 S256 D128
 // 10.9 / 13.7, H24 S512 D128 14.7 / 12.1.  Eight waves: no mask H4 S2048 D64 12.7 (four) / 11.1, D128 22.0 / 17.3, H8 S1024 D64 8.1 / 7.9,
 // causal 8.4 / 9.4.
@@ -427,7 +431,8 @@ int small_waves_for(const fa_fwd_params *p, int compute_units, int *first_parts)
     int L, R;
     fa_mask_bounds(s_max, p->is_causal, p->window_size_left, p->window_size_right, &L, &R);
     const bool uneven = R == 0 && L >= s_max && sk == p->S && p->S >= 2048;
-    if (items > (uneven ? 2 : 1) * slots || (items > compute_units && sk <= 128 && p->S % 128 == 0)) return 0;
+    const bool one_whole_tile = sk == kBlockKeysHost && L >= s_max && R >= s_max && (p->d == 128 || p->S <= 96);
+    if (items > (uneven ? 2 : 1) * slots || (items > compute_units && ((sk <= 128 && p->S % 128 == 0) || one_whole_tile))) return 0;
     if (first_rows_few_keys(p, R)) {              // (in workgroups of their own, or the problem stays with the tile kernels)
         const long long most = (uneven ? 2 : 1) * slots + slots / 4;
         const int parts = items + 8 * heads <= most ? 8 : 4;

@@ -42,8 +42,8 @@ def small(fa, B, H, S, Skv, D, causal=True, wl=-1, wr=-1, splits=1, sched=0, cus
 
 
 def test_line_between_32_row_blocks_and_the_tile_kernels(fa):
-    """Two blocks to a compute unit, four where a causal walk of 2048 queries and more is uneven; key splits, dropout, two key tiles on
-    most units; whatever schedule is named, on other devices too."""
+    """Two blocks to a compute unit, four where a causal walk of 2048 queries and more is uneven; key splits, dropout, one and two key
+    tiles on most units; whatever schedule is named, on other devices too."""
     for D in (64, 128):
         assert [small(fa, 1, h, 320, 320, D, causal=False)[0] for h in (1, 51, 52)] == [4, 4, 0]                  # 510 and 520 blocks
         assert [small(fa, 1, h, 500, 500, D, wl=100, exact=True)[0] for h in (32, 33)] == [4, 0]                   # 512 and 528
@@ -51,6 +51,9 @@ def test_line_between_32_row_blocks_and_the_tile_kernels(fa):
         assert [small(fa, 1, h, 2048, 2048, D, causal=False)[0] for h in (8, 9)] == [4, 0]
         assert [small(fa, 1, h, 2048, 2048, D, wl=2000, exact=True)[0] for h in (8, 9)] == [4, 0]
         assert [small(fa, 1, h, 128, 128, D, causal=False)[0] for h in (64, 65)] == [4, 0] and small(fa, 1, 100, 129, 129, D, causal=False)[0] == 4
+        assert [small(fa, 1, h, 64, 64, D, causal=False)[0] for h in (128, 129)] == [4, 0] and small(fa, 1, 256, 64, 65, D, causal=False)[0] == 4
+        assert [small(fa, 1, 100, s, 64, D, causal=False)[0] for s in (96, 97)] == [0, 0 if D == 128 else 4]
+        assert small(fa, 1, 200, 64, 64, D, causal=False, wl=40)[0] == 4 and small(fa, 1, 200, 64, 64, D, causal=False, wl=64, wr=64)[0] == 0
         assert small(fa, 1, 4, 256, 2000, D, splits=2)[0] == 0 and small(fa, 1, 4, 256, 256, D, dropout=0.1)[0] == 0
         assert [small(fa, 1, 8, 256, 256, D, sched=n)[0] for n in range(4)] == [4] * 4
         assert [small(fa, 1, 16, 320, 320, D, causal=False, cus=c)[0] for c in (64, 80)] == [0, 4]
