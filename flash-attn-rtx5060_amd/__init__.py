@@ -340,7 +340,7 @@ def flash_attention_forward(q, k, v, softmax_scale=None, causal=False, window_le
     ``alibi_slopes``: fp32 GPU tensor [N]; slope[h]*|i-j| is subtracted from every scaled score (mask.h:21-26).
     ``exact_first_rows``: see fa_fwd_params.exact_first_rows.  ``static_scratch``: go through
     fa_fwd_split_static (the key splits' partial results in the library's own static device array)."""
-    torch = _torch()
+    torch = _torch_module or _torch()
     key = None
     if (out is None and lse is None and {type(window_left), type(window_right), type(sched), type(seed)} <= _WHOLE and
             {type(softmax_scale), type(causal), type(return_lse), type(dropout_prob), type(splits), type(exact_first_rows),
@@ -349,8 +349,11 @@ def flash_attention_forward(q, k, v, softmax_scale=None, causal=False, window_le
                            static_scratch, alibi_slopes)
         plan = _plans.get(key)
         if plan is not None:
-            out = None if type(q) in _plain_tensors else torch.empty_like(q)         # (of q's class)
-            st, out, lse = _native().forward_planned(plan[0], q, k, v, alibi_slopes, seed & _SEEDS, bool(return_lse), plan[1], bool(static_scratch), out)
+            if type(q) in _plain_tensors:
+                st, out, lse = _native().forward_planned(plan[0], q, k, v, alibi_slopes, seed & _SEEDS, bool(return_lse), plan[1], bool(static_scratch))
+            else:                       # (O is of q's class)
+                st, out, lse = _native().forward_planned_into(torch.empty_like(q), plan[0], q, k, v, alibi_slopes, seed & _SEEDS, bool(return_lse),
+                                                              plan[1], bool(static_scratch))
             if st != FA_OK:
                 raise FaError(st, lib().fa_last_device_error().decode() if st == FA_ERR_DEVICE else "")
             return (out, lse) if return_lse else out

@@ -37,17 +37,17 @@ PyObject *g_first_forward = nullptr, *g_first_backward = nullptr;
 void *raw_stream(const Tensor &t) { return c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(t.device().index()).stream(); }
 Tensor bytes_like(const Tensor &t, int64_t n) { return at::empty({n}, t.options().dtype(at::kByte)); }
 
-// flash_attention_forward with its plan at hand: the status, O and the logsumexp (or None).  `given`: the tensor for O where q is of a
-// subclass (made in Python, whose empty_like returns one of that class).
-std::tuple<int, Tensor, c10::optional<Tensor>> forward_planned(const std::string &block, const Tensor &q, const Tensor &k, const Tensor &v,
-                                                               const c10::optional<Tensor> &slopes, unsigned long long seed, bool want_lse,
-                                                               int64_t workspace_bytes, bool static_scratch, const c10::optional<Tensor> &given)
+// flash_attention_forward with its plan at hand, into a tensor for O that the caller has made (of q's class, where that is a subclass):
+// the status, O and the logsumexp (or None).
+typedef std::tuple<int, Tensor, c10::optional<Tensor>> Planned;
+Planned forward_planned_into(Tensor out, const std::string &block, const Tensor &q, const Tensor &k, const Tensor &v, const c10::optional<Tensor> &slopes,
+                             unsigned long long seed, bool want_lse, int64_t workspace_bytes, bool static_scratch)
 {
     py::gil_scoped_release release;
     fa_fwd_params p;
     TORCH_CHECK(block.size() == sizeof(p), "not a forward plan");
     std::memcpy(&p, block.data(), sizeof(p));
-    Tensor out = given ? *given : at::empty_like(q);
+    if (!out.defined()) out = at::empty_like(q);
     c10::optional<Tensor> lse;
     p.Q = q.data_ptr(); p.K = k.data_ptr(); p.V = v.data_ptr(); p.O = out.data_ptr();
     p.seed = seed;
@@ -63,6 +63,11 @@ std::tuple<int, Tensor, c10::optional<Tensor>> forward_planned(const std::string
     }
     const int status = (static_scratch ? g_forward_static : g_forward)(&p, raw_stream(q));
     return {status, out, lse};
+}
+Planned forward_planned(const std::string &block, const Tensor &q, const Tensor &k, const Tensor &v, const c10::optional<Tensor> &slopes, unsigned long long seed,
+                        bool want_lse, int64_t workspace_bytes, bool static_scratch)
+{
+    return forward_planned_into(Tensor(), block, q, k, v, slopes, seed, want_lse, workspace_bytes, static_scratch);
 }
 
 // ---- the differentiable operator
@@ -236,5 +241,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
 {
     m.def("set_up", &set_up);
     m.def("forward_planned", &forward_planned);
+    m.def("forward_planned_into", &forward_planned_into);
     m.def("attention", &attention);
 }
