@@ -8,9 +8,9 @@
 constexpr int kFaMaxDevices = 64;
 constexpr int kFaEagerQueueSlots = 16;                         // counter sets for eager launches, one per stream
 constexpr int kFaQueueSlots = 256;                             // work-queue counter sets per device; the rest serve captured launches
-// Counters of the decoding kernel that merges its key splits itself: sets like the work queue's, a word per K/V head, each
-// in a cache line of its own (in neighbouring words the workgroups' additions queue up behind each other: B1 H16 S_kv 3000, 368
-// of them, 10.5 us instead of 8.8)
+// Counters of the decoding kernel that merges its key splits itself: sets like the work queue's, a word per K/V head, 64
+// bytes apart, two to a line of the L2 (in neighbouring words the workgroups' additions queue up behind each other: B1 H16 S_kv
+// 3000, 368 of them, 10.5 us instead of 8.8)
 constexpr int kFaEagerMergeSlots = 64, kFaMergeSlots = 256, kFaMergeHeads = 512, kFaMergeStride = 16;
 constexpr unsigned long long kFaStaticScratchBytes = 32ull << 20;   // key-split scratch per device
 

@@ -62,7 +62,9 @@ hipError_t fa_configure_backward_strided();
 
 namespace {
 constexpr int kBlockKeysHost = 64;
-constexpr int kComputeUnits = 256;      // MI355X; the persistent grid is sized from the device at run time
+// MI355X; the persistent grid, and which problems are small, go by the device at run time.  (Split counts are chosen without a device, for
+// this many: on one with fewer, a chunk that is left whole for the kernel of 32-row blocks may be the tile kernels'.)
+constexpr int kComputeUnits = 256;
 
 // Workgroup shape for a problem.  The 8-wave kernel (256 query rows, one workgroup per CU) shares every K/V
 // tile among more rows; the 4-wave kernel (128 rows, two workgroups per CU, each with its own barrier, so that the

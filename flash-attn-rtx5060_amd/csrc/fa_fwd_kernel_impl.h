@@ -226,8 +226,8 @@ __device__ __forceinline__ DropWords dropout_words(uint32_t seed_lo, uint32_t se
     return DropWords{{c0, c1, c2, c3}};
 }
 // The same words for a group of keys and a head that stay while the queries change: what does not depend on the query, four of the
-// first three rounds' six products among it, is formed once (DropAhead), three of twenty products fewer per draw than the compiler
-// leaves (it hoists the head's first one).
+// first three rounds' six products among it, is formed once (DropAhead): sixteen of the ten rounds' twenty products are left per draw, where the
+// compiler, which hoists the head's first one, left nineteen.
 struct DropAhead { uint32_t x0, x1, x2, x3, x4; };
 __device__ __forceinline__ DropAhead dropout_ahead(uint32_t seed_lo, uint32_t seed_hi, uint32_t bh, uint32_t group)
 {
@@ -1115,7 +1115,7 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
             // A lane's sum beyond kTileSum, or a NaN: the reference points of the rows whose maximum asks for it move up to it, and
             // the tile's exponentials are taken again (P(tile) has not been used yet).  A row moves by its own maximum alone, by
             // the rule that a tile with maxima follows too: what it gives does not depend on the rows it shares a wave with, nor
-            // on which of the two loops its tiles went through.
+            // on which of the two loops its tiles went through (nor on the call's other heads, as long as the tile kernels run it).
             if (!BY_MAX && __builtin_expect(__builtin_amdgcn_ballot_w64(!(t_a + t_b <= kTileSum)) != 0, 0)) {
                 mx = row_max();
                 const bool grow = __builtin_fmaf(mx, c, nmc) > kRescaleLog2;
