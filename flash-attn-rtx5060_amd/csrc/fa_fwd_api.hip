@@ -420,9 +420,14 @@ int small_tiles(const fa_fwd_params *p)
 // keys, no mask H72 to H128 D64 5.5 to 5.7 / 5.7 to 5.9, D128 7.2 to 7.5 / 7.7 to 8.1, causal H96 7.4 / 7.8 and 9.8 / 10.2; 64 keys that are a
 // whole tile without a mask, D128 H130 S64 6.4 / 7.1, H256 6.7 / 7.7, H110 S96 6.6 / 7.4, H33 S320 6.8 / 7.4, D64 H165 S40 4.9 / 5.4, H256 S64
 // 5.2 / 5.6, H170 S96 5.5 / 5.6, but H82 S100 5.4 / 5.35, H66 S160 5.6 / 5.4; with a mask 40 to the left D128 H165 S64 7.8 / 7.5, with 48 keys
-// 7.8 / 7.5, with 100 9.2 / 8.0, with 128 7.8 / 7.7.  First rows in fewer parts than eight (four at
-// head dimension 64, or where all are resident) would be what the call waits for: causal H64 S256 D64 8.7 / 10.9, H48 S256 D128
-// 10.9 / 13.7, H24 S512 D128 14.7 / 12.1.  Eight waves: no mask H4 S2048 D64 12.7 (four) / 11.1, D128 22.0 / 17.3, H8 S1024 D64 8.1 / 7.9,
+// 7.8 / 7.5, with 100 9.2 / 8.0, with 128 7.8 / 7.7.
+// First rows go in four parts of eight, a row to each half-wave: in eight parts half of their waves have none, and beside short blocks the
+// workgroups that do not fit any more are what the call waits for (tile kernels / eight / four parts: bf16 H56 S64 D64 6.2 / 8.0 / 5.6, H52
+// S97 D128 10.0 / 11.8 / 8.2, H40 S256 D64 9.1 / 9.5 / 6.7, fp16 H64 S169 D64 9.0 / 8.5 / 7.8, H16 S1024 D128 22.3 / 16.6 / 16.6).  Where a quarter
+// of the slots more does not hold them (head dimension 128: eight of them per head, or all at once), the tile kernels are level: H64
+// S256 D128 11.0 / 11.2.  Their bf16 products take longer: two 128-row blocks at head dimension 64 whose first rows do not fit
+// beside them stay too, H60 S192 8.6 / 9.4, H64 S148 8.5 / 9.1.  (1900 random causal problems, us: none slower than the tile
+// kernels by more than 1 %, 1.40 times as fast on average.)  Eight waves: no mask H4 S2048 D64 12.7 (four) / 11.1, D128 22.0 / 17.3, H8 S1024 D64 8.1 / 7.9,
 // causal 8.4 / 9.4.
 int small_waves_for(const fa_fwd_params *p, int compute_units, int *first_parts)
 {
@@ -436,10 +441,12 @@ int small_waves_for(const fa_fwd_params *p, int compute_units, int *first_parts)
     const bool one_whole_tile = sk == kBlockKeysHost && L >= s_max && R >= s_max && (p->d == 128 || p->S <= 96);
     if (items > (uneven ? 2 : 1) * slots || (items > compute_units && ((sk <= 128 && p->S % 128 == 0) || one_whole_tile))) return 0;
     if (first_rows_few_keys(p, R)) {              // (in workgroups of their own, or the problem stays with the tile kernels)
+        const int rows = 32 - (sk - p->S) < p->S ? 32 - (sk - p->S) : p->S;
         const long long most = (uneven ? 2 : 1) * slots + slots / 4;
-        const int parts = items + 8 * heads <= most ? 8 : 4;
-        if (parts == 4 && items + 4 * heads > (p->d == 64 ? most : slots)) return 0;
-        *first_parts = parts;
+        if (p->d == 64 ? items + 4 * heads > most : items + 8 * heads > most && items + 4 * heads > slots) return 0;
+        const bool beside = items + heads * ((rows + 7) / 8) <= slots;
+        if (!beside && p->d == 64 && p->dtype == FA_DTYPE_BF16 && p->S > 128 && p->S <= 256) return 0;
+        *first_parts = 4;
     }
     return items <= compute_units && small_tiles(p) >= 24 ? 8 : 4;
 }

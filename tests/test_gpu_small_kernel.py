@@ -1,6 +1,6 @@
 """The kernel of 32-row blocks whose waves share the keys, against the tile kernels: the same heads once as a small problem and
 once among enough others that the tile kernels take the call.  Edges of its tiles (64 keys, 32 at head dimension 128), of its blocks
-and of what a wave gets; every mask, with four waves and with eight; the first rows in eight parts and in four; and both sides of the
+and of what a wave gets; every mask, with four waves and with eight; and both sides of the
 rule's line (on the host: tests/test_launch_rules.py)."""
 import pytest
 
@@ -50,7 +50,7 @@ def test_small_against_tile_kernels(fa, dtype, S, Sk, D, group, bshd, kw):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("H,S,D,parts,kw", [(16, 1024, 64, 0, dict()), (51, 320, 128, 0, dict()), (8, 4096, 64, 8, dict(causal=True)), (16, 2048, 128, 8, dict(causal=True)),
+@pytest.mark.parametrize("H,S,D,parts,kw", [(16, 1024, 64, 0, dict()), (51, 320, 128, 0, dict()), (8, 4096, 64, 4, dict(causal=True)), (16, 2048, 128, 4, dict(causal=True)),
                                             (53, 256, 64, 4, dict(causal=True)), (42, 256, 128, 4, dict(causal=True))])
 def test_both_sides_of_the_line(fa, H, S, D, parts, kw):
     """The most heads that the small kernel takes, and one more, with which the tile kernels do: the same heads agree."""

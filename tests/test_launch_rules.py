@@ -29,11 +29,11 @@ def test_schedules_of_the_tile_kernels(fa):
     assert launch(fa, 1, 4, 3, 512, 512, 64)[0] == fa.FA_ERR_LAYOUT
 
 
-def small(fa, B, H, S, Skv, D, causal=True, wl=-1, wr=-1, splits=1, sched=0, cus=CUS, Hk=None, dropout=0.0, exact=False):
+def small(fa, B, H, S, Skv, D, causal=True, wl=-1, wr=-1, splits=1, sched=0, cus=CUS, Hk=None, dropout=0.0, exact=False, dtype=0):
     """(waves of the kernel of 32-row blocks, parts of the first rows)"""
     p = fa.make_params(B, H, S, D, 0x1000, 0x2000, 0x3000, 0x4000, causal=causal, window_left=wl, window_right=wr, n_kv_heads=Hk or 0, sched=sched,
                        S_kv=0 if Skv == S else Skv, split_num=splits, workspace_ptr=0x5000, workspace_bytes=1 << 62, dropout_prob=dropout,
-                       exact_first_rows=exact)
+                       exact_first_rows=exact, dtype=dtype)
     parts = ctypes.c_int(-1)
     waves = fa.lib().fa_sched_small(ctypes.byref(p), cus, ctypes.byref(parts))
     if waves > 0:
@@ -66,14 +66,18 @@ def test_line_between_32_row_blocks_and_the_tile_kernels(fa):
 
 
 def test_parts_of_the_first_rows(fa):
-    """Eight per head beside 32-row blocks where a quarter of the slots more holds them, else four at head dimension 64 or where all are
-    resident, else the tile kernels; these in as many as fit into twice the slots (head dimension 64: 7/4); none where there are none."""
-    assert [small(fa, 1, h, 256, 256, 64) for h in (40, 41, 53, 54)] == [(4, 8), (4, 4), (4, 4), (0, 8)]
-    assert [small(fa, 1, h, 256, 256, 128) for h in (40, 41, 42, 43)] == [(4, 8), (4, 4), (4, 4), (0, 8)]
+    """Four per head beside 32-row blocks where a quarter of the slots more holds them (head dimension 128: eight, or where all are
+    resident; 64 in bf16, two 128-row blocks: where those that have rows are), else the tile kernels; these in as many as fit into
+    twice the slots (head dimension 64: 7/4); none where there are none."""
+    assert [small(fa, 1, h, 256, 256, 64) for h in (40, 41, 53, 54)] == [(4, 4), (4, 4), (4, 4), (0, 8)]
+    assert [small(fa, 1, h, 256, 256, 128) for h in (40, 41, 42, 43)] == [(4, 4), (4, 4), (4, 4), (0, 8)]
+    assert [small(fa, 1, h, 256, 256, 64, dtype=1) for h in (42, 43)] == [(4, 4), (0, 8)] and small(fa, 1, 53, 257, 257, 64, dtype=1)[0] == 0
+    assert [small(fa, 1, 60, s, k, 64, dtype=1)[0] for s, k in ((128, 129), (129, 129), (192, 192), (192, 208), (192, 207))] == [4, 0, 0, 4, 0]
+    assert small(fa, 1, 44, 257, 257, 64, dtype=1) == (4, 4)
     assert [small(fa, 1, h, 256, 256, 128)[1] for h in (100, 180, 256, 257)] == [8, 2, 2, 0]
-    assert small(fa, 1, 8, 2048, 2048, 64) == (4, 8) and small(fa, 1, 16, 2048, 2048, 64) == (4, 8) and small(fa, 1, 16, 4096, 4096, 64) == (0, 8)
-    assert small(fa, 1, 8, 256, 256, 64, exact=True) == (4, 0) and small(fa, 1, 8, 256, 288, 64) == (4, 0) and small(fa, 1, 8, 256, 287, 64) == (4, 8)
-    assert small(fa, 1, 8, 256, 256, 64, causal=False) == (4, 0) and small(fa, 1, 8, 256, 256, 64, causal=False, wr=0) == (4, 8)
+    assert small(fa, 1, 8, 2048, 2048, 64) == (4, 4) and small(fa, 1, 16, 2048, 2048, 64) == (4, 4) and small(fa, 1, 16, 4096, 4096, 64) == (0, 8)
+    assert small(fa, 1, 8, 256, 256, 64, exact=True) == (4, 0) and small(fa, 1, 8, 256, 288, 64) == (4, 0) and small(fa, 1, 8, 256, 287, 64) == (4, 4)
+    assert small(fa, 1, 8, 256, 256, 64, causal=False) == (4, 0) and small(fa, 1, 8, 256, 256, 64, causal=False, wr=0) == (4, 4)
     assert small(fa, 1, 8, 256, 200, 64) == (4, 0) and small(fa, 1, 8, 10, 20, 64, Hk=1) == (4, 0)                 # (a group's rows in one block)
 
 
