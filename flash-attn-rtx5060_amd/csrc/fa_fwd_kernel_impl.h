@@ -562,15 +562,15 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
     constexpr int FIRST_AT = BY_ROWS ? 0 : LA * TILEB, ROWS_AT = BY_ROWS ? FirstRows<BF16, D, NW>::LDS_BYTES : LA * TILEB;
     static_assert(NST <= 3 && FIRST_AT + FirstRows<BF16, D, NW>::LDS_BYTES <= STAGES * TILEB - 64, "first-rows path does not fit behind the requested stages");
     static_assert(!BY_ROWS || (ROWS_AT >= LA * TILEB && ROWS_AT + NW * 4096 <= STAGES * TILEB - 64), "the epilogue's rows do not fit behind the requested stages");
-    // (see the item loop; the kernels left out spill a dozen vector registers with it, those with ALiBi and a mask without it)
-    constexpr bool TIED = !(GENERAL && DROPOUT && D == 128) || (MASKED && ALIBI);
+    // (see the item loop; the kernels left out spill more vector registers with it than their scratch may hold, six)
+    constexpr bool TIED = !(GENERAL && DROPOUT && D == 128 && MASKED && !ALIBI);
     static_assert(NSTV == NST || (NSTV == NST - 1 && NSTV >= 2), "V stages: as many as K stages, or one fewer");
     constexpr uint32_t LDS_V = NST * TILEB;       // K stages first, then V stages
     static_assert(INSTR % NW == 0, "tile must divide over the waves");
     static_assert(NST >= 2 && NST * TILEB <= 65536, "stage offsets must fit the 16-bit LDS immediate");
     typedef Num<BF16> N;
 
-    if (TIED) fetch_args<FaKernelArgs>();
+    fetch_args<FaKernelArgs>();
     extern __shared__ __attribute__((aligned(1024))) char smem[];
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)smem;
 
@@ -655,8 +655,9 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
     // divisions' reciprocals, conditions of the epilogue, ... -- is formed in front of the first item and parked in lanes of vector
     // registers: 175 of them in the general 128-wide kernels, 72 with it, of the strided 64-wide ones 132 and 90, and 0.5 to 1 us of
     // every launch.  Causal B8 H16 S1024 D64 [B,S,H,D] 35.3 against 38.0 us, with four K/V heads 35.5 against 37.5, S500 19.2 against
-    // 20.2, D128 ALiBi 31.3 against 32.1, S512 17.0 against 17.5, D128 29.3 against 29.5, B4 H16 S2048 53.0 against 53.6.  In
-    // launches of more items it costs nothing.)
+    // 20.2, D128 ALiBi 31.3 against 32.1, S512 17.0 against 17.5, D128 29.3 against 29.5, B4 H16 S2048 53.0 against 53.6.
+    // Dropout, D128, general: H53 S64 bf16 8.2 against 7.25, H333 S64 10.2 against 9.5; with a mask the arguments and the requests'
+    // addresses alone, H37 S64 9.7 against 9.3, H64 S200 15.9 against 15.2.  In launches of more items it costs nothing.)
     typedef const __attribute__((address_space(4))) FaKernelArgs KernelArgs;
     KernelArgs *tied_args = (KernelArgs *)__builtin_amdgcn_kernarg_segment_ptr();
     if (TIED) asm volatile("" : "+s"(tied_args));
@@ -810,7 +811,7 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
         const char *src = reinterpret_cast<const char *>(k_head) + (size_t)tile * (kBlockKeys * 2) * k_rs;
         const bool ragged = GENERAL && (tile + 1) * kBlockKeys > Sk;
         uint32_t to = lds0 + (uint32_t)(wave * 1024);
-        if (TIED) asm volatile("" : "+s"(to));             // (or the stages' addresses are all formed in front of the loop)
+        asm volatile("" : "+s"(to));                       // (or the stages' addresses are all formed in front of the loop)
 #pragma unroll
         for (int i = 0; i < IPW; ++i)
             dma_16(src, ragged ? ragged_source(tile, i, k_rs, true) : gk[i], to + stage * TILEB + i * NW * 1024);
@@ -820,7 +821,7 @@ __global__ void __launch_bounds__(NW * 64, 2) fa_fwd_pipelined(const FaKernelArg
         const char *src = reinterpret_cast<const char *>(v_head) + (size_t)tile * (kBlockKeys * 2) * v_rs;
         const bool ragged = GENERAL && (tile + 1) * kBlockKeys > Sk;
         uint32_t to = lds0 + (uint32_t)(wave * 1024);
-        if (TIED) asm volatile("" : "+s"(to));             // (or the stages' addresses are all formed in front of the loop)
+        asm volatile("" : "+s"(to));                       // (or the stages' addresses are all formed in front of the loop)
 #pragma unroll
         for (int i = 0; i < IPW; ++i)
             dma_16(src, ragged ? ragged_source(tile, i, v_rs, false) : gv[i], to + LDS_V + stage * TILEB + i * NW * 1024);

@@ -65,7 +65,8 @@ MORE = {
     # (masked, ALiBi, general, dropout: once per work item)
     ("fa_fwd_pipelined", "128", "true", "false", "true", "false"): 16,
     ("fa_fwd_pipelined", "128", "true", "true", "true", "false"): 20,
-    ("fa_fwd_pipelined", "128", "false", "true", "true", "true"): 12,
+    ("fa_fwd_pipelined", "128", "false", "false", "true", "true"): 16,
+    ("fa_fwd_pipelined", "128", "false", "true", "true", "true"): 24,
     ("fa_fwd_pipelined", "128", "true", "true", "true", "true"): 16,
     # (row blocks, waves, ALiBi, streaming)
     ("fa_fwd_decode", "128", "1", "4", "true", "false"): 8,
